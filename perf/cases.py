@@ -191,7 +191,7 @@ def _prepare_sim(case, seed):
         got = C.c_uint64()
         plain = abi.CondParams(100, 1, 50, 1e-6, 1e-8, 0.001, 0, 10)
         d.check(L.cleo_mlp_make_samples(d.h, C.byref(plain), x.data_ptr(), y.data_ptr(), cap, C.byref(got)), "samples")
-        tp = abi.MLPTrainParams(4, min(16384, int(got.value)), 3e-3, 0.9, 0.999, 1e-8, 11)
+        tp = abi.MLPTrainParams(40, min(8192, int(got.value)), 2e-3, 0.9, 0.999, 1e-8, 11)
         loss = C.c_float()
         d.check(L.cleo_mlp_train(d.h, x.data_ptr(), y.data_ptr(), got.value, C.byref(tp), C.byref(loss)), "train")
     return s
