@@ -41,7 +41,7 @@ BYTES = {
     "k_cond_queue": (44, 2 * 8 + 8 + 8),
     # read xi, r, msol of every paired drop; write its slot of the shuffled order (the drops stay
     # in place; enacted pairs, a few per cent, also write their attributes) | refs, nact, volume
-    "k_collisions": (28, 8 + 4 + 8),
+    "k_coll_team": (28, 8 + 4 + 8),
     "k_coll_tiles": (28, 8 + 4 + 8),
     # read coords, radius, sdgbxindex; write coords, sdgbxindex | bounds, winds, counts
     "k_motion": (64, 6 * 8 + 6 * 8 + 28 * 4),
@@ -78,7 +78,7 @@ def stage_kernel(stage, tiles):
     if stage == 0:
         return {0: "k_condensation", 1: "k_cond_drops", 2: "k_cond_queue"}[tiles.cond_flat]
     if stage == 1:
-        return "k_coll_tiles" if tiles.coll_flat else "k_collisions"
+        return "k_coll_tiles" if tiles.coll_flat else "k_coll_team"
     return {0: "k_motion", 1: "k_motion_flat", 2: "k_motion_scatter", 3: "k_motion_keys"}[tiles.motion_flat]
 
 

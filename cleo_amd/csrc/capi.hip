@@ -230,6 +230,7 @@ int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p) {
   a.inj_oj = c->inj_oj;
   a.inj_op = c->inj_op;
   a.big = c->big_scratch;
+  a.big2 = reinterpret_cast<uint32_t*>(c->dm);
   launch_collisions(c, a);
   launch_advance_event(c);
   if (compose) std::swap(c->order, c->order_alt);
@@ -1117,6 +1118,7 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
       a.inj_oj = c->inj_oj;
       a.inj_op = c->inj_op;
       a.big = c->big_scratch;
+      a.big2 = reinterpret_cast<uint32_t*>(c->dm);
       launch_collisions(c, a);
     } else if (kern == 3) {  // motion, sort and condensation with the solves in the sort's gather
       MotionArgs a{};

@@ -852,16 +852,14 @@ __device__ __forceinline__ uint32_t enact_pair(const CollCfg& k, DropAttrs& d1, 
 __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
-    const uint32_t hi0 = __umulhi(0xD2511F53u, c[0]);
-    const uint32_t lo0 = 0xD2511F53u * c[0];
-    const uint32_t hi1 = __umulhi(0xCD9E8D57u, c[2]);
-    const uint32_t lo1 = 0xCD9E8D57u * c[2];
-    const uint32_t n0 = hi1 ^ c[1] ^ k0;
-    const uint32_t n2 = hi0 ^ c[3] ^ k1;
+    const uint64_t p0 = static_cast<uint64_t>(c[0]) * 0xD2511F53u;  // one 32x32 -> 64 product each
+    const uint64_t p1 = static_cast<uint64_t>(c[2]) * 0xCD9E8D57u;
+    const uint32_t n0 = static_cast<uint32_t>(p1 >> 32) ^ c[1] ^ k0;
+    const uint32_t n2 = static_cast<uint32_t>(p0 >> 32) ^ c[3] ^ k1;
     c[0] = n0;
-    c[1] = lo1;
+    c[1] = static_cast<uint32_t>(p1);
     c[2] = n2;
-    c[3] = lo0;
+    c[3] = static_cast<uint32_t>(p0);
     k0 += 0x9E3779B9u;
     k1 += 0xBB67AE85u;
   }

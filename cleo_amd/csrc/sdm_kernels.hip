@@ -5,6 +5,7 @@
 // SoA store (sorted by sdgbxindex), so every per-drop load and store of a wave is a coalesced run.  No kernel uses atomics on drop data: sums keep the
 // reference's sequential order and the sort is stable by construction.
 #include <algorithm>
+#include <cmath>
 
 #include "kernels.hpp"
 #include "sdm_kernels.hpp"
@@ -227,23 +228,15 @@ __device__ __forceinline__ uint32_t rng_word(const uint32_t r4[4], uint32_t t) {
 __device__ __forceinline__ uint32_t fy_scale(uint32_t u, uint32_t iter) {
   return static_cast<uint32_t>((static_cast<uint64_t>(u) * (iter + 1ull)) >> 32);
 }
-// j_t of Fisher-Yates swap t < n-1 of gridbox g: uniform in [0, iter], iter = n-1-t
-// (shuffle.hpp:80-87), from the counter stream (word t%4 of the block for item t/4, so one block
-// serves four consecutive swaps) or the injected indices
-__device__ __forceinline__ uint32_t fy_index(const CollArgs& a, uint32_t g, uint32_t base, uint32_t n, uint32_t t,
-                                             uint64_t event) {
+// The index j_t of Fisher-Yates swap t < n-1 of gridbox g is uniform in [0, iter], iter = n-1-t
+// (shuffle.hpp:80-87): from the counter stream, word t%4 of the block for item t/4 (one block serves
+// four consecutive swaps), or an injected index
+__device__ __forceinline__ uint32_t inj_index(const CollArgs& a, uint32_t g, uint32_t base, uint32_t n, uint32_t t) {
   const uint32_t iter = n - 1 - t;
-  uint32_t j;
-  if (a.inj_j) {
-    j = a.inj_j[a.inj_oj[g] + t];
-    if (j > iter) {  // an injected index outside [0, iter] is an argument error
-      set_error(a.ctl, CLEO_ERR_INJECTED_INDEX, g, base + iter);
-      j = iter;
-    }
-  } else {
-    uint32_t r4[4];
-    rng_block(a.seed, event, 0u, g, t >> 2, r4);
-    j = fy_scale(rng_word(r4, t), iter);
+  uint32_t j = a.inj_j[a.inj_oj[g] + t];
+  if (j > iter) {  // an injected index outside [0, iter] is an argument error
+    set_error(a.ctl, CLEO_ERR_INJECTED_INDEX, g, base + iter);
+    j = iter;
   }
   return j;
 }
@@ -360,116 +353,6 @@ __device__ __forceinline__ void coll_order_nulls(const CollArgs& a, uint32_t g, 
   }
 }
 
-// The permutation `perm` and the drawn indices `jb` live in LDS (kLds) or, for gridboxes above
-// kCollLdsCap drops, in HBM scratch; the two instantiations keep LDS accesses as ds_* instructions.
-template <bool kLds, bool Kinetic>
-__device__ __forceinline__ void coll_gbx(const CollArgs& a, int lane, uint32_t g, uint32_t base, uint32_t nfull,
-                                         uint32_t n, uint32_t* perm, uint32_t* jb, uint32_t (&acc)[3]) {
-  wave_sync();  // the previous gridbox of this wave is done with perm / jb
-  const uint64_t event = a.ctl->event;
-  auto draw = [&](uint32_t t) -> uint32_t { return fy_index(a, g, base, n, t, event); };
-  if (kLds && n <= 2 * kWave) {
-    // Fisher-Yates in registers: element e of the permutation is lane e % 64 of P[e / 64]; the
-    // n-1 swaps are wave-uniform readlane / writelane pairs instead of a dependent LDS chain.
-    uint32_t P0 = static_cast<uint32_t>(lane), P1 = static_cast<uint32_t>(lane) + kWave;
-    const uint32_t J0 = (n >= 2 && static_cast<uint32_t>(lane) < n - 1) ? draw(lane) : 0u;
-    const uint32_t J1 = (n >= 2 && static_cast<uint32_t>(lane) + kWave < n - 1) ? draw(lane + kWave) : 0u;
-    for (uint32_t t = 0; t + 1 < n; ++t) {
-      const uint32_t iter = n - 1 - t;
-      const uint32_t j = t < kWave ? readlane_u32(J0, t) : readlane_u32(J1, t - kWave);
-      const uint32_t vi = iter < kWave ? readlane_u32(P0, iter) : readlane_u32(P1, iter - kWave);
-      const uint32_t vj = j < kWave ? readlane_u32(P0, j) : readlane_u32(P1, j - kWave);
-      if (iter < kWave)
-        P0 = writelane_u32(P0, vj, iter);
-      else
-        P1 = writelane_u32(P1, vj, iter - kWave);
-      if (j < kWave)
-        P0 = writelane_u32(P0, vi, j);
-      else
-        P1 = writelane_u32(P1, vi, j - kWave);
-    }
-    perm[lane] = P0;
-    perm[lane + kWave] = P1;
-    wave_sync();
-  } else {
-    for (uint32_t k = lane; k < n; k += kWave) perm[k] = k;
-    if (n >= 2) {
-      for (uint32_t t = lane; t < n - 1; t += kWave) jb[t] = draw(t);
-      if (!kLds) __threadfence_block();
-      wave_sync();
-      if (lane == 0) {  // fisher_yates_shuffle (shuffle.hpp:80-87)
-        for (uint32_t t = 0; t + 1 < n; ++t) {
-          const uint32_t iter = n - 1 - t;
-          const uint32_t j = jb[t];
-          const uint32_t pi = perm[iter];
-          perm[iter] = perm[j];
-          perm[j] = pi;
-        }
-      }
-    }
-    if (!kLds) __threadfence_block();
-    wave_sync();
-  }
-
-  const uint32_t npairs = n / 2;
-  uint32_t nulls = 0, events = 0;
-  for (uint32_t c = 0; c < npairs; c += kWave) {
-    const uint32_t jj = c + lane;
-    bool nul = false;
-    if (jj < npairs)
-      nul = coll_pair<Kinetic>(a, g, base, n, jj, coll_pos(a, base, perm[2 * jj]), coll_pos(a, base, perm[2 * jj + 1]),
-                               event, events);
-    nulls += static_cast<uint32_t>(__popcll(__ballot(nul)));
-  }
-  // unpaired last drop and the inactive tail (nulls of earlier sub-steps) keep their places
-  for (uint32_t k = 2 * npairs + lane; k < nfull; k += kWave) a.order[base + k] = coll_pos(a, base, k < n ? perm[k] : k);
-  if (nulls > 0) coll_order_nulls(a, g, base, n, nulls, lane);
-  acc[0] += npairs;
-  acc[1] += wave_sum_u32(events);
-  acc[2] += nulls;
-}
-
-template <bool Kinetic>
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_collisions(CollArgs a) {
-  extern __shared__ uint32_t lds_dyn[];
-  const int lane = lane_id();
-  const int w = static_cast<int>(threadIdx.x >> 6);
-  uint32_t acc[3] = {0, 0, 0};
-  for (uint32_t g = wave_index(); g < a.ngbx; g += wave_count()) {
-    const uint32_t base = a.off[g];
-    const uint32_t nfull = a.off[g + 1] - base;
-    const uint32_t n = a.nact[g];
-    if (n <= kCollLdsCap) {
-      uint32_t* perm = lds_dyn + static_cast<uint32_t>(w) * 2u * kCollLdsCap;
-      coll_gbx<true, Kinetic>(a, lane, g, base, nfull, n, perm, perm + kCollLdsCap, acc);
-    } else {
-      uint32_t* perm = a.big + 2ull * base;
-      coll_gbx<false, Kinetic>(a, lane, g, base, nfull, n, perm, perm + n, acc);
-    }
-  }
-  if (lane == 0)
-    for (int j = 0; j < 3; ++j) put_stat(a.stat, j, wave_index(), acc[j]);
-}
-
-// ---- tiled collisions: 64 gridboxes per wave ---------------------------------------------------
-// Lane i shuffles gridbox 64*tile + i: its permutation (one byte per drop) lives in the wave's LDS
-// tile and the swaps of all 64 gridboxes run side by side, with the same index sequence as the
-// per-gridbox path.  The tile's pairs are then flattened over the lanes (a lane finds its gridbox
-// by binary search over the prefix of per-gridbox pair counts), so every lane evaluates a pair
-// whatever the gridbox sizes.  Gridboxes above kTileMaxN drops, or beyond the tile's LDS, take the
-// per-gridbox path through HBM scratch.  The constant-kinetics instantiation runs at four waves per
-// SIMD (20 registers spilled, their scratch accesses mostly outside the tile loop: 1.18 -> 1.07 ms on
-// the coupled workload); the kinetic-energy one, which spills more, at three.
-struct CollTileLds {
-  uint32_t perm32[kTilePermBytes / 4];  // byte permutations, gridbox i from byte loff[i]
-  uint32_t ppre[kWave + 1];             // first pair of gridbox i among the tile's pairs
-  uint32_t base[kWave];                 // first drop of gridbox i
-  uint32_t loff[kWave];                 // kBigGbx: the gridbox takes the per-gridbox path
-  uint32_t n[kWave];
-  uint32_t nulls[kWave];
-};
-static_assert(sizeof(CollTileLds) == kCollTileLdsBytes, "tile LDS size");
-
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_t& total) {
   uint32_t x = v;
 #pragma unroll
@@ -480,9 +363,58 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_
   total = readlane_u32(x, kWave - 1);
   return x - v;
 }
-// the i with pre[i] <= f < pre[i+1], given pre[0] <= f < pre[kWave]
-__device__ __forceinline__ uint32_t tile_owner(const uint32_t* pre, uint32_t f) {
-  uint32_t lo = 0, hi = kWave;
+// ---- Fisher-Yates without its serial chain -----------------------------------------------------
+// Swap `iter` (iter = n-1 .. 1, with index j <= iter) moves the element at place j to place iter for
+// good and the one at place iter to place j, so the shuffled order follows from the indices alone.
+// With L(x) = { iter : j_iter = x } (all >= x), the element at place x just before swap x is
+//   U(x) = x                          when L(x) \ {x} is empty,
+//   U(x) = U(min(L(x) \ {x}))         otherwise (the last swap that put something there took it from
+//                                     its own place), and
+//   order[iter] = U(min{ e in L(j) : e > iter })   when there is such a swap,
+//               = U(iter) when j = iter, else j;      order[0] = U(0).
+// The lists L are built by all lanes at once with atomic exchanges on their heads; their walks (three
+// entries long on average) only take minima, so the result does not depend on the order of the
+// entries.  The chains of U are one hop long on average (11 at most in 8192 drops).  Serial swaps take
+// one dependent memory round trip each: a gridbox of 8192 drops 1.68 ms for its collisions against
+// 22 us here, 24679 gridboxes of 300 drops 4.9 ms against 0.13 ms.  What bounds it: LDS (about 30
+// accesses per 64 drops, with bank conflicts) and the latency of its four passes.
+//
+// A team of B lanes (a wave, or a whole workgroup) shuffles the drops of one or more gridboxes, its
+// items flattened over the lanes.  The lists of a team live in LDS as 16-bit places (kLdsIdx), or,
+// for a gridbox above the team's LDS, in HBM scratch as 32-bit ones.
+template <int B>
+__device__ __forceinline__ void team_sync() {
+  if constexpr (B == kWave) {
+    __threadfence_block();  // lists in HBM scratch: this wave's stores before its loads
+    wave_sync();
+  } else {
+    __syncthreads();
+  }
+}
+// per item (drop): the list head of its place, the next swap in the list it is on, its index j and
+// later the start of its chain, and the first hop of its place's chain
+struct FyLds {
+  using Idx = uint16_t;
+  uint32_t* head;
+  Idx *nxt, *jst, *hop;
+  __device__ __forceinline__ uint32_t exch(uint32_t at, uint32_t v) const { return atomicExch(&head[at], v); }
+  __device__ __forceinline__ uint32_t first(uint32_t at) const { return head[at]; }
+};
+struct FyHbm {
+  using Idx = uint32_t;
+  uint32_t* head;
+  Idx *nxt, *jst, *hop;
+  // the atomics act in L2, so the heads are read there too
+  __device__ __forceinline__ uint32_t exch(uint32_t at, uint32_t v) const { return atomicExch(&head[at], v); }
+  __device__ __forceinline__ uint32_t first(uint32_t at) const {
+    return __hip_atomic_load(&head[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
+constexpr uint32_t kTeamMaxItems = 15360;  // 150 KB of lists
+constexpr uint32_t kFyItemBytes = 10;  // LDS of one item: a 32-bit head and three 16-bit places
+// the i < cnt with pre[i] <= f < pre[i+1] (pre[0] <= f < pre[cnt])
+__device__ __forceinline__ uint32_t tile_owner(const uint32_t* pre, uint32_t cnt, uint32_t f) {
+  uint32_t lo = 0, hi = cnt;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
     if (pre[mid] <= f)
@@ -492,6 +424,190 @@ __device__ __forceinline__ uint32_t tile_owner(const uint32_t* pre, uint32_t f) 
   }
   return lo;
 }
+// gridboxes g0 .. g0 + cnt - 1 of a team: their drops, the prefixes of their active drops, of their
+// blocks of four swaps and of their pairs
+struct TeamGbx {
+  uint32_t ipre[kWave + 1], qpre[kWave + 1], ppre[kWave + 1];
+  uint32_t base[kWave], n[kWave], nfull[kWave], nulls[kWave];
+};
+// Shuffled order of the `cnt` gridboxes from entry i0 of T on, into M.nxt (gridbox i's from entry
+// T.ipre[i] - T.ipre[i0] on).  Every lane of the team calls it.
+template <int B, class Mem>
+__device__ __forceinline__ void team_shuffle(const CollArgs& a, const Mem& M, const TeamGbx& T, uint32_t g0, uint32_t i0,
+                                             uint32_t cnt, uint64_t event, uint32_t tid) {
+  using Idx = typename Mem::Idx;
+  constexpr uint32_t kNone = static_cast<uint32_t>(static_cast<Idx>(~Idx(0)));
+  constexpr uint32_t kChain = kNone / 2u + 1u;  // top bit: the place to chase from, not the element
+  const uint32_t off0 = T.ipre[i0], total = T.ipre[i0 + cnt] - off0;
+  const uint32_t nquad = T.qpre[i0 + cnt] - T.qpre[i0];
+  for (uint32_t f = tid; f < total; f += B) M.head[f] = kNone;
+  team_sync<B>();
+  // a lane draws one block of the counter stream and links its four swaps
+  for (uint32_t f = tid; f < nquad; f += B) {
+    const uint32_t i = i0 + tile_owner(T.qpre + i0, cnt, T.qpre[i0] + f);
+    const uint32_t q = T.qpre[i0] + f - T.qpre[i], g = g0 + i, n = T.n[i], o = T.ipre[i] - off0;
+    uint32_t r4[4] = {0u, 0u, 0u, 0u};
+    if (!a.inj_j) rng_block(a.seed, event, 0u, g, q, r4);
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w) {
+      const uint32_t t = 4u * q + w;
+      if (t + 1 < n) {
+        const uint32_t iter = n - 1 - t;
+        const uint32_t j = a.inj_j ? inj_index(a, g, T.base[i], n, t) : fy_scale(r4[w], iter);
+        M.jst[o + iter] = static_cast<Idx>(j);
+        M.nxt[o + iter] = static_cast<Idx>(M.exch(o + j, iter));
+      }
+    }
+  }
+  team_sync<B>();
+  for (uint32_t f = tid; f < total; f += B) {
+    const uint32_t i = i0 + tile_owner(T.ipre + i0, cnt, off0 + f);
+    const uint32_t o = T.ipre[i] - off0, k = f - o;
+    uint32_t m = kNone;  // min(L(k) \ {k})
+    for (uint32_t e = M.first(f); e != kNone; e = M.nxt[o + e])
+      if (e != k && e < m) m = e;
+    M.hop[f] = static_cast<Idx>(m);
+    uint32_t start = k | kChain;
+    if (k > 0) {
+      const uint32_t j = M.jst[f];
+      if (j != k) {
+        uint32_t s = kNone;  // min{ e in L(j) : e > k }
+        for (uint32_t e = M.first(o + j); e != kNone; e = M.nxt[o + e])
+          if (e > k && e < s) s = e;
+        start = s != kNone ? (s | kChain) : j;
+      }
+    }
+    M.jst[f] = static_cast<Idx>(start);
+  }
+  team_sync<B>();
+  for (uint32_t f = tid; f < total; f += B) {
+    const uint32_t i = i0 + tile_owner(T.ipre + i0, cnt, off0 + f);
+    const uint32_t o = T.ipre[i] - off0, v = M.jst[f];
+    uint32_t x = v & ~kChain;
+    if (v & kChain)
+      for (uint32_t h = M.hop[o + x]; h != kNone; h = M.hop[o + x]) x = h;
+    M.nxt[f] = static_cast<Idx>(x);
+  }
+  team_sync<B>();
+}
+
+// Collisions of the `cnt` gridboxes from entry i0 of T on, by one team: the shuffle, the pairs
+// flattened over the lanes, the unpaired drops, then the nulls.  lds: the lists are in L, else in
+// the gridbox's HBM scratch (cnt is 1 then).
+template <int B, bool Kinetic>
+__device__ __forceinline__ void team_collide(const CollArgs& a, bool lds, const FyLds& L, TeamGbx& T, uint32_t g0,
+                                             uint32_t i0, uint32_t cnt, uint64_t event, uint32_t tid, uint32_t& events) {
+  FyHbm H{};
+  if (lds) {
+    team_shuffle<B>(a, L, T, g0, i0, cnt, event, tid);
+  } else {
+    // two words per drop of the collision scratch, two of the per-drop condensation scratch (free
+    // during collisions)
+    const uint64_t b2 = 2ull * T.base[i0];
+    const uint32_t n = T.n[i0];
+    H = FyHbm{a.big2 + b2, a.big + b2, a.big + b2 + n, a.big2 + b2 + n};
+    team_shuffle<B>(a, H, T, g0, i0, cnt, event, tid);
+  }
+  const uint32_t off0 = T.ipre[i0], p0 = T.ppre[i0], npairs = T.ppre[i0 + cnt] - p0;
+  auto place = [&](uint32_t f) -> uint32_t { return lds ? static_cast<uint32_t>(L.nxt[f]) : H.nxt[f]; };
+  for (uint32_t f = tid; f < npairs; f += B) {
+    const uint32_t i = i0 + tile_owner(T.ppre + i0, cnt, p0 + f);
+    const uint32_t jj = p0 + f - T.ppre[i], o = T.ipre[i] - off0 + 2 * jj, bi = T.base[i];
+    if (coll_pair<Kinetic>(a, g0 + i, bi, T.n[i], jj, coll_pos(a, bi, place(o)), coll_pos(a, bi, place(o + 1)), event,
+                           events))
+      atomicAdd(&T.nulls[i], 1u);
+  }
+  // unpaired last drop and the inactive tail (nulls of earlier sub-steps) keep their places
+  auto tail = [&](uint32_t i, uint32_t k0, uint32_t step) {
+    const uint32_t bi = T.base[i], n = T.n[i], o = T.ipre[i] - off0;
+    for (uint32_t k = 2 * (n / 2) + k0; k < T.nfull[i]; k += step)
+      a.order[bi + k] = coll_pos(a, bi, k < n ? place(o + k) : k);
+  };
+  if (cnt == 1)
+    tail(i0, tid, B);
+  else if (tid < cnt)
+    tail(i0 + tid, 0u, 1u);
+  team_sync<B>();
+  for (uint32_t i = i0 + tid / kWave; i < i0 + cnt; i += B / kWave)
+    if (T.nulls[i]) coll_order_nulls(a, g0 + i, T.base[i], T.n[i], T.nulls[i], lane_id());
+}
+
+// A team per workgroup of B lanes, `gpt` consecutive gridboxes at a time, whose lists fit `cap` items
+// of LDS together, else one after the other (and through HBM scratch above cap drops).
+template <int B, bool Kinetic>
+__global__ void __launch_bounds__(B) CLEO_OCCUPANCY(Kinetic && B <= 256 ? 3 : 4) k_coll_team(CollArgs a, uint32_t gpt, uint32_t cap) {
+  extern __shared__ uint32_t lds_dyn[];
+  __shared__ TeamGbx T;
+  const uint32_t tid = threadIdx.x;
+  uint16_t* half = reinterpret_cast<uint16_t*>(lds_dyn + cap);
+  const FyLds L{lds_dyn, half, half + cap, half + 2 * cap};
+  const uint64_t event = a.ctl->event;
+  uint32_t pairs = 0, events = 0, nulls = 0;
+  for (uint64_t g0 = static_cast<uint64_t>(blockIdx.x) * gpt; g0 < a.ngbx; g0 += static_cast<uint64_t>(gridDim.x) * gpt) {
+    const uint32_t cnt = static_cast<uint32_t>(min(static_cast<uint64_t>(gpt), a.ngbx - g0));
+    team_sync<B>();  // the previous gridboxes are done with T and L
+    if (tid < kWave) {
+      uint32_t base = 0, nfull = 0, n = 0;
+      if (tid < cnt) {
+        base = a.off[g0 + tid];
+        nfull = a.off[g0 + tid + 1] - base;
+        n = a.nact[g0 + tid];
+      }
+      uint32_t it, qt, pt;
+      T.ipre[tid] = wave_excl_scan(n, static_cast<int>(tid), it);
+      T.qpre[tid] = wave_excl_scan((n + 2u) / 4u, static_cast<int>(tid), qt);
+      T.ppre[tid] = wave_excl_scan(n / 2u, static_cast<int>(tid), pt);
+      if (tid == 0) {
+        T.ipre[kWave] = it;
+        T.qpre[kWave] = qt;
+        T.ppre[kWave] = pt;
+      }
+      T.base[tid] = base;
+      T.n[tid] = n;
+      T.nfull[tid] = nfull;
+      T.nulls[tid] = 0u;
+    }
+    team_sync<B>();
+    const bool whole = T.ipre[cnt] <= cap;
+    for (uint32_t i = 0; i < cnt;) {
+      const uint32_t m = whole ? cnt : 1u;
+      team_collide<B, Kinetic>(a, whole || T.n[i] <= cap, L, T, static_cast<uint32_t>(g0), i, m, event, tid, events);
+      i += m;
+      if (i < cnt) team_sync<B>();  // the lists are reused
+    }
+    if (tid < cnt) nulls += T.nulls[tid];
+    if (tid == 0) pairs += T.ppre[cnt];
+  }
+  pairs = wave_sum_u32(pairs);
+  events = wave_sum_u32(events);
+  nulls = wave_sum_u32(nulls);
+  if (lane_id() == 0) {
+    put_stat(a.stat, 0, wave_index(), pairs);
+    put_stat(a.stat, 1, wave_index(), events);
+    put_stat(a.stat, 2, wave_index(), nulls);
+  }
+}
+
+// ---- tiled collisions: 64 gridboxes per wave ---------------------------------------------------
+// Lane i shuffles gridbox 64*tile + i: its permutation (one byte per drop) lives in the wave's LDS
+// tile and the serial swaps of all 64 gridboxes run side by side.  The tile's pairs are then
+// flattened over the lanes (a lane finds its gridbox by binary search over the prefix of per-gridbox
+// pair counts), so every lane evaluates a pair whatever the gridbox sizes.  Gridboxes above kTileMaxN drops, or beyond the tile's LDS, follow one
+// after the other with the whole wave as their team (64^3 gridboxes of 128 drops, where a few of each
+// tile overflow: 433 -> 316 us against their serial swaps in HBM scratch).  The constant-kinetics
+// instantiation runs at four waves per SIMD (1.18 -> 1.07 ms on 134M drops against three), the
+// kinetic-energy one at three.
+struct CollTileLds {
+  uint32_t perm32[kTilePermBytes / 4];  // byte permutations, gridbox i from byte loff[i]
+  uint32_t ppre[kWave + 1];             // first pair of gridbox i among the tile's pairs
+  uint32_t base[kWave];                 // first drop of gridbox i
+  uint32_t loff[kWave];                 // kBigGbx: the gridbox is shuffled by the whole wave
+  uint32_t n[kWave];
+  uint32_t nulls[kWave];
+};
+static_assert(sizeof(CollTileLds) == kCollTileLdsBytes, "tile LDS size");
+// drops of a large gridbox whose lists fit the tile's permutation bytes behind its TeamGbx
+constexpr uint32_t kTileTeamCap = (kTilePermBytes - sizeof(TeamGbx)) / kFyItemBytes / 4u * 4u;
 
 template <bool Kinetic>
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(Kinetic ? 3 : 4) k_coll_tiles(CollArgs a) {
@@ -500,7 +616,6 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(Kinetic ? 3 : 4) k_coll_ti
   CollTileLds& L = reinterpret_cast<CollTileLds*>(lds_dyn)[threadIdx.x >> 6];
   uint8_t* pb = reinterpret_cast<uint8_t*>(L.perm32);
   const uint64_t event = a.ctl->event;
-  uint32_t acc[3] = {0, 0, 0};
   uint32_t pairs = 0, events = 0, nulls = 0;
   const uint32_t ntiles = (a.ngbx + kWave - 1) / kWave;
   for (uint32_t tile = wave_index(); tile < ntiles; tile += wave_count()) {
@@ -526,7 +641,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(Kinetic ? 3 : 4) k_coll_ti
         const uint32_t iter = n - 1 - t;
         uint32_t j;
         if (a.inj_j) {
-          j = fy_index(a, g, base, n, t, event);
+          j = inj_index(a, g, base, n, t);
         } else {
           // t is the same for every lane still shuffling, so the block is drawn once per 4 swaps
           if ((t & 3u) == 0u) rng_block(a.seed, event, 0u, g, t >> 2, r4);
@@ -551,7 +666,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(Kinetic ? 3 : 4) k_coll_ti
     // ppre[i] <= f < ppre[i+1]): each pair is evaluated once, by one lane, which records its two
     // slots of the logical order and stores the drops' new attributes when it was enacted
     for (uint32_t f = lane; f < ptot; f += kWave) {
-      const uint32_t i = tile_owner(L.ppre, f);
+      const uint32_t i = tile_owner(L.ppre, kWave, f);
       const uint32_t jj = f - L.ppre[i], bi = L.base[i];
       const uint8_t* pi = pb + L.loff[i];
       if (coll_pair<Kinetic>(a, tile * kWave + i, bi, L.n[i], jj, coll_pos(a, bi, pi[2 * jj]),
@@ -575,20 +690,45 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(Kinetic ? 3 : 4) k_coll_ti
       coll_order_nulls(a, tile * kWave + static_cast<uint32_t>(i), readlane_u32(base, i), readlane_u32(n, i),
                        readlane_u32(mynulls, i), lane);
     }
+    // the gridboxes that are too large: one after the other by the whole wave, in the tile's LDS
+    // (its permutations are done with) or HBM scratch
+    TeamGbx& T = *reinterpret_cast<TeamGbx*>(L.perm32);
+    uint32_t* head = L.perm32 + sizeof(TeamGbx) / 4;
+    uint16_t* half = reinterpret_cast<uint16_t*>(head + kTileTeamCap);
+    const FyLds lists{head, half, half + kTileTeamCap, half + 2 * kTileTeamCap};
     uint64_t mb = __ballot(valid && !small);
     while (mb) {
       const int i = __ffsll(static_cast<unsigned long long>(mb)) - 1;
       mb &= mb - 1;
-      const uint32_t bb = readlane_u32(base, i), nb = readlane_u32(n, i);
-      coll_gbx<false, Kinetic>(a, lane, tile * kWave + static_cast<uint32_t>(i), bb, readlane_u32(nfull, i), nb,
-                      a.big + 2ull * bb, a.big + 2ull * bb + nb, acc);
+      const uint32_t nb = readlane_u32(n, i), bb = readlane_u32(base, i), fb = readlane_u32(nfull, i);
+      wave_sync();
+      if (lane == 0) {
+        T.ipre[0] = T.qpre[0] = T.ppre[0] = 0u;
+        T.ipre[1] = nb;
+        T.qpre[1] = (nb + 2u) / 4u;
+        T.ppre[1] = nb / 2u;
+        T.base[0] = bb;
+        T.n[0] = nb;
+        T.nfull[0] = fb;
+        T.nulls[0] = 0u;
+      }
+      wave_sync();
+      team_collide<kWave, Kinetic>(a, nb <= kTileTeamCap, lists, T, tile * kWave + static_cast<uint32_t>(i), 0u, 1u, event,
+                                   static_cast<uint32_t>(lane), events);
+      if (lane == 0) {
+        pairs += nb / 2u;
+        nulls += T.nulls[0];
+      }
     }
   }
-  acc[0] += wave_sum_u32(pairs);
-  acc[1] += wave_sum_u32(events);
-  acc[2] += wave_sum_u32(nulls);
-  if (lane == 0)
-    for (int j = 0; j < 3; ++j) put_stat(a.stat, j, wave_index(), acc[j]);
+  pairs = wave_sum_u32(pairs);
+  events = wave_sum_u32(events);
+  nulls = wave_sum_u32(nulls);
+  if (lane == 0) {
+    put_stat(a.stat, 0, wave_index(), pairs);
+    put_stat(a.stat, 1, wave_index(), events);
+    put_stat(a.stat, 2, wave_index(), nulls);
+  }
 }
 
 // per-gridbox sizes of the injected stream: n-1 indices and 2*floor(n/2) phis
@@ -1567,10 +1707,34 @@ void launch_qcond(cleo_ctx* c, const QcondArgs& a) {
   hipLaunchKernelGGL(k_qcond, dim3(gbx_blocks((a.ngbx + kWave - 1) / kWave, 4, c->tiles.cond_grid_waves)), dim3(256), 0,
                      c->stream, a);
 }
+template <int B, bool Kinetic>
+static void launch_coll_team_k(cleo_ctx* c, const CollArgs& a, unsigned nb, uint32_t gpt, uint32_t cap) {
+  const size_t lds = static_cast<size_t>(cap) * kFyItemBytes;
+  kev_mark(c, 0);
+  hipLaunchKernelGGL((k_coll_team<B, Kinetic>), dim3(nb), dim3(B), lds, c->stream, a, gpt, cap);
+  kev_mark(c, 1);
+}
+template <int B>
+static void launch_coll_team(cleo_ctx* c, const CollArgs& args, uint32_t gpt, uint64_t items) {
+  CollArgs a = args;
+  const uint32_t cap = static_cast<uint32_t>(std::min<uint64_t>(kTeamMaxItems, (items + 63) / 64 * 64));
+  const unsigned nb = gbx_blocks(a.ngbx, gpt, 0);
+  a.stat = stat_slots(c, static_cast<uint64_t>(nb) * (B / kWave));
+  if (coll_is_kinetic(a.k))
+    launch_coll_team_k<B, true>(c, a, nb, gpt, cap);
+  else
+    launch_coll_team_k<B, false>(c, a, nb, gpt, cap);
+  launch_stats_reduce(c, nb * (B / kWave), ST_COLL_PAIRS, 3);
+}
 void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   if (args.ngbx == 0) return;
   CollArgs a = args;
-  if (c->tiles.coll_flat) {
+  const uint64_t mean = std::max<uint64_t>(1, c->ntot / a.ngbx);
+  // Tiles give the least work per drop (33.5M drops: 0.29 ms against 0.56 ms for the teams), but a
+  // wave walks through its 64 gridboxes' swaps and pairs in about 1.2 us per drop of the mean, so
+  // they need enough gridboxes to fill the chip (32^3 gridboxes of 64: 81 us against 45 us; the
+  // lines cross near 75,000 gridboxes at any mean) whose drops fit a tile's 8 KB of permutations.
+  if (c->tiles.coll_flat && a.ngbx >= kTileMinGbx && mean <= kTilePermBytes / kWave + 4) {
     const unsigned nb = gbx_blocks((a.ngbx + kWave - 1) / kWave, a.wpb, c->tiles.coll_grid_waves);
     a.stat = stat_slots(c, static_cast<uint64_t>(nb) * a.wpb);
     kev_mark(c, 0);
@@ -1582,16 +1746,19 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
     launch_stats_reduce(c, nb * a.wpb, ST_COLL_PAIRS, 3);
     return;
   }
-  const unsigned nb = gbx_blocks(a.ngbx, a.wpb, c->tiles.coll_grid_waves);
-  a.stat = stat_slots(c, static_cast<uint64_t>(nb) * a.wpb);
-  const size_t lds = static_cast<size_t>(a.wpb) * 2u * kCollLdsCap * sizeof(uint32_t);
-  kev_mark(c, 0);
-  if (coll_is_kinetic(a.k))
-    hipLaunchKernelGGL(k_collisions<true>, dim3(nb), dim3(64 * a.wpb), lds, c->stream, a);
-  else
-    hipLaunchKernelGGL(k_collisions<false>, dim3(nb), dim3(64 * a.wpb), lds, c->stream, a);
-  kev_mark(c, 1);
-  launch_stats_reduce(c, nb * a.wpb, ST_COLL_PAIRS, 3);
+  // Teams, one workgroup each.  A wave takes as many gridboxes as make 512 drops (128 to 1024 tried:
+  // 55, 49, 45, 68 us on 32^3 gridboxes of 64), but no more than leave 4096 teams (3750 gridboxes of
+  // 128: 18 us with one each, 33 us with four).  With few gridboxes, or large ones, the pairs of one
+  // gridbox are spread over the waves of a workgroup instead.
+  if (mean <= 512 && (mean <= 96 || a.ngbx > 512)) {
+    const uint64_t gpt = std::min<uint64_t>(kWave, std::max<uint64_t>(1, std::min<uint64_t>(512 / mean, a.ngbx / 4096)));
+    const double items = static_cast<double>(gpt * mean);
+    launch_coll_team<kWave>(c, a, static_cast<uint32_t>(gpt), static_cast<uint64_t>(items + 6.0 * std::sqrt(items)) + 128);
+  } else if (mean <= 2048) {
+    launch_coll_team<256>(c, a, 1u, 2 * mean);
+  } else {
+    launch_coll_team<1024>(c, a, 1u, 2 * mean);
+  }
 }
 void launch_motion(cleo_ctx* c, const MotionArgs& args) {
   if (args.grid.ngbx == 0) return;

@@ -5,14 +5,13 @@
 
 namespace cleo {
 
-constexpr int kCollMaxWpb = 4;
-constexpr uint32_t kCollLdsCap = 512;  // drops per gridbox held in LDS; larger gridboxes use HBM scratch
 constexpr int kStatSlotsMax = 4;       // counters per wave of one kernel
 // tiled collisions: byte permutations of up to kTileMaxN drops, kTilePermBytes of them per wave
 constexpr uint32_t kTileMaxN = 255;
 constexpr uint32_t kTilePermBytes = 8192;
+constexpr uint32_t kTileMinGbx = 75000;  // gridboxes from which the tiles are the faster variant
 constexpr uint32_t kCollTileLdsBytes = kTilePermBytes + 4u * (65u + 4u * 64u);
-constexpr uint32_t kBigGbx = 0xFFFFFFFFu;  // tile LDS marker of a gridbox on the per-gridbox path
+constexpr uint32_t kBigGbx = 0xFFFFFFFFu;  // tile LDS marker of a gridbox the whole wave shuffles
 // condensation task ring: prepared drops per wave, and waves per CU of the default grid
 constexpr uint32_t kRing = 128;
 constexpr uint32_t kCondRingBytes = kRing * (11u * 8u + 8u + 2u * 4u);
@@ -71,7 +70,8 @@ struct CollArgs {
   const double* inj_phi;
   const uint32_t* inj_oj;
   const uint32_t* inj_op;
-  uint32_t* big;
+  uint32_t* big;   // scratch, two words per drop
+  uint32_t* big2;  // the same again
   StatSlots stat;   // ST_COLL_PAIRS .. ST_NULLS
 };
 

@@ -407,7 +407,9 @@ typedef struct {
   uint32_t cond_grid_waves;        /* waves per launch; each loops over gridboxes (or drops) */
   uint32_t coll_grid_waves;        /*   0: one wave per gridbox (one thread per drop) */
   uint32_t motion_grid_waves;
-  uint32_t coll_flat;              /* 1: 64 gridboxes per wave, pairs flattened over the lanes */
+  uint32_t coll_flat;              /* 1: 64 gridboxes per wave, pairs flattened over the lanes, on
+                                      domains that fill the chip that way (else as 0: a wave or a
+                                      workgroup per gridbox or few) */
   uint32_t cond_defer;             /* cond_flat 1: Newton iterations after which a drop is set
                                       aside and solved by a second launch (0: never) */
 } cleo_tiles;
