@@ -434,14 +434,8 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   // a gridbox launch has at most ngbx + 3 waves, a drop launch 4 per 256 drops
   c->sp_slots = std::max<uint64_t>(ngbx + 4, 4 * ((maxn + 255) / 256) + 4);
   HIP_TRY(c, dalloc(&c->sp, kStatSlotsMax * c->sp_slots));
-  // deferred drops of the condensation: per-wave segments (waves of a drop launch times a quarter
-  // of their drops + 16), the shared list they move to and its counter.  The list has room for
-  // every drop (a launch defers each drop at most once), so no deferred drop is ever solved in
-  // the launch that deferred it.
-  HIP_TRY(c, dalloc(&c->dcount, 1));
-  c->dlist_cap = static_cast<uint32_t>(std::min<uint64_t>(maxn + 64, 0xFFFFFFFFull));
-  HIP_TRY(c, dalloc(&c->dlist, c->dlist_cap));
-  HIP_TRY(c, dalloc(&c->dseg, std::min<uint64_t>(maxn / 4 + 20 * c->sp_slots + 64, 0xFFFFFFFFull)));
+  HIP_TRY(c, dalloc(&c->dlist, maxn));
+  HIP_TRY(c, dalloc(&c->dcount, maxn / 256 + 1));
   HIP_TRY(c, dalloc(&c->perm, std::max<uint64_t>(maxn, 1)));
   HIP_TRY(c, dalloc(&c->dstep, std::max<uint64_t>(maxn, 1)));
   HIP_TRY(c, dalloc(&c->order, std::max<uint64_t>(maxn, 1)));
@@ -475,8 +469,7 @@ int cleo_destroy(cleo_ctx* c) {
                   static_cast<void*>(c->niters), static_cast<void*>(c->guess), static_cast<void*>(c->rs_key[0]),
                   static_cast<void*>(c->rs_key[1]), static_cast<void*>(c->rs_idx[0]), static_cast<void*>(c->rs_idx[1]),
                   static_cast<void*>(c->rs_cnt), static_cast<void*>(c->gs), static_cast<void*>(c->dm),
-                  static_cast<void*>(c->sp), static_cast<void*>(c->dlist), static_cast<void*>(c->dcount),
-                  static_cast<void*>(c->dseg), c->mom, static_cast<void*>(c->perm), static_cast<void*>(c->dstep), static_cast<void*>(c->order), static_cast<void*>(c->order_alt),
+                  static_cast<void*>(c->sp), static_cast<void*>(c->dlist), static_cast<void*>(c->dcount), c->mom, static_cast<void*>(c->perm), static_cast<void*>(c->dstep), static_cast<void*>(c->order), static_cast<void*>(c->order_alt),
                   static_cast<void*>(c->qm)})
     if (p) hipFree(p);
   if (c->h_ctl) hipHostFree(c->h_ctl);

@@ -120,11 +120,9 @@ struct cleo_ctx {
   double* dm = nullptr;  // maxn: per-drop condensed mass (flat condensation)
   // per-wave statistics: up to kStatSlotsMax counters per wave, reduced into DevCtl::stats
   uint32_t* sp = nullptr;
-  // deferred-drop list of the thread-per-drop condensation (segments per wave) and their counts
+  // drops set aside by the workgroups of the thread-per-drop condensation (maxn positions)
   uint32_t* dlist = nullptr;
-  uint32_t* dcount = nullptr;
-  uint32_t dlist_cap = 0;
-  uint32_t* dseg = nullptr;
+  uint32_t* dcount = nullptr;  // their number per workgroup (at most one per 256 drops)
   // neighbour sort: source position of every destination position (maxn), and the step each drop
   // took in the last thread-per-drop motion (maxn bytes, 27 = left the domain)
   uint32_t* perm = nullptr;

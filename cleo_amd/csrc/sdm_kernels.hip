@@ -2050,7 +2050,6 @@ namespace cleo {
 // per gridbox: optional qcond recompute (ordered, before any radius changes), then the
 // saturation ratio and diffusion factor condensation uses (condensation.cpp:44-56)
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_prep(CondFlatArgs a) {
-  if (a.dcount && blockIdx.x == 0 && threadIdx.x == 0) *a.dcount = 0u;  // the deferred list starts empty
   __shared__ double win_all[4][kSumWin];
   double* win = win_all[threadIdx.x >> 6];
   const int lane = lane_id();
@@ -2084,7 +2083,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_prep(CondFlatArg
 
 // One active drop k of gridbox g: Koehler factors, Newton solve, radius update, mass change * xi
 // into dm[k] (condensation.cpp:44-125).  With cfg.budget the solve may give up (returns false,
-// nothing written) so that the drop is solved again, without a budget, by k_cond_deferred.
+// nothing written) so that the drop is solved again, without a budget, by solve_listed.
 struct CondStats {
   uint32_t solved, iters, subs, restarts;
 };
@@ -2179,59 +2178,71 @@ __global__ void __launch_bounds__(256) k_cond_guess(CondFlatArgs a) {
   }
 }
 
-// Deferred drops of a wave are first listed in the wave's own segment of a.dseg (`dsegcap` each,
-// no contention); defer_drop appends those of the wave's deferring lanes (position q), and a
-// deferring lane whose drop finds the segment full appends it to the shared list at once, with
-// an atomic of its own.  The shared list holds dcap >= ntot entries and a launch defers each drop
-// at most once, so every deferred drop is listed (an overflow would be recorded as a bounds
-// error).  Every lane of the wave calls it.
-__device__ __forceinline__ void defer_drop(const CondFlatArgs& a, uint32_t* seg, uint32_t& ndef, bool deferred,
-                                           uint32_t q) {
-  const uint64_t m = __ballot(deferred);
+// Drops whose solve outlives cfg.budget iterations (a few per cent; their lanes would hold the other
+// 63 of the wave) are set aside by their workgroup and solved later, without a budget, packed into
+// whole waves.  A workgroup takes a contiguous range of drops and lists its deferred ones in that range
+// of a.dlist, so there is room for all of them, and counts them in LDS.  (One list for all workgroups,
+// with an atomic per wave on its counter, took 238 us for the gather with the solves on 2.1M drops,
+// 591 us on 8.4M, and 18 and 31 us more for a launch that solved the list; same-address atomics take
+// about 5 ns each.)  Who solves them:
+// - kTail: the workgroup itself at the end of its range, about 60 drops of 2048, while others fill the
+//   CU: no further launch (2.1M drops: 104 us against 110).
+// - else k_cond_deferred, which packs the lists of several workgroups and keeps the second copy of
+//   the solve, with its registers, out of the main loop (33.5M drops: 1155 us against 1209, 134M:
+//   4.44 ms against 4.64; equal at 8.4M).
+__device__ __forceinline__ void defer_drop(uint32_t* ndef, uint32_t* list, bool deferred, uint32_t q) {
+  const uint64_t m = ballot(deferred);
   if (!m) return;
-  const uint32_t idx = ndef + static_cast<uint32_t>(__popcll(m & lanemask_lt()));
-  ndef = min(a.dsegcap, ndef + static_cast<uint32_t>(__popcll(m)));
-  if (!deferred) return;
-  if (idx < a.dsegcap) {
-    seg[idx] = q;
-    return;
-  }
-  const uint32_t j = atomicAdd(a.dcount, 1u);
-  if (j < a.dcap)
-    a.dlist[j] = q;
-  else
-    set_error(a.ctl, CLEO_ERR_BOUNDS, kOOB, q);
-}
-// At the end of the kernel the wave moves its segment to the shared list with one atomic, so that
-// k_cond_deferred finds the deferred drops of all waves packed 64 to a wave.  The shared list has
-// room for every segment, so nothing is lost.
-__device__ __forceinline__ void defer_flush(const CondFlatArgs& a, const uint32_t* seg, uint32_t ndef, int lane) {
-  if (ndef == 0) return;
-  wave_sync();  // the segment's entries were written by other lanes of this wave
   uint32_t base = 0;
-  if (lane == 0) base = atomicAdd(a.dcount, ndef);
-  base = readlane_u32(base, 0);
-  for (uint32_t i = static_cast<uint32_t>(lane); i < ndef; i += kWave) {
-    const uint64_t j = static_cast<uint64_t>(base) + i;
-    if (j < a.dcap) a.dlist[j] = seg[i];
+  const int leader = __ffsll(static_cast<unsigned long long>(m)) - 1;
+  if (lane_id() == leader) base = atomicAdd(ndef, static_cast<uint32_t>(__popcll(m)));
+  base = readlane_u32(base, leader);
+  if (deferred) list[base + lanes_below(m)] = q;
+}
+// the workgroup's range of n drops: whole chunks of its threads, consecutive ranges on one XCD
+__device__ __forceinline__ uint64_t block_span(uint64_t n, uint32_t blocks, uint32_t threads) {
+  return ((n + blocks - 1) / blocks + threads - 1) / threads * threads;
+}
+__device__ __forceinline__ void block_range(uint64_t n, uint64_t& lo, uint64_t& hi) {
+  const uint64_t per = block_span(n, gridDim.x, blockDim.x);
+  lo = min(static_cast<uint64_t>(xcd_block()) * per, n);
+  hi = min(lo + per, n);
+}
+
+__device__ __forceinline__ void solve_listed(const CondFlatArgs& a, uint32_t k, CondStats& st) {
+  NewtonCfg nobudget = a.cfg;
+  nobudget.budget = 0;
+  const double warm =
+      a.warm ? a.warm[a.warm_perm ? a.warm_perm[k] : k] : __longlong_as_double(0x7FF8000000000000ll);
+  cond_drop(a, nobudget, a.s.gbx[k], k, warm, st);
+}
+// Every thread of the workgroup calls it, after its last defer_drop.
+template <bool kTail>
+__device__ __forceinline__ void finish_deferred(const CondFlatArgs& a, const uint32_t* ndef, const uint32_t* list,
+                                                CondStats& st) {
+  __syncthreads();  // the entries, and the drops' records, were written by the workgroup's other waves
+  const uint32_t n = *ndef;
+  if constexpr (kTail) {
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) solve_listed(a, list[i], st);
+  } else {
+    if (threadIdx.x == 0) a.dcount[xcd_block()] = n;
   }
 }
 
-// per active drop, one thread each.  Drops whose solve outlives cfg.budget iterations (a few per
-// cent; their lanes would hold the other 63 of the wave) go to the deferred list, up to `dcap`
-// of them, and are solved by k_cond_deferred, 64 to a wave.
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_drops(CondFlatArgs a) {
-  const uint32_t ndom = a.off[a.ngbx];
-  const int lane = lane_id();
+// per active drop, one thread each
+template <bool kTail>
+__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(5) k_cond_drops(CondFlatArgs a) {
+  __shared__ uint32_t ndef;
+  if (threadIdx.x == 0) ndef = 0u;
+  __syncthreads();
   CondStats st{0, 0, 0, 0};
-  uint32_t ndef = 0;
-  uint32_t* seg = a.dseg + static_cast<uint64_t>(wave_index()) * a.dsegcap;
-  for (uint64_t k0 = static_cast<uint64_t>(blockIdx.x) * blockDim.x; k0 < ndom;
-       k0 += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
+  uint64_t k_lo, k_hi;
+  block_range(a.off[a.ngbx], k_lo, k_hi);
+  for (uint64_t k0 = k_lo; k0 < k_hi; k0 += blockDim.x) {
     const uint64_t k = k0 + threadIdx.x;
     bool active = false;
     uint32_t g = 0;
-    if (k < ndom) {
+    if (k < k_hi) {
       g = a.s.gbx[k];
       active = g < a.ngbx && k < a.off[g] + a.nact[g];
     }
@@ -2239,25 +2250,34 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_drops(CondFlatAr
     if (active && a.warm) warm = a.warm[k];
     bool deferred = false;
     if (active) deferred = !cond_drop(a, a.cfg, g, k, warm, st);
-    defer_drop(a, seg, ndef, deferred, static_cast<uint32_t>(k));
+    defer_drop(&ndef, a.dlist + k_lo, deferred, static_cast<uint32_t>(k));
   }
-  if (a.dcount) defer_flush(a, seg, ndef, lane);
+  finish_deferred<kTail>(a, &ndef, a.dlist + k_lo, st);
   put_cond_stats(a.stat, st);
 }
 
-// the deferred drops, thread i taking entry i of the list (grid-stride), solved without a budget;
-// every wave writes its statistics slot
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_deferred(CondFlatArgs a) {
+// The deferred drops of a solving pass of `nlists` workgroups over n drops, kListsPerBlock lists
+// flattened over a workgroup's threads.
+constexpr uint32_t kListsPerBlock = 8;
+__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(5) k_cond_deferred(CondFlatArgs a, uint32_t nlists) {
+  __shared__ uint32_t pre[kListsPerBlock + 1];
   CondStats st{0, 0, 0, 0};
-  NewtonCfg nobudget = a.cfg;
-  nobudget.budget = 0;
-  const uint64_t n = min(static_cast<uint64_t>(*a.dcount), static_cast<uint64_t>(a.dcap));
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    const uint32_t k = a.dlist[i];
-    const double warm =
-        a.warm ? a.warm[a.warm_perm ? a.warm_perm[k] : k] : __longlong_as_double(0x7FF8000000000000ll);
-    cond_drop(a, nobudget, a.s.gbx[k], k, warm, st);
+  const uint64_t per = block_span(a.off[a.ngbx], nlists, 256u);
+  for (uint32_t l0 = blockIdx.x * kListsPerBlock; l0 < nlists; l0 += gridDim.x * kListsPerBlock) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t t = 0;
+      for (uint32_t i = 0; i < kListsPerBlock; ++i) {
+        pre[i] = t;
+        t += l0 + i < nlists ? a.dcount[l0 + i] : 0u;
+      }
+      pre[kListsPerBlock] = t;
+    }
+    __syncthreads();
+    for (uint32_t f = threadIdx.x; f < pre[kListsPerBlock]; f += blockDim.x) {
+      const uint32_t i = tile_owner(pre, kListsPerBlock, f);
+      solve_listed(a, a.dlist[(l0 + i) * per + f - pre[i]], st);
+    }
   }
   put_cond_stats(a.stat, st);
 }
@@ -2267,13 +2287,13 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_deferred(CondFla
 // solves it before writing its record (with the new radius) and dm[q], qm[q] to the sorted store.
 // The solve does not depend on the order of the drops; the per-gridbox sums run afterwards on the
 // sorted store (k_cond_state).  Drops that outlive cfg.budget iterations are written unsolved and
-// listed by their sorted position for k_cond_deferred, as in k_cond_drops.  The memory traffic of
+// set aside, as in k_cond_drops.  The memory traffic of
 // the gather and the FP64 arithmetic of the solves overlap in one pass.
 // kMove: the unsorted store holds the drops before motion (the counting pass k_motion_drops<false>
 // only recorded their steps); each drop moves here, with the same arithmetic, before its solve in
 // the gridbox it reaches, so motion writes nothing of its own.  kLds: the coordinate bounds are read
 // from an LDS copy (dynamic shared memory of nz + nx + ny + 3 doubles).
-template <bool kMove, bool kLds>
+template <bool kMove, bool kLds, bool kTail>
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gather_cond(NsortArgs n, CondFlatArgs a, MotionArgs m) {
   extern __shared__ double bounds_lds[];
   MotionArgs b = m;
@@ -2286,11 +2306,11 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gath
     b.grid.xh = bounds_lds + nzh;
     b.grid.yh = bounds_lds + nzh + nxh;
   }
+  __shared__ uint32_t ndef;
+  if (threadIdx.x == 0) ndef = 0u;
+  __syncthreads();
   const uint64_t nsrc = n.off[n.grid.ngbx];
-  const int lane = lane_id();
   CondStats st{0, 0, 0, 0};
-  uint32_t ndef = 0;
-  uint32_t* seg = a.dseg + static_cast<uint64_t>(wave_index()) * a.dsegcap;
   const double nowarm = __longlong_as_double(0x7FF8000000000000ll);
   // Each block takes one contiguous range of destinations, in block-uniform chunks (every wave
   // of the block stays in the loop for the ballots below).  A drop that changed gridbox is read
@@ -2298,11 +2318,11 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gath
   // readers run on the same CU at about the same time, and with the ranges in xcd_block() order
   // the neighbouring ranges run on the same XCD, behind one L2 (measured 4.82 -> 4.61 -> 4.49 ms
   // against chunks strided over the grid).
-  const uint64_t per = ((nsrc + gridDim.x - 1) / gridDim.x + blockDim.x - 1) / blockDim.x * blockDim.x;
-  const uint64_t c0 = static_cast<uint64_t>(xcd_block()) * per, c1 = min(c0 + per, nsrc);
-  for (uint64_t q0 = c0; q0 < c1; q0 += blockDim.x) {
+  uint64_t q_lo, q_hi;
+  block_range(nsrc, q_lo, q_hi);
+  for (uint64_t q0 = q_lo; q0 < q_hi; q0 += blockDim.x) {
     const uint64_t q = q0 + threadIdx.x;
-    const bool inq = q < nsrc;
+    const bool inq = q < q_hi;
     const uint32_t p = inq ? n.perm[q] : 0u;
     const bool okp = inq && p < nsrc;
     if (inq && !okp) set_error(n.ctl, CLEO_ERR_SORT_NONLOCAL, kOOB, q);
@@ -2339,14 +2359,14 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gath
     double rnew = r, dm = 0.0, qm = 0.0;
     bool solved = false;
     if (active) solved = cond_solve(a, a.cfg, g, q, r, msol, [&] { return xi; }, warm, st, rnew, dm, qm);
-    defer_drop(a, seg, ndef, active && !solved, static_cast<uint32_t>(q));
+    defer_drop(&ndef, a.dlist + q_lo, active && !solved, static_cast<uint32_t>(q));
     if (okp) __builtin_nontemporal_store(solved ? rnew : r, &n.dst.r[q]);
     if (solved) {
       __builtin_nontemporal_store(dm, &a.dm[q]);
       if (a.qm) __builtin_nontemporal_store(qm, &a.qm[q]);
     }
   }
-  if (a.dcount) defer_flush(a, seg, ndef, lane);
+  finish_deferred<kTail>(a, &ndef, a.dlist + q_lo, st);
   put_cond_stats(a.stat, st);
 }
 
@@ -2934,26 +2954,38 @@ static void launch_gather_move(cleo_ctx* c, const NsortArgs& n, const MotionArgs
 }
 
 // the gather with the solves; with m, the drops also move in it (k_sort_gather_cond<true, ...>)
+template <bool kTail>
 static void launch_gather_cond(cleo_ctx* c, const NsortArgs& n, const CondFlatArgs& a, const MotionArgs* m,
                                unsigned nb) {
   if (!m) {
-    hipLaunchKernelGGL((k_sort_gather_cond<false, false>), dim3(nb), dim3(256), 0, c->stream, n, a, MotionArgs{});
+    hipLaunchKernelGGL((k_sort_gather_cond<false, false, kTail>), dim3(nb), dim3(256), 0, c->stream, n, a, MotionArgs{});
     return;
   }
   const uint32_t nb_ = m->grid.nz + m->grid.nx + m->grid.ny + 3;
   if (nb_ <= kMotionLdsBounds)
-    hipLaunchKernelGGL((k_sort_gather_cond<true, true>), dim3(nb), dim3(256), nb_ * sizeof(double), c->stream, n, a,
-                       *m);
+    hipLaunchKernelGGL((k_sort_gather_cond<true, true, kTail>), dim3(nb), dim3(256), nb_ * sizeof(double), c->stream, n,
+                       a, *m);
   else
-    hipLaunchKernelGGL((k_sort_gather_cond<true, false>), dim3(nb), dim3(256), 0, c->stream, n, a, *m);
+    hipLaunchKernelGGL((k_sort_gather_cond<true, false, kTail>), dim3(nb), dim3(256), 0, c->stream, n, a, *m);
+}
+static void launch_deferred(cleo_ctx* c, CondFlatArgs a, unsigned nlists) {
+  const unsigned nb = nblocks(nlists, kListsPerBlock);
+  a.stat = stat_slots(c, 4ull * nb);
+  hipLaunchKernelGGL(k_cond_deferred, dim3(nb), dim3(256), 0, c->stream, a, nlists);
+  launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
 }
 
-// per-wave segments of the deferred list for a drop launch of nb blocks: a quarter of a wave's
-// drops, at least 16
-static void set_defer_segments(const cleo_ctx* c, CondFlatArgs& a, unsigned nb) {
-  const uint64_t per_wave = (c->ntot + 4ull * nb - 1) / (4ull * nb);
-  a.dseg = c->dseg;
-  a.dsegcap = a.dcount ? static_cast<uint32_t>(per_wave / 4 + 16) : 0u;
+// whether the workgroups of a solving pass solve their deferred drops themselves (finish_deferred)
+static bool tail_solves(const cleo_ctx* c, uint32_t budget) { return budget == 0 || c->ntot < 6000000u; }
+// Blocks of a solving pass: ranges of 8 to 16 chunks of 256 drops, long enough to pack the deferred
+// drops, short enough to balance (33.5M drops in ranges of 4 / 8 / 16 / 32 chunks: 1190 / 1155 / 1181 /
+// 1277 us; 134M: 4.69 / 4.58 / 4.44 / 4.60 ms), but never fewer than fill the chip at five workgroups
+// per CU; at most grid_waves waves when that is set.
+static unsigned solve_blocks(const cleo_ctx* c, uint32_t grid_waves) {
+  const uint64_t chunks = std::max<uint64_t>(1, (c->ntot + 255) / 256);
+  const uint64_t per = std::min<uint64_t>(16, std::max<uint64_t>(8, chunks / 16384));
+  const uint64_t nb = std::min(chunks, std::max<uint64_t>(5ull * c->num_cu, (chunks + per - 1) / per));
+  return static_cast<unsigned>(grid_waves ? std::min<uint64_t>(nb, std::max<uint32_t>(1u, grid_waves / 4)) : nb);
 }
 
 void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
@@ -2966,9 +2998,8 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
   const uint64_t ntiles = (a.ngbx + kWave - 1) / kWave;
   const uint32_t budget = c->tiles.cond_flat == 2 ? 0u : c->tiles.cond_defer;
   a.cfg.budget = budget;
-  a.dcap = budget ? c->dlist_cap : 0u;
   a.dlist = c->dlist;
-  a.dcount = budget ? c->dcount : nullptr;  // zeroed by k_cond_prep
+  a.dcount = c->dcount;
   hipLaunchKernelGGL(k_cond_prep, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
   if (c->tiles.cond_flat == 2) {
     // task-ring kernel: waves of 4 per block; by default as many waves as fit on the device at once
@@ -2980,21 +3011,21 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
     kev_mark(c, 1);
     launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
   } else {
-    const unsigned nb = drop_blocks(c->ntot, gw);
+    const unsigned nb = solve_blocks(c, gw);
     a.stat = stat_slots(c, 4ull * nb);  // every wave of k_cond_drops writes its slot
-    set_defer_segments(c, a, nb);
     if (a.mlp_inline) {  // the learned guesses, from the saturation ratios k_cond_prep left
       hipLaunchKernelGGL(k_cond_guess, dim3(drop_blocks(c->ntot, gw ? gw : 32768)), dim3(256), 0, c->stream, a);
       a.warm = a.warm_buf;
     }
     kev_mark(c, 0);
-    hipLaunchKernelGGL(k_cond_drops, dim3(nb), dim3(256), 0, c->stream, a);
-    if (budget) {
-      launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
-      hipLaunchKernelGGL(k_cond_deferred, dim3(nb), dim3(256), 0, c->stream, a);
-    }
-    kev_mark(c, 1);
+    const bool tail = tail_solves(c, budget);
+    if (tail)
+      hipLaunchKernelGGL(k_cond_drops<true>, dim3(nb), dim3(256), 0, c->stream, a);
+    else
+      hipLaunchKernelGGL(k_cond_drops<false>, dim3(nb), dim3(256), 0, c->stream, a);
     launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
+    if (!tail) launch_deferred(c, a, nb);
+    kev_mark(c, 1);
   }
   hipLaunchKernelGGL(k_cond_state, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
 }
@@ -3036,14 +3067,10 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   a.qm = c->qm;  // the qcond recompute joins k_cond_state
   const uint32_t gw = c->tiles.cond_grid_waves;
   const uint64_t ntiles = (ngbx + kWave - 1) / kWave;
-  // a deferred drop is solved again by its sorted position k; its learned guess is that of source
-  // position perm[k]
   const uint32_t budget = c->tiles.cond_defer;
-  if (a.mlp_inline) a.warm_perm = n.perm;
   a.cfg.budget = budget;
-  a.dcap = budget ? c->dlist_cap : 0u;
   a.dlist = c->dlist;
-  a.dcount = budget ? c->dcount : nullptr;  // zeroed by k_cond_prep
+  a.dcount = c->dcount;
   hipLaunchKernelGGL(k_cond_prep, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
   if (a.mlp_inline) {  // learned guesses of the drops where motion left them
     CondFlatArgs ga = a;
@@ -3052,18 +3079,19 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
     ga.guess_out = nullptr;
     hipLaunchKernelGGL(k_cond_guess, dim3(drop_blocks(c->ntot, gw ? gw : 32768)), dim3(256), 0, c->stream, ga);
     a.warm = a.warm_buf;
+    a.warm_perm = n.perm;
   }
-  const unsigned nb = drop_blocks(c->ntot, gw);
+  const unsigned nb = solve_blocks(c, gw);
   a.stat = stat_slots(c, 4ull * nb);
-  set_defer_segments(c, a, nb);
   kev_mark(c, 0);
-  launch_gather_cond(c, n, a, move_in_gather ? &m : nullptr, nb);
+  const bool tail = tail_solves(c, budget);
+  if (tail)
+    launch_gather_cond<true>(c, n, a, move_in_gather ? &m : nullptr, nb);
+  else
+    launch_gather_cond<false>(c, n, a, move_in_gather ? &m : nullptr, nb);
   kev_mark(c, 1);
-  if (budget) {
-    launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
-    hipLaunchKernelGGL(k_cond_deferred, dim3(nb), dim3(256), 0, c->stream, a);
-  }
   launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
+  if (!tail) launch_deferred(c, a, nb);
   hipLaunchKernelGGL(k_nsort_oob, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, n, c->ntot);
   hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, static_cast<const uint32_t*>(nullptr));
   if (commit_dst >= 0) nsort_commit(c, commit_dst);

@@ -129,18 +129,15 @@ struct CondFlatArgs {
   // recomputes the gridbox qcond from it instead of a separate pass in k_cond_prep
   double* qm;
   StatSlots stat;  // ST_COND_DROPS .. ST_WARM_RESTARTS
-  uint32_t* dlist;   // deferred drops (positions) of all waves, room for `dcap`
-  uint32_t* dcount;  // one counter: entries claimed in dlist, zeroed by k_cond_prep (null: no deferral)
-  uint32_t dcap;
-  uint32_t* dseg;    // per-wave segments where a wave lists its deferred drops first, `dsegcap` each
-  uint32_t dsegcap;
+  uint32_t* dlist;  // positions of the drops each workgroup sets aside, from its range's start on
+  uint32_t* dcount;  // their number per workgroup, where a second launch solves them
   // mlp_inline: the learned guesses are evaluated by k_cond_guess into warm_buf inside the launch
   // sequence (after the saturation ratios exist) and read from there
   int32_t mlp_inline;
   MLPWeights W;
   double* warm_buf;
   // warm (learned guesses) indexed by the drop's source position perm[k] rather than by k: the
-  // guesses of the sort's gather with the solves, read again by k_cond_deferred
+  // guesses of the sort's gather with the solves, read again for its deferred drops
   const uint32_t* warm_perm;
   double* guess_out;  // non-null: the guesses are recorded here too (array position order)
   // k_cond_guess on the store as motion left it (before the sort): a drop is active when its new
