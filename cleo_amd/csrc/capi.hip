@@ -431,9 +431,7 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   HIP_TRY(c, dalloc(&c->big_scratch, 2 * maxn));
   HIP_TRY(c, dalloc(&c->gs, kGsStride * ngbx));
   HIP_TRY(c, dalloc(&c->dm, maxn));
-  // a gridbox launch has at most ngbx + 3 waves, a drop launch 4 per 256 drops
-  c->sp_slots = std::max<uint64_t>(ngbx + 4, 4 * ((maxn + 255) / 256) + 4);
-  HIP_TRY(c, dalloc(&c->sp, kStatSlotsMax * c->sp_slots));
+  HIP_TRY(c, dalloc(&c->sp, kStatRow * kStatRows));
   HIP_TRY(c, dalloc(&c->dlist, maxn));
   HIP_TRY(c, dalloc(&c->dcount, maxn / 256 + 1));
   HIP_TRY(c, dalloc(&c->perm, std::max<uint64_t>(maxn, 1)));
@@ -445,6 +443,7 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   HIP_TRY(c, dalloc(&c->ctl, 1));
   HIP_TRY(c, hipHostMalloc(reinterpret_cast<void**>(&c->h_ctl), sizeof(DevCtl), hipHostMallocDefault));
   HIP_TRY(c, ctx_fill(c, c->ctl, 0, sizeof(DevCtl)));
+  HIP_TRY(c, ctx_fill(c, c->sp, 0, kStatRow * kStatRows * 8));
   HIP_TRY(c, ctx_fill(c, c->off, 0, (ngbx + 1) * 4));
   HIP_TRY(c, ctx_fill(c, c->off_alt, 0, (ngbx + 1) * 4));
   HIP_TRY(c, ctx_fill(c, c->nact, 0, ngbx * 4));
@@ -941,7 +940,13 @@ int cleo_get_stats(cleo_ctx* c, cleo_stats* s) {
   if (!c || !s) return CLEO_E_ARG;
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   HIP_TRY(c, ctx_copy(c, c->h_ctl, c->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost));
-  const unsigned long long* v = c->h_ctl->stats;
+  std::vector<unsigned long long> rows(kStatRow * kStatRows);
+  HIP_TRY(c, ctx_copy(c, rows.data(), c->sp, rows.size() * 8, hipMemcpyDeviceToHost));
+  unsigned long long v[ST_COUNT];
+  for (uint32_t j = 0; j < ST_COUNT; ++j) {
+    v[j] = c->h_ctl->stats[j];
+    for (uint32_t r = 0; r < kStatRows; ++r) v[j] += rows[r * kStatRow + j];
+  }
   s->cond_drops = v[ST_COND_DROPS];
   s->newton_iters = v[ST_NEWTON_ITERS];
   s->substep_drops = v[ST_SUBSTEP_DROPS];
@@ -958,6 +963,7 @@ int cleo_reset_stats(cleo_ctx* c) {
   if (!c) return CLEO_E_ARG;
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   HIP_TRY(c, ctx_fill(c, c->ctl->stats, 0, sizeof(c->ctl->stats)));
+  HIP_TRY(c, ctx_fill(c, c->sp, 0, kStatRow * kStatRows * 8));
   return CLEO_OK;
 }
 
@@ -1052,6 +1058,8 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
   HIP_TRY(c, hipMemcpyAsync(saved_nact, c->nact, ngbx * 4ull, hipMemcpyDeviceToDevice, c->stream));
   DevCtl saved_ctl;
   HIP_TRY(c, ctx_copy(c, &saved_ctl, c->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost));
+  std::vector<unsigned long long> saved_rows(kStatRow * kStatRows);
+  HIP_TRY(c, ctx_copy(c, saved_rows.data(), c->sp, saved_rows.size() * 8, hipMemcpyDeviceToHost));
   const cleo_cond_params cp = c->sdm.first_cond() ? *c->sdm.first_cond()
                                                    : cleo_cond_params{100, 1, 50, 1e-6, 1e-8, 0.001, 0, 10};
   const cleo_coll_params kp = c->sdm.first_coll()
@@ -1176,6 +1184,7 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
   hipFree(saved);
   hipFree(saved_nact);
   HIP_TRY(c, ctx_copy(c, c->ctl, &saved_ctl, sizeof(DevCtl), hipMemcpyHostToDevice));
+  HIP_TRY(c, ctx_copy(c, c->sp, saved_rows.data(), saved_rows.size() * 8, hipMemcpyHostToDevice));
   if (rc != CLEO_OK) return rc;
   if (tmin) *tmin = best;
   if (tmean) *tmean = total / static_cast<float>(reps);

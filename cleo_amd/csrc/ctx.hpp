@@ -44,10 +44,11 @@ struct GState {
   double* vhi;
 };
 
-// Per-wave statistics slots: counter j of the wave in slot i is sp[j * nslot + i].
+// Statistics: kStatRows rows of one 128-byte line, each with a partial sum of every counter (StatIdx).
+constexpr uint32_t kStatRow = 16, kStatRows = 256;
+static_assert(ST_COUNT <= kStatRow, "counters of a row");
 struct StatSlots {
-  uint32_t* sp;
-  uint32_t nslot;
+  unsigned long long* rows;
 };
 
 struct MLPDev;  // mlp.hip
@@ -118,8 +119,7 @@ struct cleo_ctx {
   cleo_tiles tiles{1, 1, 1, 0, 0, 0, 0, 0, 0, 0};
   double* gs = nullptr;  // kGsStride*ngbx: per gridbox saturation ratio, diffusion factor, Koehler a, 1/a
   double* dm = nullptr;  // maxn: per-drop condensed mass (flat condensation)
-  // per-wave statistics: up to kStatSlotsMax counters per wave, reduced into DevCtl::stats
-  uint32_t* sp = nullptr;
+  unsigned long long* sp = nullptr;  // statistics: kStatRows rows of kStatRow partial sums
   // drops set aside by the workgroups of the thread-per-drop condensation (maxn positions)
   uint32_t* dlist = nullptr;
   uint32_t* dcount = nullptr;  // their number per workgroup (at most one per 256 drops)
@@ -139,7 +139,6 @@ struct cleo_ctx {
   double* qm = nullptr;
   // mass-moment observer results (ngbx uint64 + 2 * ngbx float, allocated at first use)
   void* mom = nullptr;
-  uint64_t sp_slots = 0;  // slots per counter: max(ngbx, waves of a thread-per-drop launch)
   // per-drop Newton iteration record
   bool rec_niters = false;
   uint32_t* niters = nullptr;

@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_condensation(CondArgs
   uint32_t acc[4] = {0, 0, 0, 0};
   for (uint32_t g = wave_index(); g < a.ngbx; g += wave_count()) cond_gbx<kFuseQcond>(a, g, lane, acc);
   if (lane == 0)
-    for (int j = 0; j < 4; ++j) put_stat(a.stat, j, wave_index(), acc[j]);
+    for (int j = 0; j < 4; ++j) put_stat(a.stat, ST_COND_DROPS + j, acc[j]);
 }
 
 // EffectOnHydrometeorStatesFunctor (movesupersindomain.hpp:95-136), standalone: 64 gridboxes per
@@ -582,9 +582,9 @@ __global__ void __launch_bounds__(B) CLEO_OCCUPANCY(Kinetic && B <= 256 ? 3 : 4)
   events = wave_sum_u32(events);
   nulls = wave_sum_u32(nulls);
   if (lane_id() == 0) {
-    put_stat(a.stat, 0, wave_index(), pairs);
-    put_stat(a.stat, 1, wave_index(), events);
-    put_stat(a.stat, 2, wave_index(), nulls);
+    put_stat(a.stat, ST_COLL_PAIRS, pairs);
+    put_stat(a.stat, ST_COLL_EVENTS, events);
+    put_stat(a.stat, ST_NULLS, nulls);
   }
 }
 
@@ -725,9 +725,9 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(Kinetic ? 3 : 4) k_coll_ti
   events = wave_sum_u32(events);
   nulls = wave_sum_u32(nulls);
   if (lane == 0) {
-    put_stat(a.stat, 0, wave_index(), pairs);
-    put_stat(a.stat, 1, wave_index(), events);
-    put_stat(a.stat, 2, wave_index(), nulls);
+    put_stat(a.stat, ST_COLL_PAIRS, pairs);
+    put_stat(a.stat, ST_COLL_EVENTS, events);
+    put_stat(a.stat, ST_NULLS, nulls);
   }
 }
 
@@ -741,22 +741,6 @@ __global__ void k_inj_sizes(const uint32_t* nact, uint32_t ngbx, uint32_t* nj, u
 }
 
 __global__ void k_advance_event(DevCtl* ctl) { ctl->event += 1; }
-
-// DevCtl::stats[first + blockIdx.y] += sum of the nslot slots of counter blockIdx.y; each block
-// sums a strided share and adds it with one atomic (a few hundred atomics per launch).
-__global__ void __launch_bounds__(256) k_stats_reduce(const uint32_t* sp, uint32_t nslot, int first, DevCtl* ctl) {
-  __shared__ unsigned long long part[4];
-  const uint32_t* col = sp + static_cast<uint64_t>(blockIdx.y) * nslot;
-  unsigned long long v = 0;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nslot; i += gridDim.x * blockDim.x) v += col[i];
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  if (lane_id() == 0) part[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned long long t = part[0] + part[1] + part[2] + part[3];
-    if (t) atomicAdd(&ctl->stats[first + static_cast<int>(blockIdx.y)], t);
-  }
-}
 
 // ============================ motion ==========================================================
 // Source gridbox that reaches `d` by the neighbour step `s` (s = (dz+1) + 3(dx+1) + 9(dy+1)),
@@ -979,7 +963,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_motion(MotionArgs a) 
   const int lane = lane_id();
   uint32_t moved = 0;
   for (uint32_t g = wave_index(); g < a.grid.ngbx; g += wave_count()) moved += motion_gbx(a, g, lane);
-  if (lane == 0) put_stat(a.stat, 0, wave_index(), moved);
+  if (lane == 0) put_stat(a.stat, ST_MOTION_DROPS, moved);
 }
 
 // ============================ neighbour sort ==================================================
@@ -1693,14 +1677,13 @@ void launch_condensation(cleo_ctx* c, const CondArgs& args) {
   CondArgs a = args;
   hipLaunchKernelGGL(k_gbx_thermo, dim3(stride_blocks(a.ngbx)), dim3(256), 0, c->stream, a.st, a.ngbx, a.gs);
   const unsigned nb = gbx_blocks(a.ngbx, a.wpb, c->tiles.cond_grid_waves);
-  a.stat = stat_slots(c, static_cast<uint64_t>(nb) * a.wpb);
+  a.stat = stat_slots(c);
   kev_mark(c, 0);
   if (a.fuse_qcond)
     hipLaunchKernelGGL(k_condensation<true>, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
   else
     hipLaunchKernelGGL(k_condensation<false>, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
   kev_mark(c, 1);
-  launch_stats_reduce(c, nb * a.wpb, ST_COND_DROPS, 4);
 }
 void launch_qcond(cleo_ctx* c, const QcondArgs& a) {
   if (a.ngbx == 0) return;
@@ -1719,12 +1702,11 @@ static void launch_coll_team(cleo_ctx* c, const CollArgs& args, uint32_t gpt, ui
   CollArgs a = args;
   const uint32_t cap = static_cast<uint32_t>(std::min<uint64_t>(kTeamMaxItems, (items + 63) / 64 * 64));
   const unsigned nb = gbx_blocks(a.ngbx, gpt, 0);
-  a.stat = stat_slots(c, static_cast<uint64_t>(nb) * (B / kWave));
+  a.stat = stat_slots(c);
   if (coll_is_kinetic(a.k))
     launch_coll_team_k<B, true>(c, a, nb, gpt, cap);
   else
     launch_coll_team_k<B, false>(c, a, nb, gpt, cap);
-  launch_stats_reduce(c, nb * (B / kWave), ST_COLL_PAIRS, 3);
 }
 void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   if (args.ngbx == 0) return;
@@ -1736,14 +1718,13 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   // lines cross near 75,000 gridboxes at any mean) whose drops fit a tile's 8 KB of permutations.
   if (c->tiles.coll_flat && a.ngbx >= kTileMinGbx && mean <= kTilePermBytes / kWave + 4) {
     const unsigned nb = gbx_blocks((a.ngbx + kWave - 1) / kWave, a.wpb, c->tiles.coll_grid_waves);
-    a.stat = stat_slots(c, static_cast<uint64_t>(nb) * a.wpb);
+    a.stat = stat_slots(c);
     kev_mark(c, 0);
     if (coll_is_kinetic(a.k))
       hipLaunchKernelGGL(k_coll_tiles<true>, dim3(nb), dim3(64 * a.wpb), a.wpb * kCollTileLdsBytes, c->stream, a);
     else
       hipLaunchKernelGGL(k_coll_tiles<false>, dim3(nb), dim3(64 * a.wpb), a.wpb * kCollTileLdsBytes, c->stream, a);
     kev_mark(c, 1);
-    launch_stats_reduce(c, nb * a.wpb, ST_COLL_PAIRS, 3);
     return;
   }
   // Teams, one workgroup each.  A wave takes as many gridboxes as make 512 drops (128 to 1024 tried:
@@ -1764,21 +1745,14 @@ void launch_motion(cleo_ctx* c, const MotionArgs& args) {
   if (args.grid.ngbx == 0) return;
   MotionArgs a = args;
   const unsigned nb = gbx_blocks(a.grid.ngbx, a.wpb, c->tiles.motion_grid_waves);
-  a.stat = stat_slots(c, static_cast<uint64_t>(nb) * a.wpb);
+  a.stat = stat_slots(c);
   hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * a.grid.ngbx)), dim3(256), 0, c->stream, a.cnt,
                      28ull * a.grid.ngbx, 0u);
   kev_mark(c, 0);
   hipLaunchKernelGGL(k_motion, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
   kev_mark(c, 1);
-  launch_stats_reduce(c, nb * a.wpb, ST_MOTION_DROPS, 1);
 }
-void launch_stats_reduce(cleo_ctx* c, uint32_t nslot, int first, int ncount) {
-  if (nslot == 0) return;
-  const unsigned nb = static_cast<unsigned>(std::min<uint64_t>(128, (nslot + 1023) / 1024));
-  hipLaunchKernelGGL(k_stats_reduce, dim3(nb, static_cast<unsigned>(ncount)), dim3(256), 0, c->stream,
-                     static_cast<const uint32_t*>(c->sp), nslot, first, c->ctl);
-}
-StatSlots stat_slots(cleo_ctx* c, uint64_t nslot) { return StatSlots{c->sp, static_cast<uint32_t>(nslot)}; }
+StatSlots stat_slots(cleo_ctx* c) { return StatSlots{c->sp}; }
 void launch_advance_event(cleo_ctx* c) { hipLaunchKernelGGL(k_advance_event, dim3(1), dim3(1), 0, c->stream, c->ctl); }
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np) {
   hipLaunchKernelGGL(k_inj_sizes, dim3(nblocks(c->grid.ngbx, 256)), dim3(256), 0, c->stream, c->nact, c->grid.ngbx, nj, np);
@@ -1937,9 +1911,8 @@ void motion_sort_fused(cleo_ctx* c, const MotionArgs& args, const SoA& dst, int 
   MotionArgs a = args;
   hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * ngbx)), dim3(256), 0, c->stream, a.cnt, 28ull * ngbx, 0u);
   const unsigned nb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
-  a.stat = stat_slots(c, 4ull * nb);
+  a.stat = stat_slots(c);
   launch_motion_drops<false>(c, a, nb);
-  launch_stats_reduce(c, 4u * nb, ST_MOTION_DROPS, 1);
   NsortArgs n = nsort_args(c, a.s, dst, nullptr);
   nsort_tables(c, n, nullptr);
   kev_mark(c, 0);
@@ -1962,11 +1935,10 @@ void motion_sort_gather(cleo_ctx* c, const MotionArgs& args, const SoA& dst, int
   a.step = c->dstep;
   hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * ngbx)), dim3(256), 0, c->stream, a.cnt, 28ull * ngbx, 0u);
   const unsigned nb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
-  a.stat = stat_slots(c, 4ull * nb);
+  a.stat = stat_slots(c);
   kev_mark(c, 0);
   launch_motion_drops<false>(c, a, nb);
   kev_mark(c, 1);
-  launch_stats_reduce(c, 4u * nb, ST_MOTION_DROPS, 1);
   NsortArgs n = nsort_args(c, a.s, dst, nullptr);
   n.step = c->dstep;
   nsort_tables(c, n, nullptr);
@@ -2134,11 +2106,10 @@ __device__ __forceinline__ void put_cond_stats(const StatSlots& sl, CondStats st
   st.subs = wave_sum_u32(st.subs);
   st.restarts = wave_sum_u32(st.restarts);
   if (lane_id() == 0) {
-    const uint32_t slot = wave_index();
-    put_stat(sl, 0, slot, st.solved);
-    put_stat(sl, 1, slot, st.iters);
-    put_stat(sl, 2, slot, st.subs);
-    put_stat(sl, 3, slot, st.restarts);
+    put_stat(sl, ST_COND_DROPS, st.solved);
+    put_stat(sl, ST_NEWTON_ITERS, st.iters);
+    put_stat(sl, ST_SUBSTEP_DROPS, st.subs);
+    put_stat(sl, ST_WARM_RESTARTS, st.restarts);
   }
 }
 
@@ -2603,10 +2574,10 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_cond_queue(CondFlatAr
   st_subs = wave_sum_u32(st_subs);
   st_restarts = wave_sum_u32(st_restarts);
   if (lane == 0) {
-    put_stat(a.stat, 0, wave_index(), st_solved);
-    put_stat(a.stat, 1, wave_index(), st_iters);
-    put_stat(a.stat, 2, wave_index(), st_subs);
-    put_stat(a.stat, 3, wave_index(), st_restarts);
+    put_stat(a.stat, ST_COND_DROPS, st_solved);
+    put_stat(a.stat, ST_NEWTON_ITERS, st_iters);
+    put_stat(a.stat, ST_SUBSTEP_DROPS, st_subs);
+    put_stat(a.stat, ST_WARM_RESTARTS, st_restarts);
   }
 }
 
@@ -2888,7 +2859,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_motion_drops(MotionAr
     count_keys(a.cnt, motion_key(Ma, ga), acta, lane);
     count_keys(a.cnt, motion_key(Mb, gb), actb, lane);
   }
-  if (lane == 0) put_stat(a.stat, 0, wave_index(), nmoved);
+  if (lane == 0) put_stat(a.stat, ST_MOTION_DROPS, nmoved);
 }
 
 // launches k_motion_drops with the bounds in LDS when they fit
@@ -2970,9 +2941,8 @@ static void launch_gather_cond(cleo_ctx* c, const NsortArgs& n, const CondFlatAr
 }
 static void launch_deferred(cleo_ctx* c, CondFlatArgs a, unsigned nlists) {
   const unsigned nb = nblocks(nlists, kListsPerBlock);
-  a.stat = stat_slots(c, 4ull * nb);
+  a.stat = stat_slots(c);
   hipLaunchKernelGGL(k_cond_deferred, dim3(nb), dim3(256), 0, c->stream, a, nlists);
-  launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
 }
 
 // whether the workgroups of a solving pass solve their deferred drops themselves (finish_deferred)
@@ -3005,14 +2975,13 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
     // task-ring kernel: waves of 4 per block; by default as many waves as fit on the device at once
     const uint64_t waves = gw ? gw : static_cast<uint64_t>(c->num_cu) * kCondQueueWavesPerCu;
     const unsigned nb = static_cast<unsigned>(std::max<uint64_t>(1, std::min<uint64_t>(waves / 4, (c->ntot + 255) / 256)));
-    a.stat = stat_slots(c, 4ull * nb);
+    a.stat = stat_slots(c);
     kev_mark(c, 0);
     hipLaunchKernelGGL(k_cond_queue, dim3(nb), dim3(256), 4 * kCondRingBytes, c->stream, a);
     kev_mark(c, 1);
-    launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
   } else {
     const unsigned nb = solve_blocks(c, gw);
-    a.stat = stat_slots(c, 4ull * nb);  // every wave of k_cond_drops writes its slot
+    a.stat = stat_slots(c);
     if (a.mlp_inline) {  // the learned guesses, from the saturation ratios k_cond_prep left
       hipLaunchKernelGGL(k_cond_guess, dim3(drop_blocks(c->ntot, gw ? gw : 32768)), dim3(256), 0, c->stream, a);
       a.warm = a.warm_buf;
@@ -3023,7 +2992,6 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
       hipLaunchKernelGGL(k_cond_drops<true>, dim3(nb), dim3(256), 0, c->stream, a);
     else
       hipLaunchKernelGGL(k_cond_drops<false>, dim3(nb), dim3(256), 0, c->stream, a);
-    launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
     if (!tail) launch_deferred(c, a, nb);
     kev_mark(c, 1);
   }
@@ -3051,9 +3019,8 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
     hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * ngbx)), dim3(256), 0, c->stream, m.cnt, 28ull * ngbx,
                        0u);
     const unsigned mb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
-    m.stat = stat_slots(c, 4ull * mb);
+    m.stat = stat_slots(c);
     launch_motion_drops<false>(c, m, mb);
-    launch_stats_reduce(c, 4u * mb, ST_MOTION_DROPS, 1);
   } else {
     launch_motion_flat(c, m);
   }
@@ -3082,7 +3049,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
     a.warm_perm = n.perm;
   }
   const unsigned nb = solve_blocks(c, gw);
-  a.stat = stat_slots(c, 4ull * nb);
+  a.stat = stat_slots(c);
   kev_mark(c, 0);
   const bool tail = tail_solves(c, budget);
   if (tail)
@@ -3090,7 +3057,6 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   else
     launch_gather_cond<false>(c, n, a, move_in_gather ? &m : nullptr, nb);
   kev_mark(c, 1);
-  launch_stats_reduce(c, 4u * nb, ST_COND_DROPS, 4);
   if (!tail) launch_deferred(c, a, nb);
   hipLaunchKernelGGL(k_nsort_oob, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, n, c->ntot);
   hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, static_cast<const uint32_t*>(nullptr));
@@ -3102,13 +3068,12 @@ void launch_motion_flat(cleo_ctx* c, const MotionArgs& args) {
   if (args.grid.ngbx == 0) return;
   MotionArgs a = args;
   const unsigned nb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
-  a.stat = stat_slots(c, 4ull * nb);  // every wave of k_motion_drops writes its slot
+  a.stat = stat_slots(c);
   hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * a.grid.ngbx)), dim3(256), 0, c->stream, a.cnt,
                      28ull * a.grid.ngbx, 0u);
   kev_mark(c, 0);
   launch_motion_drops<true>(c, a, nb);
   kev_mark(c, 1);
-  launch_stats_reduce(c, 4u * nb, ST_MOTION_DROPS, 1);
 }
 
 }  // namespace cleo

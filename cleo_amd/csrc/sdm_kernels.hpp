@@ -5,7 +5,6 @@
 
 namespace cleo {
 
-constexpr int kStatSlotsMax = 4;       // counters per wave of one kernel
 // tiled collisions: byte permutations of up to kTileMaxN drops, kTilePermBytes of them per wave
 constexpr uint32_t kTileMaxN = 255;
 constexpr uint32_t kTilePermBytes = 8192;
@@ -153,10 +152,8 @@ void launch_qcond(cleo_ctx* c, const QcondArgs& a);
 void launch_collisions(cleo_ctx* c, const CollArgs& a);
 void launch_motion(cleo_ctx* c, const MotionArgs& a);
 void launch_advance_event(cleo_ctx* c);
-// DevCtl::stats[first + j] += sum over the nslot slots of counter j, j < ncount
-void launch_stats_reduce(cleo_ctx* c, uint32_t nslot, int first, int ncount);
-// slot block of the context for a launch with `nslot` waves
-StatSlots stat_slots(cleo_ctx* c, uint64_t nslot);
+// the statistics rows of the context
+StatSlots stat_slots(cleo_ctx* c);
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np);
 // exclusive scan of in[i*stride+offset], i < len, into out[0..len] (out[len] = total)
 void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset, uint32_t* out,
