@@ -158,8 +158,8 @@ int enqueue_condensation(cleo_ctx* c, const cleo_cond_params& p, bool fuse_qcond
 // offsets of the injected stream per gridbox; validates the sizes the caller gave
 int prepare_injected(cleo_ctx* c) {
   launch_inj_sizes(c, c->tot, c->oobpre);
-  scan_u32(c, c->tot, c->grid.ngbx, 1u, 0u, c->inj_oj, nullptr);
-  scan_u32(c, c->oobpre, c->grid.ngbx, 1u, 0u, c->inj_op, nullptr);
+  scan_u32(c, c->tot, c->grid.ngbx, 1u, 0u, c->inj_oj);
+  scan_u32(c, c->oobpre, c->grid.ngbx, 1u, 0u, c->inj_op);
   uint32_t tj = 0, tp = 0;
   HIP_TRY(c, hipMemcpyAsync(&tj, c->inj_oj + c->grid.ngbx, 4, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipMemcpyAsync(&tp, c->inj_op + c->grid.ngbx, 4, hipMemcpyDeviceToHost, c->stream));
@@ -231,12 +231,18 @@ int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p) {
   a.inj_op = c->inj_op;
   a.big = c->big_scratch;
   a.big2 = reinterpret_cast<uint32_t*>(c->dm);
+  a.event_ofs = c->events_pending++;
   launch_collisions(c, a);
-  launch_advance_event(c);
   if (compose) std::swap(c->order, c->order_alt);
   c->order_live = true;
   if (inj) c->rng_mode = 0;  // consumed
   return launch_check(c);
+}
+
+// the end of a microphysics pass with collision events
+void end_collisions(cleo_ctx* c) {
+  resort_nulls(c, c->events_pending);
+  c->events_pending = 0;
 }
 
 // MoveSupersInDomain::run_step body: motion, stable sort + refs, (qcond unless fused later)
@@ -265,7 +271,7 @@ int enqueue_motion(cleo_ctx* c, const cleo_motion_params& p, bool qcond) {
     } else {
       launch_motion(c, a);
     }
-    neighbour_sort(c, c->cur, 1 - c->cur, nullptr, false, a.step);
+    neighbour_sort_to(c, c->buf[c->cur], c->buf[1 - c->cur], 1 - c->cur, a.step);
   }
   if (qcond) {
     QcondArgs q{c->buf[c->cur], c->off, c->st, c->solute, c->grid.ngbx, wpb_or1(c->tiles.cond_waves_per_block), c->ctl};
@@ -371,7 +377,7 @@ int enqueue_run_step(cleo_ctx* c, uint32_t t_mdl, uint32_t t_mdl_next) {
       subt = nxt;
     }
     if (pending_qcond) qcond_now();
-    if (any_coll) neighbour_sort(c, c->cur, 1 - c->cur, &c->ctl->resort_flag, true);
+    if (any_coll) end_collisions(c);
     t_sdm = t_sdm_next;
   }
   return launch_check(c);
@@ -423,7 +429,7 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   HIP_TRY(c, dalloc(&c->cnt, 56 * ngbx));  // counts, then the run offsets of the neighbour sort
   HIP_TRY(c, dalloc(&c->tot, ngbx + 1));
   HIP_TRY(c, dalloc(&c->oobpre, ngbx + 1));
-  HIP_TRY(c, dalloc(&c->oobcnt, ngbx));
+  HIP_TRY(c, dalloc(&c->part, 2 * ((ngbx + kTabBlock - 1) / kTabBlock) + 1));
   HIP_TRY(c, dalloc(&c->inj_oj, ngbx + 1));
   HIP_TRY(c, dalloc(&c->inj_op, ngbx + 1));
   c->scan_tmp_n = scan_tmp_words(28 * ngbx + 1);
@@ -447,6 +453,8 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   HIP_TRY(c, ctx_fill(c, c->off, 0, (ngbx + 1) * 4));
   HIP_TRY(c, ctx_fill(c, c->off_alt, 0, (ngbx + 1) * 4));
   HIP_TRY(c, ctx_fill(c, c->nact, 0, ngbx * 4));
+  HIP_TRY(c, ctx_fill(c, c->cnt, 0, 28 * ngbx * 4));
+  HIP_TRY(c, ctx_fill(c, c->tot, 0, (ngbx + 1) * 4));
   HIP_TRY(c, ctx_fill(c, c->d_state, 0, 11 * ngbx * 8));
   c->solute = make_solute(2016.5 / dimless::RHO0, 0.05844277 / dimless::MR0, 2.0);
   HIP_TRY(c, mlp_create(c));
@@ -462,7 +470,7 @@ int cleo_destroy(cleo_ctx* c) {
   free_soa(c->buf[1]);
   for (void* p : {static_cast<void*>(c->d_halves), static_cast<void*>(c->off), static_cast<void*>(c->off_alt),
                   static_cast<void*>(c->nact), static_cast<void*>(c->d_state), static_cast<void*>(c->cnt),
-                  static_cast<void*>(c->tot), static_cast<void*>(c->oobpre), static_cast<void*>(c->oobcnt), static_cast<void*>(c->inj_oj),
+                  static_cast<void*>(c->tot), static_cast<void*>(c->oobpre), static_cast<void*>(c->part), static_cast<void*>(c->inj_oj),
                   static_cast<void*>(c->inj_op), static_cast<void*>(c->scan_tmp), static_cast<void*>(c->big_scratch),
                   static_cast<void*>(c->ctl), static_cast<void*>(c->inj_j), static_cast<void*>(c->inj_phi),
                   static_cast<void*>(c->niters), static_cast<void*>(c->guess), static_cast<void*>(c->rs_key[0]),
@@ -685,6 +693,7 @@ int cleo_set_rng_counter(cleo_ctx* c, uint64_t seed, uint64_t first_event) {
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   c->rng_mode = 1;
   c->seed = seed;
+  c->events_pending = 0;
   HIP_TRY(c, ctx_copy(c, &c->ctl->event, &first_event, 8, hipMemcpyHostToDevice));
   return CLEO_OK;
 }
@@ -788,7 +797,7 @@ int cleo_collisions(cleo_ctx* c, const cleo_coll_params* p) {
   if (!c || !p) return CLEO_E_ARG;
   const int rc = enqueue_collision_event(c, *p);
   if (rc != CLEO_OK) return rc;
-  neighbour_sort(c, c->cur, 1 - c->cur, &c->ctl->resort_flag, true);
+  end_collisions(c);
   return launch_check(c);
 }
 
@@ -820,6 +829,13 @@ int cleo_run_steps_graph(cleo_ctx* c, uint32_t t_mdl, uint32_t span, uint32_t ns
     }
   }
   HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (c->events_pending) {  // events of a call that failed before its end: count them now
+    uint64_t ev = 0;
+    HIP_TRY(c, ctx_copy(c, &ev, &c->ctl->event, 8, hipMemcpyDeviceToHost));
+    ev += c->events_pending;
+    HIP_TRY(c, ctx_copy(c, &c->ctl->event, &ev, 8, hipMemcpyHostToDevice));
+    c->events_pending = 0;
+  }
   // The launches a step enqueues depend on the store's state when it starts (which buffer is
   // current, whether a collision order is pending), so every replay must start in the state the
   // previous one ended in.  One step is captured, or two when one step changes the state; if two
@@ -829,18 +845,21 @@ int cleo_run_steps_graph(cleo_ctx* c, uint32_t t_mdl, uint32_t span, uint32_t ns
   int cur0 = c->cur;
   bool live0 = c->order_live;
   uint32_t* ord0 = c->order;  // which of the two order buffers holds the pending order
-  auto set_order = [&](uint32_t* ord) {
+  uint32_t* off0 = c->off;    // and which of the two ref buffers is current
+  auto set_buffers = [&](uint32_t* ord, uint32_t* off) {
     if (c->order != ord) std::swap(c->order, c->order_alt);
+    if (c->off != off) std::swap(c->off, c->off_alt);
   };
   int rc = CLEO_OK;
   for (int attempt = 0; attempt < 3; ++attempt) {
     cur0 = c->cur;
     live0 = c->order_live;
     ord0 = c->order;
+    off0 = c->off;
     HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     rc = enqueue_run_step(c, t_mdl, t_mdl + span);
     per_graph = 1;
-    if (rc == CLEO_OK && (c->cur != cur0 || c->order_live != live0 || c->order != ord0)) {
+    if (rc == CLEO_OK && (c->cur != cur0 || c->order_live != live0 || c->order != ord0 || c->off != off0)) {
       rc = enqueue_run_step(c, t_mdl + span, t_mdl + 2 * span);
       per_graph = 2;
     }
@@ -848,15 +867,17 @@ int cleo_run_steps_graph(cleo_ctx* c, uint32_t t_mdl, uint32_t span, uint32_t ns
     const int cur1 = c->cur;
     const bool live1 = c->order_live;
     uint32_t* const ord1 = c->order;
+    uint32_t* const off1 = c->off;
+    c->events_pending = 0;
     c->cur = cur0;
     c->order_live = live0;
-    set_order(ord0);
+    set_buffers(ord0, off0);
     if (rc != CLEO_OK || e != hipSuccess) {
       if (graph) hipGraphDestroy(graph);
       if (rc != CLEO_OK) return rc;
       return fail(c, CLEO_E_HIP, std::string("capture: ") + hipGetErrorString(e));
     }
-    if (cur1 == cur0 && live1 == live0 && ord1 == ord0) break;
+    if (cur1 == cur0 && live1 == live0 && ord1 == ord0 && off1 == off0) break;
     hipGraphDestroy(graph);
     graph = nullptr;
     if (live1 && !live0) {
@@ -877,7 +898,7 @@ int cleo_run_steps_graph(cleo_ctx* c, uint32_t t_mdl, uint32_t span, uint32_t ns
   }
   c->cur = cur0;  // every replay starts and ends in the same state
   c->order_live = live0;
-  set_order(ord0);
+  set_buffers(ord0, off0);
   const uint32_t nreplay = nsteps / per_graph;
   for (uint32_t i = 0; i < nreplay; ++i) {
     e = hipGraphLaunch(exec, c->stream);

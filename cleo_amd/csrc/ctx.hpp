@@ -66,16 +66,16 @@ struct cleo_ctx {
   cleo::SoA buf[2]{};
   int cur = 0;
   uint32_t* off = nullptr;      // ngbx+1: gridbox refs, off[ngbx] = in-domain count
-  uint32_t* off_alt = nullptr;  // ngbx+1: next refs while sorting
+  uint32_t* off_alt = nullptr;  // ngbx+1: next refs while sorting; the two swap with each sort after motion
   uint32_t* nact = nullptr;     // ngbx: active drops per gridbox (subview extent)
   cleo::GState st{};
   double* d_state = nullptr;
   cleo::Solute solute{};
   // neighbour-sort scratch
-  uint32_t* cnt = nullptr;      // ngbx*56: sort counts (ngbx*28), then run offsets (ngbx*28)
+  uint32_t* cnt = nullptr;      // ngbx*56: sort counts (ngbx*28, zero between sorts), then run offsets (ngbx*28)
   uint32_t* tot = nullptr;      // ngbx+1
   uint32_t* oobpre = nullptr;   // ngbx+1
-  uint32_t* oobcnt = nullptr;   // ngbx: out-of-domain count per gridbox (compact copy for its scan)
+  uint32_t* part = nullptr;     // the sort's sums per block of gridboxes
   uint32_t* scan_tmp = nullptr;
   size_t scan_tmp_n = 0;
   // generic radix sort scratch (lazily allocated)
@@ -135,6 +135,7 @@ struct cleo_ctx {
   uint32_t* order = nullptr;
   uint32_t* order_alt = nullptr;  // the other buffer: a collision event composes order into it
   bool order_live = false;
+  uint32_t events_pending = 0;  // collision events since the device's event counter last moved on
   // per drop: condensed mass * xi before a condensation solve (the qcond recompute after motion)
   double* qm = nullptr;
   // mass-moment observer results (ngbx uint64 + 2 * ngbx float, allocated at first use)

@@ -537,7 +537,7 @@ int cleo_mlp_make_samples(cleo_ctx* c, const cleo_cond_params* p, float* x_out, 
     c->scan_tmp = tmp;
     c->scan_tmp_n = need;
   }
-  scan_u32(c, flag, n, 1u, 0u, pos, nullptr);
+  scan_u32(c, flag, n, 1u, 0u, pos);
   uint32_t total = 0;
   MLP_TRY(c, hipMemcpyAsync(&total, pos + n, 4, hipMemcpyDeviceToHost, c->stream));
   MLP_TRY(c, hipStreamSynchronize(c->stream));

@@ -82,9 +82,11 @@ struct DevCtl {
   uint32_t err_gbx;
   uint64_t err_drop;
   uint32_t resort_flag;  // nulls appeared in this microphysics pass
-  uint32_t pad0;
+  uint32_t resort_go;    // the re-sort under way has nulls to move
   uint64_t event;        // collision events so far (counter RNG)
   unsigned long long stats[ST_COUNT];
+  uint32_t resort_nsrc;  // drops in the domain before that re-sort
+  uint32_t pad0;
 };
 
 __device__ __forceinline__ void record_error(DevCtl* ctl, int code, uint32_t gbx, uint64_t drop) {

@@ -541,7 +541,7 @@ __global__ void __launch_bounds__(B) CLEO_OCCUPANCY(Kinetic && B <= 256 ? 3 : 4)
   const uint32_t tid = threadIdx.x;
   uint16_t* half = reinterpret_cast<uint16_t*>(lds_dyn + cap);
   const FyLds L{lds_dyn, half, half + cap, half + 2 * cap};
-  const uint64_t event = a.ctl->event;
+  const uint64_t event = a.ctl->event + a.event_ofs;
   uint32_t pairs = 0, events = 0, nulls = 0;
   for (uint64_t g0 = static_cast<uint64_t>(blockIdx.x) * gpt; g0 < a.ngbx; g0 += static_cast<uint64_t>(gridDim.x) * gpt) {
     const uint32_t cnt = static_cast<uint32_t>(min(static_cast<uint64_t>(gpt), a.ngbx - g0));
@@ -615,7 +615,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(Kinetic ? 3 : 4) k_coll_ti
   const int lane = lane_id();
   CollTileLds& L = reinterpret_cast<CollTileLds*>(lds_dyn)[threadIdx.x >> 6];
   uint8_t* pb = reinterpret_cast<uint8_t*>(L.perm32);
-  const uint64_t event = a.ctl->event;
+  const uint64_t event = a.ctl->event + a.event_ofs;
   uint32_t pairs = 0, events = 0, nulls = 0;
   const uint32_t ntiles = (a.ngbx + kWave - 1) / kWave;
   for (uint32_t tile = wave_index(); tile < ntiles; tile += wave_count()) {
@@ -739,8 +739,6 @@ __global__ void k_inj_sizes(const uint32_t* nact, uint32_t ngbx, uint32_t* nj, u
   nj[g] = n >= 2 ? n - 1 : 0;
   np[g] = 2 * (n / 2);
 }
-
-__global__ void k_advance_event(DevCtl* ctl) { ctl->event += 1; }
 
 // ============================ motion ==========================================================
 // Source gridbox that reaches `d` by the neighbour step `s` (s = (dz+1) + 3(dx+1) + 9(dy+1)),
@@ -967,67 +965,152 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_motion(MotionArgs a) 
 }
 
 // ============================ neighbour sort ==================================================
-__device__ __forceinline__ bool guard_off(const uint32_t* flag) { return flag && *flag == 0u; }
+
+// base[] of the sorted store, the first place of each gridbox (and of each gridbox's drops that leave
+// the domain), as the sum of a prefix within its block of kTabBlock gridboxes and the block's start
+__device__ __forceinline__ uint32_t new_base(const NsortArgs& a, uint32_t d) {
+  return a.tot[d] + a.part[2u * (d / kTabBlock)];
+}
+__device__ __forceinline__ uint32_t oob_base(const NsortArgs& a, uint32_t g) {
+  return a.part[2u * a.nblk] + a.oobpre[g] + a.part[2u * (g / kTabBlock) + 1u];
+}
+// exclusive prefix of v over the block's kTabBlock threads, and the block's total
+__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* ws, uint32_t& total) {
+  uint32_t wt;
+  const uint32_t x = wave_excl_scan(v, lane_id(), wt);
+  const uint32_t w = threadIdx.x / kWave, nw = blockDim.x / kWave;
+  __syncthreads();  // the previous scan is done with ws
+  if (lane_id() == 0) ws[w] = wt;
+  __syncthreads();
+  uint32_t pre = 0;
+  total = 0;
+  for (uint32_t i = 0; i < nw; ++i) {
+    pre += i < w ? ws[i] : 0u;
+    total += ws[i];
+  }
+  return pre + x;
+}
+// the condensation inputs of a gridbox (condensation.cpp:44-56)
+__device__ __forceinline__ void gbx_thermo(const GState& st, uint32_t g, double* gs) {
+  const double temp = st.temp[g], press = st.press[g];
+  const double psat = saturation_pressure(temp);
+  gs[kGsStride * g] = supersaturation_ratio(press, st.qv[g], psat);
+  gs[kGsStride * g + 1] = diffusion_factor(press, temp, psat);
+  const double akoh = kohler_a(temp);
+  gs[kGsStride * g + 2] = akoh;
+  gs[kGsStride * g + 3] = rcp_nr(akoh);
+}
 
 // Per destination d (thread per d): the drops arriving in d, and for each step s the drops that
 // reach d from source gridboxes of lower index than the source of s (the stable order puts them
-// first).  The counts are destination-major (row d, column s: arrivals at d by the step s) and
-// read as one row; the run offsets are written source-major into `runs` (row g, column s: the
-// offset of g's drops taking the step s), so the rank pass reads its gridbox's 27 offsets as one
-// contiguous row.  Every entry of `runs` belongs to one destination (g + step s): no two threads
-// write the same entry.  Only the entries of steps that some drop takes are written (a source off
-// a finite axis has none); the others keep older values that no pass reads.
-__global__ void k_nsort_tot(NsortArgs a) {
-  if (guard_off(a.flag)) return;
-  const uint32_t d = blockIdx.x * blockDim.x + threadIdx.x;
-  if (d >= a.grid.ngbx) return;
-  const uint32_t* row = a.cnt + 28ull * d;
-  a.oobcnt[d] = row[27];  // the out-of-domain count, compact for its scan
-  uint32_t cnt[27];
-  uint32_t t = 0;
+// first).  The counts are destination-major (row d, column s: arrivals at d by the step s), read as
+// one row and left zero for the next motion.  The run offsets are written source-major into `runs`
+// (row g, column s: the offset of g's drops taking the step s), so the rank pass reads its gridbox's
+// 27 offsets as one contiguous row.  Every entry of `runs` belongs to one destination (g + step s): no
+// two threads write the same entry.  Only the entries of steps that some drop takes are written (a
+// source off a finite axis has none); the others keep older values that no pass reads.
+// The arrivals and the drops that leave the domain are scanned here within the block of gridboxes;
+// k_nsort_part scans the blocks' totals, and the rank pass, which reads base[] anyway, writes the new
+// refs.  (Separate launches for the fill of the counts, two three-level scans, the refs, the active
+// counts and the condensation inputs, with the same for the re-sort after collisions, made 34 launches
+// of a coupled step, 11 now: 409 -> 349 us on 32^3 gridboxes of 64 drops.)  kThermo: the gridbox's condensation inputs too, for a
+// condensation in the sort's gather (the State is that of before the sort).
+template <bool kThermo>
+__global__ void __launch_bounds__(kTabBlock) k_nsort_tot(NsortArgs a, GState st, double* gs) {
+  __shared__ uint32_t ws[kTabBlock / kWave];
+  const uint32_t d = blockIdx.x * kTabBlock + threadIdx.x;
+  uint32_t t = 0, gone = 0;
+  if (d < a.grid.ngbx) {
+    uint4* row = reinterpret_cast<uint4*>(a.cnt + 28ull * d);
+    uint32_t cnt[28];
 #pragma unroll
-  for (int s = 0; s < 27; ++s) {
-    cnt[s] = row[s];
-    t += cnt[s];
-  }
-  const Grid& gr = a.grid;
-  const int nz = static_cast<int>(gr.nz), nx = static_cast<int>(gr.nx), ny = static_cast<int>(gr.ny);
-  const int gz = static_cast<int>(d % gr.nz), gx = static_cast<int>((d / gr.nz) % gr.nx),
-            gy = static_cast<int>(d / (gr.nz * gr.nx));
-  auto axis = [](int i, int dd, int n, bool per) {
-    int j = i - dd;
-    if (j < 0) j = per ? j + n : -1;
-    if (j >= n) j = per ? j - n : -1;
-    return j;
-  };
-  uint32_t src[27];  // the source of each step (kOOB: off a finite axis, no drops)
-#pragma unroll
-  for (int s = 0; s < 27; ++s) {
-    const int jz = axis(gz, s % 3 - 1, nz, gr.per[0] != 0), jx = axis(gx, (s / 3) % 3 - 1, nx, gr.per[1] != 0),
-              jy = axis(gy, s / 9 - 1, ny, gr.per[2] != 0);
-    src[s] = (jz >= 0 && jx >= 0 && jy >= 0) ? static_cast<uint32_t>(jz + nz * (jx + nx * jy)) : kOOB;
-  }
-  const bool wraps = (gr.per[0] && (gz == 0 || gz + 1 == nz)) || (gr.per[1] && (gx == 0 || gx + 1 == nx)) ||
-                     (gr.per[2] && (gy == 0 || gy + 1 == ny));
-  if (!wraps) {
-    // no step wraps: the source of step s is d - (dz + nz dx + nz nx dy), so the sources in index
-    // order are the steps in decreasing order
-    uint32_t before = 0;
-#pragma unroll
-    for (int s = 26; s >= 0; --s) {
-      if (cnt[s] > 0u && src[s] != kOOB) a.runs[28ull * src[s] + static_cast<uint32_t>(s)] = before;
-      before += cnt[s];
+    for (int i = 0; i < 7; ++i) {
+      const uint4 v = row[i];
+      cnt[4 * i] = v.x;
+      cnt[4 * i + 1] = v.y;
+      cnt[4 * i + 2] = v.z;
+      cnt[4 * i + 3] = v.w;
     }
-  } else {
+#pragma unroll
+    for (int i = 0; i < 7; ++i) row[i] = uint4{0u, 0u, 0u, 0u};
+    gone = cnt[27];
+#pragma unroll
+    for (int s = 0; s < 27; ++s) t += cnt[s];
+    const Grid& gr = a.grid;
+    const int nz = static_cast<int>(gr.nz), nx = static_cast<int>(gr.nx), ny = static_cast<int>(gr.ny);
+    const int gz = static_cast<int>(d % gr.nz), gx = static_cast<int>((d / gr.nz) % gr.nx),
+              gy = static_cast<int>(d / (gr.nz * gr.nx));
+    auto axis = [](int i, int dd, int n, bool per) {
+      int j = i - dd;
+      if (j < 0) j = per ? j + n : -1;
+      if (j >= n) j = per ? j - n : -1;
+      return j;
+    };
+    uint32_t src[27];  // the source of each step (kOOB: off a finite axis, no drops)
 #pragma unroll
     for (int s = 0; s < 27; ++s) {
+      const int jz = axis(gz, s % 3 - 1, nz, gr.per[0] != 0), jx = axis(gx, (s / 3) % 3 - 1, nx, gr.per[1] != 0),
+                jy = axis(gy, s / 9 - 1, ny, gr.per[2] != 0);
+      src[s] = (jz >= 0 && jx >= 0 && jy >= 0) ? static_cast<uint32_t>(jz + nz * (jx + nx * jy)) : kOOB;
+    }
+    const bool wraps = (gr.per[0] && (gz == 0 || gz + 1 == nz)) || (gr.per[1] && (gx == 0 || gx + 1 == nx)) ||
+                       (gr.per[2] && (gy == 0 || gy + 1 == ny));
+    if (!wraps) {
+      // no step wraps: the source of step s is d - (dz + nz dx + nz nx dy), so the sources in index
+      // order are the steps in decreasing order
       uint32_t before = 0;
 #pragma unroll
-      for (int q = 0; q < 27; ++q) before += src[q] < src[s] ? cnt[q] : 0u;
-      if (cnt[s] > 0u && src[s] != kOOB) a.runs[28ull * src[s] + static_cast<uint32_t>(s)] = before;
+      for (int s = 26; s >= 0; --s) {
+        if (cnt[s] > 0u && src[s] != kOOB) a.runs[28ull * src[s] + static_cast<uint32_t>(s)] = before;
+        before += cnt[s];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 27; ++s) {
+        uint32_t before = 0;
+#pragma unroll
+        for (int q = 0; q < 27; ++q) before += src[q] < src[s] ? cnt[q] : 0u;
+        if (cnt[s] > 0u && src[s] != kOOB) a.runs[28ull * src[s] + static_cast<uint32_t>(s)] = before;
+      }
+    }
+    a.nact[d] = t;
+    if constexpr (kThermo) {
+      if (st.temp[d] <= 0) set_error(a.ctl, CLEO_ERR_TEMP_NONPOSITIVE, d, a.off[d]);
+      gbx_thermo(st, d, gs);
     }
   }
-  a.tot[d] = t;
+  uint32_t tsum, gsum;
+  const uint32_t tpre = block_excl_scan(t, ws, tsum), gpre = block_excl_scan(gone, ws, gsum);
+  if (d < a.grid.ngbx) {
+    a.tot[d] = tpre;
+    a.oobpre[d] = gpre;
+  }
+  if (threadIdx.x == 0) {
+    const bool only = gridDim.x == 1;  // no k_nsort_part follows
+    a.part[2u * blockIdx.x] = only ? 0u : tsum;
+    a.part[2u * blockIdx.x + 1u] = only ? 0u : gsum;
+    if (only) a.part[2u] = tsum;
+    if (blockIdx.x == 0) a.ctl->stats[ST_SORTS] += 1;
+  }
+}
+// the blocks' totals of k_nsort_tot to their starts (one workgroup); part[2 nblk] gets the drops in the
+// domain
+__global__ void __launch_bounds__(1024) k_nsort_part(uint32_t* part, uint32_t nblk) {
+  __shared__ uint32_t ws[16];
+  uint32_t t0 = 0, g0 = 0;
+  for (uint32_t b0 = 0; b0 < nblk; b0 += 1024u) {
+    const uint32_t b = b0 + threadIdx.x;
+    const uint32_t t = b < nblk ? part[2u * b] : 0u, g = b < nblk ? part[2u * b + 1u] : 0u;
+    uint32_t ts, gs;
+    const uint32_t tp = block_excl_scan(t, ws, ts), gp = block_excl_scan(g, ws, gs);
+    if (b < nblk) {
+      part[2u * b] = t0 + tp;
+      part[2u * b + 1u] = g0 + gp;
+    }
+    t0 += ts;
+    g0 += gs;
+  }
+  if (threadIdx.x == 0) part[2u * nblk] = t0;
 }
 
 // Stable scatter (sortsupers.hpp:63-76,167-193 under Serial): drop p of source gridbox g with
@@ -1052,7 +1135,7 @@ __global__ void k_nsort_tot(NsortArgs a) {
 // 9(dy+1) is g + noff away from the edges, else wrapped on periodic axes (the same gridbox as
 // neighbour_of, without a division per lane).  A g past the last gridbox gives an empty head.
 struct RankHead {
-  uint32_t g, sbase, nfull, trun;
+  uint32_t g, sbase, nfull, trun, base;
   int gz, gx, gy;
 };
 __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, int gz, int gx, int gy, int32_t noff,
@@ -1061,11 +1144,11 @@ __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, in
   const int nz = static_cast<int>(a.grid.nz), nx = static_cast<int>(a.grid.nx), ny = static_cast<int>(a.grid.ny);
   const bool valid = g < ngbx;
   const uint32_t gc = valid ? static_cast<uint32_t>(g) : ngbx - 1u;
-  RankHead h{gc, 0u, 0u, 0u, gz, gx, gy};
+  RankHead h{gc, 0u, 0u, 0u, 0u, gz, gx, gy};
   const uint32_t lo = a.off[gc], hi = a.off[gc + 1];
   h.sbase = lo;
   h.nfull = valid ? hi - lo : 0u;
-  uint32_t d = ngbx;  // lanes 27..63: the out-of-domain run (base[ngbx] + oobpre[g])
+  uint32_t d = ngbx;  // lanes 27..63: the out-of-domain run
   bool ok = valid && lane == 27;
   if (lane < 27 && !valid) {
     d = 0u;  // no gridbox: a harmless load, discarded
@@ -1087,8 +1170,12 @@ __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, in
       d = ok ? static_cast<uint32_t>(jz + nz * (jx + nx * jy)) : 0u;
     }
   }
-  const uint32_t b = a.base[d];
-  const uint32_t extra = lane < 27 ? a.runs[28ull * gc + static_cast<uint32_t>(lane)] : a.oobpre[gc];
+  // new_base(d) + the run's offset, or oob_base(gc); tot[ngbx] is 0
+  const bool in = d < ngbx;
+  const uint32_t b = a.tot[d] + a.part[in ? 2u * (d / kTabBlock) : 2u * a.nblk];
+  const uint32_t extra = lane < 27 ? a.runs[28ull * gc + static_cast<uint32_t>(lane)]
+                                   : a.oobpre[gc] + a.part[2u * (gc / kTabBlock) + 1u];
+  h.base = b;
   h.trun = ok ? b + extra : 0u;
   return h;
 }
@@ -1134,6 +1221,7 @@ __device__ __forceinline__ void rank_gbx(const NsortArgs& a, const RankHead& h, 
   const int nz = static_cast<int>(a.grid.nz), nx = static_cast<int>(a.grid.nx), ny = static_cast<int>(a.grid.ny);
   const int gz = h.gz, gx = h.gx, gy = h.gy;
   uint32_t trun = h.trun;
+  if (lane == 13) a.off_new[g] = h.base;  // step 13 stays: the new refs
   auto near = [](int q, int r, int nd, bool per) {
     const int dd = q - r;
     if (dd >= -1 && dd <= 1) return true;
@@ -1212,13 +1300,17 @@ __device__ __forceinline__ void rank_gbx(const NsortArgs& a, const RankHead& h, 
 // (z, x, y) advance by the stride's with carries (no division per gridbox).
 template <bool kOrder, bool kStep>
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kStep ? 6 : 4) k_nsort_perm(NsortArgs a) {
-  if (guard_off(a.flag)) return;
   const int lane = lane_id();
   const uint32_t nz = a.grid.nz, nx = a.grid.nx;
   const uint64_t ngbx = a.grid.ngbx;
   const uint32_t g0 = xcd_wave_index(), stride = wave_count();
   const uint32_t nsrc = a.off[ngbx];
-  if (g0 >= ngbx || nsrc == 0) return;
+  if (g0 == 0 && lane == 0) a.off_new[ngbx] = a.part[2u * a.nblk];
+  if (g0 >= ngbx) return;
+  if (nsrc == 0) {  // no drops to rank: the new refs only
+    for (uint64_t g = g0 + static_cast<uint64_t>(lane) * stride; g < ngbx; g += static_cast<uint64_t>(kWave) * stride) a.off_new[g] = 0u;
+    return;
+  }
   uint32_t gz = g0 % nz, gx = (g0 / nz) % nx, gy = g0 / (nz * nx);
   const uint32_t sz = stride % nz, sx = (stride / nz) % nx, sy = stride / (nz * nx);
   const int32_t noff = (lane % 3 - 1) + static_cast<int32_t>(nz) * ((lane / 3) % 3 - 1) +
@@ -1263,13 +1355,32 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kStep ? 6 : 4) k_nsort_per
   }
 }
 
+// record p of src to position q of dst
+__device__ __forceinline__ void copy_drop(const SoA& src, const SoA& dst, uint64_t p, uint64_t q) {
+  dst.gbx[q] = src.gbx[p];
+  dst.c3[q] = src.c3[p];
+  dst.c1[q] = src.c1[p];
+  dst.c2[q] = src.c2[p];
+  dst.xi[q] = src.xi[p];
+  dst.r[q] = src.r[p];
+  dst.msol[q] = src.msol[p];
+  dst.id[q] = src.id[p];
+}
+// The drops that were out of the domain before (positions nsrc on) follow the newly out-of-domain
+// ones; the domain's drops fill the first nsrc positions of the sorted store either way, so they keep
+// their positions.
+__device__ __forceinline__ void copy_oob(const NsortArgs& a, uint64_t nsrc) {
+  for (uint64_t p = nsrc + blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; p < a.ntot;
+       p += static_cast<uint64_t>(gridDim.x) * blockDim.x)
+    copy_drop(a.src, a.dst, p, p);
+}
+
 // Second pass: destination position q takes the record at source position perm[q].  Consecutive
 // threads write consecutive positions, so each cache line of the sorted store is written whole by
 // one wave; the reads follow the runs of the source order.  Two positions per thread, all loads of
 // both issued before the stores.  A position whose perm entry is not a source position of the
 // domain (counts inconsistent with the keys) is reported and skipped, so no read leaves the store.
 __global__ void __launch_bounds__(256) k_nsort_gather(NsortArgs a) {
-  if (guard_off(a.flag)) return;
   const uint64_t nsrc = a.off[a.grid.ngbx];
   for (uint64_t q0 = 2ull * blockIdx.x * blockDim.x; q0 < nsrc; q0 += 2ull * gridDim.x * blockDim.x) {
     const uint64_t qa = q0 + threadIdx.x, qb = qa + blockDim.x;
@@ -1307,29 +1418,7 @@ __global__ void __launch_bounds__(256) k_nsort_gather(NsortArgs a) {
       a.dst.id[qb] = idb;
     }
   }
-}
-
-// drops already out of the domain stay behind the newly out-of-domain ones, in order
-__global__ void k_nsort_oob(NsortArgs a, uint64_t ntot) {
-  if (guard_off(a.flag)) return;
-  const uint64_t old_end = a.off[a.grid.ngbx];
-  const uint64_t dst0 = static_cast<uint64_t>(a.base[a.grid.ngbx]) + a.oobpre[a.grid.ngbx];
-  for (uint64_t p = old_end + blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; p < ntot;
-       p += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    const uint64_t d = dst0 + (p - old_end);
-    if (d >= ntot) {
-      set_error(a.ctl, CLEO_ERR_SORT_NONLOCAL, kOOB, p);
-      continue;
-    }
-    a.dst.gbx[d] = a.src.gbx[p];
-    a.dst.c3[d] = a.src.c3[p];
-    a.dst.c1[d] = a.src.c1[p];
-    a.dst.c2[d] = a.src.c2[p];
-    a.dst.xi[d] = a.src.xi[p];
-    a.dst.r[d] = a.src.r[p];
-    a.dst.msol[d] = a.src.msol[p];
-    a.dst.id[d] = a.src.id[p];
-  }
+  copy_oob(a, nsrc);
 }
 
 // Second pass of the fused motion + sort (the first is k_motion_drops<false>): the drops of
@@ -1361,10 +1450,10 @@ __device__ __forceinline__ void motion_scatter_gbx(const MotionArgs& a, const Ns
     const uint32_t need = present & ~have;
     if (lane < 28 && ((need >> lane) & 1u)) {
       if (lane == 27) {
-        run = n.base[a.grid.ngbx] + n.oobpre[g];
+        run = oob_base(n, g);
       } else {
         const uint32_t d = neighbour_of(a.grid, g, lane);
-        run = n.base[d] + n.runs[28ull * g + lane];
+        run = new_base(n, d) + n.runs[28ull * g + lane];
       }
     }
     have |= need;
@@ -1395,69 +1484,87 @@ __device__ __forceinline__ void motion_scatter_gbx(const MotionArgs& a, const Ns
 }
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_motion_scatter(MotionArgs a, NsortArgs n) {
   const int lane = lane_id();
-  for (uint32_t g = wave_index(); g < a.grid.ngbx; g += wave_count()) motion_scatter_gbx(a, n, g, lane);
-}
-
-// counts of the re-sort after collisions: active drops stay, nulls leave the domain
-__global__ void k_cnt_from_nact(const uint32_t* off, const uint32_t* nact, uint32_t ngbx, uint32_t* cnt,
-                                const uint32_t* flag) {
-  if (guard_off(flag)) return;
-  for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < 28ull * ngbx;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    const uint32_t g = static_cast<uint32_t>(i / 28), s = static_cast<uint32_t>(i % 28);
-    const uint32_t n = nact[g], nfull = off[g + 1] - off[g];
-    cnt[i] = s == 13 ? n : (s == 27 ? nfull - n : 0u);
+  for (uint32_t g = wave_index(); g < a.grid.ngbx; g += wave_count()) {
+    if (lane == 0) n.off_new[g] = new_base(n, g);
+    motion_scatter_gbx(a, n, g, lane);
   }
+  if (wave_index() == 0 && lane == 0) n.off_new[a.grid.ngbx] = n.part[2u * n.nblk];
+  copy_oob(n, n.off[a.grid.ngbx]);
 }
 
-__global__ void k_set_nact(const uint32_t* off, uint32_t ngbx, uint32_t* nact, const uint32_t* flag) {
-  if (guard_off(flag)) return;
+__global__ void k_set_nact(const uint32_t* off, uint32_t ngbx, uint32_t* nact, DevCtl* ctl) {
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g < ngbx) nact[g] = off[g + 1] - off[g];
+  if (g == 0) ctl->stats[ST_SORTS] += 1;
 }
 
-__global__ void k_copy_u32(const uint32_t* src, uint32_t* dst, uint64_t n, const uint32_t* flag) {
-  if (guard_off(flag)) return;
-  for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
-    dst[i] = src[i];
+// ============================ re-sort after collisions ========================================
+// When collisions left nulls, SDMMethods sorts again: the active drops of each gridbox move together
+// and the nulls of all gridboxes, in order, go behind the domain (before the drops that were out of it
+// already, which keep their positions).  Three launches that end at once when there are no nulls, so
+// that a captured graph needs no host decision: the plan (one workgroup), the records in their new
+// places in the other buffer, and their way back with the new refs.
+//
+// The plan also advances the event counter past the events of this microphysics pass.
+__global__ void __launch_bounds__(1024) k_resort_plan(DevCtl* ctl, const uint32_t* off, const uint32_t* nact, uint32_t ngbx,
+                                                      uint32_t* off_new, uint32_t events) {
+  __shared__ uint32_t ws[16];
+  const uint32_t flag = ctl->resort_flag;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    ctl->event += events;
+    ctl->resort_flag = 0u;
+    ctl->resort_go = flag;
+    ctl->resort_nsrc = off[ngbx];
+    if (flag) ctl->stats[ST_SORTS] += 1;
+  }
+  if (!flag) return;
+  uint32_t run = 0;
+  for (uint64_t g0 = 0; g0 < ngbx; g0 += 4096u) {  // four gridboxes per thread
+    const uint64_t g = g0 + 4u * threadIdx.x;
+    uint32_t n[4], sum = 0, all;
+    for (uint32_t i = 0; i < 4; ++i) {
+      n[i] = g + i < ngbx ? nact[g + i] : 0u;
+      sum += n[i];
+    }
+    uint32_t at = run + block_excl_scan(sum, ws, all);
+    for (uint32_t i = 0; i < 4; ++i) {
+      if (g + i < ngbx) off_new[g + i] = at;
+      at += n[i];
+    }
+    run += all;
+  }
+  if (threadIdx.x == 0) off_new[ngbx] = run;
 }
-
-__global__ void k_copy_soa(SoA src, SoA dst, uint64_t lo, uint64_t hi, const uint32_t* flag) {
-  if (guard_off(flag)) return;
-  for (uint64_t p = lo + blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; p < hi;
-       p += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    dst.gbx[p] = src.gbx[p];
-    dst.c3[p] = src.c3[p];
-    dst.c1[p] = src.c1[p];
-    dst.c2[p] = src.c2[p];
-    dst.xi[p] = src.xi[p];
-    dst.r[p] = src.r[p];
-    dst.msol[p] = src.msol[p];
-    dst.id[p] = src.id[p];
+// slot k of gridbox g: place off_new[g] + k when active, else behind the active drops of the domain
+// and the nulls of the gridboxes before (off[g] - off_new[g] of them)
+__global__ void __launch_bounds__(256) k_resort_gather(const DevCtl* ctl, SoA src, SoA dst, const uint32_t* off,
+                                                       const uint32_t* nact, const uint32_t* off_new, uint32_t ngbx,
+                                                       const uint32_t* order) {
+  if (!ctl->resort_go) return;
+  const uint32_t nsrc = ctl->resort_nsrc, active = off_new[ngbx];
+  for (uint32_t g = wave_index(); g < ngbx; g += wave_count()) {
+    const uint32_t lo = off[g], n = nact[g], nfull = off[g + 1] - lo, to = off_new[g];
+    for (uint32_t k = static_cast<uint32_t>(lane_id()); k < nfull; k += kWave) {
+      const uint32_t p = order[lo + k];
+      const uint32_t q = k < n ? to + k : active + (lo - to) + (k - n);
+      if (p < nsrc && q < nsrc) copy_drop(src, dst, p, q);
+    }
   }
 }
-
-// copies [off_old[ngbx], ntot) from src to dst (the out-of-domain region after collisions)
-__global__ void k_copy_oob_region(SoA src, SoA dst, const uint32_t* off, uint32_t ngbx, uint64_t ntot) {
-  const uint64_t lo = off[ngbx];
-  for (uint64_t p = lo + blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; p < ntot;
-       p += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    dst.gbx[p] = src.gbx[p];
-    dst.c3[p] = src.c3[p];
-    dst.c1[p] = src.c1[p];
-    dst.c2[p] = src.c2[p];
-    dst.xi[p] = src.xi[p];
-    dst.r[p] = src.r[p];
-    dst.msol[p] = src.msol[p];
-    dst.id[p] = src.id[p];
+__global__ void __launch_bounds__(256) k_resort_back(const DevCtl* ctl, SoA src, SoA dst, uint32_t* off, uint32_t* nact,
+                                                     const uint32_t* off_new, uint32_t ngbx, uint32_t* order) {
+  if (!ctl->resort_go) return;
+  const uint64_t first = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x,
+                 stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  for (uint64_t q = first; q < ctl->resort_nsrc; q += stride) {
+    copy_drop(src, dst, q, q);
+    order[q] = static_cast<uint32_t>(q);
   }
-}
-
-__global__ void k_clear_flag(DevCtl* ctl) { ctl->resort_flag = 0u; }
-__global__ void k_sorts_stat(DevCtl* ctl, const uint32_t* flag) {
-  if (guard_off(flag)) return;
-  ctl->stats[ST_SORTS] += 1;
+  for (uint64_t g = first; g <= ngbx; g += stride) {
+    off[g] = off_new[g];
+    if (g < ngbx) nact[g] = off_new[g + 1] - off_new[g];
+  }
 }
 
 // ============================ generic stable radix sort =======================================
@@ -1517,15 +1624,7 @@ __global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* key, const u
 __global__ void k_gather_soa(SoA src, SoA dst, const uint32_t* idx, uint64_t n) {
   for (uint64_t p = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; p < n;
        p += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    const uint32_t s = idx[p];
-    dst.gbx[p] = src.gbx[s];
-    dst.c3[p] = src.c3[s];
-    dst.c1[p] = src.c1[s];
-    dst.c2[p] = src.c2[s];
-    dst.xi[p] = src.xi[s];
-    dst.r[p] = src.r[s];
-    dst.msol[p] = src.msol[s];
-    dst.id[p] = src.id[s];
+    copy_drop(src, dst, idx[p], p);
   }
 }
 
@@ -1550,9 +1649,7 @@ __device__ __forceinline__ uint32_t load_in(const uint32_t* in, uint64_t i, uint
 }
 
 __global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const uint32_t* in, uint64_t len, uint32_t stride,
-                                                              uint32_t offset, uint32_t* partial,
-                                                              const uint32_t* flag) {
-  if (guard_off(flag)) return;
+                                                              uint32_t offset, uint32_t* partial) {
   __shared__ uint32_t ws[4];
   const uint64_t t0 = static_cast<uint64_t>(blockIdx.x) * kScanTile;
   uint32_t s = 0;
@@ -1565,8 +1662,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const uint32_t* in
 
 __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const uint32_t* in, uint64_t len, uint32_t stride,
                                                              uint32_t offset, const uint32_t* block_off,
-                                                             uint32_t* out, const uint32_t* flag) {
-  if (guard_off(flag)) return;
+                                                             uint32_t* out) {
   __shared__ uint32_t ws[4];
   const uint64_t t0 = static_cast<uint64_t>(blockIdx.x) * kScanTile;
   // each thread owns kScanItems consecutive items
@@ -1606,8 +1702,7 @@ static inline unsigned nblocks(uint64_t n, uint64_t per) {
   const uint64_t b = (n + per - 1) / per;
   return static_cast<unsigned>(b == 0 ? 1 : b);
 }
-__global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v);
-__global__ void k_iota_u32(uint32_t* p, uint64_t n, const uint32_t* flag);
+__global__ void k_iota_u32(uint32_t* p, uint64_t n);
 template <bool kWrite>
 static void launch_motion_drops(cleo_ctx* c, const MotionArgs& a, unsigned nb);
 static void launch_gather_move(cleo_ctx* c, const NsortArgs& n, const MotionArgs& m);
@@ -1647,30 +1742,18 @@ static inline unsigned stride_blocks(uint64_t n) {
   const uint64_t b = (n + 255) / 256;
   return static_cast<unsigned>(b == 0 ? 1 : (b > 65536 ? 65536 : b));
 }
-// blocks of a grid-stride loop that usually has little or nothing to do: a launch guarded by a
-// device flag that is mostly clear (the re-sort after collisions), or the out-of-domain tail.
+// blocks of a grid-stride loop that usually has nothing to do (the re-sort after collisions).
 // 2048 blocks of 256 threads still fill every CU when the work is there; a launch of many
 // thousands of blocks that exit at once costs tens of microseconds.
 static inline unsigned sparse_blocks(uint64_t n) { return std::min<unsigned>(stride_blocks(n), 2048u); }
 
-__global__ void k_set_u32(uint32_t* out, uint32_t v, const uint32_t* flag) {
-  if (guard_off(flag)) return;
-  *out = v;
-}
+__global__ void k_set_u32(uint32_t* out, uint32_t v) { *out = v; }
 
 // supersaturation ratio and diffusion factor of every gridbox (thread per gridbox) for
 // k_condensation: the correctly rounded exp of the saturation pressure, evaluated here, would
 // otherwise cost the per-gridbox solve kernel its registers
 __global__ void k_gbx_thermo(GState st, uint32_t ngbx, double* gs) {
-  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < ngbx; g += gridDim.x * blockDim.x) {
-    const double temp = st.temp[g], press = st.press[g];
-    const double psat = saturation_pressure(temp);
-    gs[kGsStride * g] = supersaturation_ratio(press, st.qv[g], psat);
-    gs[kGsStride * g + 1] = diffusion_factor(press, temp, psat);
-    const double akoh = kohler_a(temp);
-    gs[kGsStride * g + 2] = akoh;
-    gs[kGsStride * g + 3] = rcp_nr(akoh);
-  }
+  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < ngbx; g += gridDim.x * blockDim.x) gbx_thermo(st, g, gs);
 }
 void launch_condensation(cleo_ctx* c, const CondArgs& args) {
   if (args.ngbx == 0) return;
@@ -1746,20 +1829,13 @@ void launch_motion(cleo_ctx* c, const MotionArgs& args) {
   MotionArgs a = args;
   const unsigned nb = gbx_blocks(a.grid.ngbx, a.wpb, c->tiles.motion_grid_waves);
   a.stat = stat_slots(c);
-  hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * a.grid.ngbx)), dim3(256), 0, c->stream, a.cnt,
-                     28ull * a.grid.ngbx, 0u);
   kev_mark(c, 0);
   hipLaunchKernelGGL(k_motion, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
   kev_mark(c, 1);
 }
 StatSlots stat_slots(cleo_ctx* c) { return StatSlots{c->sp}; }
-void launch_advance_event(cleo_ctx* c) { hipLaunchKernelGGL(k_advance_event, dim3(1), dim3(1), 0, c->stream, c->ctl); }
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np) {
   hipLaunchKernelGGL(k_inj_sizes, dim3(nblocks(c->grid.ngbx, 256)), dim3(256), 0, c->stream, c->nact, c->grid.ngbx, nj, np);
-}
-void launch_copy_oob_region(cleo_ctx* c, int src, int dst) {
-  hipLaunchKernelGGL(k_copy_oob_region, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, c->buf[src],
-                     c->buf[dst], c->off, c->grid.ngbx, c->ntot);
 }
 
 static size_t scan_words_rec(uint64_t len) {
@@ -1770,117 +1846,85 @@ static size_t scan_words_rec(uint64_t len) {
 size_t scan_tmp_words(uint64_t len) { return scan_words_rec(len) + 16; }
 
 static void scan_rec(hipStream_t stream, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset,
-                     uint32_t* out, const uint32_t* flag, uint32_t* tmp) {
+                     uint32_t* out, uint32_t* tmp) {
   if (len == 0) {
-    hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, stream, out, 0u, flag);
+    hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, stream, out, 0u);
     return;
   }
   const uint64_t nb = (len + kScanTile - 1) / kScanTile;
   if (nb == 1) {
     hipLaunchKernelGGL(k_scan_apply, dim3(1), dim3(kScanThreads), 0, stream, in, len, stride, offset,
-                       static_cast<const uint32_t*>(nullptr), out, flag);
+                       static_cast<const uint32_t*>(nullptr), out);
     return;
   }
   uint32_t* partial = tmp;
   uint32_t* pscan = tmp + nb;
   hipLaunchKernelGGL(k_scan_reduce, dim3(static_cast<unsigned>(nb)), dim3(kScanThreads), 0, stream, in, len, stride,
-                     offset, partial, flag);
-  scan_rec(stream, partial, nb, 1u, 0u, pscan, flag, tmp + nb + nb + 1);
+                     offset, partial);
+  scan_rec(stream, partial, nb, 1u, 0u, pscan, tmp + nb + nb + 1);
   hipLaunchKernelGGL(k_scan_apply, dim3(static_cast<unsigned>(nb)), dim3(kScanThreads), 0, stream, in, len, stride,
-                     offset, static_cast<const uint32_t*>(pscan), out, flag);
+                     offset, static_cast<const uint32_t*>(pscan), out);
 }
-void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset, uint32_t* out,
-              const uint32_t* flag) {
-  scan_rec(c->stream, in, len, stride, offset, out, flag, c->scan_tmp);
+void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset, uint32_t* out) {
+  scan_rec(c->stream, in, len, stride, offset, out, c->scan_tmp);
 }
 
 // argument block of the neighbour-sort kernels reading `src` and writing `dst`
-static NsortArgs nsort_args(cleo_ctx* c, const SoA& src, const SoA& dst, const uint32_t* flag) {
+static NsortArgs nsort_args(cleo_ctx* c, const SoA& src, const SoA& dst) {
   NsortArgs a{};
   a.src = src;
   a.dst = dst;
   a.off = c->off;
-  a.base = c->off_alt;
+  a.off_new = c->off_alt;
+  a.nact = c->nact;
   a.cnt = c->cnt;
   a.runs = c->cnt + 28ull * c->grid.ngbx;
-  a.oobpre = c->oobpre;
   a.tot = c->tot;
-  a.oobcnt = c->oobcnt;
+  a.oobpre = c->oobpre;
+  a.part = c->part;
+  a.nblk = nblocks(c->grid.ngbx, kTabBlock);
   a.grid = c->grid;
   a.wpb = c->tiles.motion_waves_per_block ? c->tiles.motion_waves_per_block : 1;
   a.ctl = c->ctl;
-  a.flag = flag;
   a.ntot = c->ntot;
   a.perm = c->perm;
   a.order = c->order_live ? c->order : nullptr;
   return a;
 }
-// the drops of the domain to their sorted places: destinations, then the records
-static void nsort_move(cleo_ctx* c, const NsortArgs& a) {
-  const uint32_t ngbx = c->grid.ngbx;
-  launch_nsort_perm(c, a, ngbx);
-  // streaming copy: one pair of positions per thread (measured faster than a capped grid), except
-  // under a device flag that is mostly clear
-  const unsigned nb = a.flag ? sparse_blocks(c->ntot) : motion_blocks(c->ntot, 0);
-  hipLaunchKernelGGL(k_nsort_gather, dim3(nb), dim3(256), 0, c->stream, a);
+// totals per destination, run offsets and the prefixes they start from; with `gs`, the condensation
+// inputs of every gridbox too
+static void nsort_tables(cleo_ctx* c, const NsortArgs& a, double* gs = nullptr) {
+  if (gs)
+    hipLaunchKernelGGL(k_nsort_tot<true>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a, c->st, gs);
+  else
+    hipLaunchKernelGGL(k_nsort_tot<false>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a, GState{}, gs);
+  if (a.nblk > 1) hipLaunchKernelGGL(k_nsort_part, dim3(1), dim3(1024), 0, c->stream, a.part, a.nblk);
 }
-// totals per destination, start offsets in the count table, new refs and the out-of-domain prefix
-static void nsort_tables(cleo_ctx* c, const NsortArgs& a, const uint32_t* flag) {
-  const uint32_t ngbx = c->grid.ngbx;
-  hipLaunchKernelGGL(k_nsort_tot, dim3(nblocks(ngbx, 256)), dim3(256), 0, c->stream, a);
-  scan_u32(c, c->tot, ngbx, 1u, 0u, c->off_alt, flag);
-  scan_u32(c, c->oobcnt, ngbx, 1u, 0u, c->oobpre, flag);
-}
-// the sorted store in buffer `dst` becomes current: refs and active counts follow
+// the sorted store in buffer `dst` becomes current, with the refs its sort wrote
 static void nsort_commit(cleo_ctx* c, int dst) {
-  const uint32_t ngbx = c->grid.ngbx;
   c->cur = dst;
   c->order_live = false;  // the sorted store is in its logical order
-  hipLaunchKernelGGL(k_copy_u32, dim3(stride_blocks(ngbx + 1ull)), dim3(256), 0, c->stream, c->off_alt, c->off,
-                     ngbx + 1ull, static_cast<const uint32_t*>(nullptr));
-  hipLaunchKernelGGL(k_set_nact, dim3(nblocks(ngbx, 256)), dim3(256), 0, c->stream, c->off, ngbx, c->nact,
-                     static_cast<const uint32_t*>(nullptr));
+  std::swap(c->off, c->off_alt);
 }
 
 void neighbour_sort_to(cleo_ctx* c, const SoA& src, const SoA& dst, int commit_dst, const uint8_t* step) {
-  const uint32_t ngbx = c->grid.ngbx;
-  NsortArgs a = nsort_args(c, src, dst, nullptr);
+  NsortArgs a = nsort_args(c, src, dst);
   a.step = step;
-  nsort_tables(c, a, nullptr);
-  nsort_move(c, a);
-  hipLaunchKernelGGL(k_nsort_oob, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, a, c->ntot);
-  hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, static_cast<const uint32_t*>(nullptr));
+  nsort_tables(c, a);
+  launch_nsort_perm(c, a, c->grid.ngbx);
+  // streaming copy: one pair of positions per thread (measured faster than a capped grid)
+  hipLaunchKernelGGL(k_nsort_gather, dim3(motion_blocks(c->ntot, 0)), dim3(256), 0, c->stream, a);
   if (commit_dst >= 0) nsort_commit(c, commit_dst);
 }
 
-void neighbour_sort(cleo_ctx* c, int src, int dst, const uint32_t* flag, bool from_nact, const uint8_t* step) {
-  if (flag == nullptr && !from_nact) {
-    neighbour_sort_to(c, c->buf[src], c->buf[dst], dst, step);
-    return;
-  }
+void resort_nulls(cleo_ctx* c, uint32_t events) {
   const uint32_t ngbx = c->grid.ngbx;
-  NsortArgs a = nsort_args(c, c->buf[src], c->buf[dst], flag);
-  if (from_nact) {
-    const unsigned nb = flag ? sparse_blocks(28ull * ngbx) : nblocks(28ull * ngbx, 256);
-    hipLaunchKernelGGL(k_cnt_from_nact, dim3(nb), dim3(256), 0, c->stream, c->off, c->nact, ngbx, c->cnt, flag);
-  }
-  nsort_tables(c, a, flag);
-  nsort_move(c, a);
-  hipLaunchKernelGGL(k_nsort_oob, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, a, c->ntot);
-  hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, flag);
-  if (flag == nullptr) {
-    nsort_commit(c, dst);
-  } else {
-    hipLaunchKernelGGL(k_copy_soa, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, c->buf[dst], c->buf[src],
-                       0ull, c->ntot, flag);
-    // the copied-back store is in its logical order: if the sort ran, the order becomes the identity
-    if (c->order_live)
-      hipLaunchKernelGGL(k_iota_u32, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, c->order, c->ntot, flag);
-    hipLaunchKernelGGL(k_copy_u32, dim3(stride_blocks(ngbx + 1ull)), dim3(256), 0, c->stream, c->off_alt, c->off,
-                       ngbx + 1ull, flag);
-    hipLaunchKernelGGL(k_set_nact, dim3(nblocks(ngbx, 256)), dim3(256), 0, c->stream, c->off, ngbx, c->nact, flag);
-    hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, c->stream, c->ctl);
-  }
+  const SoA &s = c->buf[c->cur], &t = c->buf[1 - c->cur];
+  hipLaunchKernelGGL(k_resort_plan, dim3(1), dim3(1024), 0, c->stream, c->ctl, c->off, c->nact, ngbx, c->off_alt, events);
+  hipLaunchKernelGGL(k_resort_gather, dim3(sparse_blocks(64ull * ngbx)), dim3(256), 0, c->stream, c->ctl, s, t, c->off,
+                     c->nact, c->off_alt, ngbx, c->order);
+  hipLaunchKernelGGL(k_resort_back, dim3(sparse_blocks(std::max<uint64_t>(c->ntot, ngbx + 1ull))), dim3(256), 0, c->stream,
+                     c->ctl, t, s, c->off, c->nact, c->off_alt, ngbx, c->order);
 }
 
 // A pending collision order applied: the domain's drops are gathered into the other buffer in
@@ -1888,17 +1932,15 @@ void neighbour_sort(cleo_ctx* c, int src, int dst, const uint32_t* flag, bool fr
 // current.  Nothing happens when the store is already in order.
 // the store as it is, with the identity as its pending order
 void pending_identity_order(cleo_ctx* c) {
-  hipLaunchKernelGGL(k_iota_u32, dim3(stride_blocks(c->ntot)), dim3(256), 0, c->stream, c->order, c->ntot,
-                     static_cast<const uint32_t*>(nullptr));
+  hipLaunchKernelGGL(k_iota_u32, dim3(stride_blocks(c->ntot)), dim3(256), 0, c->stream, c->order, c->ntot);
   c->order_live = true;
 }
 void materialize_order(cleo_ctx* c) {
   if (!c->order_live) return;
   const int src = c->cur, dst = 1 - c->cur;
-  NsortArgs a = nsort_args(c, c->buf[src], c->buf[dst], nullptr);
+  NsortArgs a = nsort_args(c, c->buf[src], c->buf[dst]);
   a.perm = c->order;
   hipLaunchKernelGGL(k_nsort_gather, dim3(motion_blocks(c->ntot, 0)), dim3(256), 0, c->stream, a);
-  launch_copy_oob_region(c, src, dst);
   c->cur = dst;
   c->order_live = false;
 }
@@ -1909,18 +1951,15 @@ void materialize_order(cleo_ctx* c) {
 void motion_sort_fused(cleo_ctx* c, const MotionArgs& args, const SoA& dst, int commit_dst) {
   const uint32_t ngbx = c->grid.ngbx;
   MotionArgs a = args;
-  hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * ngbx)), dim3(256), 0, c->stream, a.cnt, 28ull * ngbx, 0u);
   const unsigned nb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
   a.stat = stat_slots(c);
   launch_motion_drops<false>(c, a, nb);
-  NsortArgs n = nsort_args(c, a.s, dst, nullptr);
-  nsort_tables(c, n, nullptr);
+  NsortArgs n = nsort_args(c, a.s, dst);
+  nsort_tables(c, n);
   kev_mark(c, 0);
   hipLaunchKernelGGL(k_motion_scatter, dim3(gbx_blocks(ngbx, n.wpb, c->tiles.motion_grid_waves)), dim3(64 * n.wpb), 0,
                      c->stream, a, n);
   kev_mark(c, 1);
-  hipLaunchKernelGGL(k_nsort_oob, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, n, c->ntot);
-  hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, static_cast<const uint32_t*>(nullptr));
   if (commit_dst >= 0) nsort_commit(c, commit_dst);
 }
 
@@ -1933,19 +1972,16 @@ void motion_sort_gather(cleo_ctx* c, const MotionArgs& args, const SoA& dst, int
   if (ngbx == 0) return;
   MotionArgs a = args;
   a.step = c->dstep;
-  hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * ngbx)), dim3(256), 0, c->stream, a.cnt, 28ull * ngbx, 0u);
   const unsigned nb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
   a.stat = stat_slots(c);
   kev_mark(c, 0);
   launch_motion_drops<false>(c, a, nb);
   kev_mark(c, 1);
-  NsortArgs n = nsort_args(c, a.s, dst, nullptr);
+  NsortArgs n = nsort_args(c, a.s, dst);
   n.step = c->dstep;
-  nsort_tables(c, n, nullptr);
+  nsort_tables(c, n);
   launch_nsort_perm(c, n, ngbx);
   launch_gather_move(c, n, a);
-  hipLaunchKernelGGL(k_nsort_oob, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, n, c->ntot);
-  hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, static_cast<const uint32_t*>(nullptr));
   if (commit_dst >= 0) nsort_commit(c, commit_dst);
 }
 
@@ -1985,7 +2021,7 @@ void radix_sort_soa(hipStream_t stream, const SoA& src, const SoA& dst, uint64_t
   for (int p = 0; p < passes; ++p) {
     const int shift = 4 * p;
     hipLaunchKernelGGL(k_rs_count, dim3(ntiles), dim3(256), 0, stream, sc.key[cur], n, shift, ntiles, counts);
-    scan_rec(stream, counts, 16ull * ntiles, 1u, 0u, offs, nullptr, sc.scan_tmp);
+    scan_rec(stream, counts, 16ull * ntiles, 1u, 0u, offs, sc.scan_tmp);
     hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(256), 0, stream, sc.key[cur], sc.idx[cur], n, shift, ntiles,
                        static_cast<const uint32_t*>(offs), sc.key[1 - cur], sc.idx[1 - cur]);
     cur = 1 - cur;
@@ -2009,9 +2045,7 @@ void generic_sort(cleo_ctx* c) {
   sc.scan_tmp = c->scan_tmp;
   radix_sort_soa(c->stream, c->buf[src], c->buf[dst], n, ngbx, c->off, sc);
   if (n > 0) c->cur = dst;
-  hipLaunchKernelGGL(k_set_nact, dim3(nblocks(ngbx, 256)), dim3(256), 0, c->stream, c->off, ngbx, c->nact,
-                     static_cast<const uint32_t*>(nullptr));
-  hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, static_cast<const uint32_t*>(nullptr));
+  hipLaunchKernelGGL(k_set_nact, dim3(nblocks(ngbx, 256)), dim3(256), 0, c->stream, c->off, ngbx, c->nact, c->ctl);
 }
 
 }  // namespace cleo
@@ -2043,12 +2077,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_prep(CondFlatArg
         a.st.qc[g] = rho_cond / dry_air_density(press, temp, qv);
       }
       if (temp <= 0) set_error(a.ctl, CLEO_ERR_TEMP_NONPOSITIVE, g, a.off[g]);
-      const double psat = saturation_pressure(temp);
-      a.gs[kGsStride * g] = supersaturation_ratio(press, qv, psat);
-      a.gs[kGsStride * g + 1] = diffusion_factor(press, temp, psat);
-      const double akoh = kohler_a(temp);
-      a.gs[kGsStride * g + 2] = akoh;
-      a.gs[kGsStride * g + 3] = rcp_nr(akoh);
+      gbx_thermo(a.st, g, a.gs);
     }
   }
 }
@@ -2338,6 +2367,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gath
     }
   }
   finish_deferred<kTail>(a, &ndef, a.dlist + q_lo, st);
+  copy_oob(n, nsrc);
   put_cond_stats(a.stat, st);
 }
 
@@ -2773,18 +2803,11 @@ void launch_thermo_eval(cleo_ctx* c, uint64_t n, const double* temp, const doubl
                      s_ratio, ffactor);
 }
 
-// p[i] = i for i < n, skipped unless *flag when flag is non-null
-__global__ void k_iota_u32(uint32_t* p, uint64_t n, const uint32_t* flag) {
-  if (flag && *flag == 0u) return;
+// p[i] = i for i < n
+__global__ void k_iota_u32(uint32_t* p, uint64_t n) {
   for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
     p[i] = static_cast<uint32_t>(i);
-}
-
-__global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
-  for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
-    p[i] = v;
 }
 
 // count-table key of a moved drop: 28*d + step for destination d, 28*g + 27 when it left the domain
@@ -2914,6 +2937,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_nsort_gather_move(Nso
     n.dst.msol[q] = n.src.msol[p];
     n.dst.id[q] = n.src.id[p];
   }
+  copy_oob(n, nsrc);
 }
 static void launch_gather_move(cleo_ctx* c, const NsortArgs& n, const MotionArgs& m) {
   const uint32_t nb_ = m.grid.nz + m.grid.nx + m.grid.ny + 3;
@@ -3016,18 +3040,16 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   const bool on = c->kev_on;
   c->kev_on = false;  // the main kernel of this sequence is the gather with the solves
   if (move_in_gather) {
-    hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * ngbx)), dim3(256), 0, c->stream, m.cnt, 28ull * ngbx,
-                       0u);
-    const unsigned mb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
+      const unsigned mb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
     m.stat = stat_slots(c);
     launch_motion_drops<false>(c, m, mb);
   } else {
     launch_motion_flat(c, m);
   }
   c->kev_on = on;
-  NsortArgs n = nsort_args(c, m.s, dst, nullptr);
+  NsortArgs n = nsort_args(c, m.s, dst);
   n.step = c->dstep;
-  nsort_tables(c, n, nullptr);
+  nsort_tables(c, n, cond.gs);
   launch_nsort_perm(c, n, ngbx);
   CondFlatArgs a = cond;
   a.s = dst;
@@ -3038,7 +3060,6 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   a.cfg.budget = budget;
   a.dlist = c->dlist;
   a.dcount = c->dcount;
-  hipLaunchKernelGGL(k_cond_prep, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
   if (a.mlp_inline) {  // learned guesses of the drops where motion left them
     CondFlatArgs ga = a;
     ga.s = m.s;
@@ -3058,9 +3079,10 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
     launch_gather_cond<false>(c, n, a, move_in_gather ? &m : nullptr, nb);
   kev_mark(c, 1);
   if (!tail) launch_deferred(c, a, nb);
-  hipLaunchKernelGGL(k_nsort_oob, dim3(sparse_blocks(c->ntot)), dim3(256), 0, c->stream, n, c->ntot);
-  hipLaunchKernelGGL(k_sorts_stat, dim3(1), dim3(1), 0, c->stream, c->ctl, static_cast<const uint32_t*>(nullptr));
-  if (commit_dst >= 0) nsort_commit(c, commit_dst);
+  if (commit_dst >= 0) {
+    nsort_commit(c, commit_dst);
+    a.off = c->off;  // the sorted store's refs
+  }
   hipLaunchKernelGGL(k_cond_state, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
 }
 
@@ -3069,8 +3091,6 @@ void launch_motion_flat(cleo_ctx* c, const MotionArgs& args) {
   MotionArgs a = args;
   const unsigned nb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
   a.stat = stat_slots(c);
-  hipLaunchKernelGGL(k_fill_u32, dim3(stride_blocks(28ull * a.grid.ngbx)), dim3(256), 0, c->stream, a.cnt,
-                     28ull * a.grid.ngbx, 0u);
   kev_mark(c, 0);
   launch_motion_drops<true>(c, a, nb);
   kev_mark(c, 1);

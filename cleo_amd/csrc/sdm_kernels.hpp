@@ -18,6 +18,8 @@ constexpr uint32_t kCondQueueWavesPerCu = 12;
 // per-gridbox condensation inputs in gs: saturation ratio, diffusion factor, Koehler a and its
 // refined reciprocal (one 32-byte line each)
 constexpr uint32_t kGsStride = 4;
+// gridboxes whose sort totals are scanned together (threads of k_nsort_tot)
+constexpr uint32_t kTabBlock = 256;
 // LDS window (values) of the per-gridbox drop-order sums
 constexpr uint32_t kSumWin = 1024;
 
@@ -65,6 +67,7 @@ struct CollArgs {
   uint32_t wpb;
   DevCtl* ctl;
   uint64_t seed;
+  uint64_t event_ofs;  // this event's number after ctl->event
   const uint32_t* inj_j;
   const double* inj_phi;
   const uint32_t* inj_oj;
@@ -90,17 +93,18 @@ struct MotionArgs {
 
 struct NsortArgs {
   SoA src, dst;
-  const uint32_t* off;     // current refs (ngbx+1)
-  const uint32_t* base;    // new refs (ngbx+1)
-  uint32_t* cnt;           // ngbx*28: arrivals per (destination, step)
-  uint32_t* runs;          // ngbx*28: per (source, step) the run's offset among its destination's arrivals
-  const uint32_t* oobpre;  // ngbx+1
-  uint32_t* tot;
-  uint32_t* oobcnt;        // ngbx: drops of each gridbox that leave the domain (row d's last count)
+  const uint32_t* off;  // current refs (ngbx+1)
+  uint32_t* off_new;    // refs of the sorted store (ngbx+1), written by the rank pass
+  uint32_t* nact;       // the sorted store's drops per gridbox
+  uint32_t* cnt;        // ngbx*28: arrivals per (destination, step); left zero by k_nsort_tot
+  uint32_t* runs;       // ngbx*28: per (source, step) the run's offset among its destination's arrivals
+  uint32_t* tot;        // ngbx+1: arrivals before each destination in its block of kTabBlock; tot[ngbx] = 0
+  uint32_t* oobpre;     // ngbx: drops leaving the domain before each gridbox in its block
+  uint32_t* part;       // nblk pairs: both sums before each block; then the sorted store's domain drops
+  uint32_t nblk;
   Grid grid;
   uint32_t wpb;
   DevCtl* ctl;
-  const uint32_t* flag;    // non-null: skip unless *flag
   uint64_t ntot;
   uint32_t* perm;          // source position of each destination position of the domain's drops
   const uint8_t* step;     // non-null: each drop's step from motion, read instead of its key
@@ -151,18 +155,15 @@ void launch_condensation(cleo_ctx* c, const CondArgs& a);
 void launch_qcond(cleo_ctx* c, const QcondArgs& a);
 void launch_collisions(cleo_ctx* c, const CollArgs& a);
 void launch_motion(cleo_ctx* c, const MotionArgs& a);
-void launch_advance_event(cleo_ctx* c);
 // the statistics rows of the context
 StatSlots stat_slots(cleo_ctx* c);
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np);
 // exclusive scan of in[i*stride+offset], i < len, into out[0..len] (out[len] = total)
-void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset, uint32_t* out,
-              const uint32_t* flag);
+void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset, uint32_t* out);
 size_t scan_tmp_words(uint64_t len);
-// stable neighbour sort of buf[src] into buf[dst] after motion (flag == nullptr) or after
-// collisions (flag = &ctl->resort_flag, data ends back in buf[src] and refs in c->off)
-void neighbour_sort(cleo_ctx* c, int src, int dst, const uint32_t* flag, bool from_nact,
-                    const uint8_t* step = nullptr);
+// after the collision events of a microphysics pass (which leave a pending order): the event counter
+// moves on by `events`, and if nulls appeared the store is sorted again (SDMMethods, sdmmethods.hpp:213-230)
+void resort_nulls(cleo_ctx* c, uint32_t events);
 // the neighbour sort of `src` (after motion) into `dst`; commit_dst >= 0: that buffer becomes current
 void neighbour_sort_to(cleo_ctx* c, const SoA& src, const SoA& dst, int commit_dst, const uint8_t* step = nullptr);
 // motion + neighbour sort + a condensation that follows at once, the solve in the sort's gather
@@ -189,7 +190,6 @@ uint64_t radix_scratch_words(uint64_t n);
 RadixScratch radix_scratch_at(uint32_t* base, uint64_t n);
 void radix_sort_soa(hipStream_t stream, const SoA& src, const SoA& dst, uint64_t n, uint32_t ngbx, uint32_t* off,
                     const RadixScratch& sc);
-void launch_copy_oob_region(cleo_ctx* c, int src, int dst);
 // applies a pending collision order to the store (buf[cur] then holds the drops in order)
 void materialize_order(cleo_ctx* c);
 // 0th, 1st and 2nd mass moments of every gridbox into device arrays of ngbx entries (raindrops
