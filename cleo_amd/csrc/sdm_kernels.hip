@@ -13,7 +13,26 @@
 namespace cleo {
 
 // ============================ per-gridbox sums ================================================
-// Drop-order sums of v(k) over [lo, lo + len) for the gridboxes of a tile of 64 (lane i passes its
+// A wave sums a tile of `gpt` consecutive gridboxes, one per lane (at most 64).  Its lanes add their
+// gridboxes' values one after the other, so a tile takes the time of its drops' loads plus its longest
+// sum; tiles of 64 gridboxes leave most of the chip idle below half a million gridboxes (sum_gpt).
+__host__ __device__ __forceinline__ uint32_t sum_tiles(uint32_t ngbx, uint32_t gpt) { return (ngbx + gpt - 1) / gpt; }
+// acc + v[i0] + v[i0+1] + ... + v[i1-1], left to right, eight LDS reads in flight at a time (a read per
+// add waits about 100 cycles for each value)
+template <class T>
+__device__ __forceinline__ T add_in_order(T acc, const T* v, uint32_t i0, uint32_t i1) {
+  uint32_t i = i0;
+  for (; i + 8 <= i1; i += 8) {
+    T r[8];
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) r[j] = v[i + j];
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) acc += r[j];
+  }
+  for (; i < i1; ++i) acc += v[i];
+  return acc;
+}
+// Drop-order sums of v(k) over [lo, lo + len) for the gridboxes of a tile (lane i passes its
 // own gridbox's range and gets its sum).  The tile's drops [t_lo, t_hi) are staged through an LDS
 // window of kSumWin values with coalesced loads (the next window's loads in flight while the current
 // one is added); each lane then adds its gridbox's values left to right, exactly as a serial loop
@@ -37,7 +56,7 @@ __device__ __forceinline__ double tile_sum(double* win, uint32_t t_lo, uint32_t 
     wave_sync();
     if (we < t_hi) load(we);
     const uint32_t a0 = max(lo, w), a1 = min(lo + len, we);
-    for (uint32_t k = a0; k < a1; ++k) acc += win[k - w];
+    if (a0 < a1) acc = add_in_order(acc, win, a0 - w, a1 - w);
     wave_sync();
   }
   return acc;
@@ -74,9 +93,9 @@ __device__ __forceinline__ void tile_sum2(double* win, uint32_t t_lo, uint32_t t
     wave_sync();
     if (we < t_hi) load(we);
     const uint32_t b0 = max(lo, w), b1 = min(lo + len, we);
-    for (uint32_t k = b0; k < b1; ++k) {
-      a1 += win[k - w];
-      a2 += win[kHalf + k - w];
+    if (b0 < b1) {
+      a1 = add_in_order(a1, win, b0 - w, b1 - w);
+      a2 = add_in_order(a2, win + kHalf, b0 - w, b1 - w);
     }
     wave_sync();
   }
@@ -196,11 +215,11 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_qcond(QcondArgs a) {
   __shared__ double win_all[4][kSumWin];
   double* win = win_all[threadIdx.x >> 6];
   const int lane = lane_id();
-  const uint32_t ntiles = (a.ngbx + kWave - 1) / kWave;
+  const uint32_t gpt = a.gpt, ntiles = sum_tiles(a.ngbx, gpt);
   for (uint32_t tile = wave_index(); tile < ntiles; tile += wave_count()) {
-    const uint32_t g0 = tile * kWave, g = g0 + static_cast<uint32_t>(lane);
-    const bool valid = g < a.ngbx;
-    const uint32_t t_lo = a.off[g0], t_hi = a.off[min(g0 + kWave, a.ngbx)];
+    const uint32_t g0 = tile * gpt, g = g0 + static_cast<uint32_t>(lane);
+    const bool valid = static_cast<uint32_t>(lane) < gpt && g < a.ngbx;
+    const uint32_t t_lo = a.off[g0], t_hi = a.off[min(g0 + gpt, a.ngbx)];
     const uint32_t lo = valid ? a.off[g] : t_hi, hi = valid ? a.off[g + 1] : t_hi;
     const double tot = tile_sum(win, t_lo, t_hi, lo, hi - lo, [&](uint32_t k) { return qcond_term(a.s, a.sol, a.ctl, k); },
                                 lane);
@@ -1768,10 +1787,22 @@ void launch_condensation(cleo_ctx* c, const CondArgs& args) {
     hipLaunchKernelGGL(k_condensation<false>, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
   kev_mark(c, 1);
 }
-void launch_qcond(cleo_ctx* c, const QcondArgs& a) {
-  if (a.ngbx == 0) return;
-  hipLaunchKernelGGL(k_qcond, dim3(gbx_blocks((a.ngbx + kWave - 1) / kWave, 4, c->tiles.cond_grid_waves)), dim3(256), 0,
-                     c->stream, a);
+// Gridboxes per tile of the per-gridbox sums: as many as leave 8192 waves, but at least the 512 drops
+// of a window.  Mass moments with 64 / by this rule / 1 gridbox per tile: 32^3 gridboxes of 64 drops
+// 41 / 17 / 51 us, 24679 of 300 drops 478 (at 256 waves) / 96 / 115 us, 3750 of 128 drops 160 / 12 /
+// 14 us; from 64^3 gridboxes on the passes are bound by HBM at any width (134M drops: 0.59 ms).
+static uint32_t sum_gpt(const cleo_ctx* c) {
+  const uint64_t ngbx = c->grid.ngbx, mean = std::max<uint64_t>(1, c->ntot / ngbx);
+  return static_cast<uint32_t>(std::min<uint64_t>(kWave, std::max<uint64_t>({1, ngbx / 8192, 512 / mean})));
+}
+static unsigned sum_blocks(const cleo_ctx* c, uint32_t grid_waves) {
+  return gbx_blocks(sum_tiles(c->grid.ngbx, sum_gpt(c)), 4, grid_waves);
+}
+void launch_qcond(cleo_ctx* c, const QcondArgs& args) {
+  if (args.ngbx == 0) return;
+  QcondArgs a = args;
+  a.gpt = sum_gpt(c);
+  hipLaunchKernelGGL(k_qcond, dim3(sum_blocks(c, c->tiles.cond_grid_waves)), dim3(256), 0, c->stream, a);
 }
 template <int B, bool Kinetic>
 static void launch_coll_team_k(cleo_ctx* c, const CollArgs& a, unsigned nb, uint32_t gpt, uint32_t cap) {
@@ -2059,14 +2090,14 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_prep(CondFlatArg
   __shared__ double win_all[4][kSumWin];
   double* win = win_all[threadIdx.x >> 6];
   const int lane = lane_id();
-  const uint32_t ntiles = (a.ngbx + kWave - 1) / kWave;
+  const uint32_t gpt = a.gpt, ntiles = sum_tiles(a.ngbx, gpt);
   for (uint32_t tile = wave_index(); tile < ntiles; tile += wave_count()) {
-    const uint32_t g0 = tile * kWave, g = g0 + static_cast<uint32_t>(lane);
-    const bool valid = g < a.ngbx;
+    const uint32_t g0 = tile * gpt, g = g0 + static_cast<uint32_t>(lane);
+    const bool valid = static_cast<uint32_t>(lane) < gpt && g < a.ngbx;
     double tot = 0.0;
     const bool qcond_here = a.fuse_qcond && !a.qm;  // else k_cond_state recomputes it from qm
     if (qcond_here) {
-      const uint32_t t_lo = a.off[g0], t_hi = a.off[min(g0 + kWave, a.ngbx)];
+      const uint32_t t_lo = a.off[g0], t_hi = a.off[min(g0 + gpt, a.ngbx)];
       const uint32_t lo = valid ? a.off[g] : t_hi, hi = valid ? a.off[g + 1] : t_hi;
       tot = tile_sum(win, t_lo, t_hi, lo, hi - lo, [&](uint32_t k) { return qcond_term(a.s, a.sol, a.ctl, k); }, lane);
     }
@@ -2618,11 +2649,11 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_state(CondFlatAr
   __shared__ double win_all[4][kSumWin];
   double* win = win_all[threadIdx.x >> 6];
   const int lane = lane_id();
-  const uint32_t ntiles = (a.ngbx + kWave - 1) / kWave;
+  const uint32_t gpt = a.gpt, ntiles = sum_tiles(a.ngbx, gpt);
   for (uint32_t tile = wave_index(); tile < ntiles; tile += wave_count()) {
-    const uint32_t g0 = tile * kWave, g = g0 + static_cast<uint32_t>(lane);
-    const bool valid = g < a.ngbx;
-    const uint32_t t_lo = a.off[g0], t_hi = a.off[min(g0 + kWave, a.ngbx)];
+    const uint32_t g0 = tile * gpt, g = g0 + static_cast<uint32_t>(lane);
+    const bool valid = static_cast<uint32_t>(lane) < gpt && g < a.ngbx;
+    const uint32_t t_lo = a.off[g0], t_hi = a.off[min(g0 + gpt, a.ngbx)];
     const uint32_t lo = valid ? a.off[g] : t_hi, n = valid ? a.nact[g] : 0u;
     double qc_new = 0.0, tot = 0.0;
     if (a.qm) {
@@ -2693,15 +2724,15 @@ void launch_receive_dynamics(cleo_ctx* c, const cleo_dynamics_step& dyn) {
 
 // ============================ observers =======================================================
 // Mass moments per gridbox (observers/massmoments_observer.cpp:23-73): one lane per gridbox of a
-// 64-gridbox tile.  The tile's drops pass through an LDS window with coalesced loads (the next
+// tile.  The tile's drops pass through an LDS window with coalesced loads (the next
 // window's loads in flight while the current one is added); the loading lane turns each drop into
 // its three terms (xi; (float)(xi m); (float)(xi m m), m the drop mass,
 // zero for a drop below the raindrop radius when kRain), and each lane then adds its gridbox's
 // terms left to right, so the float sums are the reference's serial ones.
 constexpr uint32_t kMomWin = 512;
 template <bool kRain>
-__global__ void __launch_bounds__(256) k_mass_moments(SoA s, const uint32_t* off, uint32_t ngbx, Solute sol,
-                                                      DevCtl* ctl, uint64_t* mom0, float* mom1, float* mom2) {
+__global__ void __launch_bounds__(256) k_mass_moments(SoA s, const uint32_t* off, uint32_t ngbx, uint32_t gpt,
+                                                      Solute sol, DevCtl* ctl, uint64_t* mom0, float* mom1, float* mom2) {
   __shared__ uint64_t w0_all[4][kMomWin];
   __shared__ float w1_all[4][kMomWin], w2_all[4][kMomWin];
   const uint32_t wv = threadIdx.x >> 6;
@@ -2710,11 +2741,11 @@ __global__ void __launch_bounds__(256) k_mass_moments(SoA s, const uint32_t* off
   float* w2 = w2_all[wv];
   const int lane = lane_id();
   constexpr double rlim(40e-6 / dimless::R0);  // calculate_rainmassmoments: raindrop radius
-  const uint32_t ntiles = (ngbx + kWave - 1) / kWave;
+  const uint32_t ntiles = sum_tiles(ngbx, gpt);
   for (uint32_t tile = wave_index(); tile < ntiles; tile += wave_count()) {
-    const uint32_t g0 = tile * kWave, g = g0 + static_cast<uint32_t>(lane);
-    const bool valid = g < ngbx;
-    const uint32_t t_lo = off[g0], t_hi = off[min(g0 + kWave, ngbx)];
+    const uint32_t g0 = tile * gpt, g = g0 + static_cast<uint32_t>(lane);
+    const bool valid = static_cast<uint32_t>(lane) < gpt && g < ngbx;
+    const uint32_t t_lo = off[g0], t_hi = off[min(g0 + gpt, ngbx)];
     const uint32_t lo = valid ? off[g] : t_hi, hi = valid ? off[g + 1] : t_hi;
     uint64_t m0 = 0;
     float m1 = 0.f, m2 = 0.f;
@@ -2757,10 +2788,10 @@ __global__ void __launch_bounds__(256) k_mass_moments(SoA s, const uint32_t* off
       wave_sync();
       if (we < t_hi) load(we);
       const uint32_t b0 = max(lo, w), b1 = min(hi, we);
-      for (uint32_t k = b0; k < b1; ++k) {
-        m0 += w0[k - w];
-        m1 += w1[k - w];
-        m2 += w2[k - w];
+      if (b0 < b1) {
+        m0 = add_in_order(m0, w0, b0 - w, b1 - w);
+        m1 = add_in_order(m1, w1, b0 - w, b1 - w);
+        m2 = add_in_order(m2, w2, b0 - w, b1 - w);
       }
       wave_sync();
     }
@@ -2775,13 +2806,13 @@ void launch_mass_moments(cleo_ctx* c, bool rain, uint64_t* mom0, float* mom1, fl
   const uint32_t ngbx = c->grid.ngbx;
   if (ngbx == 0) return;
   materialize_order(c);  // the sums follow the drops' logical order
-  const uint64_t ntiles = (ngbx + kWave - 1) / kWave;
-  const unsigned nb = gbx_blocks(ntiles, 4, 0);
+  const uint32_t gpt = sum_gpt(c);
+  const unsigned nb = sum_blocks(c, 0);
   if (rain)
-    hipLaunchKernelGGL(k_mass_moments<true>, dim3(nb), dim3(256), 0, c->stream, c->buf[c->cur], c->off, ngbx,
+    hipLaunchKernelGGL(k_mass_moments<true>, dim3(nb), dim3(256), 0, c->stream, c->buf[c->cur], c->off, ngbx, gpt,
                        c->solute, c->ctl, mom0, mom1, mom2);
   else
-    hipLaunchKernelGGL(k_mass_moments<false>, dim3(nb), dim3(256), 0, c->stream, c->buf[c->cur], c->off, ngbx,
+    hipLaunchKernelGGL(k_mass_moments<false>, dim3(nb), dim3(256), 0, c->stream, c->buf[c->cur], c->off, ngbx, gpt,
                        c->solute, c->ctl, mom0, mom1, mom2);
 }
 
@@ -2989,12 +3020,12 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
   // joins k_cond_state (the task ring keeps it in k_cond_prep)
   a.qm = (a.fuse_qcond && c->tiles.cond_flat == 1) ? c->qm : nullptr;
   const uint32_t gw = c->tiles.cond_grid_waves;
-  const uint64_t ntiles = (a.ngbx + kWave - 1) / kWave;
+  a.gpt = sum_gpt(c);
   const uint32_t budget = c->tiles.cond_flat == 2 ? 0u : c->tiles.cond_defer;
   a.cfg.budget = budget;
   a.dlist = c->dlist;
   a.dcount = c->dcount;
-  hipLaunchKernelGGL(k_cond_prep, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_cond_prep, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
   if (c->tiles.cond_flat == 2) {
     // task-ring kernel: waves of 4 per block; by default as many waves as fit on the device at once
     const uint64_t waves = gw ? gw : static_cast<uint64_t>(c->num_cu) * kCondQueueWavesPerCu;
@@ -3019,7 +3050,7 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
     if (!tail) launch_deferred(c, a, nb);
     kev_mark(c, 1);
   }
-  hipLaunchKernelGGL(k_cond_state, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_cond_state, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
 }
 
 // Motion, the neighbour sort and a condensation that follows at once, with the condensation solve
@@ -3055,7 +3086,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   a.s = dst;
   a.qm = c->qm;  // the qcond recompute joins k_cond_state
   const uint32_t gw = c->tiles.cond_grid_waves;
-  const uint64_t ntiles = (ngbx + kWave - 1) / kWave;
+  a.gpt = sum_gpt(c);
   const uint32_t budget = c->tiles.cond_defer;
   a.cfg.budget = budget;
   a.dlist = c->dlist;
@@ -3083,7 +3114,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
     nsort_commit(c, commit_dst);
     a.off = c->off;  // the sorted store's refs
   }
-  hipLaunchKernelGGL(k_cond_state, dim3(gbx_blocks(ntiles, 4, gw)), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_cond_state, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
 }
 
 void launch_motion_flat(cleo_ctx* c, const MotionArgs& args) {

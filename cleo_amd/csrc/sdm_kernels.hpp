@@ -50,6 +50,7 @@ struct QcondArgs {
   uint32_t ngbx;
   uint32_t wpb;
   DevCtl* ctl;
+  uint32_t gpt;  // gridboxes per tile of the sums
 };
 
 struct CollArgs {
@@ -146,6 +147,7 @@ struct CondFlatArgs {
   // k_cond_guess on the store as motion left it (before the sort): a drop is active when its new
   // gridbox is in the domain (the refs still describe the unsorted store)
   int32_t unsorted;
+  uint32_t gpt;  // gridboxes per tile of the sums
 };
 
 // launchers (sdm_kernels.hip); all enqueue on ctx->stream
