@@ -84,18 +84,11 @@ int ensure_radix(cleo_ctx* c, uint64_t n) {
     hipFree(c->rs_idx[i]);
   }
   hipFree(c->rs_cnt);
-  const uint64_t ntiles = (n + 255) / 256;
   for (int i = 0; i < 2; ++i) {
     HIP_TRY(c, dalloc(&c->rs_key[i], n));
     HIP_TRY(c, dalloc(&c->rs_idx[i], n));
   }
-  HIP_TRY(c, dalloc(&c->rs_cnt, 32 * ntiles + 1));
-  const size_t need = scan_tmp_words(16 * ntiles);
-  if (need > c->scan_tmp_n) {
-    hipFree(c->scan_tmp);
-    HIP_TRY(c, dalloc(&c->scan_tmp, need));
-    c->scan_tmp_n = need;
-  }
+  HIP_TRY(c, dalloc(&c->rs_cnt, radix_count_words(n)));
   c->rs_n = n;
   return CLEO_OK;
 }

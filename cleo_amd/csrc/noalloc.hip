@@ -1,7 +1,6 @@
 // noalloc.hip -- the entry point of libcleo_hip.so that allocates no device memory:
 // cleo_sort_supers_noalloc, the generic superdroplet sort of cleo_upload_supers_device on
-// caller-owned device arrays.  Its scratch (radix keys, indices, digit counts and the scan's
-// partials) lives in `scratch`, a fixed device array of this file; every GPU the library runs on
+// caller-owned device arrays.  Its scratch (a row per drop, radix keys, indices and digit counts) lives in `scratch`, a fixed device array of this file; every GPU the library runs on
 // holds one copy until the process ends.  Calls that overlap on one GPU share that copy and race.
 #include <hip/hip_runtime.h>
 
@@ -12,9 +11,7 @@
 namespace {
 
 constexpr uint64_t kMaxSupers = CLEO_NOALLOC_MAX_SUPERS;
-// radix_scratch_words(kMaxSupers) = 4 n + 32 ceil(n / 256) + 1 + the scan's partials (a few hundred
-// words); the margin covers the last
-constexpr uint64_t kScratchWords = 4 * kMaxSupers + 32 * ((kMaxSupers + 255) / 256) + 1 + 4096;
+constexpr uint64_t kScratchWords = cleo::radix_scratch_words(kMaxSupers);
 
 __device__ __align__(256) uint32_t scratch[kScratchWords];
 

@@ -321,7 +321,7 @@ int cleo_thermo_eval(cleo_ctx* ctx, uint64_t n, const double* temp, const double
    device SoA `in` to the device SoA `out` (n drops each, not overlapping), with refs (device, ngbx+1
    entries) the first position of each gridbox and refs[ngbx] the in-domain count, enqueued on
    `stream` (a hipStream_t; NULL is the null stream) without synchronising.  No context, no
-   hipMalloc: the scratch is a fixed device array of the library (about 17 MB per GPU, held until the
+   hipMalloc: the scratch is a fixed device array of the library (about 85 MB per GPU, held until the
    process ends), so n <= CLEO_NOALLOC_MAX_SUPERS (CLEO_E_ARG beyond).  Calls that overlap on one GPU
    share that array and race; calls in one stream order themselves. */
 #define CLEO_NOALLOC_MAX_SUPERS (1u << 20)
