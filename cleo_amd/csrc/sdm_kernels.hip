@@ -800,7 +800,9 @@ __device__ __forceinline__ double interpolation(double blo, double bhi, double i
 // One axis of CartesianMaps::get_local_bounding_gridbox_index (cartesianmaps.cpp:68-286,
 // domainboundaries.hpp:34-109): step to the backward/forward neighbour when the coordinate left
 // [lower, upper) and wrap the coordinate at a periodic domain edge.  i is the drop's index along
-// the axis, updated to the neighbour's.  Returns the step taken.
+// the axis, updated to the neighbour's.  Returns the step taken; on a periodic axis of one or two
+// gridboxes several steps lead to one neighbour, and the step is then the change of the index, so that
+// drops with the same source and destination have the same step (the sort places drops by their step).
 __device__ __forceinline__ int axis_step(uint32_t& idx, double& coord, uint32_t& i, uint32_t nd, uint32_t inc,
                                          bool periodic, const double* h) {
   const double lo = h[i], hi = h[i + 1];
@@ -811,6 +813,7 @@ __device__ __forceinline__ int axis_step(uint32_t& idx, double& coord, uint32_t&
         coord = coord + h[nd] - lo;  // lim1 = upper bound of the backward neighbour
         idx = nb;
         i = nd - 1;
+        if (nd <= 2) return static_cast<int>(nd) - 1;
       } else {
         idx = kOOB;
       }
@@ -827,6 +830,7 @@ __device__ __forceinline__ int axis_step(uint32_t& idx, double& coord, uint32_t&
         coord = coord + h[0] - hi;  // lim1 = lower bound of the forward neighbour
         idx = nb;
         i = 0;
+        if (nd <= 2) return 1 - static_cast<int>(nd);
       } else {
         idx = kOOB;
       }
