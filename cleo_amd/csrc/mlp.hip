@@ -27,13 +27,13 @@
 
 namespace cleo {
 
-struct WaveLds {
-  static constexpr bool kHasXs = true;
+struct GradLds {
   float xs[64][kInPad];           // normalised inputs (fp32)
   uint16_t xb[64][kInPad];        // same, bf16 (A operand of layer 1)
   uint16_t h1[64][kH1Stride];     // SiLU(z1), bf16 (A operand of layer 2, B operand of dW2)
   uint16_t dz2[64][kH1Stride];    // dL/dz2, bf16
-  float ys[64];
+  float part[2][16][64];          // layer 3 products on their way to the other wave
+  float ys[64], dy[64];
 };
 
 struct GuessArgs {
@@ -147,136 +147,160 @@ struct TrainArgs {
   float* partial;        // [waves][NPARAM + 1]
 };
 
-// loss gradient of 64 samples (one wave) -> partial[wave]
-__global__ void __launch_bounds__(64) k_mlp_grad(TrainArgs a) {
-  __shared__ WaveLds L;
-  const int lane = lane_id();
+// Loss gradient of 64 samples -> partial[workgroup], by two waves, each with the hidden units of one
+// half (and, in the first layer's gradient, the weights of one half).  Bound by instruction issue and
+// latency, not by its 100 MFMAs: one wave with all 64 units, computing each sigmoid three times over and
+// rounding to bf16 in integer steps, took 30 us a batch of 8192 samples and 40 us of 65536; two waves,
+// the sigmoids kept from the forward pass and hardware rounding take 18.5 and 29 us, with the same
+// results bit for bit.
+__global__ void __launch_bounds__(128) k_mlp_grad(TrainArgs a) {
+  __shared__ GradLds L;
+  const int lane = lane_id(), ni = static_cast<int>(threadIdx.x >> 6);
   const int col = lane % 32;
   const uint32_t s0 = blockIdx.x * 64;
   const bool valid = s0 + lane < a.count;
-  float f[kIn] = {0, 0, 0, 0, 0, 0};
   float t = 0.0f;
-  if (valid) {
-    const uint64_t idx = a.perm ? a.perm[a.first + s0 + lane] : a.first + s0 + lane;
-    for (int j = 0; j < kIn; ++j) f[j] = a.x[idx * kInPad + j];
-    t = (a.y[idx] - a.W.p[P_YMEAN]) / a.W.p[P_YSTD];
+  {
+    float f[kInPad] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (valid) {
+      const uint64_t idx = a.perm ? a.perm[a.first + s0 + lane] : a.first + s0 + lane;
+      for (int j = 0; j < kIn; ++j) f[j] = a.x[idx * kInPad + j];
+      t = (a.y[idx] - a.W.p[P_YMEAN]) / a.W.p[P_YSTD];
+    }
+    if (ni == 0) {
+      for (int k = 0; k < kInPad; ++k) {
+        const float v = k < kIn && valid ? (f[k] - a.W.p[P_XMEAN + k]) / a.W.p[P_XSTD + k] : 0.0f;
+        L.xs[lane][k] = v;
+        L.xb[lane][k] = f2bf(v);
+      }
+    }
   }
-  load_normalised(L, a.W.p, f, valid);
-  f32x16 z1[2][2], z2[2][2];
-  const float yp = mlp_forward_wave(a.W, L, z1, z2);
+  __syncthreads();
+  f32x16 z1[2], s1[2], z2[2], s2[2];
+  const float yp = mlp_forward_pair(a.W, L, ni, z1, s1, z2, s2);
   const float dy = valid ? a.gscale * (yp - t) : 0.0f;
   float* out = a.partial + static_cast<uint64_t>(blockIdx.x) * (NPARAM + 1);
-  // loss partial: sum of squared errors
-  float se = valid ? (yp - t) * (yp - t) : 0.0f;
-  for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o);
-  L.ys[lane] = dy;
-  wave_sync();
-  // dW3, db3, dz2
-  float gw3[2] = {0.0f, 0.0f};
-  float gb2[2] = {0.0f, 0.0f};
-  const float w3v[2] = {a.W.p[P_W3 + col], a.W.p[P_W3 + 32 + col]};
+  if (ni == 0) {
+    L.dy[lane] = dy;
+    // loss partial: sum of squared errors, and db3
+    float se = valid ? (yp - t) * (yp - t) : 0.0f, db3 = dy;
+    for (int o = 32; o > 0; o >>= 1) {
+      se += __shfl_xor(se, o);
+      db3 += __shfl_xor(db3, o);
+    }
+    if (lane == 0) {
+      out[P_B3] = db3;
+      out[NPARAM] = se;
+    }
+  }
+  __syncthreads();
+  // dW3, dz2
+  float gw3 = 0.0f, gb2 = 0.0f;
+  const float w3v = a.W.p[P_W3 + ni * 32 + col];
   for (int mi = 0; mi < 2; ++mi) {
     for (int v = 0; v < 16; ++v) {
       const int s = mi * 32 + drow(v, lane);
-      const float dys = L.ys[s];
-      for (int ni = 0; ni < 2; ++ni) {
-        const float z = z2[mi][ni][v];
-        gw3[ni] += dys * silu(z);
-        const float d = dys * w3v[ni] * dsilu(z);
-        gb2[ni] += d;
-        L.dz2[s][ni * 32 + col] = f2bf(d);
-      }
+      const float dys = L.dy[s], z = z2[mi][v], sg = s2[mi][v];
+      gw3 += dys * (z * sg);
+      const float d = dys * w3v * dsilu(z, sg);
+      gb2 += d;
+      L.dz2[s][ni * 32 + col] = f2bf(d);
     }
   }
-  for (int ni = 0; ni < 2; ++ni) {
-    gw3[ni] += __shfl_xor(gw3[ni], 32);
-    gb2[ni] += __shfl_xor(gb2[ni], 32);
-  }
-  float db3 = dy;
-  for (int o = 32; o > 0; o >>= 1) db3 += __shfl_xor(db3, o);
+  gw3 += __shfl_xor(gw3, 32);
+  gb2 += __shfl_xor(gb2, 32);
   if (lane < 32) {
-    for (int ni = 0; ni < 2; ++ni) {
-      out[P_W3 + ni * 32 + col] = gw3[ni];
-      out[P_B2 + ni * 32 + col] = gb2[ni];
-    }
+    out[P_W3 + ni * 32 + col] = gw3;
+    out[P_B2 + ni * 32 + col] = gb2;
   }
-  if (lane == 0) {
-    out[P_B3] = db3;
-    out[NPARAM] = se;
-  }
-  wave_sync();
+  __syncthreads();
   const int kq = 4 * (lane / 32);
-  // dW2[o][i] = sum_s dz2[s][o] h1[s][i]  (A = dz2^T, B = h1, K = samples)
+  // dW2[o][i] = sum_s dz2[s][o] h1[s][i]  (A = dz2^T, B = h1, K = samples), i of this wave's half
   for (int mi = 0; mi < 2; ++mi) {
-    for (int ni = 0; ni < 2; ++ni) {
-      f32x16 acc = {};
-      for (int kk = 0; kk < 8; ++kk) {
-        const int sb = kk * 8 + kq;
-        const bf16x4 av = {static_cast<short>(L.dz2[sb][mi * 32 + col]), static_cast<short>(L.dz2[sb + 1][mi * 32 + col]),
-                           static_cast<short>(L.dz2[sb + 2][mi * 32 + col]), static_cast<short>(L.dz2[sb + 3][mi * 32 + col])};
-        const bf16x4 bv = {static_cast<short>(L.h1[sb][ni * 32 + col]), static_cast<short>(L.h1[sb + 1][ni * 32 + col]),
-                           static_cast<short>(L.h1[sb + 2][ni * 32 + col]), static_cast<short>(L.h1[sb + 3][ni * 32 + col])};
-        acc = mfma(av, bv, acc);
-      }
-      for (int v = 0; v < 16; ++v) out[P_W2 + (mi * 32 + drow(v, lane)) * kHid + ni * 32 + col] = acc[v];
+    f32x16 acc = {};
+    for (int kk = 0; kk < 8; ++kk) {
+      const int sb = kk * 8 + kq;
+      const bf16x4 av = {static_cast<short>(L.dz2[sb][mi * 32 + col]), static_cast<short>(L.dz2[sb + 1][mi * 32 + col]),
+                         static_cast<short>(L.dz2[sb + 2][mi * 32 + col]), static_cast<short>(L.dz2[sb + 3][mi * 32 + col])};
+      const bf16x4 bv = {static_cast<short>(L.h1[sb][ni * 32 + col]), static_cast<short>(L.h1[sb + 1][ni * 32 + col]),
+                         static_cast<short>(L.h1[sb + 2][ni * 32 + col]), static_cast<short>(L.h1[sb + 3][ni * 32 + col])};
+      acc = mfma(av, bv, acc);
     }
+    for (int v = 0; v < 16; ++v) out[P_W2 + (mi * 32 + drow(v, lane)) * kHid + ni * 32 + col] = acc[v];
   }
   // dh1[s][i] = sum_o dz2[s][o] W2[o][i]  (A = dz2, B = W2 via its transpose copy), dz1 = dh1 * SiLU'(z1)
-  float gb1[2] = {0.0f, 0.0f};
-  float gw1[2][kIn] = {};
+  float gb1 = 0.0f, gw1[kIn] = {};
   for (int mi = 0; mi < 2; ++mi) {
-    for (int ni = 0; ni < 2; ++ni) {
-      f32x16 acc = {};
-      for (int kk = 0; kk < 8; ++kk) {
-        const uint16_t* ar = &L.dz2[mi * 32 + col][kk * 8 + kq];
-        const bf16x4 av = {static_cast<short>(ar[0]), static_cast<short>(ar[1]), static_cast<short>(ar[2]),
-                           static_cast<short>(ar[3])};
-        const uint16_t* br = a.W.w2t + (ni * 32 + col) * kHid + kk * 8 + kq;
-        const bf16x4 bv = {static_cast<short>(br[0]), static_cast<short>(br[1]), static_cast<short>(br[2]),
-                           static_cast<short>(br[3])};
-        acc = mfma(av, bv, acc);
-      }
-      for (int v = 0; v < 16; ++v) {
-        const int s = mi * 32 + drow(v, lane);
-        const float d = acc[v] * dsilu(z1[mi][ni][v]);
-        gb1[ni] += d;
-        for (int j = 0; j < kIn; ++j) gw1[ni][j] += d * L.xs[s][j];
-      }
+    f32x16 acc = {};
+    for (int kk = 0; kk < 8; ++kk) {
+      const uint16_t* ar = &L.dz2[mi * 32 + col][kk * 8 + kq];
+      const bf16x4 av = {static_cast<short>(ar[0]), static_cast<short>(ar[1]), static_cast<short>(ar[2]),
+                         static_cast<short>(ar[3])};
+      const uint16_t* br = a.W.w2t + (ni * 32 + col) * kHid + kk * 8 + kq;
+      const bf16x4 bv = {static_cast<short>(br[0]), static_cast<short>(br[1]), static_cast<short>(br[2]),
+                         static_cast<short>(br[3])};
+      acc = mfma(av, bv, acc);
+    }
+    for (int v = 0; v < 16; ++v) {
+      const int s = mi * 32 + drow(v, lane);
+      const float d = acc[v] * dsilu(z1[mi][v], s1[mi][v]);
+      gb1 += d;
+      for (int j = 0; j < kIn; ++j) gw1[j] += d * L.xs[s][j];
     }
   }
-  for (int ni = 0; ni < 2; ++ni) {
-    gb1[ni] += __shfl_xor(gb1[ni], 32);
-    for (int j = 0; j < kIn; ++j) gw1[ni][j] += __shfl_xor(gw1[ni][j], 32);
-  }
+  gb1 += __shfl_xor(gb1, 32);
+  for (int j = 0; j < kIn; ++j) gw1[j] += __shfl_xor(gw1[j], 32);
   if (lane < 32) {
-    for (int ni = 0; ni < 2; ++ni) {
-      out[P_B1 + ni * 32 + col] = gb1[ni];
-      for (int j = 0; j < kIn; ++j) out[P_W1 + (ni * 32 + col) * kIn + j] = gw1[ni][j];
-    }
+    out[P_B1 + ni * 32 + col] = gb1;
+    for (int j = 0; j < kIn; ++j) out[P_W1 + (ni * 32 + col) * kIn + j] = gw1[j];
   }
 }
 
-// first level of the gradient sum: chunk c of kReduceChunk waves, summed in wave order, for every
-// parameter (and the loss, entry NPARAM); one thread per (parameter, chunk)
+// rows w0 .. w1 - 1 of column p, added in order; the loads of a full chunk are all in flight at once
 constexpr uint32_t kReduceChunk = 32;
+__device__ __forceinline__ float sum_rows(const float* rows, uint32_t w0, uint32_t w1, int p) {
+  const float* r = rows + static_cast<uint64_t>(w0) * (NPARAM + 1) + p;
+  float s = 0.0f;
+  if (w1 - w0 == kReduceChunk) {
+    float v[kReduceChunk];
+#pragma unroll
+    for (uint32_t i = 0; i < kReduceChunk; ++i) v[i] = r[i * (NPARAM + 1)];
+#pragma unroll
+    for (uint32_t i = 0; i < kReduceChunk; ++i) s += v[i];
+    return s;
+  }
+  for (uint32_t i = 0; i < w1 - w0; ++i) s += r[static_cast<uint64_t>(i) * (NPARAM + 1)];
+  return s;
+}
+// a level of the gradient sum: chunk c of kReduceChunk rows, summed in row order, for every
+// parameter (and the loss, entry NPARAM); one thread per (parameter, chunk)
 __global__ void k_mlp_reduce_chunks(const float* partial, uint32_t nwaves, float* chunks) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p > NPARAM) return;
   const uint32_t w0 = blockIdx.y * kReduceChunk, w1 = min(w0 + kReduceChunk, nwaves);
-  float s = 0.0f;
-  for (uint32_t w = w0; w < w1; ++w) s += partial[static_cast<uint64_t>(w) * (NPARAM + 1) + p];
-  chunks[static_cast<uint64_t>(blockIdx.y) * (NPARAM + 1) + p] = s;
+  chunks[static_cast<uint64_t>(blockIdx.y) * (NPARAM + 1) + p] = sum_rows(partial, w0, w1, p);
 }
 
+// bf16 copies of the weights where the kernels read them: W1 (padded), W2 and W2^T
+__device__ __forceinline__ void pack_weight(int p, float w, uint16_t* w1p, uint16_t* w2, uint16_t* w2t) {
+  const uint16_t b = f2bf(w);
+  if (p < P_B1) {
+    w1p[(p / kIn) * kInPad + p % kIn] = b;
+  } else if (p >= P_W2 && p < P_B2) {
+    const int o = (p - P_W2) / kHid, i = (p - P_W2) % kHid;
+    w2[o * kHid + i] = b;
+    w2t[i * kHid + o] = b;
+  }
+}
 // grad[p] = the chunk sums added in chunk order (a fixed order: training is deterministic); then
-// Adam on the fp32 master weights
-__global__ void k_mlp_reduce_adam(const float* chunks, uint32_t nchunks, float* grad, float* loss, float* master,
-                                  float* m, float* v, int32_t apply, float lr, float b1, float b2, float eps,
-                                  float bc1, float bc2) {
+// Adam on the fp32 master weights, and their bf16 copies
+__global__ void __launch_bounds__(64) k_mlp_reduce_adam(const float* chunks, uint32_t nchunks, float* grad, float* loss,
+                                                        float* master, float* m, float* v, int32_t apply, float lr,
+                                                        float b1, float b2, float eps, float bc1, float bc2,
+                                                        uint16_t* w1p, uint16_t* w2, uint16_t* w2t) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p > NPARAM) return;
-  float s = 0.0f;
-  for (uint32_t w = 0; w < nchunks; ++w) s += chunks[static_cast<uint64_t>(w) * (NPARAM + 1) + p];
+  const float s = sum_rows(chunks, 0u, nchunks, p);
   if (p == NPARAM) {
     *loss = s;
     return;
@@ -287,22 +311,17 @@ __global__ void k_mlp_reduce_adam(const float* chunks, uint32_t nchunks, float* 
   const float vv = b2 * v[p] + (1.0f - b2) * s * s;
   m[p] = mm;
   v[p] = vv;
-  master[p] -= lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+  const float w = master[p] - lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+  master[p] = w;
+  pack_weight(p, w, w1p, w2, w2t);
 }
 
-// bf16 copies of W1 (padded), W2 and W2^T from the fp32 master blob
+// all bf16 copies from the fp32 master blob, and the zero columns of the padded W1
 __global__ void k_mlp_pack(const float* master, uint16_t* w1p, uint16_t* w2, uint16_t* w2t) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < kHid * kInPad) {
-    const int o = t / kInPad, k = t % kInPad;
-    w1p[t] = k < kIn ? f2bf(master[P_W1 + o * kIn + k]) : 0;
-  }
-  if (t < kHid * kHid) {
-    const int o = t / kHid, i = t % kHid;
-    const uint16_t b = f2bf(master[P_W2 + o * kHid + i]);
-    w2[o * kHid + i] = b;
-    w2t[i * kHid + o] = b;
-  }
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < kHid)
+    for (int k = kIn; k < kInPad; ++k) w1p[p * kInPad + k] = 0;
+  if (p < P_B2) pack_weight(p, master[p], w1p, w2, w2t);
 }
 
 // per-column sums of x (6 columns) and y in double, one partial per block
@@ -371,27 +390,37 @@ struct MLPDev {
   MLPWeights weights() const { return MLPWeights{w1p, w2, w2t, master}; }
 };
 
-// per-wave partial gradients, followed by room for the chunk sums of k_mlp_reduce_chunks
+// the partial gradients of each workgroup, followed by the chunk sums of every level
 static uint32_t reduce_nchunks(uint32_t waves) { return (waves + kReduceChunk - 1) / kReduceChunk; }
+static uint64_t reduce_rows(uint32_t waves) {
+  uint64_t rows = waves;
+  for (uint32_t n = waves; n > 1; rows += n) n = reduce_nchunks(n);
+  return rows + 1;
+}
 static hipError_t ensure_partial(MLPDev* m, uint32_t waves) {
   if (m->partial_waves >= waves) return hipSuccess;
   hipFree(m->partial);
   m->partial = nullptr;
   m->partial_waves = 0;
-  const size_t rows = static_cast<size_t>(waves) + reduce_nchunks(waves);
-  hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->partial), rows * (NPARAM + 1) * 4);
+  hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->partial), reduce_rows(waves) * (NPARAM + 1) * 4);
   if (e == hipSuccess) m->partial_waves = waves;
   return e;
 }
-// the two-level gradient sum of `waves` per-wave partials, then Adam when `apply`
+// The sum of `waves` partials, in levels of chunks of 32 rows until one chunk is left, which the last
+// launch adds (batches up to 65536 samples: one level before it); then Adam when `apply`.
 static void launch_reduce_adam(hipStream_t s, MLPDev* m, uint32_t waves, int32_t apply, float lr, float b1, float b2,
                                float eps, float bc1, float bc2) {
-  const uint32_t nch = reduce_nchunks(waves);
-  float* ch = m->partial + static_cast<uint64_t>(m->partial_waves) * (NPARAM + 1);
-  hipLaunchKernelGGL(k_mlp_reduce_chunks, dim3((NPARAM + 256) / 256, nch), dim3(256), 0, s,
-                     static_cast<const float*>(m->partial), waves, ch);
-  hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 256) / 256), dim3(256), 0, s, static_cast<const float*>(ch),
-                     nch, m->grad, m->loss, m->master, m->adam_m, m->adam_v, apply, lr, b1, b2, eps, bc1, bc2);
+  const float* rows = m->partial;
+  uint32_t n = waves;
+  do {
+    float* next = const_cast<float*>(rows) + static_cast<uint64_t>(n) * (NPARAM + 1);
+    const uint32_t nch = reduce_nchunks(n);
+    hipLaunchKernelGGL(k_mlp_reduce_chunks, dim3((NPARAM + 256) / 256, nch), dim3(256), 0, s, rows, n, next);
+    rows = next;
+    n = nch;
+  } while (n > kReduceChunk);
+  hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 64) / 64), dim3(64), 0, s, rows, n, m->grad, m->loss, m->master,
+                     m->adam_m, m->adam_v, apply, lr, b1, b2, eps, bc1, bc2, m->w1p, m->w2, m->w2t);
 }
 
 hipError_t mlp_create(cleo_ctx* c) {
@@ -474,7 +503,7 @@ using namespace cleo;
 
 static void launch_pack(cleo_ctx* c) {
   MLPDev* m = c->mlp;
-  hipLaunchKernelGGL(k_mlp_pack, dim3(16), dim3(256), 0, c->stream, m->master, m->w1p, m->w2, m->w2t);
+  hipLaunchKernelGGL(k_mlp_pack, dim3((P_B2 + 255) / 256), dim3(256), 0, c->stream, m->master, m->w1p, m->w2, m->w2t);
 }
 
 extern "C" {
@@ -569,7 +598,7 @@ int cleo_mlp_loss_grad(cleo_ctx* c, const float* x, const float* y, uint64_t n, 
   const uint32_t waves = static_cast<uint32_t>((n + 63) / 64);
   MLP_TRY(c, ensure_partial(m, waves));
   TrainArgs a{x, y, nullptr, 0, static_cast<uint32_t>(n), 2.0f / static_cast<float>(n), m->weights(), m->partial};
-  hipLaunchKernelGGL(k_mlp_grad, dim3(waves), dim3(64), 0, c->stream, a);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(waves), dim3(128), 0, c->stream, a);
   launch_reduce_adam(c->stream, m, waves, 0, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
   MLP_TRY(c, hipGetLastError());
   MLP_TRY(c, hipStreamSynchronize(c->stream));
@@ -672,11 +701,10 @@ int cleo_mlp_train(cleo_ctx* c, const float* x, const float* y, uint64_t n, cons
     for (uint64_t bi = 0; bi < nbatch; ++bi) {
       ++step;
       TrainArgs a{x, y, dperm, order[bi] * bsz, bsz, 2.0f / static_cast<float>(bsz), m->weights(), m->partial};
-      hipLaunchKernelGGL(k_mlp_grad, dim3(waves), dim3(64), 0, c->stream, a);
+      hipLaunchKernelGGL(k_mlp_grad, dim3(waves), dim3(128), 0, c->stream, a);
       const float bc1 = 1.0f - std::pow(tp->beta1, static_cast<float>(step));
       const float bc2 = 1.0f - std::pow(tp->beta2, static_cast<float>(step));
       launch_reduce_adam(c->stream, m, waves, 1, tp->lr, tp->beta1, tp->beta2, tp->eps, bc1, bc2);
-      launch_pack(c);
     }
   }
   MLP_TRY(c, hipGetLastError());

@@ -40,19 +40,12 @@ struct MLPWeights {
   const float* p;        // fp32 blob (biases, W3, normalisation)
 };
 
-__device__ __forceinline__ uint16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return static_cast<uint16_t>((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
-}
+// round to nearest even (v_cvt_pk_bf16_f32; integer rounding with its NaN branch took 14 instructions,
+// 134 times in the gradient kernel)
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(static_cast<uint32_t>(h) << 16); }
 __device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + __expf(-z)); }
-__device__ __forceinline__ float silu(float z) { return z * sigm(z); }
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = sigm(z);
-  return s * (1.0f + z * (1.0f - s));
-}
+__device__ __forceinline__ float dsilu(float z, float s) { return s * (1.0f + z * (1.0f - s)); }  // s = sigm(z)
 __device__ __forceinline__ int drow(int v, int lane) { return 8 * (v / 4) + 4 * (lane / 32) + (v % 4); }
 
 __device__ __forceinline__ f32x16 mfma(bf16x4 a, bf16x4 b, f32x16 c) {
@@ -61,15 +54,18 @@ __device__ __forceinline__ f32x16 mfma(bf16x4 a, bf16x4 b, f32x16 c) {
 
 
 
-// Forward pass of the 64 samples held in L.xb; returns z1, z2 in accumulator layout (tile
-// [mi][ni], element v: row drow(v,lane) + 32 mi, column lane%32 + 32 ni) and y for sample `lane`
-// (lane < 64).  Each output row depends on its own input row only.  `Lds` holds xb, h1 and ys.
+// Forward pass of the 64 samples held in L.xb by a workgroup of two waves: wave `ni` (0, 1) has the
+// hidden units 32 ni .. 32 ni + 31 of both layers.  Returns z1, z2 in accumulator layout (tile mi,
+// element v: sample row drow(v,lane) + 32 mi, unit lane%32 + 32 ni), their sigmoids s1, s2 (the
+// backward pass needs them again; each costs an exponential and a division) and y for sample `lane`.
+// Every thread of the workgroup calls it.
 template <class Lds>
-__device__ __forceinline__ float mlp_forward_wave(const MLPWeights& W, Lds& L, f32x16 z1[2][2], f32x16 z2[2][2]) {
+__device__ __forceinline__ float mlp_forward_pair(const MLPWeights& W, Lds& L, int ni, f32x16 z1[2], f32x16 s1[2],
+                                                  f32x16 z2[2], f32x16 s2[2]) {
   const int lane = lane_id();
   const int col = lane % 32, kq = 4 * (lane / 32);
   // layer 1: [64 x 8] . [8 x 64]
-  for (int ni = 0; ni < 2; ++ni) {
+  {
     const uint16_t* wr = W.w1p + (ni * 32 + col) * kInPad + kq;
     const bf16x4 b = {static_cast<short>(wr[0]), static_cast<short>(wr[1]), static_cast<short>(wr[2]),
                       static_cast<short>(wr[3])};
@@ -82,40 +78,45 @@ __device__ __forceinline__ float mlp_forward_wave(const MLPWeights& W, Lds& L, f
       acc = mfma(a, b, acc);
       for (int v = 0; v < 16; ++v) {
         acc[v] += bias;
-        L.h1[mi * 32 + drow(v, lane)][ni * 32 + col] = f2bf(silu(acc[v]));
+        s1[mi][v] = sigm(acc[v]);
+        L.h1[mi * 32 + drow(v, lane)][ni * 32 + col] = f2bf(acc[v] * s1[mi][v]);
       }
-      z1[mi][ni] = acc;
+      z1[mi] = acc;
     }
   }
-  wave_sync();
-  // layer 2: [64 x 64] . [64 x 64]
+  __syncthreads();
+  // layer 2: [64 x 64] . [64 x 64]; then the products of layer 3, y[s] = sum_n SiLU(z2[s][n]) w3[n] + b3
+  const float bias = W.p[P_B2 + ni * 32 + col], w3 = W.p[P_W3 + ni * 32 + col];
+  float t[2][16];
   for (int mi = 0; mi < 2; ++mi) {
-    for (int ni = 0; ni < 2; ++ni) {
-      f32x16 acc = {};
-      for (int kk = 0; kk < 8; ++kk) {
-        const uint16_t* ar = &L.h1[mi * 32 + col][kk * 8 + kq];
-        const bf16x4 a = {static_cast<short>(ar[0]), static_cast<short>(ar[1]), static_cast<short>(ar[2]),
-                          static_cast<short>(ar[3])};
-        const uint16_t* br = W.w2 + (ni * 32 + col) * kHid + kk * 8 + kq;
-        const bf16x4 b = {static_cast<short>(br[0]), static_cast<short>(br[1]), static_cast<short>(br[2]),
-                          static_cast<short>(br[3])};
-        acc = mfma(a, b, acc);
-      }
-      const float bias = W.p[P_B2 + ni * 32 + col];
-      for (int v = 0; v < 16; ++v) acc[v] += bias;
-      z2[mi][ni] = acc;
+    f32x16 acc = {};
+    for (int kk = 0; kk < 8; ++kk) {
+      const uint16_t* ar = &L.h1[mi * 32 + col][kk * 8 + kq];
+      const bf16x4 a = {static_cast<short>(ar[0]), static_cast<short>(ar[1]), static_cast<short>(ar[2]),
+                        static_cast<short>(ar[3])};
+      const uint16_t* br = W.w2 + (ni * 32 + col) * kHid + kk * 8 + kq;
+      const bf16x4 b = {static_cast<short>(br[0]), static_cast<short>(br[1]), static_cast<short>(br[2]),
+                        static_cast<short>(br[3])};
+      acc = mfma(a, b, acc);
     }
-  }
-  // layer 3: y[s] = sum_n SiLU(z2[s][n]) w3[n] + b3, reduced over the 32 lanes of a half-wave
-  const float w3a = W.p[P_W3 + col], w3b = W.p[P_W3 + 32 + col];
-  for (int mi = 0; mi < 2; ++mi) {
     for (int v = 0; v < 16; ++v) {
-      float t = silu(z2[mi][0][v]) * w3a + silu(z2[mi][1][v]) * w3b;
-      for (int o = 16; o > 0; o >>= 1) t += __shfl_xor(t, o);
-      if (col == 0) L.ys[mi * 32 + drow(v, lane)] = t;
+      acc[v] += bias;
+      s2[mi][v] = sigm(acc[v]);
+      t[mi][v] = acc[v] * s2[mi][v] * w3;
     }
+    z2[mi] = acc;
   }
-  wave_sync();
+  // the two waves' products meet in LDS (wave 1 hands over tile 0's and takes tile 1's); wave mi then
+  // reduces the 32 samples of tile mi over the 32 lanes of a half-wave
+  for (int v = 0; v < 16; ++v) L.part[ni][v][lane] = t[1 - ni][v];
+  __syncthreads();
+  for (int v = 0; v < 16; ++v) {
+    const float other = L.part[1 - ni][v][lane];
+    float u = ni == 0 ? t[0][v] + other : other + t[1][v];
+    for (int o = 16; o > 0; o >>= 1) u += __shfl_xor(u, o);
+    if (col == 0) L.ys[ni * 32 + drow(v, lane)] = u;
+  }
+  __syncthreads();
   return L.ys[lane] + W.p[P_B3];
 }
 
@@ -266,20 +267,5 @@ __device__ __forceinline__ void drop_features(double r, double msol, double s_ra
   f[4] = static_cast<float>(press);
   f[5] = static_cast<float>(delt);
 }
-
-// the lane's normalised inputs into L.xb (bf16) and, when the LDS block has one, L.xs (fp32)
-template <class Lds>
-__device__ __forceinline__ void load_normalised(Lds& L, const float* p, const float f[kIn], bool valid) {
-  const int lane = lane_id();
-  for (int k = 0; k < kInPad; ++k) {
-    float v = 0.0f;
-    if (k < kIn && valid) v = (f[k] - p[P_XMEAN + k]) / p[P_XSTD + k];
-    if constexpr (Lds::kHasXs) L.xs[lane][k] = v;
-    L.xb[lane][k] = f2bf(v);
-  }
-  wave_sync();
-}
-
-
 
 }  // namespace cleo
