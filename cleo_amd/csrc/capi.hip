@@ -441,14 +441,15 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   c->big_scratch_n = 2 * maxn;
   HIP_TRY(c, dalloc(&c->ctl, 1));
   HIP_TRY(c, hipHostMalloc(reinterpret_cast<void**>(&c->h_ctl), sizeof(DevCtl), hipHostMallocDefault));
-  HIP_TRY(c, ctx_fill(c, c->ctl, 0, sizeof(DevCtl)));
-  HIP_TRY(c, ctx_fill(c, c->sp, 0, kStatRow * kStatRows * 8));
-  HIP_TRY(c, ctx_fill(c, c->off, 0, (ngbx + 1) * 4));
-  HIP_TRY(c, ctx_fill(c, c->off_alt, 0, (ngbx + 1) * 4));
-  HIP_TRY(c, ctx_fill(c, c->nact, 0, ngbx * 4));
-  HIP_TRY(c, ctx_fill(c, c->cnt, 0, 28 * ngbx * 4));
-  HIP_TRY(c, ctx_fill(c, c->tot, 0, (ngbx + 1) * 4));
-  HIP_TRY(c, ctx_fill(c, c->d_state, 0, 11 * ngbx * 8));
+  HIP_TRY(c, hipMemsetAsync(c->ctl, 0, sizeof(DevCtl), c->stream));
+  HIP_TRY(c, hipMemsetAsync(c->sp, 0, kStatRow * kStatRows * 8, c->stream));
+  HIP_TRY(c, hipMemsetAsync(c->off, 0, (ngbx + 1) * 4, c->stream));
+  HIP_TRY(c, hipMemsetAsync(c->off_alt, 0, (ngbx + 1) * 4, c->stream));
+  HIP_TRY(c, hipMemsetAsync(c->nact, 0, ngbx * 4, c->stream));
+  HIP_TRY(c, hipMemsetAsync(c->cnt, 0, 28 * ngbx * 4, c->stream));
+  HIP_TRY(c, hipMemsetAsync(c->tot, 0, (ngbx + 1) * 4, c->stream));
+  HIP_TRY(c, hipMemsetAsync(c->d_state, 0, 11 * ngbx * 8, c->stream));
+  HIP_TRY(c, hipStreamSynchronize(c->stream));
   c->solute = make_solute(2016.5 / dimless::RHO0, 0.05844277 / dimless::MR0, 2.0);
   HIP_TRY(c, mlp_create(c));
   *out = c;

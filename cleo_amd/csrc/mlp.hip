@@ -373,6 +373,105 @@ __global__ void __launch_bounds__(256) k_mlp_forward(ForwardArgs a) {
   }
 }
 
+// ---- the sample order: a Fisher-Yates shuffle from a xorshift64 stream --------------------------
+// The order is that of the serial shuffle `for i = n-1 .. 1: swap(perm[i], perm[x() % (i+1)])` (5 ms
+// for 2M samples on one host core with the copy of its result, 0.26 ms here, most of it the random
+// accesses of the atomic exchanges and list walks).  xorshift64 is linear over the bits of its state, so a thread gets its place in the stream by 64 x 64 bit matrices:
+// jump[b] is the one of kDrawsPerThread << b steps.  The order follows from the drawn indices by the
+// lists of the swaps that hit each place, as in the collisions' shuffle (sdm_kernels.hip), here over
+// several launches.
+constexpr uint32_t kDrawsPerThread = 16, kJumps = 29;
+__host__ __device__ inline uint64_t xorshift64(uint64_t s) {
+  s ^= s << 13;
+  s ^= s >> 7;
+  s ^= s << 17;
+  return s;
+}
+// the matrix with columns m applied to s
+__host__ __device__ inline uint64_t apply_bits(const uint64_t* m, uint64_t s) {
+  uint64_t r = 0;
+  for (int b = 0; b < 64; ++b) r ^= m[b] & (0ull - ((s >> b) & 1ull));
+  return r;
+}
+struct Jumps {
+  uint64_t m[kJumps][64];
+  Jumps() {
+    for (int b = 0; b < 64; ++b) {
+      uint64_t s = 1ull << b;
+      for (uint32_t k = 0; k < kDrawsPerThread; ++k) s = xorshift64(s);
+      m[0][b] = s;
+    }
+    for (uint32_t j = 1; j < kJumps; ++j)
+      for (int b = 0; b < 64; ++b) m[j][b] = apply_bits(m[j - 1], m[j - 1][b]);
+  }
+};
+static const Jumps& jumps() {
+  static const Jumps j;
+  return j;
+}
+// the state after `steps` steps from s
+static uint64_t xorshift64_after(uint64_t s, uint64_t steps) {
+  for (uint32_t j = 0; j < kJumps; ++j)
+    if ((steps / kDrawsPerThread) >> j & 1u) s = apply_bits(jumps().m[j], s);
+  for (uint64_t k = 0; k < steps % kDrawsPerThread; ++k) s = xorshift64(s);
+  return s;
+}
+constexpr uint32_t kNoEntry = 0xFFFFFFFFu;
+struct OrderArgs {
+  uint32_t n;
+  uint64_t state;
+  const uint64_t* jump;  // [kJumps][64]
+  // per place: the last swap listed there, the next swap in the list a swap is on, the swap's index and
+  // later the place its element comes from (kNoEntry: known at once), the first hop of the place's chain
+  uint32_t *head, *nxt, *src, *hop;
+  uint32_t* perm;
+};
+__global__ void __launch_bounds__(256) k_order_clear(OrderArgs a) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) a.head[i] = kNoEntry;
+}
+__global__ void __launch_bounds__(256) k_order_draw(OrderArgs a) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t c0 = static_cast<uint64_t>(t) * kDrawsPerThread;  // draw c is that of swap n-1-c
+  if (c0 + 1 >= a.n) return;
+  uint64_t s = a.state;
+  for (uint32_t j = 0; j < kJumps; ++j)
+    if ((t >> j) & 1u) s = apply_bits(a.jump + 64u * j, s);
+  for (uint32_t k = 0; k < kDrawsPerThread && c0 + k + 1 < a.n; ++k) {
+    const uint32_t i = a.n - 1u - static_cast<uint32_t>(c0 + k);
+    s = xorshift64(s);
+    const uint32_t j = static_cast<uint32_t>(s % (static_cast<uint64_t>(i) + 1ull));
+    a.src[i] = j;
+    a.nxt[i] = atomicExch(&a.head[j], i);
+  }
+}
+__global__ void __launch_bounds__(256) k_order_link(OrderArgs a) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
+    uint32_t hop = kNoEntry;
+    for (uint32_t e = a.head[i]; e != kNoEntry; e = a.nxt[e])
+      if (e != i && e < hop) hop = e;
+    a.hop[i] = hop;
+    uint32_t from = i;
+    if (i > 0) {
+      const uint32_t j = a.src[i];
+      if (j != i) {
+        from = kNoEntry;  // the first swap after i that hit place j; without one, j's own element
+        for (uint32_t e = a.head[j]; e != kNoEntry; e = a.nxt[e])
+          if (e > i && e < from) from = e;
+        if (from == kNoEntry) a.perm[i] = j;
+      }
+    }
+    a.src[i] = from;
+  }
+}
+__global__ void __launch_bounds__(256) k_order_chase(OrderArgs a) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
+    uint32_t x = a.src[i];
+    if (x == kNoEntry) continue;
+    for (uint32_t h = a.hop[x]; h != kNoEntry; h = a.hop[x]) x = h;
+    a.perm[i] = x;
+  }
+}
+
 // ------------------------------------------------------------------------------------------------
 struct MLPDev {
   bool ready = false;
@@ -387,6 +486,10 @@ struct MLPDev {
   double* warm = nullptr;   // maxn
   float* partial = nullptr;
   uint32_t partial_waves = 0;
+  double* moments = nullptr;      // per-block sums of k_mlp_moments
+  uint64_t* jump = nullptr;       // the sample order's jump matrices
+  uint32_t* order = nullptr;      // the sample order and its scratch: five words per sample
+  uint64_t order_n = 0;
   MLPWeights weights() const { return MLPWeights{w1p, w2, w2t, master}; }
 };
 
@@ -444,7 +547,8 @@ void mlp_destroy(cleo_ctx* c) {
   for (void* p : {static_cast<void*>(m->master), static_cast<void*>(m->adam_m), static_cast<void*>(m->adam_v),
                   static_cast<void*>(m->grad), static_cast<void*>(m->loss), static_cast<void*>(m->w1p),
                   static_cast<void*>(m->w2), static_cast<void*>(m->w2t), static_cast<void*>(m->warm),
-                  static_cast<void*>(m->partial)})
+                  static_cast<void*>(m->partial), static_cast<void*>(m->moments), static_cast<void*>(m->jump),
+                  static_cast<void*>(m->order)})
     if (p) hipFree(p);
   delete m;
   c->mlp = nullptr;
@@ -500,6 +604,35 @@ using namespace cleo;
       return CLEO_E_HIP;                                                   \
     }                                                                      \
   } while (0)
+
+constexpr unsigned kMomentBlocks = 256;
+
+// the shuffled order of n samples on the device (see k_order_draw) and the stream's state behind it
+static int sample_order(cleo_ctx* c, uint64_t n, uint64_t state, const uint32_t** perm, uint64_t* state_after) {
+  MLPDev* m = c->mlp;
+  if (!m->jump) {
+    MLP_TRY(c, hipMalloc(reinterpret_cast<void**>(&m->jump), sizeof(Jumps)));
+    MLP_TRY(c, ctx_copy(c, m->jump, jumps().m, sizeof(Jumps), hipMemcpyHostToDevice));
+  }
+  if (m->order_n < n) {
+    hipFree(m->order);
+    m->order = nullptr;
+    m->order_n = 0;
+    MLP_TRY(c, hipMalloc(reinterpret_cast<void**>(&m->order), 5 * n * 4));
+    m->order_n = n;
+  }
+  uint32_t* w = m->order;
+  const OrderArgs a{static_cast<uint32_t>(n), state, m->jump, w, w + n, w + 2 * n, w + 3 * n, w + 4 * n};
+  const unsigned nb = static_cast<unsigned>(std::min<uint64_t>((n + 255) / 256, 16384));
+  const uint64_t threads = (n + kDrawsPerThread - 1) / kDrawsPerThread;
+  hipLaunchKernelGGL(k_order_clear, dim3(nb), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_order_draw, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_order_link, dim3(nb), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_order_chase, dim3(nb), dim3(256), 0, c->stream, a);
+  *perm = a.perm;
+  *state_after = xorshift64_after(state, n - 1);
+  return CLEO_OK;
+}
 
 static void launch_pack(cleo_ctx* c) {
   MLPDev* m = c->mlp;
@@ -628,15 +761,13 @@ int cleo_mlp_train(cleo_ctx* c, const float* x, const float* y, uint64_t n, cons
                    float* final_loss) {
   if (!c || !x || !y || !tp || n < 64 || tp->batch == 0 || tp->epochs == 0) return CLEO_E_ARG;
   MLPDev* m = c->mlp;
+  if (n >= kNoEntry) return CLEO_E_ARG;
   // normalisation from the sample moments
-  const unsigned mb = 256;
-  double* part = nullptr;
-  MLP_TRY(c, hipMalloc(reinterpret_cast<void**>(&part), mb * 14 * 8));
-  hipLaunchKernelGGL(k_mlp_moments, dim3(mb), dim3(256), 0, c->stream, x, y, n, part);
+  const unsigned mb = kMomentBlocks;
+  if (!m->moments) MLP_TRY(c, hipMalloc(reinterpret_cast<void**>(&m->moments), mb * 14 * 8));
+  hipLaunchKernelGGL(k_mlp_moments, dim3(mb), dim3(256), 0, c->stream, x, y, n, m->moments);
   std::vector<double> hp(mb * 14);
-  MLP_TRY(c, hipMemcpyAsync(hp.data(), part, mb * 14 * 8, hipMemcpyDeviceToHost, c->stream));
-  MLP_TRY(c, hipStreamSynchronize(c->stream));
-  hipFree(part);
+  MLP_TRY(c, ctx_copy(c, hp.data(), m->moments, mb * 14 * 8, hipMemcpyDeviceToHost));
   double mom[14] = {};
   for (unsigned b = 0; b < mb; ++b)
     for (int j = 0; j < 14; ++j) mom[j] += hp[b * 14 + j];
@@ -676,19 +807,11 @@ int cleo_mlp_train(cleo_ctx* c, const float* x, const float* y, uint64_t n, cons
   launch_pack(c);
   m->ready = true;
   // sample order: one seeded permutation, batches visited in a seeded order each epoch
-  std::vector<uint32_t> perm(n);
-  for (uint64_t i = 0; i < n; ++i) perm[i] = static_cast<uint32_t>(i);
-  uint64_t st = tp->seed ^ 0xD1B54A32D192ED03ull;
-  auto next = [&st]() {
-    st ^= st << 13;
-    st ^= st >> 7;
-    st ^= st << 17;
-    return st;
-  };
-  for (uint64_t i = n - 1; i > 0; --i) std::swap(perm[i], perm[next() % (i + 1)]);
-  uint32_t* dperm = nullptr;
-  MLP_TRY(c, hipMalloc(reinterpret_cast<void**>(&dperm), n * 4));
-  MLP_TRY(c, ctx_copy(c, dperm, perm.data(), n * 4, hipMemcpyHostToDevice));
+  uint64_t st = 0;
+  const uint32_t* dperm = nullptr;
+  const int ro = sample_order(c, n, tp->seed ^ 0xD1B54A32D192ED03ull, &dperm, &st);
+  if (ro != CLEO_OK) return ro;
+  auto next = [&st]() { return st = xorshift64(st); };
   const uint64_t nbatch = n / tp->batch ? n / tp->batch : 1;
   const uint32_t bsz = static_cast<uint32_t>(std::min<uint64_t>(tp->batch, n));
   const uint32_t waves = (bsz + 63) / 64;
@@ -709,7 +832,6 @@ int cleo_mlp_train(cleo_ctx* c, const float* x, const float* y, uint64_t n, cons
   }
   MLP_TRY(c, hipGetLastError());
   MLP_TRY(c, hipStreamSynchronize(c->stream));
-  hipFree(dperm);
   const int rc = mlp_check_ready(c);
   if (rc != CLEO_OK) return rc;
   if (final_loss) {

@@ -165,3 +165,49 @@ def test_fused_warm_start_matches_unfused(gpu):
     for st in stats[1:]:
         assert st["newton_iters"] == stats[0]["newton_iters"] and st["warm_restarts"] == stats[0]["warm_restarts"]
     _say(f"  Newton iterations {stats[0]['newton_iters']}, warm restarts {stats[0]['warm_restarts']}")
+
+
+@pytest.mark.parametrize("n", [64, 65, 127, 1000, 4096, 4097, 100003])
+def test_sample_order_is_the_serial_shuffle(gpu, n):
+    """With a learning rate of 0 the reported loss is that of the last batch under the given weights: it
+    must be the loss of the samples the serial xorshift64 shuffle puts there."""
+    print(f"case: sample order of {n} samples", flush=True)
+    batch, mask = max(1, n // 7), (1 << 64) - 1
+    st = 0xD1B54A32D192ED03
+
+    def draw():
+        nonlocal st
+        st = (st ^ (st << 13)) & mask
+        st ^= st >> 7
+        st = (st ^ (st << 17)) & mask
+        return st
+
+    perm = list(range(n))
+    for i in range(n - 1, 0, -1):
+        j = draw() % (i + 1)
+        perm[i], perm[j] = perm[j], perm[i]
+    nbatch = max(1, n // batch)
+    order = list(range(nbatch))
+    for b in range(nbatch - 1, 0, -1):
+        j = draw() % (b + 1)
+        order[b], order[j] = order[j], order[b]
+    last = perm[order[-1] * batch:order[-1] * batch + batch]
+    rng = np.random.default_rng(n)
+    blob = np.zeros(abi.MLP_NBLOB, dtype=np.float32)
+    blob[:abi.MLP_NPARAMS] = rng.uniform(-0.3, 0.3, abi.MLP_NPARAMS)
+    blob[abi.MLP_NPARAMS + 6:abi.MLP_NPARAMS + 12] = 1.0
+    blob[-1] = 1.0
+    x = torch.zeros((n, 8), device="cuda", dtype=torch.float32)
+    x[:, :6] = torch.from_numpy(rng.normal(size=(n, 6)).astype(np.float32)).cuda()
+    y = torch.from_numpy(rng.normal(size=n).astype(np.float32) * 3).cuda()
+    xb, yb = x[torch.tensor(last, device="cuda")].contiguous(), y[torch.tensor(last, device="cuda")].contiguous()
+    torch.cuda.synchronize()
+    d = abi.Domain(gpu, 64, (1, 1, 1), [0.0, 1.0], [0.0, 1.0], [0.0, 1.0])
+    fp = C.POINTER(C.c_float)
+    got, want = C.c_float(), C.c_float()
+    grad = np.zeros(abi.MLP_NPARAMS, dtype=np.float32)
+    d.check(gpu.lib.cleo_mlp_set_weights(d.h, blob.ctypes.data_as(fp)), "set_weights")
+    d.check(gpu.lib.cleo_mlp_loss_grad(d.h, xb.data_ptr(), yb.data_ptr(), batch, C.byref(want), grad.ctypes.data_as(fp)), "grad")
+    tp = abi.MLPTrainParams(1, batch, 0.0, 0.9, 0.999, 1e-8, 0)
+    d.check(gpu.lib.cleo_mlp_train(d.h, x.data_ptr(), y.data_ptr(), n, C.byref(tp), C.byref(got)), "train")
+    assert got.value == want.value  # the same samples in the same order through the same kernels
