@@ -34,8 +34,6 @@ FP64_PEAK_TFLOPS = 78.6
 
 # algorithmic HBM bytes (per drop, per gridbox) of each stage's main kernel, by variant
 BYTES = {
-    # read r, msol, xi; write r | read State (press, temp, qv, qc, vol), refs; write temp, qv, qc
-    "k_condensation": (32, 5 * 8 + 8 + 3 * 8),
     # read sdgbxindex, r, msol, xi; write r, dm | saturation ratio and diffusion factor, temp, refs
     "k_cond_drops": (44, 2 * 8 + 8 + 8),
     "k_cond_queue": (44, 2 * 8 + 8 + 8),
@@ -44,7 +42,6 @@ BYTES = {
     "k_coll_team": (28, 8 + 4 + 8),
     "k_coll_tiles": (28, 8 + 4 + 8),
     # read coords, radius, sdgbxindex; write coords, sdgbxindex | bounds, winds, counts
-    "k_motion": (64, 6 * 8 + 6 * 8 + 28 * 4),
     "k_motion_flat": (64, 6 * 8 + 6 * 8 + 28 * 4),
     # fused motion + sort, moving pass: read coords, radius, xi, msol, id; write the 60-byte record
     # at its sorted place | bounds, winds, refs, run starts
@@ -76,10 +73,10 @@ def measured_traffic(kernel, ndims):
 def stage_kernel(stage, tiles):
     """Name of the main kernel of a stage (0 condensation, 1 collisions, 2 motion) under a tiling."""
     if stage == 0:
-        return {0: "k_condensation", 1: "k_cond_drops", 2: "k_cond_queue"}[tiles.cond_flat]
+        return {0: "k_cond_drops", 1: "k_cond_drops", 2: "k_cond_queue"}[tiles.cond_flat]
     if stage == 1:
         return "k_coll_tiles" if tiles.coll_flat else "k_coll_team"
-    return {0: "k_motion", 1: "k_motion_flat", 2: "k_motion_scatter", 3: "k_motion_keys"}[tiles.motion_flat]
+    return {0: "k_motion_flat", 1: "k_motion_flat", 2: "k_motion_scatter", 3: "k_motion_keys"}[tiles.motion_flat]
 
 
 def host_cpu():

@@ -95,8 +95,8 @@ int ensure_radix(cleo_ctx* c, uint64_t n) {
 
 uint32_t wpb_or1(uint32_t v) { return v == 0 ? 1u : std::min<uint32_t>(v, 4u); }
 
-CondArgs cond_args(cleo_ctx* c, const cleo_cond_params& p, bool fuse_qcond) {
-  CondArgs a{};
+CondFlatArgs cond_args(cleo_ctx* c, const cleo_cond_params& p, bool fuse_qcond) {
+  CondFlatArgs a{};
   a.s = c->buf[c->cur];
   a.off = c->off;
   a.nact = c->nact;
@@ -104,14 +104,13 @@ CondArgs cond_args(cleo_ctx* c, const cleo_cond_params& p, bool fuse_qcond) {
   a.sol = c->solute;
   a.cfg = NewtonCfg{step2dimlesstime(p.interval), p.minsubdelt_s / dimless::TIME0, p.rtol, p.atol, p.maxniters, 0u};
   a.ngbx = c->grid.ngbx;
-  a.wpb = wpb_or1(c->tiles.cond_waves_per_block);
   a.alter = p.do_alter_thermo;
   a.fuse_qcond = fuse_qcond ? 1 : 0;
   a.ctl = c->ctl;
   a.niters = c->rec_niters ? c->niters : nullptr;
-  a.warm = nullptr;
   a.warm_limit = p.warm_restart_iters;
   a.gs = c->gs;
+  a.dm = c->dm;
   return a;
 }
 
@@ -120,31 +119,23 @@ int enqueue_condensation(cleo_ctx* c, const cleo_cond_params& p, bool fuse_qcond
   if (p.interval == 0) return fail(c, CLEO_E_ARG, "condensation interval 0");
   if (!(p.minsubdelt_s > 0.0)) return fail(c, CLEO_E_ARG, "MINSUBTSTEP must be positive");
   materialize_order(c);  // the per-gridbox sums run in drop order
-  CondArgs a = cond_args(c, p, fuse_qcond);
-  // the thread-per-drop sequence evaluates the learned guesses itself (after the saturation
-  // ratios are known); the others read them from a separate guess pass
-  const bool inline_mlp = p.warm_start && c->tiles.cond_flat == 1;
-  if (p.warm_start && !inline_mlp) {
-    const int rc = mlp_enqueue_guess(c, p, &a.warm);
+  CondFlatArgs f = cond_args(c, p, fuse_qcond);
+  if (p.warm_start && c->cond_variant() == 1) {
+    // the thread-per-drop sequence evaluates the learned guesses itself (after the saturation
+    // ratios are known); the task ring reads them from a separate guess pass
+    const int rc = mlp_check_ready(c);
+    if (rc != CLEO_OK) return rc;
+    f.mlp_inline = 1;
+    f.W = mlp_weights(c);
+    f.warm_buf = mlp_warm_buffer(c);
+    f.guess_out = (c->rec_guess && c->guess) ? c->guess : nullptr;
+  } else if (p.warm_start) {
+    const int rc = mlp_enqueue_guess(c, p, &f.warm);
     if (rc != CLEO_OK) return rc;
     if (c->rec_guess && c->guess)
-      HIP_TRY(c, hipMemcpyAsync(c->guess, a.warm, c->ntot * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+      HIP_TRY(c, hipMemcpyAsync(c->guess, f.warm, c->ntot * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   }
-  if (c->tiles.cond_flat) {
-    CondFlatArgs f{a.s, a.off, a.nact, a.st, a.sol, a.cfg, a.ngbx, a.alter, a.fuse_qcond, a.ctl, a.niters,
-                   a.warm, a.warm_limit, c->gs, c->dm};
-    if (inline_mlp) {
-      const int rc = mlp_check_ready(c);
-      if (rc != CLEO_OK) return rc;
-      f.mlp_inline = 1;
-      f.W = mlp_weights(c);
-      f.warm_buf = mlp_warm_buffer(c);
-      f.guess_out = (c->rec_guess && c->guess) ? c->guess : nullptr;
-    }
-    launch_condensation_flat(c, f);
-  } else {
-    launch_condensation(c, a);
-  }
+  launch_condensation_flat(c, f);
   return launch_check(c);
 }
 
@@ -251,19 +242,15 @@ int enqueue_motion(cleo_ctx* c, const cleo_motion_params& p, bool qcond) {
   a.wpb = wpb_or1(c->tiles.motion_waves_per_block);
   a.cnt = c->cnt;
   a.ctl = c->ctl;
-  if (c->tiles.motion_flat == 2) {
+  if (c->motion_variant() == 2) {
     materialize_order(c);  // the fused pass ranks the drops in store order
     a.s = c->buf[c->cur];
     motion_sort_fused(c, a, c->buf[1 - c->cur], 1 - c->cur);
-  } else if (c->tiles.motion_flat == 3) {
+  } else if (c->motion_variant() == 3) {
     motion_sort_gather(c, a, c->buf[1 - c->cur], 1 - c->cur);
   } else {
-    if (c->tiles.motion_flat) {
-      a.step = c->dstep;  // the sort reads each drop's step instead of decoding its new key
-      launch_motion_flat(c, a);
-    } else {
-      launch_motion(c, a);
-    }
+    a.step = c->dstep;  // the sort reads each drop's step
+    launch_motion_flat(c, a);
     neighbour_sort_to(c, c->buf[c->cur], c->buf[1 - c->cur], 1 - c->cur, a.step);
   }
   if (qcond) {
@@ -289,9 +276,7 @@ int enqueue_motion_condensation(cleo_ctx* c, const cleo_motion_params& mp, const
   a.wpb = wpb_or1(c->tiles.motion_waves_per_block);
   a.cnt = c->cnt;
   a.ctl = c->ctl;
-  const CondArgs ca = cond_args(c, cp, true);
-  CondFlatArgs f{ca.s, ca.off, ca.nact, ca.st, ca.sol, ca.cfg, ca.ngbx, ca.alter, ca.fuse_qcond, ca.ctl, ca.niters,
-                 nullptr, ca.warm_limit, c->gs, c->dm};
+  CondFlatArgs f = cond_args(c, cp, true);
   if (cp.warm_start) {  // learned guesses, evaluated on the moved drops before the gather
     const int rc = mlp_check_ready(c);
     if (rc != CLEO_OK) return rc;
@@ -337,7 +322,7 @@ int enqueue_run_step(cleo_ctx* c, uint32_t t_mdl, uint32_t t_mdl_next) {
       for (uint32_t i = 0; i < p.n && first < 0; ++i)
         if (on_step(i, t_sdm)) first = static_cast<int>(i);
       const bool fuse = first >= 0 && p.proc[first].kind == CLEO_PROCESS_CONDENSATION &&
-                        (c->tiles.motion_flat == 1 || c->tiles.motion_flat == 3) && c->tiles.cond_flat == 1 &&
+                        (c->motion_variant() == 1 || c->motion_variant() == 3) && c->cond_variant() == 1 &&
                         !(p.proc[first].cond.warm_start && c->rec_guess);
       const int rc = fuse ? enqueue_motion_condensation(c, p.motion, p.proc[first].cond)
                           : enqueue_motion(c, p.motion, false);
@@ -1108,16 +1093,10 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
     c->kev_on = kernel_only;
     hipEventRecord(c->ev[14], c->stream);
     if (kern == 0) {
-      CondArgs a = cond_args(c, cp, false);
-      a.s = c->buf[spare];
-      a.niters = nullptr;
-      if (t.cond_flat) {
-        CondFlatArgs f{a.s, a.off, a.nact, a.st, a.sol, a.cfg, a.ngbx, a.alter, a.fuse_qcond, a.ctl, nullptr,
-                       nullptr, a.warm_limit, c->gs, c->dm};
-        launch_condensation_flat(c, f);
-      } else {
-        launch_condensation(c, a);
-      }
+      CondFlatArgs f = cond_args(c, cp, false);
+      f.s = c->buf[spare];
+      f.niters = nullptr;
+      launch_condensation_flat(c, f);
     } else if (kern == 1) {
       CollArgs a{};
       a.s = c->buf[spare];
@@ -1147,9 +1126,8 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
       a.wpb = t.motion_waves_per_block ? t.motion_waves_per_block : 1;
       a.cnt = c->cnt;
       a.ctl = c->ctl;
-      const CondArgs ca = cond_args(c, cp, true);
-      CondFlatArgs f{ca.s, ca.off, ca.nact, ca.st, ca.sol, ca.cfg, ca.ngbx, ca.alter, ca.fuse_qcond, ca.ctl, nullptr,
-                     nullptr, ca.warm_limit, c->gs, c->dm};
+      CondFlatArgs f = cond_args(c, cp, true);
+      f.niters = nullptr;
       motion_sort_condense(c, a, f, sorted, -1);
     } else {
       MotionArgs a{};
@@ -1162,17 +1140,13 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
       a.wpb = t.motion_waves_per_block ? t.motion_waves_per_block : 1;
       a.cnt = c->cnt;
       a.ctl = c->ctl;
-      if (t.motion_flat == 2) {
+      if (c->motion_variant() == 2) {
         motion_sort_fused(c, a, sorted, -1);
-      } else if (t.motion_flat == 3) {
+      } else if (c->motion_variant() == 3) {
         motion_sort_gather(c, a, sorted, -1);
       } else {
-        if (t.motion_flat) {
-          a.step = c->dstep;
-          launch_motion_flat(c, a);
-        } else {
-          launch_motion(c, a);
-        }
+        a.step = c->dstep;
+        launch_motion_flat(c, a);
         const bool on = c->kev_on;
         c->kev_on = false;  // the main kernel of the unfused stage is the motion kernel
         neighbour_sort_to(c, c->buf[spare], sorted, -1, a.step);
@@ -1206,40 +1180,31 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
   return CLEO_OK;
 }
 
-// Times each stage at 1, 2 and 4 waves (gridboxes) per workgroup, the thread-per-drop, tiled and
-// task-ring variants, and grids of one wave per gridbox or of 8192 / 32768 looping waves, on the
-// resident population, and keeps the fastest.  Drops and State are left unchanged.
+// Times each stage's variants (thread per drop and task ring; motion also fused with the sort and in
+// its gather; collisions with 1 or 4 tiles per workgroup), and grids of one wave per gridbox or of
+// 8192 / 32768 looping waves, on the resident population, and keeps the fastest.  Drops and State are
+// left unchanged.
 int cleo_autotune(cleo_ctx* c, cleo_tiles* chosen) {
   if (!c) return CLEO_E_ARG;
   if (c->ntot == 0) return fail(c, CLEO_E_STATE, "no superdroplets resident");
   HIP_TRY(c, hipStreamSynchronize(c->stream));
-  struct Cand {
-    uint32_t wpb, flat;
-  };
-  constexpr int kNC = 7;
-  const Cand cands[kNC] = {{1, 0}, {2, 0}, {4, 0}, {1, 1}, {4, 1}, {1, 2}, {1, 3}};  // {waves per block, variant}
   const uint32_t grid_waves[3] = {0, 8192, 32768};
   cleo_tiles best_t = c->tiles;
   for (int kern = 0; kern < 3; ++kern) {
     float best = 1e30f;
-    for (int gi = 0; gi < 3 * kNC; ++gi) {
-      const Cand& cd = cands[gi % kNC];
-      const uint32_t gw = grid_waves[gi / kNC];
-      if (kern != 1 && cd.flat && cd.wpb != 1) continue;  // thread-per-drop kernels ignore wpb
-      if (kern == 1 && cd.flat >= 2) continue;              // collisions have two variants
-      if (kern == 0 && cd.flat == 3) continue;              // condensation has three
+    const uint32_t nvar = kern == 2 ? 3u : 2u;
+    for (uint32_t i = 0; i < 3 * nvar; ++i) {
+      const uint32_t var = i % nvar + 1u, gw = grid_waves[i / nvar];
       cleo_tiles t = best_t;
       if (kern == 0) {
-        t.cond_waves_per_block = cd.wpb;
-        t.cond_flat = cd.flat;
+        t.cond_flat = var;
         t.cond_grid_waves = gw;
       } else if (kern == 1) {
-        t.coll_waves_per_block = cd.wpb;
-        t.coll_flat = cd.flat;
+        t.coll_flat = 1;
+        t.coll_waves_per_block = var == 1 ? 1 : 4;
         t.coll_grid_waves = gw;
       } else {
-        t.motion_waves_per_block = cd.wpb;
-        t.motion_flat = cd.flat;
+        t.motion_flat = var;
         t.motion_grid_waves = gw;
       }
       float tmin = 0.f;

@@ -48,19 +48,6 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 __device__ __forceinline__ uint32_t writelane_u32(uint32_t v, uint32_t x, uint32_t l) {
   return static_cast<uint32_t>(lane_id()) == l ? x : v;
 }
-__device__ __forceinline__ double readlane_f64(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-  return __hiloint2double(hi, lo);
-}
-
-// Adds the per-lane values v of lanes 0..m-1 to `acc` strictly in lane order, so a
-// gridbox sum keeps the sequential order of the reference's Serial reduction.
-__device__ __forceinline__ double ordered_add(double acc, double v, int m) {
-  for (int i = 0; i < m; ++i) acc += readlane_f64(v, i);
-  return acc;
-}
-
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);

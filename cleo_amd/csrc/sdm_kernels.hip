@@ -1,9 +1,10 @@
 // sdm_kernels.hip -- gfx950 kernels of the super-droplet step.
 //
-// Launch shape: one wave64 per gridbox, `wpb` waves per workgroup; with a capped grid each wave
-// loops over gridboxes g, g + (waves in the grid), ...  Drops of a gridbox are contiguous in the
-// SoA store (sorted by sdgbxindex), so every per-drop load and store of a wave is a coalesced run.  No kernel uses atomics on drop data: sums keep the
-// reference's sequential order and the sort is stable by construction.
+// Launch shapes: a thread per drop, or a wave64 per gridbox or few (with a capped grid each wave loops
+// over gridboxes g, g + (waves in the grid), ...).  Drops of a gridbox are contiguous in the SoA store
+// (sorted by sdgbxindex), so every per-drop load and store of a wave is a coalesced run.  No kernel
+// uses atomics on drop data: sums keep the reference's sequential order and the sort is stable by
+// construction.
 #include <algorithm>
 #include <cmath>
 
@@ -110,105 +111,7 @@ __device__ __forceinline__ double qcond_term(const SoA& s, const Solute& sol, De
   return m;
 }
 
-// ============================ condensation ====================================================
-// DoCondensation::do_condensation for one gridbox per wave (condensation.hpp:141-150,
-// condensation.cpp:44-137).  With `fuse_qcond`, the gridbox qcond of
-// EffectOnHydrometeorStatesFunctor (movesupersindomain.hpp:95-136) is recomputed first, as
-// happens between motion and condensation in the reference step.
-template <bool kFuseQcond>
-__device__ __forceinline__ void cond_gbx(const CondArgs& a, uint32_t g, int lane, uint32_t (&acc)[4]) {
-  const uint32_t base = a.off[g];
-  const uint32_t nfull = a.off[g + 1] - base;
-  const uint32_t n = a.nact[g];
-  const double temp = a.st.temp[g];
-  const double press = a.st.press[g];
-  double qv = a.st.qv[g];
-  double qc = a.st.qc[g];
-  const double volume = a.st.vol[g];
-  bool bad_cm = false;
-
-  if (kFuseQcond) {
-    double tot = 0.0;
-    for (uint32_t c = 0; c < nfull; c += kWave) {
-      const uint32_t k = base + c + lane;
-      double v = 0.0;
-      if (c + lane < nfull) {
-        v = condensate_mass(a.s.r[k], a.s.msol[k], a.sol, &bad_cm) * static_cast<double>(a.s.xi[k]);
-      }
-      const int m = static_cast<int>(min(static_cast<uint32_t>(kWave), nfull - c));
-      tot = ordered_add(tot, v, m);
-    }
-    const double rho_cond = tot / volume * dimless::R0cubed_VOL0;
-    const double rho_dry = dry_air_density(press, temp, qv);
-    qc = rho_cond / rho_dry;
-  }
-  if (temp <= 0 && lane == 0) set_error(a.ctl, CLEO_ERR_TEMP_NONPOSITIVE, g, base);
-  const double s_ratio = a.gs[kGsStride * g], ffactor = a.gs[kGsStride * g + 1];  // from k_gbx_thermo
-  const double akoh_g = a.gs[kGsStride * g + 2], inv_akoh_g = a.gs[kGsStride * g + 3];
-
-  double tot = 0.0;
-  uint32_t iters = 0, subs = 0, restarts = 0;
-  for (uint32_t c = 0; c < n; c += kWave) {
-    const uint32_t k = base + c + lane;
-    double dm = 0.0;
-    if (c + lane < n) {
-      const double r = a.s.r[k];
-      const double msol = a.s.msol[k];
-      const uint64_t xi = a.s.xi[k];
-      const double old_m = condensate_mass(r, msol, a.sol, &bad_cm);
-      const double akoh = akoh_g, bkoh = kohler_b(msol, a.sol);
-      const double warm = a.warm ? a.warm[k] : __longlong_as_double(0x7FF8000000000000ll);
-      SolveOut o{0, false, false, false, false};
-      const double newr = solve_condensation(a.cfg, s_ratio, akoh, bkoh, inv_akoh_g, ffactor, r, warm, a.warm_limit, o);
-      const double rnew = at_least_dry(newr, msol, a.sol);
-      a.s.r[k] = rnew;
-      dm = (condensate_mass(rnew, msol, a.sol, &bad_cm) - old_m) * static_cast<double>(xi);
-      if (o.maxed) set_error(a.ctl, CLEO_ERR_NEWTON_MAXITERS, g, k);
-      if (a.niters) a.niters[k] = o.iters;
-      iters += o.iters;
-      subs += o.substep ? 1u : 0u;
-      restarts += o.restarted ? 1u : 0u;
-    }
-    const int m = static_cast<int>(min(static_cast<uint32_t>(kWave), n - c));
-    tot = ordered_add(tot, dm, m);
-  }
-  if (bad_cm) set_error(a.ctl, CLEO_ERR_NEG_CONDENSATE, g, base);
-
-  // EffectOnThermodynamicStateFunctor::state_change (condensation.cpp:126-137)
-  double tnew = temp;
-  if (a.alter) {
-    const double totrho = tot / volume * dimless::R0cubed_VOL0;
-    const double rho_dry = dry_air_density(press, temp, qv);
-    const double dq = totrho / rho_dry;
-    qv -= dq;
-    qc += dq;
-    const double dtemp = (dimless::Latent_v / moist_specific_heat(qv, qc)) * dq;
-    tnew += dtemp;
-  }
-  iters = wave_sum_u32(iters);
-  subs = wave_sum_u32(subs);
-  restarts = wave_sum_u32(restarts);
-  if (lane == 0) {
-    if (a.alter) {
-      a.st.temp[g] = tnew;
-      a.st.qv[g] = qv;
-    }
-    if (a.alter || kFuseQcond) a.st.qc[g] = qc;
-  }
-  acc[0] += n;
-  acc[1] += iters;
-  acc[2] += subs;
-  acc[3] += restarts;
-}
-template <bool kFuseQcond>
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_condensation(CondArgs a) {
-  const int lane = lane_id();
-  uint32_t acc[4] = {0, 0, 0, 0};
-  for (uint32_t g = wave_index(); g < a.ngbx; g += wave_count()) cond_gbx<kFuseQcond>(a, g, lane, acc);
-  if (lane == 0)
-    for (int j = 0; j < 4; ++j) put_stat(a.stat, ST_COND_DROPS + j, acc[j]);
-}
-
+// ============================ qcond ===========================================================
 // EffectOnHydrometeorStatesFunctor (movesupersindomain.hpp:95-136), standalone: 64 gridboxes per
 // wave, drop-order sums of condensed mass, then one lane per gridbox for its qcond
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_qcond(QcondArgs a) {
@@ -943,50 +846,6 @@ __device__ __forceinline__ Moved move_drop(const MotionArgs& a, uint32_t g, cons
   return move_drop(a, g, G, drop_pos(a, k), k, report);
 }
 
-// MoveSupersInGridboxesFunctor (movesupersindomain.hpp:47-93) with PredCorrMotion over
-// CartesianMaps; also counts, per gridbox, how many drops go to each of the 27 neighbour
-// directions (and out of the domain) for the stable neighbour sort.
-__device__ __forceinline__ uint32_t motion_gbx(const MotionArgs& a, uint32_t g, int lane) {
-  const uint32_t base = a.off[g];
-  const uint32_t nfull = a.off[g + 1] - base;
-  const GbxGeom G = gbx_geom(a, g);
-  uint32_t mycount = 0;
-  for (uint32_t c = 0; c < nfull; c += kWave) {
-    const uint32_t k = base + c + lane;
-    const bool act = c + lane < nfull;
-    int dir = 0;
-    if (act) {
-      const Moved M = move_drop(a, g, G, k, true);
-      a.s.c3[k] = M.c3;
-      a.s.c1[k] = M.c1;
-      a.s.c2[k] = M.c2;
-      a.s.gbx[k] = M.idx;
-      dir = M.dir;
-    }
-    uint64_t mask = __ballot(act);
-    while (mask) {
-      const int leader = __ffsll(static_cast<unsigned long long>(mask)) - 1;
-      const int v = static_cast<int>(readlane_u32(static_cast<uint32_t>(dir), leader));
-      const uint64_t m = __ballot(act && dir == v);
-      if (lane == v) mycount += static_cast<uint32_t>(__popcll(m));
-      mask &= ~m;
-    }
-  }
-  // destination-major counts: row d column s = drops arriving at d by the step s; column 27 of the
-  // source's own row = drops leaving the domain (the table is zero-filled before motion)
-  if (lane == 27)
-    a.cnt[28ull * g + 27] = mycount;
-  else if (lane < 27 && mycount > 0)
-    a.cnt[28ull * neighbour_of(a.grid, g, lane) + lane] = mycount;
-  return nfull;
-}
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_motion(MotionArgs a) {
-  const int lane = lane_id();
-  uint32_t moved = 0;
-  for (uint32_t g = wave_index(); g < a.grid.ngbx; g += wave_count()) moved += motion_gbx(a, g, lane);
-  if (lane == 0) put_stat(a.stat, ST_MOTION_DROPS, moved);
-}
-
 // ============================ neighbour sort ==================================================
 
 // base[] of the sorted store, the first place of each gridbox (and of each gridbox's drops that leave
@@ -1159,7 +1018,6 @@ __global__ void __launch_bounds__(1024) k_nsort_part(uint32_t* part, uint32_t nb
 // neighbour_of, without a division per lane).  A g past the last gridbox gives an empty head.
 struct RankHead {
   uint32_t g, sbase, nfull, trun, base;
-  int gz, gx, gy;
 };
 __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, int gz, int gx, int gy, int32_t noff,
                                               int lane) {
@@ -1167,7 +1025,7 @@ __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, in
   const int nz = static_cast<int>(a.grid.nz), nx = static_cast<int>(a.grid.nx), ny = static_cast<int>(a.grid.ny);
   const bool valid = g < ngbx;
   const uint32_t gc = valid ? static_cast<uint32_t>(g) : ngbx - 1u;
-  RankHead h{gc, 0u, 0u, 0u, 0u, gz, gx, gy};
+  RankHead h{gc, 0u, 0u, 0u, 0u};
   const uint32_t lo = a.off[gc], hi = a.off[gc + 1];
   h.sbase = lo;
   h.nfull = valid ? hi - lo : 0u;
@@ -1218,68 +1076,37 @@ __device__ __forceinline__ RankSlots rank_slots(const NsortArgs& a, const RankHe
   }
   return RankSlots{i0 < h.nfull ? p0 : kOOB, i1 < h.nfull ? p1 : kOOB};
 }
-// the step recorded for each of those drops (kStep), or its gridbox key; 0 for no drop
+// the step recorded for each of those drops
 struct RankKeys {
   uint32_t k0, k1;
 };
-template <bool kStep>
 __device__ __forceinline__ RankKeys rank_keys(const NsortArgs& a, const RankSlots& s, uint32_t nsrc) {
   const uint32_t c0 = s.p0 < nsrc ? s.p0 : 0u, c1 = s.p1 < nsrc ? s.p1 : 0u;
-  uint32_t k0, k1;
-  if constexpr (kStep) {
-    k0 = a.step[c0];
-    k1 = a.step[c1];
-  } else {
-    k0 = a.src.gbx[c0];
-    k1 = a.src.gbx[c1];
-  }
-  return RankKeys{k0, k1};
+  return RankKeys{a.step[c0], a.step[c1]};
 }
 // ranks the drops of the head's gridbox and records perm[dest] = p (stable scatter above); the
 // first two chunks use the preloaded positions and keys, later chunks load their own
-template <bool kOrder, bool kStep>
+template <bool kOrder>
 __device__ __forceinline__ void rank_gbx(const NsortArgs& a, const RankHead& h, const RankSlots& s, const RankKeys& k,
                                          uint32_t nsrc, int lane) {
-  const uint32_t g = h.g, sbase = h.sbase, nfull = h.nfull, ngbx = a.grid.ngbx;
-  const int nz = static_cast<int>(a.grid.nz), nx = static_cast<int>(a.grid.nx), ny = static_cast<int>(a.grid.ny);
-  const int gz = h.gz, gx = h.gx, gy = h.gy;
+  const uint32_t g = h.g, sbase = h.sbase, nfull = h.nfull;
   uint32_t trun = h.trun;
   if (lane == 13) a.off_new[g] = h.base;  // step 13 stays: the new refs
-  auto near = [](int q, int r, int nd, bool per) {
-    const int dd = q - r;
-    if (dd >= -1 && dd <= 1) return true;
-    return per && (dd == nd - 1 || dd == 1 - nd);
-  };
-  auto step = [](int q, int r) {
-    const int dd = q - r;
-    return dd > 1 ? -1 : (dd < -1 ? 1 : dd);
-  };
   // chunk c of 64 slots: the drop of slot sbase + c + lane is at position p with key kv
   auto chunk = [&](uint32_t c, uint32_t p, uint32_t kv) {
     const uint32_t q = sbase + c + lane;
     const bool act = c + lane < nfull;
-    // the step g -> key (27: out of the domain): recorded by motion, or found from the key; a key
-    // that is no neighbour of g, or a position outside the domain, is an error
+    // the step motion recorded (27: out of the domain); another value, or a position outside the
+    // domain, is an error
     int sv = 27;
     bool ok = act;
     if (act && p >= nsrc) {
       set_error(a.ctl, CLEO_ERR_SORT_NONLOCAL, g, q);
       ok = false;
     }
-    if (ok && kStep) {
+    if (ok) {
       sv = static_cast<int>(kv);
       if (sv > 27) {
-        set_error(a.ctl, CLEO_ERR_SORT_NONLOCAL, g, p);
-        ok = false;
-      }
-    } else if (ok && kv == g) {
-      sv = 13;
-    } else if (ok && kv < ngbx) {
-      const int vz = static_cast<int>(kv % a.grid.nz), vx = static_cast<int>((kv / a.grid.nz) % a.grid.nx),
-                vy = static_cast<int>(kv / (a.grid.nz * a.grid.nx));
-      if (near(vz, gz, nz, a.grid.per[0]) && near(vx, gx, nx, a.grid.per[1]) && near(vy, gy, ny, a.grid.per[2])) {
-        sv = (step(vz, gz) + 1) + 3 * (step(vx, gx) + 1) + 9 * (step(vy, gy) + 1);
-      } else {
         set_error(a.ctl, CLEO_ERR_SORT_NONLOCAL, g, p);
         ok = false;
       }
@@ -1313,7 +1140,7 @@ __device__ __forceinline__ void rank_gbx(const NsortArgs& a, const RankHead& h, 
     const bool act = c + lane < nfull;
     const uint32_t q = sbase + c + lane;
     const uint32_t p = act ? (kOrder ? a.order[q] : q) : kOOB;
-    const uint32_t kv = (act && p < nsrc) ? (kStep ? a.step[p] : a.src.gbx[p]) : 0u;
+    const uint32_t kv = (act && p < nsrc) ? a.step[p] : 0u;
     chunk(c, p, kv);
   }
 }
@@ -1321,8 +1148,8 @@ __device__ __forceinline__ void rank_gbx(const NsortArgs& a, const RankHead& h, 
 // Gridboxes go to waves through xcd_wave_index(), so each XCD sweeps one contiguous range and the
 // count-table rows that neighbouring gridboxes share are fetched into one L2.  The gridbox's
 // (z, x, y) advance by the stride's with carries (no division per gridbox).
-template <bool kOrder, bool kStep>
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kStep ? 6 : 4) k_nsort_perm(NsortArgs a) {
+template <bool kOrder>
+__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(6) k_nsort_perm(NsortArgs a) {
   const int lane = lane_id();
   const uint32_t nz = a.grid.nz, nx = a.grid.nx;
   const uint64_t ngbx = a.grid.ngbx;
@@ -1357,14 +1184,14 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kStep ? 6 : 4) k_nsort_per
   RankSlots S0 = rank_slots<kOrder>(a, H0, nsrc, lane), S1, S2, S3;
   H2 = next_head();
   S1 = rank_slots<kOrder>(a, H1, nsrc, lane);
-  RankKeys K0 = rank_keys<kStep>(a, S0, nsrc), K1, K2, K3;
+  RankKeys K0 = rank_keys(a, S0, nsrc), K1, K2, K3;
   // gridbox i: loads the head of i + 3, the slots of i + 2, the keys of i + 1, then ranks i
   auto stage = [&](const RankHead& hu, RankHead& hl, const RankHead& hs, const RankSlots& su, RankSlots& sl,
                    const RankSlots& sk, const RankKeys& ku, RankKeys& kl) {
     hl = next_head();
     sl = rank_slots<kOrder>(a, hs, nsrc, lane);
-    kl = rank_keys<kStep>(a, sk, nsrc);
-    rank_gbx<kOrder, kStep>(a, hu, su, ku, nsrc, lane);
+    kl = rank_keys(a, sk, nsrc);
+    rank_gbx<kOrder>(a, hu, su, ku, nsrc, lane);
   };
   for (uint64_t g = g0;;) {
     stage(H0, H3, H2, S0, S2, S1, K0, K1);
@@ -1856,17 +1683,12 @@ static inline unsigned drop_blocks(uint64_t n, uint32_t grid_waves) {
   const unsigned b = nblocks(n, 256);
   return grid_waves ? std::min<unsigned>(b, std::max<unsigned>(1u, grid_waves / 4)) : b;
 }
-// launches k_nsort_perm for the order and key source of `a`
 static void launch_nsort_perm(cleo_ctx* c, const NsortArgs& a, uint32_t ngbx) {
   const dim3 grid(gbx_blocks(ngbx, a.wpb, c->tiles.motion_grid_waves)), block(64 * a.wpb);
-  if (a.order && a.step)
-    hipLaunchKernelGGL((k_nsort_perm<true, true>), grid, block, 0, c->stream, a);
-  else if (a.order)
-    hipLaunchKernelGGL((k_nsort_perm<true, false>), grid, block, 0, c->stream, a);
-  else if (a.step)
-    hipLaunchKernelGGL((k_nsort_perm<false, true>), grid, block, 0, c->stream, a);
+  if (a.order)
+    hipLaunchKernelGGL(k_nsort_perm<true>, grid, block, 0, c->stream, a);
   else
-    hipLaunchKernelGGL((k_nsort_perm<false, false>), grid, block, 0, c->stream, a);
+    hipLaunchKernelGGL(k_nsort_perm<false>, grid, block, 0, c->stream, a);
 }
 static inline unsigned stride_blocks(uint64_t n) {
   const uint64_t b = (n + 255) / 256;
@@ -1879,25 +1701,6 @@ static inline unsigned sparse_blocks(uint64_t n) { return std::min<unsigned>(str
 
 __global__ void k_set_u32(uint32_t* out, uint32_t v) { *out = v; }
 
-// supersaturation ratio and diffusion factor of every gridbox (thread per gridbox) for
-// k_condensation: the correctly rounded exp of the saturation pressure, evaluated here, would
-// otherwise cost the per-gridbox solve kernel its registers
-__global__ void k_gbx_thermo(GState st, uint32_t ngbx, double* gs) {
-  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < ngbx; g += gridDim.x * blockDim.x) gbx_thermo(st, g, gs);
-}
-void launch_condensation(cleo_ctx* c, const CondArgs& args) {
-  if (args.ngbx == 0) return;
-  CondArgs a = args;
-  hipLaunchKernelGGL(k_gbx_thermo, dim3(stride_blocks(a.ngbx)), dim3(256), 0, c->stream, a.st, a.ngbx, a.gs);
-  const unsigned nb = gbx_blocks(a.ngbx, a.wpb, c->tiles.cond_grid_waves);
-  a.stat = stat_slots(c);
-  kev_mark(c, 0);
-  if (a.fuse_qcond)
-    hipLaunchKernelGGL(k_condensation<true>, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
-  else
-    hipLaunchKernelGGL(k_condensation<false>, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
-  kev_mark(c, 1);
-}
 // Gridboxes per tile of the per-gridbox sums: as many as leave 8192 waves, but at least the 512 drops
 // of a window.  Mass moments with 64 / by this rule / 1 gridbox per tile: 32^3 gridboxes of 64 drops
 // 41 / 17 / 51 us, 24679 of 300 drops 478 (at 256 waves) / 96 / 115 us, 3750 of 128 drops 160 / 12 /
@@ -1941,7 +1744,7 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   // wave walks through its 64 gridboxes' swaps and pairs in about 1.2 us per drop of the mean, so
   // they need enough gridboxes to fill the chip (32^3 gridboxes of 64: 81 us against 45 us; the
   // lines cross near 75,000 gridboxes at any mean) whose drops fit a tile's 8 KB of permutations.
-  if (c->tiles.coll_flat && a.ngbx >= kTileMinGbx && mean <= kTilePermBytes / kWave + 4) {
+  if (a.ngbx >= kTileMinGbx && mean <= kTilePermBytes / kWave + 4) {
     const unsigned nb = gbx_blocks((a.ngbx + kWave - 1) / kWave, a.wpb, c->tiles.coll_grid_waves);
     a.stat = stat_slots(c);
     kev_mark(c, 0);
@@ -1965,15 +1768,6 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   } else {
     launch_coll_team<1024>(c, a, 1u, 2 * mean);
   }
-}
-void launch_motion(cleo_ctx* c, const MotionArgs& args) {
-  if (args.grid.ngbx == 0) return;
-  MotionArgs a = args;
-  const unsigned nb = gbx_blocks(a.grid.ngbx, a.wpb, c->tiles.motion_grid_waves);
-  a.stat = stat_slots(c);
-  kev_mark(c, 0);
-  hipLaunchKernelGGL(k_motion, dim3(nb), dim3(64 * a.wpb), 0, c->stream, a);
-  kev_mark(c, 1);
 }
 StatSlots stat_slots(cleo_ctx* c) { return StatSlots{c->sp}; }
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np) {
@@ -3127,15 +2921,15 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
   CondFlatArgs a = args;
   // the thread-per-drop solve records each drop's qcond term, so the qcond recompute after motion
   // joins k_cond_state (the task ring keeps it in k_cond_prep)
-  a.qm = (a.fuse_qcond && c->tiles.cond_flat == 1) ? c->qm : nullptr;
+  a.qm = (a.fuse_qcond && c->cond_variant() == 1) ? c->qm : nullptr;
   const uint32_t gw = c->tiles.cond_grid_waves;
   a.gpt = sum_gpt(c);
-  const uint32_t budget = c->tiles.cond_flat == 2 ? 0u : c->tiles.cond_defer;
+  const uint32_t budget = c->cond_variant() == 2 ? 0u : c->defer_budget();
   a.cfg.budget = budget;
   a.dlist = c->dlist;
   a.dcount = c->dcount;
   hipLaunchKernelGGL(k_cond_prep, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
-  if (c->tiles.cond_flat == 2) {
+  if (c->cond_variant() == 2) {
     // task-ring kernel: waves of 4 per block; by default as many waves as fit on the device at once
     const uint64_t waves = gw ? gw : static_cast<uint64_t>(c->num_cu) * kCondQueueWavesPerCu;
     const unsigned nb = static_cast<unsigned>(std::max<uint64_t>(1, std::min<uint64_t>(waves / 4, (c->ntot + 255) / 256)));
@@ -3176,7 +2970,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   m.step = c->dstep;
   // motion variant 3: the drops move inside the gather (the counting pass writes only the steps);
   // not with learned guesses, which are evaluated on the moved store before the gather
-  const bool move_in_gather = c->tiles.motion_flat == 3 && !cond.mlp_inline && !cond.warm;
+  const bool move_in_gather = c->motion_variant() == 3 && !cond.mlp_inline && !cond.warm;
   const bool on = c->kev_on;
   c->kev_on = false;  // the main kernel of this sequence is the gather with the solves
   if (move_in_gather) {
@@ -3196,7 +2990,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   a.qm = c->qm;  // the qcond recompute joins k_cond_state
   const uint32_t gw = c->tiles.cond_grid_waves;
   a.gpt = sum_gpt(c);
-  const uint32_t budget = c->tiles.cond_defer;
+  const uint32_t budget = c->defer_budget();
   a.cfg.budget = budget;
   a.dlist = c->dlist;
   a.dcount = c->dcount;

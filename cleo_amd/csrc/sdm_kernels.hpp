@@ -23,25 +23,6 @@ constexpr uint32_t kTabBlock = 256;
 // LDS window (values) of the per-gridbox drop-order sums
 constexpr uint32_t kSumWin = 1024;
 
-struct CondArgs {
-  SoA s;
-  const uint32_t* off;
-  const uint32_t* nact;
-  GState st;
-  Solute sol;
-  NewtonCfg cfg;
-  uint32_t ngbx;
-  uint32_t wpb;
-  int32_t alter;
-  int32_t fuse_qcond;
-  DevCtl* ctl;
-  uint32_t* niters;
-  const double* warm;
-  uint32_t warm_limit;
-  StatSlots stat;  // ST_COND_DROPS .. ST_WARM_RESTARTS
-  double* gs;      // per gridbox (kGsStride): supersaturation ratio, diffusion factor, Koehler a (k_gbx_thermo)
-};
-
 struct QcondArgs {
   SoA s;
   const uint32_t* off;
@@ -108,7 +89,7 @@ struct NsortArgs {
   DevCtl* ctl;
   uint64_t ntot;
   uint32_t* perm;          // source position of each destination position of the domain's drops
-  const uint8_t* step;     // non-null: each drop's step from motion, read instead of its key
+  const uint8_t* step;     // each drop's step from motion
   const uint32_t* order;   // non-null: position of the drop at each slot of the logical order
 };
 
@@ -153,10 +134,8 @@ struct CondFlatArgs {
 // launchers (sdm_kernels.hip); all enqueue on ctx->stream
 void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& a);
 void launch_motion_flat(cleo_ctx* c, const MotionArgs& a);
-void launch_condensation(cleo_ctx* c, const CondArgs& a);
 void launch_qcond(cleo_ctx* c, const QcondArgs& a);
 void launch_collisions(cleo_ctx* c, const CollArgs& a);
-void launch_motion(cleo_ctx* c, const MotionArgs& a);
 // the statistics rows of the context
 StatSlots stat_slots(cleo_ctx* c);
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np);

@@ -395,23 +395,24 @@ typedef struct {
   uint32_t cond_waves_per_block;   /* gridboxes (waves) per workgroup, 1..4 */
   uint32_t coll_waves_per_block;
   uint32_t motion_waves_per_block;
-  uint32_t cond_flat;              /* 1: one thread per drop + per-gridbox prep/sum kernels;
+  uint32_t cond_flat;              /* 0, 1: one thread per drop + per-gridbox prep/sum kernels (0:
+                                      with drops set aside after 8 iterations, whatever cond_defer);
                                       2: the same with each wave's drops fed to its lanes from a
                                          task ring (lanes do not wait for slower drops) */
-  uint32_t motion_flat;            /* 1: one thread per drop (two per thread), direction counts by
+  uint32_t motion_flat;            /* 0, 1: one thread per drop (two per thread), direction counts by
                                          atomics; 2: motion and sort fused (a counting pass, then
                                          each drop moved again straight to its sorted place);
                                       3: a counting pass, then the sort's gather moves each drop
-                                         as it copies it to its sorted place (with cond_flat 1 and
-                                         a condensation due, the same gather also solves it) */
+                                         as it copies it to its sorted place.  With 0, 1 or 3,
+                                         cond_flat 0 or 1 and a condensation due, the sort's gather
+                                         also solves it */
   uint32_t cond_grid_waves;        /* waves per launch; each loops over gridboxes (or drops) */
   uint32_t coll_grid_waves;        /*   0: one wave per gridbox (one thread per drop) */
   uint32_t motion_grid_waves;
-  uint32_t coll_flat;              /* 1: 64 gridboxes per wave, pairs flattened over the lanes, on
-                                      domains that fill the chip that way (else as 0: a wave or a
-                                      workgroup per gridbox or few) */
+  uint32_t coll_flat;              /* 0 or 1: collisions by tiles of 64 gridboxes per wave where those
+                                      fill the chip, else by a wave or a workgroup per gridbox or few */
   uint32_t cond_defer;             /* cond_flat 1: Newton iterations after which a drop is set
-                                      aside and solved by a second launch (0: never) */
+                                      aside and solved later, packed with others (0: never) */
 } cleo_tiles;
 int cleo_set_tiles(cleo_ctx* ctx, const cleo_tiles* tiles);
 int cleo_get_tiles(cleo_ctx* ctx, cleo_tiles* tiles);
