@@ -60,13 +60,19 @@ void free_soa(SoA& s) {
   s = SoA{};
 }
 
+// the work enqueued so far is done and h_ctl holds the control block as it left it
+hipError_t fetch_ctl(cleo_ctx* c) {
+  launch_publish_ctl(c);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
+}
 // synchronise, then report a recorded device error
 int sync_check(cleo_ctx* c) {
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  HIP_TRY(c, ctx_copy(c, c->h_ctl, c->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost));
-  if (c->h_ctl->err_code != 0) {
-    c->msg = "device error " + std::to_string(c->h_ctl->err_code) + " at gridbox " +
-             std::to_string(c->h_ctl->err_gbx) + " drop " + std::to_string(c->h_ctl->err_drop);
+  HIP_TRY(c, fetch_ctl(c));
+  const DevCtl& k = c->h_ctl->ctl;
+  if (k.err_code != 0) {
+    c->msg = "device error " + std::to_string(k.err_code) + " at gridbox " + std::to_string(k.err_gbx) + " drop " +
+             std::to_string(k.err_drop);
     return CLEO_E_DEVICE;
   }
   return CLEO_OK;
@@ -386,54 +392,85 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   c->grid.ny = static_cast<uint32_t>(ny);
   c->grid.ngbx = static_cast<uint32_t>(ngbx);
   for (int i = 0; i < 3; ++i) c->grid.per[i] = dom->periodic[i] ? 1 : 0;
-  const uint64_t nh = nz + nx + ny + 3;
-  HIP_TRY(c, dalloc(&c->d_halves, nh));
-  HIP_TRY(c, ctx_copy(c, c->d_halves, dom->zhalf, (nz + 1) * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, c->d_halves + nz + 1, dom->xhalf, (nx + 1) * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, c->d_halves + nz + nx + 2, dom->yhalf, (ny + 1) * 8, hipMemcpyHostToDevice));
-  c->grid.zh = c->d_halves;
-  c->grid.xh = c->d_halves + nz + 1;
-  c->grid.yh = c->d_halves + nz + nx + 2;
   c->maxn = maxn;
-  HIP_TRY(c, alloc_soa(c->buf[0], maxn));
-  HIP_TRY(c, alloc_soa(c->buf[1], maxn));
-  HIP_TRY(c, dalloc(&c->off, ngbx + 1));
-  HIP_TRY(c, dalloc(&c->off_alt, ngbx + 1));
-  HIP_TRY(c, dalloc(&c->nact, ngbx));
-  HIP_TRY(c, dalloc(&c->d_state, 11 * ngbx));
+  const uint64_t nh = nz + nx + ny + 3;
+  const uint64_t nd = std::max<uint64_t>(maxn, 1);
+  // The context's arrays: those that start from zero in one allocation, cleared at once; the others in
+  // one more unless they are large (48 allocations of a few kB took most of the time to create a small
+  // context).
+  struct Part {
+    void** p;
+    size_t bytes;
+  };
+  std::vector<Part> zero, rest;
+  auto want = [](std::vector<Part>& to, auto** p, uint64_t n) {
+    to.push_back(Part{reinterpret_cast<void**>(p), (std::max<uint64_t>(n, 1) * sizeof(**p) + 255) / 256 * 256});
+  };
+  want(zero, &c->ctl, 1);
+  want(zero, &c->sp, kStatRow * kStatRows);
+  want(zero, &c->off, ngbx + 1);
+  want(zero, &c->off_alt, ngbx + 1);
+  want(zero, &c->nact, ngbx);
+  want(zero, &c->d_state, 11 * ngbx);
+  want(zero, &c->cnt, 56 * ngbx);  // counts, then the run offsets of the neighbour sort
+  want(zero, &c->tot, ngbx + 1);
+  want(rest, &c->d_halves, nh);
+  want(rest, &c->oobpre, ngbx + 1);
+  want(rest, &c->part, 2 * ((ngbx + kTabBlock - 1) / kTabBlock) + 1);
+  want(rest, &c->inj_oj, ngbx + 1);
+  want(rest, &c->inj_op, ngbx + 1);
+  want(rest, &c->gs, kGsStride * ngbx);
+  c->scan_tmp_n = scan_tmp_words(ngbx + 1);
+  want(rest, &c->scan_tmp, c->scan_tmp_n);
+  for (SoA& b : c->buf) {
+    want(rest, &b.gbx, nd);
+    for (double** f : {&b.c3, &b.c1, &b.c2, &b.r, &b.msol}) want(rest, f, nd);
+    for (uint64_t** f : {&b.xi, &b.id}) want(rest, f, nd);
+  }
+  want(rest, &c->big_scratch, 2 * nd);
+  want(rest, &c->dm, nd);
+  want(rest, &c->qm, nd);
+  want(rest, &c->dlist, nd);
+  want(rest, &c->dcount, nd / 256 + 1);
+  want(rest, &c->perm, nd);
+  want(rest, &c->dstep, nd);
+  want(rest, &c->order, nd);
+  want(rest, &c->order_alt, nd);
+  auto allocate = [&](const std::vector<Part>& parts, bool together) -> hipError_t {
+    size_t total = 0;
+    for (const Part& q : parts) total += q.bytes;
+    unsigned char* at = nullptr;
+    for (const Part& q : parts) {
+      if (!together || !at) {
+        void* p = nullptr;
+        const hipError_t e = hipMalloc(&p, together ? total : q.bytes);
+        if (e != hipSuccess) return e;
+        c->owned.push_back(p);
+        at = static_cast<unsigned char*>(p);
+      }
+      *q.p = at;
+      at += q.bytes;
+    }
+    return hipSuccess;
+  };
+  size_t zero_bytes = 0, rest_bytes = 0;
+  for (const Part& q : zero) zero_bytes += q.bytes;
+  for (const Part& q : rest) rest_bytes += q.bytes;
+  HIP_TRY(c, allocate(zero, true));
+  HIP_TRY(c, allocate(rest, rest_bytes <= (64u << 20)));
+  HIP_TRY(c, hipHostMalloc(reinterpret_cast<void**>(&c->h_ctl), 4096 + kStageBytes, hipHostMallocDefault));
+  c->stage = reinterpret_cast<unsigned char*>(c->h_ctl) + 4096;
   double* s = c->d_state;
   c->st = GState{s, s + ngbx, s + 2 * ngbx, s + 3 * ngbx, s + 4 * ngbx, s + 5 * ngbx,
                  s + 6 * ngbx, s + 7 * ngbx, s + 8 * ngbx, s + 9 * ngbx, s + 10 * ngbx};
-  HIP_TRY(c, dalloc(&c->cnt, 56 * ngbx));  // counts, then the run offsets of the neighbour sort
-  HIP_TRY(c, dalloc(&c->tot, ngbx + 1));
-  HIP_TRY(c, dalloc(&c->oobpre, ngbx + 1));
-  HIP_TRY(c, dalloc(&c->part, 2 * ((ngbx + kTabBlock - 1) / kTabBlock) + 1));
-  HIP_TRY(c, dalloc(&c->inj_oj, ngbx + 1));
-  HIP_TRY(c, dalloc(&c->inj_op, ngbx + 1));
-  c->scan_tmp_n = scan_tmp_words(28 * ngbx + 1);
-  HIP_TRY(c, dalloc(&c->scan_tmp, c->scan_tmp_n));
-  HIP_TRY(c, dalloc(&c->big_scratch, 2 * maxn));
-  HIP_TRY(c, dalloc(&c->gs, kGsStride * ngbx));
-  HIP_TRY(c, dalloc(&c->dm, maxn));
-  HIP_TRY(c, dalloc(&c->sp, kStatRow * kStatRows));
-  HIP_TRY(c, dalloc(&c->dlist, maxn));
-  HIP_TRY(c, dalloc(&c->dcount, maxn / 256 + 1));
-  HIP_TRY(c, dalloc(&c->perm, std::max<uint64_t>(maxn, 1)));
-  HIP_TRY(c, dalloc(&c->dstep, std::max<uint64_t>(maxn, 1)));
-  HIP_TRY(c, dalloc(&c->order, std::max<uint64_t>(maxn, 1)));
-  HIP_TRY(c, dalloc(&c->order_alt, std::max<uint64_t>(maxn, 1)));
-  HIP_TRY(c, dalloc(&c->qm, std::max<uint64_t>(maxn, 1)));
-  c->big_scratch_n = 2 * maxn;
-  HIP_TRY(c, dalloc(&c->ctl, 1));
-  HIP_TRY(c, hipHostMalloc(reinterpret_cast<void**>(&c->h_ctl), sizeof(DevCtl), hipHostMallocDefault));
-  HIP_TRY(c, hipMemsetAsync(c->ctl, 0, sizeof(DevCtl), c->stream));
-  HIP_TRY(c, hipMemsetAsync(c->sp, 0, kStatRow * kStatRows * 8, c->stream));
-  HIP_TRY(c, hipMemsetAsync(c->off, 0, (ngbx + 1) * 4, c->stream));
-  HIP_TRY(c, hipMemsetAsync(c->off_alt, 0, (ngbx + 1) * 4, c->stream));
-  HIP_TRY(c, hipMemsetAsync(c->nact, 0, ngbx * 4, c->stream));
-  HIP_TRY(c, hipMemsetAsync(c->cnt, 0, 28 * ngbx * 4, c->stream));
-  HIP_TRY(c, hipMemsetAsync(c->tot, 0, (ngbx + 1) * 4, c->stream));
-  HIP_TRY(c, hipMemsetAsync(c->d_state, 0, 11 * ngbx * 8, c->stream));
+  c->grid.zh = c->d_halves;
+  c->grid.xh = c->d_halves + nz + 1;
+  c->grid.yh = c->d_halves + nz + nx + 2;
+  std::vector<double> faces(dom->zhalf, dom->zhalf + nz + 1);
+  faces.insert(faces.end(), dom->xhalf, dom->xhalf + nx + 1);
+  faces.insert(faces.end(), dom->yhalf, dom->yhalf + ny + 1);
+  HIP_TRY(c, hipMemsetAsync(c->ctl, 0, zero_bytes, c->stream));
+  HIP_TRY(c, hipMemcpyAsync(c->d_halves, faces.data(), nh * 8, hipMemcpyHostToDevice, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   c->solute = make_solute(2016.5 / dimless::RHO0, 0.05844277 / dimless::MR0, 2.0);
   HIP_TRY(c, mlp_create(c));
@@ -445,18 +482,10 @@ int cleo_destroy(cleo_ctx* c) {
   if (!c) return CLEO_OK;
   hipStreamSynchronize(c->stream);
   mlp_destroy(c);
-  free_soa(c->buf[0]);
-  free_soa(c->buf[1]);
-  for (void* p : {static_cast<void*>(c->d_halves), static_cast<void*>(c->off), static_cast<void*>(c->off_alt),
-                  static_cast<void*>(c->nact), static_cast<void*>(c->d_state), static_cast<void*>(c->cnt),
-                  static_cast<void*>(c->tot), static_cast<void*>(c->oobpre), static_cast<void*>(c->part), static_cast<void*>(c->inj_oj),
-                  static_cast<void*>(c->inj_op), static_cast<void*>(c->scan_tmp), static_cast<void*>(c->big_scratch),
-                  static_cast<void*>(c->ctl), static_cast<void*>(c->inj_j), static_cast<void*>(c->inj_phi),
-                  static_cast<void*>(c->niters), static_cast<void*>(c->guess), static_cast<void*>(c->rs_key[0]),
-                  static_cast<void*>(c->rs_key[1]), static_cast<void*>(c->rs_idx[0]), static_cast<void*>(c->rs_idx[1]),
-                  static_cast<void*>(c->rs_cnt), static_cast<void*>(c->gs), static_cast<void*>(c->dm),
-                  static_cast<void*>(c->sp), static_cast<void*>(c->dlist), static_cast<void*>(c->dcount), c->mom, static_cast<void*>(c->perm), static_cast<void*>(c->dstep), static_cast<void*>(c->order), static_cast<void*>(c->order_alt),
-                  static_cast<void*>(c->qm)})
+  for (void* p : c->owned) hipFree(p);
+  for (void* p : {static_cast<void*>(c->inj_j), static_cast<void*>(c->inj_phi), static_cast<void*>(c->niters),
+                  static_cast<void*>(c->guess), static_cast<void*>(c->rs_key[0]), static_cast<void*>(c->rs_key[1]),
+                  static_cast<void*>(c->rs_idx[0]), static_cast<void*>(c->rs_idx[1]), static_cast<void*>(c->rs_cnt), c->mom})
     if (p) hipFree(p);
   if (c->h_ctl) hipHostFree(c->h_ctl);
   for (hipEvent_t& e : c->ev)
@@ -478,53 +507,41 @@ int cleo_device_info(char* buf, size_t len) {
   return CLEO_OK;
 }
 
-int cleo_upload_supers(cleo_ctx* c, const cleo_supers_soa* h, uint64_t ntot) {
-  if (!c || !h) return CLEO_E_ARG;
-  if (ntot > c->maxn) return fail(c, CLEO_E_ARG, "ntot exceeds the context capacity");
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  c->order_live = false;  // the uploaded drops replace the store and its pending order
-  SoA& d = c->buf[c->cur];
-  HIP_TRY(c, ctx_copy(c, d.gbx, h->sdgbxindex, ntot * 4, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, d.c3, h->coord3, ntot * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, d.c1, h->coord1, ntot * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, d.c2, h->coord2, ntot * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, d.xi, h->xi, ntot * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, d.r, h->radius, ntot * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, d.msol, h->msol, ntot * 8, hipMemcpyHostToDevice));
-  HIP_TRY(c, ctx_copy(c, d.id, h->sdid, ntot * 8, hipMemcpyHostToDevice));
+static SoA as_soa(const cleo_supers_soa& s) {
+  return SoA{s.sdgbxindex, s.coord3, s.coord1, s.coord2, s.xi, s.radius, s.msol, s.sdid};
+}
+// the fields of n drops, enqueued one after the other
+static hipError_t copy_soa(cleo_ctx* c, const SoA& d, const SoA& s, uint64_t n, hipMemcpyKind kind) {
+  hipError_t e = hipMemcpyAsync(d.gbx, s.gbx, n * 4, kind, c->stream);
+  void* dst[7] = {d.c3, d.c1, d.c2, d.xi, d.r, d.msol, d.id};
+  const void* src[7] = {s.c3, s.c1, s.c2, s.xi, s.r, s.msol, s.id};
+  for (int i = 0; i < 7 && e == hipSuccess; ++i) e = hipMemcpyAsync(dst[i], src[i], n * 8, kind, c->stream);
+  return e;
+}
+// the uploaded drops `src` (device memory) replace the store and its pending order, sorted
+static int sort_upload(cleo_ctx* c, const SoA& src, uint64_t ntot) {
+  c->order_live = false;
   c->ntot = ntot;
   const int rc = ensure_radix(c, ntot);
   if (rc != CLEO_OK) return rc;
-  generic_sort(c);
+  generic_sort(c, src, true);
   HIP_TRY(c, hipGetLastError());
-  const int rs = sync_check(c);
-  // the upload's own sort is the reference's constructor sort, not a step sort
-  HIP_TRY(c, ctx_fill(c, &c->ctl->stats[ST_SORTS], 0, 8));
-  return rs;
+  return sync_check(c);
+}
+
+int cleo_upload_supers(cleo_ctx* c, const cleo_supers_soa* h, uint64_t ntot) {
+  if (!c || !h) return CLEO_E_ARG;
+  if (ntot > c->maxn) return fail(c, CLEO_E_ARG, "ntot exceeds the context capacity");
+  c->order_live = false;  // whatever comes of the copies
+  const SoA& d = c->buf[c->cur];
+  HIP_TRY(c, copy_soa(c, d, as_soa(*h), ntot, hipMemcpyHostToDevice));
+  return sort_upload(c, d, ntot);
 }
 
 int cleo_upload_supers_device(cleo_ctx* c, const cleo_supers_soa* h, uint64_t ntot) {
   if (!c || !h) return CLEO_E_ARG;
   if (ntot > c->maxn) return fail(c, CLEO_E_ARG, "ntot exceeds the context capacity");
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  c->order_live = false;  // the uploaded drops replace the store and its pending order
-  SoA& d = c->buf[c->cur];
-  HIP_TRY(c, ctx_copy(c, d.gbx, h->sdgbxindex, ntot * 4, hipMemcpyDeviceToDevice));
-  HIP_TRY(c, ctx_copy(c, d.c3, h->coord3, ntot * 8, hipMemcpyDeviceToDevice));
-  HIP_TRY(c, ctx_copy(c, d.c1, h->coord1, ntot * 8, hipMemcpyDeviceToDevice));
-  HIP_TRY(c, ctx_copy(c, d.c2, h->coord2, ntot * 8, hipMemcpyDeviceToDevice));
-  HIP_TRY(c, ctx_copy(c, d.xi, h->xi, ntot * 8, hipMemcpyDeviceToDevice));
-  HIP_TRY(c, ctx_copy(c, d.r, h->radius, ntot * 8, hipMemcpyDeviceToDevice));
-  HIP_TRY(c, ctx_copy(c, d.msol, h->msol, ntot * 8, hipMemcpyDeviceToDevice));
-  HIP_TRY(c, ctx_copy(c, d.id, h->sdid, ntot * 8, hipMemcpyDeviceToDevice));
-  c->ntot = ntot;
-  const int rc = ensure_radix(c, ntot);
-  if (rc != CLEO_OK) return rc;
-  generic_sort(c);
-  HIP_TRY(c, hipGetLastError());
-  const int rs = sync_check(c);
-  HIP_TRY(c, ctx_fill(c, &c->ctl->stats[ST_SORTS], 0, 8));
-  return rs;
+  return sort_upload(c, as_soa(*h), ntot);  // sorted from the caller's arrays straight into the store
 }
 
 // reference Superdrop layout (superdrop.hpp:36-60): u32 gbx @0, f64 coord3 @8, coord1 @16,
@@ -552,21 +569,12 @@ int cleo_upload_supers_aos(cleo_ctx* c, const void* aos, uint64_t ntot) {
 int cleo_download_supers(cleo_ctx* c, cleo_supers_soa* h, uint64_t* ntot, uint64_t* ndomain) {
   if (!c || !h) return CLEO_E_ARG;
   materialize_order(c);  // the drops in their order
-  const int rc = sync_check(c);
   const uint64_t n = c->ntot;
-  const SoA& d = c->buf[c->cur];
-  HIP_TRY(c, ctx_copy(c, h->sdgbxindex, d.gbx, n * 4, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, h->coord3, d.c3, n * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, h->coord1, d.c1, n * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, h->coord2, d.c2, n * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, h->xi, d.xi, n * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, h->radius, d.r, n * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, h->msol, d.msol, n * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, h->sdid, d.id, n * 8, hipMemcpyDeviceToHost));
-  uint32_t nd = 0;
-  HIP_TRY(c, ctx_copy(c, &nd, c->off + c->grid.ngbx, 4, hipMemcpyDeviceToHost));
+  HIP_TRY(c, copy_soa(c, as_soa(*h), c->buf[c->cur], n, hipMemcpyDeviceToHost));
+  const int rc = sync_check(c);
+  if (rc != CLEO_OK && rc != CLEO_E_DEVICE) return rc;
   if (ntot) *ntot = n;
-  if (ndomain) *ndomain = nd;
+  if (ndomain) *ndomain = c->h_ctl->ndomain;
   return rc;
 }
 
@@ -595,9 +603,8 @@ int cleo_download_supers_aos(cleo_ctx* c, void* aos, uint64_t* ntot, uint64_t* n
 
 int cleo_download_refs(cleo_ctx* c, uint32_t* refs) {
   if (!c || !refs) return CLEO_E_ARG;
-  const int rc = sync_check(c);
-  HIP_TRY(c, ctx_copy(c, refs, c->off, (c->grid.ngbx + 1ull) * 4, hipMemcpyDeviceToHost));
-  return rc;
+  HIP_TRY(c, hipMemcpyAsync(refs, c->off, (c->grid.ngbx + 1ull) * 4, hipMemcpyDeviceToHost, c->stream));
+  return sync_check(c);
 }
 
 // FromFileComms::receive_dynamics from device arrays: no host round trip of the State
@@ -612,19 +619,28 @@ int cleo_receive_dynamics(cleo_ctx* c, const cleo_dynamics_step* dyn) {
 int cleo_mass_moments(cleo_ctx* c, int32_t rain, uint64_t* mom0, float* mom1, float* mom2) {
   if (!c || !mom0 || !mom1 || !mom2) return CLEO_E_ARG;
   const uint64_t ngbx = c->grid.ngbx;
-  if (!c->mom) {
+  const bool small = 16 * ngbx <= kStageBytes;  // written to the host by the reduction itself
+  if (!small && !c->mom) {
     uint8_t* p = nullptr;
     HIP_TRY(c, dalloc(&p, 16 * ngbx));
     c->mom = p;
   }
-  uint64_t* d0 = static_cast<uint64_t*>(c->mom);
+  uint64_t* d0 = small ? reinterpret_cast<uint64_t*>(c->stage) : static_cast<uint64_t*>(c->mom);
   float* d1 = reinterpret_cast<float*>(d0 + ngbx);
   float* d2 = d1 + ngbx;
   launch_mass_moments(c, rain != 0, d0, d1, d2);
   HIP_TRY(c, hipGetLastError());
-  HIP_TRY(c, ctx_copy(c, mom0, d0, ngbx * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, mom1, d1, ngbx * 4, hipMemcpyDeviceToHost));
-  HIP_TRY(c, ctx_copy(c, mom2, d2, ngbx * 4, hipMemcpyDeviceToHost));
+  if (small) {
+    const int rc = sync_check(c);
+    if (rc != CLEO_OK && rc != CLEO_E_DEVICE) return rc;
+    std::memcpy(mom0, d0, ngbx * 8);
+    std::memcpy(mom1, d1, ngbx * 4);
+    std::memcpy(mom2, d2, ngbx * 4);
+    return rc;
+  }
+  HIP_TRY(c, hipMemcpyAsync(mom0, d0, ngbx * 8, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, hipMemcpyAsync(mom1, d1, ngbx * 4, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, hipMemcpyAsync(mom2, d2, ngbx * 4, hipMemcpyDeviceToHost, c->stream));
   return sync_check(c);
 }
 
@@ -641,23 +657,37 @@ int cleo_upload_gbx_state(cleo_ctx* c, const cleo_gbx_state* h) {
   state_fields(c, f);
   const double* src[11] = {h->volume, h->press, h->temp, h->qvap, h->qcond, h->wvel_lo,
                            h->wvel_hi, h->uvel_lo, h->uvel_hi, h->vvel_lo, h->vvel_hi};
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  for (int i = 0; i < 11; ++i) {
+  for (int i = 0; i < 11; ++i)
     if (!src[i]) return fail(c, CLEO_E_ARG, "null state field");
-    HIP_TRY(c, ctx_copy(c, f[i], src[i], c->grid.ngbx * 8ull, hipMemcpyHostToDevice));
+  const size_t bytes = c->grid.ngbx * 8ull;
+  if (11 * bytes <= kStageBytes) {  // the fields follow each other in d_state: one copy
+    for (int i = 0; i < 11; ++i) std::memcpy(c->stage + i * bytes, src[i], bytes);
+    HIP_TRY(c, ctx_copy(c, c->d_state, c->stage, 11 * bytes, hipMemcpyHostToDevice));
+    return CLEO_OK;
   }
+  for (int i = 0; i < 11; ++i) HIP_TRY(c, hipMemcpyAsync(f[i], src[i], bytes, hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(c, hipStreamSynchronize(c->stream));
   return CLEO_OK;
 }
 
 int cleo_download_gbx_state(cleo_ctx* c, cleo_gbx_state* h) {
   if (!c || !h) return CLEO_E_ARG;
-  const int rc = sync_check(c);
   double* f[11];
   state_fields(c, f);
   double* dst[11] = {h->volume, h->press, h->temp, h->qvap, h->qcond, h->wvel_lo,
                      h->wvel_hi, h->uvel_lo, h->uvel_hi, h->vvel_lo, h->vvel_hi};
-  for (int i = 0; i < 11; ++i)
-    if (dst[i]) HIP_TRY(c, ctx_copy(c, dst[i], f[i], c->grid.ngbx * 8ull, hipMemcpyDeviceToHost));
+  const size_t bytes = c->grid.ngbx * 8ull;
+  const bool small = 11 * bytes <= kStageBytes;
+  if (small) {
+    HIP_TRY(c, hipMemcpyAsync(c->stage, c->d_state, 11 * bytes, hipMemcpyDeviceToHost, c->stream));
+  } else {
+    for (int i = 0; i < 11; ++i)
+      if (dst[i]) HIP_TRY(c, hipMemcpyAsync(dst[i], f[i], bytes, hipMemcpyDeviceToHost, c->stream));
+  }
+  const int rc = sync_check(c);
+  if (small && (rc == CLEO_OK || rc == CLEO_E_DEVICE))
+    for (int i = 0; i < 11; ++i)
+      if (dst[i]) std::memcpy(dst[i], c->stage + i * bytes, bytes);
   return rc;
 }
 
@@ -669,12 +699,11 @@ int cleo_set_solute(cleo_ctx* c, const cleo_solute* s) {
 
 int cleo_set_rng_counter(cleo_ctx* c, uint64_t seed, uint64_t first_event) {
   if (!c) return CLEO_E_ARG;
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
   c->rng_mode = 1;
   c->seed = seed;
   c->events_pending = 0;
-  HIP_TRY(c, ctx_copy(c, &c->ctl->event, &first_event, 8, hipMemcpyHostToDevice));
-  return CLEO_OK;
+  launch_set_event(c, first_event);
+  return launch_check(c);
 }
 
 int cleo_set_rng_injected(cleo_ctx* c, const uint32_t* j, uint64_t nj, const double* phi, uint64_t nphi) {
@@ -744,7 +773,7 @@ int cleo_sort(cleo_ctx* c) {
   materialize_order(c);  // the generic sort is stable in the drops' order
   const int rc = ensure_radix(c, c->ntot);
   if (rc != CLEO_OK) return rc;
-  generic_sort(c);
+  generic_sort(c, c->buf[c->cur], false);
   return launch_check(c);
 }
 
@@ -755,9 +784,8 @@ int cleo_motion(cleo_ctx* c, const cleo_motion_params* p) {
 }
 
 static int set_substep_error(cleo_ctx* c) {
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  HIP_TRY(c, ctx_copy(c, c->h_ctl, c->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost));
-  if (c->h_ctl->err_code == 0) {
+  HIP_TRY(c, fetch_ctl(c));
+  if (c->h_ctl->ctl.err_code == 0) {
     int32_t code = CLEO_ERR_SUBSTEP;
     HIP_TRY(c, ctx_copy(c, &c->ctl->err_code, &code, 4, hipMemcpyHostToDevice));
   }
@@ -912,20 +940,17 @@ int cleo_event_elapsed(cleo_ctx* c, int32_t a, int32_t b, float* ms) {
 
 int cleo_ndomain(cleo_ctx* c, uint64_t* nd) {
   if (!c || !nd) return CLEO_E_ARG;
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  uint32_t v = 0;
-  HIP_TRY(c, ctx_copy(c, &v, c->off + c->grid.ngbx, 4, hipMemcpyDeviceToHost));
-  *nd = v;
+  HIP_TRY(c, fetch_ctl(c));
+  *nd = c->h_ctl->ndomain;
   return CLEO_OK;
 }
 
 int cleo_get_error(cleo_ctx* c, cleo_error* err) {
   if (!c || !err) return CLEO_E_ARG;
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  HIP_TRY(c, ctx_copy(c, c->h_ctl, c->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost));
-  err->code = c->h_ctl->err_code;
-  err->gbxindex = c->h_ctl->err_gbx;
-  err->drop = c->h_ctl->err_drop;
+  HIP_TRY(c, fetch_ctl(c));
+  err->code = c->h_ctl->ctl.err_code;
+  err->gbxindex = c->h_ctl->ctl.err_gbx;
+  err->drop = c->h_ctl->ctl.err_drop;
   return CLEO_OK;
 }
 
@@ -938,13 +963,12 @@ int cleo_clear_error(cleo_ctx* c) {
 
 int cleo_get_stats(cleo_ctx* c, cleo_stats* s) {
   if (!c || !s) return CLEO_E_ARG;
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  HIP_TRY(c, ctx_copy(c, c->h_ctl, c->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost));
+  HIP_TRY(c, fetch_ctl(c));
   std::vector<unsigned long long> rows(kStatRow * kStatRows);
   HIP_TRY(c, ctx_copy(c, rows.data(), c->sp, rows.size() * 8, hipMemcpyDeviceToHost));
   unsigned long long v[ST_COUNT];
   for (uint32_t j = 0; j < ST_COUNT; ++j) {
-    v[j] = c->h_ctl->stats[j];
+    v[j] = c->h_ctl->ctl.stats[j];
     for (uint32_t r = 0; r < kStatRows; ++r) v[j] += rows[r * kStatRow + j];
   }
   s->cond_drops = v[ST_COND_DROPS];

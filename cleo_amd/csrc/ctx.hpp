@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <vector>
 
 #include "physics.hpp"
 
@@ -51,6 +52,13 @@ struct StatSlots {
   unsigned long long* rows;
 };
 
+struct HostCtl {
+  DevCtl ctl;
+  uint32_t ndomain;
+};
+static_assert(sizeof(HostCtl) <= 4096, "page before the staging area");
+constexpr size_t kStageBytes = 512u << 10;
+
 struct MLPDev;  // mlp.hip
 
 }  // namespace cleo
@@ -60,6 +68,7 @@ struct cleo_ctx {
   int num_cu = 256;  // compute units of the device
   hipStream_t stream = nullptr;
   cleo::Grid grid{};
+  std::vector<void*> owned;  // the allocations behind the arrays that exist from the start
   double* d_halves = nullptr;
   uint64_t maxn = 0;
   uint64_t ntot = 0;
@@ -85,7 +94,11 @@ struct cleo_ctx {
   size_t rs_n = 0;
   // control
   cleo::DevCtl* ctl = nullptr;
-  cleo::DevCtl* h_ctl = nullptr;  // pinned mirror
+  // pinned mirror of the control block and the domain's number of drops, written by the device
+  // (fetch_ctl): a launch instead of copies and further waits
+  cleo::HostCtl* h_ctl = nullptr;
+  // pinned staging of small State transfers and moments (kStageBytes, behind h_ctl)
+  unsigned char* stage = nullptr;
   // RNG
   int rng_mode = 0;  // 0 none, 1 counter, 2 injected
   uint64_t seed = 0;
@@ -96,7 +109,6 @@ struct cleo_ctx {
   uint32_t* inj_op = nullptr;  // ngbx+1
   // large-gridbox collision scratch (permutation + indices for gridboxes above the LDS capacity)
   uint32_t* big_scratch = nullptr;
-  uint64_t big_scratch_n = 0;
   // configuration
   // the SDMMethods configuration: microphysics proc[0] >> ... >> proc[n-1], then motion
   struct Chain {

@@ -376,10 +376,10 @@ __global__ void __launch_bounds__(256) k_mlp_forward(ForwardArgs a) {
 // ---- the sample order: a Fisher-Yates shuffle from a xorshift64 stream --------------------------
 // The order is that of the serial shuffle `for i = n-1 .. 1: swap(perm[i], perm[x() % (i+1)])` (5 ms
 // for 2M samples on one host core with the copy of its result, 0.26 ms here, most of it the random
-// accesses of the atomic exchanges and list walks).  xorshift64 is linear over the bits of its state, so a thread gets its place in the stream by 64 x 64 bit matrices:
-// jump[b] is the one of kDrawsPerThread << b steps.  The order follows from the drawn indices by the
-// lists of the swaps that hit each place, as in the collisions' shuffle (sdm_kernels.hip), here over
-// several launches.
+// accesses of the atomic exchanges and list walks).  xorshift64 is linear over the bits of its state,
+// so a thread gets its place in the stream by 64 x 64 bit matrices: jump[b] is the one of
+// kDrawsPerThread << b steps.  The order follows from the drawn indices by the lists of the swaps that
+// hit each place, as in the collisions' shuffle (sdm_kernels.hip), here over several launches.
 constexpr uint32_t kDrawsPerThread = 16, kJumps = 29;
 __host__ __device__ inline uint64_t xorshift64(uint64_t s) {
   s ^= s << 13;
@@ -529,24 +529,25 @@ static void launch_reduce_adam(hipStream_t s, MLPDev* m, uint32_t waves, int32_t
 hipError_t mlp_create(cleo_ctx* c) {
   MLPDev* m = new MLPDev();
   c->mlp = m;
-  hipError_t e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->master), NBLOB * 4)) != hipSuccess) return e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->adam_m), NBLOB * 4)) != hipSuccess) return e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->adam_v), NBLOB * 4)) != hipSuccess) return e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->grad), NBLOB * 4)) != hipSuccess) return e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->loss), 16)) != hipSuccess) return e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->w1p), kHid * kInPad * 2)) != hipSuccess) return e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->w2), kHid * kHid * 2)) != hipSuccess) return e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->w2t), kHid * kHid * 2)) != hipSuccess) return e;
+  // one allocation: four blobs, the bf16 copies, the loss
+  constexpr size_t kBlob = (NBLOB * 4 + 255) / 256 * 256, kW1 = kHid * kInPad * 2, kW2 = kHid * kHid * 2;
+  const hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->master), 4 * kBlob + kW1 + 2 * kW2 + 16);
+  if (e != hipSuccess) return e;
+  unsigned char* p = reinterpret_cast<unsigned char*>(m->master);
+  m->adam_m = reinterpret_cast<float*>(p + kBlob);
+  m->adam_v = reinterpret_cast<float*>(p + 2 * kBlob);
+  m->grad = reinterpret_cast<float*>(p + 3 * kBlob);
+  m->w1p = reinterpret_cast<uint16_t*>(p + 4 * kBlob);
+  m->w2 = reinterpret_cast<uint16_t*>(p + 4 * kBlob + kW1);
+  m->w2t = reinterpret_cast<uint16_t*>(p + 4 * kBlob + kW1 + kW2);
+  m->loss = reinterpret_cast<float*>(p + 4 * kBlob + kW1 + 2 * kW2);
   return hipSuccess;
 }
 
 void mlp_destroy(cleo_ctx* c) {
   MLPDev* m = c->mlp;
   if (!m) return;
-  for (void* p : {static_cast<void*>(m->master), static_cast<void*>(m->adam_m), static_cast<void*>(m->adam_v),
-                  static_cast<void*>(m->grad), static_cast<void*>(m->loss), static_cast<void*>(m->w1p),
-                  static_cast<void*>(m->w2), static_cast<void*>(m->w2t), static_cast<void*>(m->warm),
+  for (void* p : {static_cast<void*>(m->master), static_cast<void*>(m->warm),
                   static_cast<void*>(m->partial), static_cast<void*>(m->moments), static_cast<void*>(m->jump),
                   static_cast<void*>(m->order)})
     if (p) hipFree(p);

@@ -1342,11 +1342,18 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_motion_scatter(Motion
   copy_oob(n, n.off[a.grid.ngbx]);
 }
 
-__global__ void k_set_nact(const uint32_t* off, uint32_t ngbx, uint32_t* nact, DevCtl* ctl) {
+__global__ void k_set_nact(const uint32_t* off, uint32_t ngbx, uint32_t* nact, DevCtl* ctl, bool upload) {
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g < ngbx) nact[g] = off[g + 1] - off[g];
-  if (g == 0) ctl->stats[ST_SORTS] += 1;
+  if (g == 0) ctl->stats[ST_SORTS] = upload ? 0 : ctl->stats[ST_SORTS] + 1;
 }
+__global__ void k_publish_ctl(const DevCtl* ctl, const uint32_t* off, uint32_t ngbx, HostCtl* out) {
+  constexpr uint32_t kWords = sizeof(DevCtl) / 4;
+  static_assert(kWords <= kWave, "one word per lane");
+  if (threadIdx.x < kWords) reinterpret_cast<uint32_t*>(&out->ctl)[threadIdx.x] = reinterpret_cast<const uint32_t*>(ctl)[threadIdx.x];
+  if (threadIdx.x == 0) out->ndomain = off[ngbx];
+}
+__global__ void k_set_event(DevCtl* ctl, uint64_t event) { ctl->event = event; }
 
 // ============================ re-sort after collisions ========================================
 // When collisions left nulls, SDMMethods sorts again: the active drops of each gridbox move together
@@ -1770,6 +1777,12 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   }
 }
 StatSlots stat_slots(cleo_ctx* c) { return StatSlots{c->sp}; }
+void launch_publish_ctl(cleo_ctx* c) {
+  hipLaunchKernelGGL(k_publish_ctl, dim3(1), dim3(64), 0, c->stream, c->ctl, c->off, c->grid.ngbx, c->h_ctl);
+}
+void launch_set_event(cleo_ctx* c, uint64_t event) {
+  hipLaunchKernelGGL(k_set_event, dim3(1), dim3(1), 0, c->stream, c->ctl, event);
+}
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np) {
   hipLaunchKernelGGL(k_inj_sizes, dim3(nblocks(c->grid.ngbx, 256)), dim3(256), 0, c->stream, c->nact, c->grid.ngbx, nj, np);
 }
@@ -1967,19 +1980,19 @@ void radix_sort_soa(hipStream_t stream, const SoA& src, const SoA& dst, uint64_t
                      dst, sc.key[cur], sc.idx[cur], n, ngbx, off);
 }
 
-void generic_sort(cleo_ctx* c) {
+void generic_sort(cleo_ctx* c, const SoA& src, bool upload) {
   const uint64_t n = c->ntot;
   const uint32_t ngbx = c->grid.ngbx;
-  const int src = c->cur, dst = 1 - c->cur;
+  const int dst = 1 - c->cur;
   RadixScratch sc{};
   for (int i = 0; i < 2; ++i) {
     sc.key[i] = c->rs_key[i];
     sc.idx[i] = c->rs_idx[i];
   }
   sc.cnt = c->rs_cnt;  // no rows: the drops of an upload mostly come in order
-  radix_sort_soa(c->stream, c->buf[src], c->buf[dst], n, ngbx, c->off, sc);
+  radix_sort_soa(c->stream, src, c->buf[dst], n, ngbx, c->off, sc);
   if (n > 0) c->cur = dst;
-  hipLaunchKernelGGL(k_set_nact, dim3(nblocks(ngbx, 256)), dim3(256), 0, c->stream, c->off, ngbx, c->nact, c->ctl);
+  hipLaunchKernelGGL(k_set_nact, dim3(nblocks(ngbx, 256)), dim3(256), 0, c->stream, c->off, ngbx, c->nact, c->ctl, upload);
 }
 
 }  // namespace cleo

@@ -157,8 +157,9 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
 void motion_sort_gather(cleo_ctx* c, const MotionArgs& args, const SoA& dst, int commit_dst);
 // motion + neighbour sort fused into two passes (motion_flat 2): src = args.s is left unchanged
 void motion_sort_fused(cleo_ctx* c, const MotionArgs& args, const SoA& dst, int commit_dst);
-// generic stable sort of buf[cur] into buf[1-cur]; swaps cur; sets off and nact
-void generic_sort(cleo_ctx* c);
+// generic stable sort of `src` (buf[cur], or the caller's device arrays) into buf[1-cur], which becomes
+// current; sets off and nact.  The sort of an upload is not counted: the sort counter starts from 0.
+void generic_sort(cleo_ctx* c, const SoA& src, bool upload);
 // the generic sort without a context: two key and two index arrays of n words, the digit counts
 // (radix_count_words(n)) and, or null, a 64-byte row per drop
 constexpr uint32_t kRadixTile = 2048, kDropRowWords = 16;
@@ -176,6 +177,10 @@ void radix_sort_soa(hipStream_t stream, const SoA& src, const SoA& dst, uint64_t
                     const RadixScratch& sc);
 // applies a pending collision order to the store (buf[cur] then holds the drops in order)
 void materialize_order(cleo_ctx* c);
+// the control block and the domain's number of drops into the pinned mirror h_ctl, in stream order
+void launch_publish_ctl(cleo_ctx* c);
+// the collision event counter, in stream order
+void launch_set_event(cleo_ctx* c, uint64_t event);
 // 0th, 1st and 2nd mass moments of every gridbox into device arrays of ngbx entries (raindrops
 // only when rain)
 void launch_mass_moments(cleo_ctx* c, bool rain, uint64_t* mom0, float* mom1, float* mom2);
