@@ -413,8 +413,8 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   want(zero, &c->nact, ngbx);
   want(zero, &c->d_state, 11 * ngbx);
   want(zero, &c->cnt, 56 * ngbx);  // counts, then the run offsets of the neighbour sort
-  want(zero, &c->tot, ngbx + 1);
   want(rest, &c->d_halves, nh);
+  want(rest, &c->tot, ngbx + 1);
   want(rest, &c->oobpre, ngbx + 1);
   want(rest, &c->part, 2 * ((ngbx + kTabBlock - 1) / kTabBlock) + 1);
   want(rest, &c->inj_oj, ngbx + 1);

@@ -81,8 +81,8 @@ struct cleo_ctx {
   double* d_state = nullptr;
   cleo::Solute solute{};
   // neighbour-sort scratch
-  uint32_t* cnt = nullptr;      // ngbx*56: sort counts (ngbx*28, zero between sorts), then run offsets (ngbx*28)
-  uint32_t* tot = nullptr;      // ngbx+1
+  uint32_t* cnt = nullptr;      // ngbx*56: sort counts (ngbx*28), then run offsets (ngbx*28)
+  uint32_t* tot = nullptr;      // ngbx+1: sizes of an injected stream
   uint32_t* oobpre = nullptr;   // ngbx+1
   uint32_t* part = nullptr;     // the sort's sums per block of gridboxes
   uint32_t* scan_tmp = nullptr;

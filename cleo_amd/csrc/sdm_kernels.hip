@@ -703,9 +703,7 @@ __device__ __forceinline__ double interpolation(double blo, double bhi, double i
 // One axis of CartesianMaps::get_local_bounding_gridbox_index (cartesianmaps.cpp:68-286,
 // domainboundaries.hpp:34-109): step to the backward/forward neighbour when the coordinate left
 // [lower, upper) and wrap the coordinate at a periodic domain edge.  i is the drop's index along
-// the axis, updated to the neighbour's.  Returns the step taken; on a periodic axis of one or two
-// gridboxes several steps lead to one neighbour, and the step is then the change of the index, so that
-// drops with the same source and destination have the same step (the sort places drops by their step).
+// the axis, updated to the neighbour's.  Returns the step taken.
 __device__ __forceinline__ int axis_step(uint32_t& idx, double& coord, uint32_t& i, uint32_t nd, uint32_t inc,
                                          bool periodic, const double* h) {
   const double lo = h[i], hi = h[i + 1];
@@ -716,7 +714,6 @@ __device__ __forceinline__ int axis_step(uint32_t& idx, double& coord, uint32_t&
         coord = coord + h[nd] - lo;  // lim1 = upper bound of the backward neighbour
         idx = nb;
         i = nd - 1;
-        if (nd <= 2) return static_cast<int>(nd) - 1;
       } else {
         idx = kOOB;
       }
@@ -733,7 +730,6 @@ __device__ __forceinline__ int axis_step(uint32_t& idx, double& coord, uint32_t&
         coord = coord + h[0] - hi;  // lim1 = lower bound of the forward neighbour
         idx = nb;
         i = 0;
-        if (nd <= 2) return 1 - static_cast<int>(nd);
       } else {
         idx = kOOB;
       }
@@ -838,7 +834,13 @@ __device__ __forceinline__ Moved move_drop(const MotionArgs& a, uint32_t g, cons
     const bool bad = (M.c3 < a.grid.zh[jz]) | (M.c3 >= a.grid.zh[jz + 1]) | (M.c1 < a.grid.xh[jx]) |
                      (M.c1 >= a.grid.xh[jx + 1]) | (M.c2 < a.grid.yh[jy]) | (M.c2 >= a.grid.yh[jy + 1]);
     if (report && bad) set_error(a.ctl, CLEO_ERR_BOUNDS, g, k);
-    M.dir = (dz + 1) + 3 * (dx + 1) + 9 * (dy + 1);
+    // on a periodic axis of one or two gridboxes several steps lead to one neighbour; the step is then
+    // the change of the index, so that drops with the same source and destination have the same step
+    // (the sort places drops by their step)
+    const int sz = nz <= 2 ? static_cast<int>(jz) - static_cast<int>(G.iz) : dz;
+    const int sx = nx <= 2 ? static_cast<int>(jx) - static_cast<int>(G.ix) : dx;
+    const int sy = ny <= 2 ? static_cast<int>(jy) - static_cast<int>(G.iy) : dy;
+    M.dir = (sz + 1) + 3 * (sx + 1) + 9 * (sy + 1);
   }
   return M;
 }
@@ -848,14 +850,6 @@ __device__ __forceinline__ Moved move_drop(const MotionArgs& a, uint32_t g, cons
 
 // ============================ neighbour sort ==================================================
 
-// base[] of the sorted store, the first place of each gridbox (and of each gridbox's drops that leave
-// the domain), as the sum of a prefix within its block of kTabBlock gridboxes and the block's start
-__device__ __forceinline__ uint32_t new_base(const NsortArgs& a, uint32_t d) {
-  return a.tot[d] + a.part[2u * (d / kTabBlock)];
-}
-__device__ __forceinline__ uint32_t oob_base(const NsortArgs& a, uint32_t g) {
-  return a.part[2u * a.nblk] + a.oobpre[g] + a.part[2u * (g / kTabBlock) + 1u];
-}
 // exclusive prefix of v over the block's kTabBlock threads, and the block's total
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* ws, uint32_t& total) {
   uint32_t wt;
@@ -886,14 +880,13 @@ __device__ __forceinline__ void gbx_thermo(const GState& st, uint32_t g, double*
 // Per destination d (thread per d): the drops arriving in d, and for each step s the drops that
 // reach d from source gridboxes of lower index than the source of s (the stable order puts them
 // first).  The counts are destination-major (row d, column s: arrivals at d by the step s), read as
-// one row and left zero for the next motion.  The run offsets are written source-major into `runs`
+// one row and, on small domains, left zero for the next motion (counts_stay_clear).  The run offsets are written source-major into `runs`
 // (row g, column s: the offset of g's drops taking the step s), so the rank pass reads its gridbox's
 // 27 offsets as one contiguous row.  Every entry of `runs` belongs to one destination (g + step s): no
 // two threads write the same entry.  Only the entries of steps that some drop takes are written (a
 // source off a finite axis has none); the others keep older values that no pass reads.
-// The arrivals and the drops that leave the domain are scanned here within the block of gridboxes;
-// k_nsort_part scans the blocks' totals, and the rank pass, which reads base[] anyway, writes the new
-// refs.  (Separate launches for the fill of the counts, two three-level scans, the refs, the active
+// The arrivals and the drops that leave the domain are scanned here within the block of gridboxes, into
+// the new refs and the out-of-domain prefix; k_nsort_apply adds what the blocks before have.  (Separate launches for the fill of the counts, two three-level scans, the refs, the active
 // counts and the condensation inputs, with the same for the re-sort after collisions, made 34 launches
 // of a coupled step, 11 now: 409 -> 349 us on 32^3 gridboxes of 64 drops.)  kThermo: the gridbox's condensation inputs too, for a
 // condensation in the sort's gather (the State is that of before the sort).
@@ -913,8 +906,10 @@ __global__ void __launch_bounds__(kTabBlock) k_nsort_tot(NsortArgs a, GState st,
       cnt[4 * i + 2] = v.z;
       cnt[4 * i + 3] = v.w;
     }
+    if (a.clear) {
 #pragma unroll
-    for (int i = 0; i < 7; ++i) row[i] = uint4{0u, 0u, 0u, 0u};
+      for (int i = 0; i < 7; ++i) row[i] = uint4{0u, 0u, 0u, 0u};
+    }
     gone = cnt[27];
 #pragma unroll
     for (int s = 0; s < 27; ++s) t += cnt[s];
@@ -964,19 +959,17 @@ __global__ void __launch_bounds__(kTabBlock) k_nsort_tot(NsortArgs a, GState st,
   uint32_t tsum, gsum;
   const uint32_t tpre = block_excl_scan(t, ws, tsum), gpre = block_excl_scan(gone, ws, gsum);
   if (d < a.grid.ngbx) {
-    a.tot[d] = tpre;
+    a.off_new[d] = tpre;
     a.oobpre[d] = gpre;
   }
   if (threadIdx.x == 0) {
-    const bool only = gridDim.x == 1;  // no k_nsort_part follows
-    a.part[2u * blockIdx.x] = only ? 0u : tsum;
-    a.part[2u * blockIdx.x + 1u] = only ? 0u : gsum;
-    if (only) a.part[2u] = tsum;
+    a.part[2u * blockIdx.x] = tsum;
+    a.part[2u * blockIdx.x + 1u] = gsum;
+    if (gridDim.x == 1) a.off_new[a.grid.ngbx] = tsum;  // no k_nsort_apply follows
     if (blockIdx.x == 0) a.ctl->stats[ST_SORTS] += 1;
   }
 }
-// the blocks' totals of k_nsort_tot to their starts (one workgroup); part[2 nblk] gets the drops in the
-// domain
+// kTabBlock blocks' totals to their prefixes (one workgroup), for domains of many blocks
 __global__ void __launch_bounds__(1024) k_nsort_part(uint32_t* part, uint32_t nblk) {
   __shared__ uint32_t ws[16];
   uint32_t t0 = 0, g0 = 0;
@@ -993,6 +986,35 @@ __global__ void __launch_bounds__(1024) k_nsort_part(uint32_t* part, uint32_t nb
     g0 += gs;
   }
   if (threadIdx.x == 0) part[2u * nblk] = t0;
+}
+// Adds the totals of the blocks before to the prefixes of block blockIdx.x: the prefixes themselves
+// (kScanned: k_nsort_part ran), or the sum of those blocks' totals, which up to kApplyBlocks blocks is
+// cheaper than a launch that scans them.
+template <bool kScanned>
+__global__ void __launch_bounds__(kTabBlock) k_nsort_apply(NsortArgs a) {
+  uint32_t t0 = 0, g0 = 0;
+  if constexpr (kScanned) {
+    t0 = a.part[2u * blockIdx.x];
+    g0 = a.part[2u * blockIdx.x + 1u];
+  } else {
+    __shared__ uint32_t ws[kTabBlock / kWave];
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kTabBlock) {
+      t0 += a.part[2u * b];
+      g0 += a.part[2u * b + 1u];
+    }
+    uint32_t all;
+    block_excl_scan(t0, ws, all);
+    t0 = all;
+    block_excl_scan(g0, ws, all);
+    g0 = all;
+  }
+  const uint32_t d = blockIdx.x * kTabBlock + threadIdx.x;
+  if (d < a.grid.ngbx) {
+    a.off_new[d] += t0;
+    a.oobpre[d] += g0;
+  }
+  if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x)
+    a.off_new[a.grid.ngbx] = kScanned ? a.part[2u * a.nblk] : t0 + a.part[2u * blockIdx.x];
 }
 
 // Stable scatter (sortsupers.hpp:63-76,167-193 under Serial): drop p of source gridbox g with
@@ -1017,7 +1039,7 @@ __global__ void __launch_bounds__(1024) k_nsort_part(uint32_t* part, uint32_t nb
 // 9(dy+1) is g + noff away from the edges, else wrapped on periodic axes (the same gridbox as
 // neighbour_of, without a division per lane).  A g past the last gridbox gives an empty head.
 struct RankHead {
-  uint32_t g, sbase, nfull, trun, base;
+  uint32_t g, sbase, nfull, trun;
 };
 __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, int gz, int gx, int gy, int32_t noff,
                                               int lane) {
@@ -1025,11 +1047,11 @@ __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, in
   const int nz = static_cast<int>(a.grid.nz), nx = static_cast<int>(a.grid.nx), ny = static_cast<int>(a.grid.ny);
   const bool valid = g < ngbx;
   const uint32_t gc = valid ? static_cast<uint32_t>(g) : ngbx - 1u;
-  RankHead h{gc, 0u, 0u, 0u, 0u};
+  RankHead h{gc, 0u, 0u, 0u};
   const uint32_t lo = a.off[gc], hi = a.off[gc + 1];
   h.sbase = lo;
   h.nfull = valid ? hi - lo : 0u;
-  uint32_t d = ngbx;  // lanes 27..63: the out-of-domain run
+  uint32_t d = ngbx;  // lanes 27..63: the out-of-domain run (off_new[ngbx] + oobpre[g])
   bool ok = valid && lane == 27;
   if (lane < 27 && !valid) {
     d = 0u;  // no gridbox: a harmless load, discarded
@@ -1051,12 +1073,8 @@ __device__ __forceinline__ RankHead rank_head(const NsortArgs& a, uint64_t g, in
       d = ok ? static_cast<uint32_t>(jz + nz * (jx + nx * jy)) : 0u;
     }
   }
-  // new_base(d) + the run's offset, or oob_base(gc); tot[ngbx] is 0
-  const bool in = d < ngbx;
-  const uint32_t b = a.tot[d] + a.part[in ? 2u * (d / kTabBlock) : 2u * a.nblk];
-  const uint32_t extra = lane < 27 ? a.runs[28ull * gc + static_cast<uint32_t>(lane)]
-                                   : a.oobpre[gc] + a.part[2u * (gc / kTabBlock) + 1u];
-  h.base = b;
+  const uint32_t b = a.off_new[d];
+  const uint32_t extra = lane < 27 ? a.runs[28ull * gc + static_cast<uint32_t>(lane)] : a.oobpre[gc];
   h.trun = ok ? b + extra : 0u;
   return h;
 }
@@ -1091,7 +1109,6 @@ __device__ __forceinline__ void rank_gbx(const NsortArgs& a, const RankHead& h, 
                                          uint32_t nsrc, int lane) {
   const uint32_t g = h.g, sbase = h.sbase, nfull = h.nfull;
   uint32_t trun = h.trun;
-  if (lane == 13) a.off_new[g] = h.base;  // step 13 stays: the new refs
   // chunk c of 64 slots: the drop of slot sbase + c + lane is at position p with key kv
   auto chunk = [&](uint32_t c, uint32_t p, uint32_t kv) {
     const uint32_t q = sbase + c + lane;
@@ -1155,12 +1172,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(6) k_nsort_perm(NsortArgs 
   const uint64_t ngbx = a.grid.ngbx;
   const uint32_t g0 = xcd_wave_index(), stride = wave_count();
   const uint32_t nsrc = a.off[ngbx];
-  if (g0 == 0 && lane == 0) a.off_new[ngbx] = a.part[2u * a.nblk];
-  if (g0 >= ngbx) return;
-  if (nsrc == 0) {  // no drops to rank: the new refs only
-    for (uint64_t g = g0 + static_cast<uint64_t>(lane) * stride; g < ngbx; g += static_cast<uint64_t>(kWave) * stride) a.off_new[g] = 0u;
-    return;
-  }
+  if (g0 >= ngbx || nsrc == 0) return;
   uint32_t gz = g0 % nz, gx = (g0 / nz) % nx, gy = g0 / (nz * nx);
   const uint32_t sz = stride % nz, sx = (stride / nz) % nx, sy = stride / (nz * nx);
   const int32_t noff = (lane % 3 - 1) + static_cast<int32_t>(nz) * ((lane / 3) % 3 - 1) +
@@ -1300,10 +1312,10 @@ __device__ __forceinline__ void motion_scatter_gbx(const MotionArgs& a, const Ns
     const uint32_t need = present & ~have;
     if (lane < 28 && ((need >> lane) & 1u)) {
       if (lane == 27) {
-        run = oob_base(n, g);
+        run = n.off_new[a.grid.ngbx] + n.oobpre[g];
       } else {
         const uint32_t d = neighbour_of(a.grid, g, lane);
-        run = new_base(n, d) + n.runs[28ull * g + lane];
+        run = n.off_new[d] + n.runs[28ull * g + lane];
       }
     }
     have |= need;
@@ -1334,11 +1346,7 @@ __device__ __forceinline__ void motion_scatter_gbx(const MotionArgs& a, const Ns
 }
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_motion_scatter(MotionArgs a, NsortArgs n) {
   const int lane = lane_id();
-  for (uint32_t g = wave_index(); g < a.grid.ngbx; g += wave_count()) {
-    if (lane == 0) n.off_new[g] = new_base(n, g);
-    motion_scatter_gbx(a, n, g, lane);
-  }
-  if (wave_index() == 0 && lane == 0) n.off_new[a.grid.ngbx] = n.part[2u * n.nblk];
+  for (uint32_t g = wave_index(); g < a.grid.ngbx; g += wave_count()) motion_scatter_gbx(a, n, g, lane);
   copy_oob(n, n.off[a.grid.ngbx]);
 }
 
@@ -1818,6 +1826,21 @@ void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, ui
   scan_rec(c->stream, in, len, stride, offset, out, c->scan_tmp);
 }
 
+// Whether the count table is left zero by the sort that reads it, rather than filled before motion: a
+// launch less, but on large domains motion's atomics then find the table in HBM and not in a cache that
+// a fill has just written (524288 gridboxes: motion 515 us against 478 us and 16 us for the fill).
+static bool counts_stay_clear(const cleo_ctx* c) { return c->grid.ngbx <= 65536u; }
+__global__ void __launch_bounds__(256) k_fill_u32x4(uint4* p, uint64_t n) {
+  for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n;
+       i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
+    p[i] = uint4{0u, 0u, 0u, 0u};
+}
+// the counts of the next motion start from zero
+static void clear_counts(cleo_ctx* c) {
+  if (counts_stay_clear(c)) return;
+  const uint64_t n = 7ull * c->grid.ngbx;
+  hipLaunchKernelGGL(k_fill_u32x4, dim3(stride_blocks(n)), dim3(256), 0, c->stream, reinterpret_cast<uint4*>(c->cnt), n);
+}
 // argument block of the neighbour-sort kernels reading `src` and writing `dst`
 static NsortArgs nsort_args(cleo_ctx* c, const SoA& src, const SoA& dst) {
   NsortArgs a{};
@@ -1828,10 +1851,10 @@ static NsortArgs nsort_args(cleo_ctx* c, const SoA& src, const SoA& dst) {
   a.nact = c->nact;
   a.cnt = c->cnt;
   a.runs = c->cnt + 28ull * c->grid.ngbx;
-  a.tot = c->tot;
   a.oobpre = c->oobpre;
   a.part = c->part;
   a.nblk = nblocks(c->grid.ngbx, kTabBlock);
+  a.clear = counts_stay_clear(c) ? 1u : 0u;
   a.grid = c->grid;
   a.wpb = c->tiles.motion_waves_per_block ? c->tiles.motion_waves_per_block : 1;
   a.ctl = c->ctl;
@@ -1847,7 +1870,12 @@ static void nsort_tables(cleo_ctx* c, const NsortArgs& a, double* gs = nullptr) 
     hipLaunchKernelGGL(k_nsort_tot<true>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a, c->st, gs);
   else
     hipLaunchKernelGGL(k_nsort_tot<false>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a, GState{}, gs);
-  if (a.nblk > 1) hipLaunchKernelGGL(k_nsort_part, dim3(1), dim3(1024), 0, c->stream, a.part, a.nblk);
+  if (a.nblk > kApplyBlocks) {
+    hipLaunchKernelGGL(k_nsort_part, dim3(1), dim3(1024), 0, c->stream, a.part, a.nblk);
+    hipLaunchKernelGGL(k_nsort_apply<true>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a);
+  } else if (a.nblk > 1) {
+    hipLaunchKernelGGL(k_nsort_apply<false>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a);
+  }
 }
 // the sorted store in buffer `dst` becomes current, with the refs its sort wrote
 static void nsort_commit(cleo_ctx* c, int dst) {
@@ -2796,7 +2824,6 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_motion_drops(MotionAr
     b.grid.yh = bounds_lds + nzh + nxh;
   }
   const uint32_t ndom = a.off[a.grid.ngbx];
-  uint32_t nmoved = 0;
   // block-uniform chunks of 512 drops keep every wave in the loop together for the ballots
   for (uint64_t k0 = 2ull * blockIdx.x * blockDim.x; k0 < ndom; k0 += 2ull * gridDim.x * blockDim.x) {
     const uint64_t ka = k0 + threadIdx.x, kb = ka + blockDim.x;
@@ -2825,16 +2852,16 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_motion_drops(MotionAr
     }
     if (a.step && acta) __builtin_nontemporal_store(static_cast<uint8_t>(Ma.dir), &a.step[ka]);
     if (a.step && actb) __builtin_nontemporal_store(static_cast<uint8_t>(Mb.dir), &a.step[kb]);
-    nmoved += static_cast<uint32_t>(__popcll(__ballot(acta))) + static_cast<uint32_t>(__popcll(__ballot(actb)));
     count_keys(a.cnt, motion_key(Ma, ga), acta, lane);
     count_keys(a.cnt, motion_key(Mb, gb), actb, lane);
   }
-  if (lane == 0) put_stat(a.stat, ST_MOTION_DROPS, nmoved);
+  if (blockIdx.x == 0 && threadIdx.x == 0) put_stat(a.stat, ST_MOTION_DROPS, ndom);  // each drop of the domain
 }
 
 // launches k_motion_drops with the bounds in LDS when they fit
 template <bool kWrite>
 static void launch_motion_drops(cleo_ctx* c, const MotionArgs& a, unsigned nb) {
+  clear_counts(c);
   const uint32_t nb_ = a.grid.nz + a.grid.nx + a.grid.ny + 3;
   if (nb_ <= kMotionLdsBounds)
     hipLaunchKernelGGL((k_motion_drops<kWrite, true>), dim3(nb), dim3(256), nb_ * sizeof(double), c->stream, a);

@@ -20,6 +20,8 @@ constexpr uint32_t kCondQueueWavesPerCu = 12;
 constexpr uint32_t kGsStride = 4;
 // gridboxes whose sort totals are scanned together (threads of k_nsort_tot)
 constexpr uint32_t kTabBlock = 256;
+// blocks of gridboxes up to which each block sums the totals before it
+constexpr uint32_t kApplyBlocks = 1024;
 // LDS window (values) of the per-gridbox drop-order sums
 constexpr uint32_t kSumWin = 1024;
 
@@ -76,13 +78,13 @@ struct MotionArgs {
 struct NsortArgs {
   SoA src, dst;
   const uint32_t* off;  // current refs (ngbx+1)
-  uint32_t* off_new;    // refs of the sorted store (ngbx+1), written by the rank pass
+  uint32_t* off_new;    // refs of the sorted store (ngbx+1)
   uint32_t* nact;       // the sorted store's drops per gridbox
-  uint32_t* cnt;        // ngbx*28: arrivals per (destination, step); left zero by k_nsort_tot
+  uint32_t* cnt;        // ngbx*28: arrivals per (destination, step)
+  uint32_t clear;       // k_nsort_tot leaves cnt zero
   uint32_t* runs;       // ngbx*28: per (source, step) the run's offset among its destination's arrivals
-  uint32_t* tot;        // ngbx+1: arrivals before each destination in its block of kTabBlock; tot[ngbx] = 0
-  uint32_t* oobpre;     // ngbx: drops leaving the domain before each gridbox in its block
-  uint32_t* part;       // nblk pairs: both sums before each block; then the sorted store's domain drops
+  uint32_t* oobpre;     // ngbx: drops leaving the domain before each gridbox
+  uint32_t* part;       // nblk pairs: arrivals and leaving drops per block of kTabBlock gridboxes
   uint32_t nblk;
   Grid grid;
   uint32_t wpb;
