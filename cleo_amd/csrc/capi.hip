@@ -191,7 +191,8 @@ CollCfg make_collcfg(const cleo_coll_params& p) {
   return k;
 }
 
-int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p) {
+// one collision event; last: nothing else follows in its microphysics pass
+int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p, bool last) {
   if (const char* m = coll_params_error(p)) return fail(c, CLEO_E_ARG, m);
   if (c->rng_mode == 0) return fail(c, CLEO_E_STATE, "no random-number stream set");
   const bool inj = c->rng_mode == 2;
@@ -222,6 +223,12 @@ int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p) {
   a.big = c->big_scratch;
   a.big2 = reinterpret_cast<uint32_t*>(c->dm);
   a.event_ofs = c->events_pending++;
+  if (last && c->grid.ngbx == 1 && c->ntot <= kResortOneDrops) {  // one gridbox: the event's own kernel ends the pass
+    a.close = c->events_pending;
+    a.alt = c->buf[1 - c->cur];
+    a.off_new = c->off_alt;
+    c->events_pending = 0;
+  }
   launch_collisions(c, a);
   if (compose) std::swap(c->order, c->order_alt);
   c->order_live = true;
@@ -231,6 +238,7 @@ int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p) {
 
 // the end of a microphysics pass with collision events
 void end_collisions(cleo_ctx* c) {
+  if (c->events_pending == 0) return;  // its last event has done it
   resort_nulls(c, c->events_pending);
   c->events_pending = 0;
 }
@@ -346,7 +354,10 @@ int enqueue_run_step(cleo_ctx* c, uint32_t t_mdl, uint32_t t_mdl_next) {
           rc = enqueue_condensation(c, q.cond, pending_qcond);  // with the qcond recompute first if due
         } else {
           if (pending_qcond) qcond_now();  // qcond after the sort comes before any drop changes
-          rc = enqueue_collision_event(c, q.coll);
+          bool last = true;  // of everything in this pass
+          for (uint32_t k = 0; k < p.n; ++k)
+            last = last && !(k > i && on_step(k, subt)) && next_of(subt, process_interval(p.proc[k])) >= t_sdm_next;
+          rc = enqueue_collision_event(c, q.coll, last);
           any_coll = true;
         }
         if (rc != CLEO_OK) return rc;
@@ -411,6 +422,7 @@ int cleo_create(cleo_ctx** out, uint64_t maxn, const cleo_domain_desc* dom) {
   want(zero, &c->off, ngbx + 1);
   want(zero, &c->off_alt, ngbx + 1);
   want(zero, &c->nact, ngbx);
+  want(zero, &c->coll_share, 2 * kSplitGbx);
   want(zero, &c->d_state, 11 * ngbx);
   want(zero, &c->cnt, 56 * ngbx);  // counts, then the run offsets of the neighbour sort
   want(rest, &c->d_halves, nh);
@@ -802,7 +814,7 @@ int cleo_condensation(cleo_ctx* c, const cleo_cond_params* p) {
 
 int cleo_collisions(cleo_ctx* c, const cleo_coll_params* p) {
   if (!c || !p) return CLEO_E_ARG;
-  const int rc = enqueue_collision_event(c, *p);
+  const int rc = enqueue_collision_event(c, *p, true);
   if (rc != CLEO_OK) return rc;
   end_collisions(c);
   return launch_check(c);

@@ -285,6 +285,134 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_
   total = readlane_u32(x, kWave - 1);
   return x - v;
 }
+__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* ws, uint32_t& total) {
+  uint32_t wt;
+  const uint32_t x = wave_excl_scan(v, lane_id(), wt);
+  const uint32_t w = threadIdx.x / kWave, nw = blockDim.x / kWave;
+  __syncthreads();  // the previous scan is done with ws
+  if (lane_id() == 0) ws[w] = wt;
+  __syncthreads();
+  uint32_t pre = 0;
+  total = 0;
+  for (uint32_t i = 0; i < nw; ++i) {
+    pre += i < w ? ws[i] : 0u;
+    total += ws[i];
+  }
+  return pre + x;
+}
+__device__ __forceinline__ void copy_drop(const SoA& src, const SoA& dst, uint64_t p, uint64_t q) {
+  dst.gbx[q] = src.gbx[p];
+  dst.c3[q] = src.c3[p];
+  dst.c1[q] = src.c1[p];
+  dst.c2[q] = src.c2[p];
+  dst.xi[q] = src.xi[p];
+  dst.r[q] = src.r[p];
+  dst.msol[q] = src.msol[p];
+  dst.id[q] = src.id[p];
+}
+// ============================ re-sort after collisions ========================================
+// When collisions left nulls, SDMMethods sorts again: the active drops of each gridbox move together
+// and the nulls of all gridboxes, in order, go behind the domain (before the drops that were out of it
+// already, which keep their positions).  Everything below ends at once when there are no nulls, so that
+// a captured graph needs no host decision.  It usually does end at once, so what it costs is launches
+// (2.3 us each in a graph): two for large domains (k_resort_gather, k_resort_back), one workgroup for
+// all of it up to kResortOneDrops drops, and none for a single gridbox, whose last collision event
+// closes the pass itself (step of one gridbox of 8192 drops 47 -> 26 us, 15 of them by the shares below).
+//
+// The re-sort also advances the event counter past the events of this microphysics pass.
+struct Resort {
+  DevCtl* ctl;
+  SoA src, dst;
+  uint32_t *off, *nact, *off_new, *order;
+  uint32_t ngbx;
+};
+__device__ __forceinline__ void resort_begin(const Resort& r, uint32_t events, uint32_t flag) {
+  r.ctl->event += events;
+  r.ctl->resort_go = flag;
+  r.ctl->resort_nsrc = r.off[r.ngbx];
+  if (flag) r.ctl->stats[ST_SORTS] += 1;
+}
+// New refs and gather of gridboxes [lo, hi) by the B lanes of a workgroup.  Slot k of gridbox g goes to
+// off_new[g] + k when active, else behind the active drops of the domain and the nulls of the gridboxes
+// before (off[g] - off_new[g] of them).  Each workgroup sums the counts before its own gridboxes itself.
+template <int B>
+__device__ __forceinline__ void resort_gather(const Resort& r, uint32_t lo, uint32_t hi, uint32_t tid) {
+  __shared__ uint32_t ws[B / kWave];
+  uint32_t before = 0, active = 0;
+  for (uint32_t g = tid; g < r.ngbx; g += B) {
+    const uint32_t v = r.nact[g];
+    active += v;
+    before += g < lo ? v : 0u;
+  }
+  uint32_t run, all;
+  block_excl_scan(before, ws, run);
+  block_excl_scan(active, ws, all);
+  active = all;
+  for (uint32_t g0 = lo; g0 < hi; g0 += B) {
+    const uint32_t g = g0 + tid;
+    const uint32_t at = run + block_excl_scan(g < hi ? r.nact[g] : 0u, ws, all);
+    if (g < hi) r.off_new[g] = at;
+    run += all;
+  }
+  if (tid == 0 && hi == r.ngbx) r.off_new[hi] = active;
+  __syncthreads();
+  const uint32_t nsrc = r.off[r.ngbx];
+  const bool wide = hi - lo < B / kWave;  // all lanes at one gridbox, else a wave each
+  const uint32_t lane = wide ? tid : tid % kWave, lanes = wide ? B : kWave;
+  for (uint32_t g = wide ? lo : lo + tid / kWave; g < hi; g += wide ? 1u : B / kWave) {
+    const uint32_t o = r.off[g], n = r.nact[g], nfull = r.off[g + 1] - o, to = r.off_new[g];
+    for (uint32_t k = lane; k < nfull; k += lanes) {
+      const uint32_t p = r.order[o + k];
+      const uint32_t q = k < n ? to + k : active + (o - to) + (k - n);
+      if (p < nsrc && q < nsrc) copy_drop(r.src, r.dst, p, q);
+    }
+  }
+}
+__device__ __forceinline__ void resort_back(const Resort& r, uint32_t nsrc, uint64_t first, uint64_t stride) {
+  for (uint64_t q = first; q < nsrc; q += stride) {
+    copy_drop(r.dst, r.src, q, q);
+    r.order[q] = static_cast<uint32_t>(q);
+  }
+  for (uint64_t g = first; g <= r.ngbx; g += stride) {
+    r.off[g] = r.off_new[g];
+    if (g < r.ngbx) r.nact[g] = r.off_new[g + 1] - r.off_new[g];
+  }
+}
+// all of it by one workgroup
+template <int B>
+__device__ __forceinline__ void resort_alone(const Resort& r, uint32_t events, uint32_t tid) {
+  const uint32_t flag = r.ctl->resort_flag;
+  __syncthreads();
+  if (tid == 0) {
+    resort_begin(r, events, flag);
+    r.ctl->resort_flag = 0u;
+  }
+  if (!flag) return;
+  const uint32_t nsrc = r.off[r.ngbx];
+  resort_gather<B>(r, 0u, r.ngbx, tid);
+  __syncthreads();
+  resort_back(r, nsrc, tid, B);
+}
+__global__ void __launch_bounds__(1024) k_resort_one(Resort r, uint32_t events) { resort_alone<1024>(r, events, threadIdx.x); }
+__global__ void __launch_bounds__(1024) k_resort_gather(Resort r, uint32_t events) {
+  const uint32_t flag = r.ctl->resort_flag;  // cleared by k_resort_back
+  if (blockIdx.x == 0 && threadIdx.x == 0) resort_begin(r, events, flag);
+  if (!flag) return;
+  const uint32_t per = (r.ngbx + gridDim.x - 1) / gridDim.x;
+  const uint32_t lo = min(r.ngbx, blockIdx.x * per), hi = min(r.ngbx, lo + per);
+  if (lo < hi) resort_gather<1024>(r, lo, hi, threadIdx.x);
+}
+__global__ void __launch_bounds__(256) k_resort_back(Resort r) {
+  if (!r.ctl->resort_go) return;
+  const uint64_t first = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
+  if (first == 0) r.ctl->resort_flag = 0u;
+  resort_back(r, r.ctl->resort_nsrc, first, static_cast<uint64_t>(gridDim.x) * blockDim.x);
+}
+
+__device__ __forceinline__ Resort coll_resort(const CollArgs& a) {
+  return Resort{a.ctl, a.s, a.alt, a.off, a.nact, a.off_new, a.order, a.ngbx};
+}
+
 // ---- Fisher-Yates without its serial chain -----------------------------------------------------
 // Swap `iter` (iter = n-1 .. 1, with index j <= iter) moves the element at place j to place iter for
 // good and the one at place iter to place j, so the shuffled order follows from the indices alone.
@@ -298,7 +426,7 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_
 // entries long on average) only take minima, so the result does not depend on the order of the
 // entries.  The chains of U are one hop long on average (11 at most in 8192 drops).  Serial swaps take
 // one dependent memory round trip each: a gridbox of 8192 drops 1.68 ms for its collisions against
-// 22 us here, 24679 gridboxes of 300 drops 4.9 ms against 0.13 ms.  What bounds it: LDS (about 30
+// 34 us here and 19 us in shares (below), 24679 gridboxes of 300 drops 4.9 ms against 0.13 ms.  What bounds it: LDS (about 30
 // accesses per 64 drops, with bank conflicts) and the latency of its four passes.
 //
 // A team of B lanes (a wave, or a whole workgroup) shuffles the drops of one or more gridboxes, its
@@ -455,7 +583,9 @@ __device__ __forceinline__ void team_collide(const CollArgs& a, bool lds, const 
 }
 
 // A team per workgroup of B lanes, `gpt` consecutive gridboxes at a time, whose lists fit `cap` items
-// of LDS together, else one after the other (and through HBM scratch above cap drops).
+// of LDS together, else one after the other (and through HBM scratch above cap drops).  For gridboxes
+// of 512 drops or fewer its flat passes are faster than the chains of k_coll_split (one of 501 drops with
+// kinetic energies 11.6 against 12.9 us), and so they are for many gridboxes up to 2048.
 template <int B, bool Kinetic>
 __global__ void __launch_bounds__(B) CLEO_OCCUPANCY(Kinetic && B <= 256 ? 3 : 4) k_coll_team(CollArgs a, uint32_t gpt, uint32_t cap) {
   extern __shared__ uint32_t lds_dyn[];
@@ -507,6 +637,141 @@ __global__ void __launch_bounds__(B) CLEO_OCCUPANCY(Kinetic && B <= 256 ? 3 : 4)
     put_stat(a.stat, ST_COLL_PAIRS, pairs);
     put_stat(a.stat, ST_COLL_EVENTS, events);
     put_stat(a.stat, ST_NULLS, nulls);
+  }
+  if (a.close) {
+    team_sync<B>();
+    resort_alone<B>(coll_resort(a), a.close, tid);
+  }
+}
+
+// ---- large gridboxes: a workgroup, or one per share of the gridbox's pairs -----------------------
+// Every workgroup builds the whole lists of its gridbox (draws and atomic exchanges, two draws of four
+// swaps per lane for 8192 drops) and follows the chains only of the drops in its share of the pairs, so
+// the shares need nothing from each other; a chain step takes the minimum of a place's list anew, and
+// three passes over the lists with their barriers go.  What bounds it: the latency of the lists' two
+// passes and of one pair per lane (k_coll_team's pairs of 8192 drops are four in series on one CU).
+// The last share to finish orders the nulls; it needs the others' stores only then, but every share
+// makes its own visible (one write-back of an L2 that holds this gridbox only).
+constexpr uint32_t kSplitMaxItems = 19200;  // 150 KB of lists
+constexpr uint32_t kSplitItemBytes = 8;     // LDS of one item: a 32-bit head and two 16-bit places
+struct FySplitLds {
+  uint32_t* head;
+  uint16_t *nxt, *jst;
+  using Idx = uint16_t;
+  __device__ __forceinline__ uint32_t exch(uint32_t at, uint32_t v) const { return atomicExch(&head[at], v); }
+  __device__ __forceinline__ uint32_t first(uint32_t at) const { return head[at]; }
+};
+template <int B, class Mem>
+__device__ __forceinline__ void split_lists(const CollArgs& a, const Mem& M, uint32_t g, uint32_t base, uint32_t n,
+                                            uint64_t event, uint32_t tid) {
+  using Idx = typename Mem::Idx;
+  constexpr uint32_t kNone = static_cast<uint32_t>(static_cast<Idx>(~Idx(0)));
+  for (uint32_t f = tid; f < n; f += B) M.head[f] = kNone;
+  __syncthreads();
+  for (uint32_t q = tid; q < (n + 2u) / 4u; q += B) {
+    uint32_t r4[4] = {0u, 0u, 0u, 0u};
+    if (!a.inj_j) rng_block(a.seed, event, 0u, g, q, r4);
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w) {
+      const uint32_t t = 4u * q + w;
+      if (t + 1 < n) {
+        const uint32_t iter = n - 1 - t;
+        const uint32_t j = a.inj_j ? inj_index(a, g, base, n, t) : fy_scale(r4[w], iter);
+        M.jst[iter] = static_cast<Idx>(j);
+        M.nxt[iter] = static_cast<Idx>(M.exch(j, iter));
+      }
+    }
+  }
+  __syncthreads();
+}
+// the shuffled order's entry k
+template <class Mem>
+__device__ __forceinline__ uint32_t split_place(const Mem& M, uint32_t k) {
+  using Idx = typename Mem::Idx;
+  constexpr uint32_t kNone = static_cast<uint32_t>(static_cast<Idx>(~Idx(0)));
+  uint32_t x = k;
+  if (k > 0) {
+    const uint32_t j = M.jst[k];
+    if (j != k) {
+      x = kNone;  // min{ e in L(j) : e > k }
+      for (uint32_t e = M.first(j); e != kNone; e = M.nxt[e])
+        if (e > k && e < x) x = e;
+      if (x == kNone) return j;
+    }
+  }
+  for (;;) {
+    uint32_t m = kNone;  // min(L(x) \ {x})
+    for (uint32_t e = M.first(x); e != kNone; e = M.nxt[e])
+      if (e != x && e < m) m = e;
+    if (m == kNone) return x;
+    x = m;
+  }
+}
+template <int B, bool Kinetic>
+__global__ void __launch_bounds__(B) CLEO_OCCUPANCY(Kinetic && B <= 512 ? 3 : 4) k_coll_split(CollArgs a, uint32_t split, uint32_t cap) {
+  extern __shared__ uint32_t lds_dyn[];
+  __shared__ uint32_t s_nulls, s_last;
+  const uint32_t tid = threadIdx.x, g = blockIdx.x / split, part = blockIdx.x % split;
+  const uint64_t event = a.ctl->event + a.event_ofs;
+  const uint32_t base = a.off[g], nfull = a.off[g + 1] - base, n = a.nact[g];
+  const bool lds = n <= cap;
+  uint16_t* const half = reinterpret_cast<uint16_t*>(lds_dyn + cap);
+  const FySplitLds L{lds_dyn, half, half + cap};
+  // two words per drop of the collision scratch, two of the per-drop condensation scratch (free
+  // during collisions)
+  const uint64_t b2 = 2ull * base;
+  const FyHbm H{a.big2 + b2, a.big + b2, a.big + b2 + n, nullptr};
+  // the lists in HBM scratch are one workgroup's, and then all of the pairs
+  const uint32_t shares = lds ? split : 1u;
+  if (tid == 0) s_nulls = 0u;
+  if (lds)
+    split_lists<B>(a, L, g, base, n, event, tid);
+  else if (part == 0)
+    split_lists<B>(a, H, g, base, n, event, tid);
+  auto place = [&](uint32_t k) -> uint32_t { return lds ? split_place(L, k) : split_place(H, k); };
+  uint32_t events = 0, nulls = 0;
+  const uint32_t npairs = n / 2, per = (npairs + shares - 1) / shares, hi = min(npairs, (part + 1) * per);
+  if (part < shares) {
+    for (uint32_t jj = part * per + tid; jj < hi; jj += B) {
+      const uint32_t ka = coll_pos(a, base, place(2 * jj)), kb = coll_pos(a, base, place(2 * jj + 1));
+      if (coll_pair<Kinetic>(a, g, base, n, jj, ka, kb, event, events)) ++nulls;
+    }
+    // unpaired last drop and the inactive tail (nulls of earlier sub-steps) keep their places
+    if (part + 1 == shares)
+      for (uint32_t k = 2 * npairs + tid; k < nfull; k += B) a.order[base + k] = coll_pos(a, base, k < n ? place(k) : k);
+  }
+  nulls = wave_sum_u32(nulls);
+  events = wave_sum_u32(events);
+  if (lane_id() == 0 && nulls) atomicAdd(&s_nulls, nulls);
+  // this workgroup's stores are in L2 before its first wave makes them visible to the other shares
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const uint32_t mine = s_nulls;
+    uint32_t all = mine, last = 1u;
+    if (split > 1) {
+      uint32_t* const share = a.share + 2u * g;  // nulls so far, shares done: zero between launches
+      if (mine) atomicAdd(&share[0], mine);
+      __threadfence();
+      last = atomicAdd(&share[1], 1u) + 1u == split ? 1u : 0u;
+      if (last) {
+        __threadfence();
+        all = atomicExch(&share[0], 0u);
+        atomicExch(&share[1], 0u);
+      }
+    }
+    s_nulls = all;
+    s_last = last;
+    if (part == 0) put_stat(a.stat, ST_COLL_PAIRS, n / 2);
+    if (last) put_stat(a.stat, ST_NULLS, all);
+  }
+  if (lane_id() == 0) put_stat(a.stat, ST_COLL_EVENTS, events);
+  __syncthreads();
+  if (!s_last) return;
+  if (s_nulls && tid < kWave) coll_order_nulls(a, g, base, n, s_nulls, static_cast<int>(tid));
+  if (a.close) {
+    __syncthreads();
+    resort_alone<B>(coll_resort(a), a.close, tid);
   }
 }
 
@@ -851,21 +1116,6 @@ __device__ __forceinline__ Moved move_drop(const MotionArgs& a, uint32_t g, cons
 // ============================ neighbour sort ==================================================
 
 // exclusive prefix of v over the block's kTabBlock threads, and the block's total
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* ws, uint32_t& total) {
-  uint32_t wt;
-  const uint32_t x = wave_excl_scan(v, lane_id(), wt);
-  const uint32_t w = threadIdx.x / kWave, nw = blockDim.x / kWave;
-  __syncthreads();  // the previous scan is done with ws
-  if (lane_id() == 0) ws[w] = wt;
-  __syncthreads();
-  uint32_t pre = 0;
-  total = 0;
-  for (uint32_t i = 0; i < nw; ++i) {
-    pre += i < w ? ws[i] : 0u;
-    total += ws[i];
-  }
-  return pre + x;
-}
 // the condensation inputs of a gridbox (condensation.cpp:44-56)
 __device__ __forceinline__ void gbx_thermo(const GState& st, uint32_t g, double* gs) {
   const double temp = st.temp[g], press = st.press[g];
@@ -1218,16 +1468,6 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(6) k_nsort_perm(NsortArgs 
 }
 
 // record p of src to position q of dst
-__device__ __forceinline__ void copy_drop(const SoA& src, const SoA& dst, uint64_t p, uint64_t q) {
-  dst.gbx[q] = src.gbx[p];
-  dst.c3[q] = src.c3[p];
-  dst.c1[q] = src.c1[p];
-  dst.c2[q] = src.c2[p];
-  dst.xi[q] = src.xi[p];
-  dst.r[q] = src.r[p];
-  dst.msol[q] = src.msol[p];
-  dst.id[q] = src.id[p];
-}
 // The drops that were out of the domain before (positions nsrc on) follow the newly out-of-domain
 // ones; the domain's drops fill the first nsrc positions of the sorted store either way, so they keep
 // their positions.
@@ -1362,75 +1602,6 @@ __global__ void k_publish_ctl(const DevCtl* ctl, const uint32_t* off, uint32_t n
   if (threadIdx.x == 0) out->ndomain = off[ngbx];
 }
 __global__ void k_set_event(DevCtl* ctl, uint64_t event) { ctl->event = event; }
-
-// ============================ re-sort after collisions ========================================
-// When collisions left nulls, SDMMethods sorts again: the active drops of each gridbox move together
-// and the nulls of all gridboxes, in order, go behind the domain (before the drops that were out of it
-// already, which keep their positions).  Three launches that end at once when there are no nulls, so
-// that a captured graph needs no host decision: the plan (one workgroup), the records in their new
-// places in the other buffer, and their way back with the new refs.
-//
-// The plan also advances the event counter past the events of this microphysics pass.
-__global__ void __launch_bounds__(1024) k_resort_plan(DevCtl* ctl, const uint32_t* off, const uint32_t* nact, uint32_t ngbx,
-                                                      uint32_t* off_new, uint32_t events) {
-  __shared__ uint32_t ws[16];
-  const uint32_t flag = ctl->resort_flag;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    ctl->event += events;
-    ctl->resort_flag = 0u;
-    ctl->resort_go = flag;
-    ctl->resort_nsrc = off[ngbx];
-    if (flag) ctl->stats[ST_SORTS] += 1;
-  }
-  if (!flag) return;
-  uint32_t run = 0;
-  for (uint64_t g0 = 0; g0 < ngbx; g0 += 4096u) {  // four gridboxes per thread
-    const uint64_t g = g0 + 4u * threadIdx.x;
-    uint32_t n[4], sum = 0, all;
-    for (uint32_t i = 0; i < 4; ++i) {
-      n[i] = g + i < ngbx ? nact[g + i] : 0u;
-      sum += n[i];
-    }
-    uint32_t at = run + block_excl_scan(sum, ws, all);
-    for (uint32_t i = 0; i < 4; ++i) {
-      if (g + i < ngbx) off_new[g + i] = at;
-      at += n[i];
-    }
-    run += all;
-  }
-  if (threadIdx.x == 0) off_new[ngbx] = run;
-}
-// slot k of gridbox g: place off_new[g] + k when active, else behind the active drops of the domain
-// and the nulls of the gridboxes before (off[g] - off_new[g] of them)
-__global__ void __launch_bounds__(256) k_resort_gather(const DevCtl* ctl, SoA src, SoA dst, const uint32_t* off,
-                                                       const uint32_t* nact, const uint32_t* off_new, uint32_t ngbx,
-                                                       const uint32_t* order) {
-  if (!ctl->resort_go) return;
-  const uint32_t nsrc = ctl->resort_nsrc, active = off_new[ngbx];
-  for (uint32_t g = wave_index(); g < ngbx; g += wave_count()) {
-    const uint32_t lo = off[g], n = nact[g], nfull = off[g + 1] - lo, to = off_new[g];
-    for (uint32_t k = static_cast<uint32_t>(lane_id()); k < nfull; k += kWave) {
-      const uint32_t p = order[lo + k];
-      const uint32_t q = k < n ? to + k : active + (lo - to) + (k - n);
-      if (p < nsrc && q < nsrc) copy_drop(src, dst, p, q);
-    }
-  }
-}
-__global__ void __launch_bounds__(256) k_resort_back(const DevCtl* ctl, SoA src, SoA dst, uint32_t* off, uint32_t* nact,
-                                                     const uint32_t* off_new, uint32_t ngbx, uint32_t* order) {
-  if (!ctl->resort_go) return;
-  const uint64_t first = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x,
-                 stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t q = first; q < ctl->resort_nsrc; q += stride) {
-    copy_drop(src, dst, q, q);
-    order[q] = static_cast<uint32_t>(q);
-  }
-  for (uint64_t g = first; g <= ngbx; g += stride) {
-    off[g] = off_new[g];
-    if (g < ngbx) nact[g] = off_new[g + 1] - off_new[g];
-  }
-}
 
 // ============================ generic stable radix sort =======================================
 // LSD radix sort of (key, position) with digits of up to 8 bits, three launches per pass: digit counts
@@ -1751,6 +1922,19 @@ static void launch_coll_team(cleo_ctx* c, const CollArgs& args, uint32_t gpt, ui
   else
     launch_coll_team_k<B, false>(c, a, nb, gpt, cap);
 }
+template <int B>
+static void launch_coll_split(cleo_ctx* c, const CollArgs& args, uint32_t split, uint64_t items) {
+  CollArgs a = args;
+  const uint32_t cap = static_cast<uint32_t>(std::min<uint64_t>(kSplitMaxItems, (items + 63) / 64 * 64));
+  a.stat = stat_slots(c);
+  a.share = c->coll_share;
+  kev_mark(c, 0);
+  if (coll_is_kinetic(a.k))
+    hipLaunchKernelGGL((k_coll_split<B, true>), dim3(a.ngbx * split), dim3(B), cap * kSplitItemBytes, c->stream, a, split, cap);
+  else
+    hipLaunchKernelGGL((k_coll_split<B, false>), dim3(a.ngbx * split), dim3(B), cap * kSplitItemBytes, c->stream, a, split, cap);
+  kev_mark(c, 1);
+}
 void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   if (args.ngbx == 0) return;
   CollArgs a = args;
@@ -1772,16 +1956,24 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   }
   // Teams, one workgroup each.  A wave takes as many gridboxes as make 512 drops (128 to 1024 tried:
   // 55, 49, 45, 68 us on 32^3 gridboxes of 64), but no more than leave 4096 teams (3750 gridboxes of
-  // 128: 18 us with one each, 33 us with four).  With few gridboxes, or large ones, the pairs of one
-  // gridbox are spread over the waves of a workgroup instead.
+  // 128: 18 us with one each, 33 us with four).  With few gridboxes, or larger ones, a workgroup takes
+  // the pairs of one gridbox.
   if (mean <= 512 && (mean <= 96 || a.ngbx > 512)) {
     const uint64_t gpt = std::min<uint64_t>(kWave, std::max<uint64_t>(1, std::min<uint64_t>(512 / mean, a.ngbx / 4096)));
     const double items = static_cast<double>(gpt * mean);
     launch_coll_team<kWave>(c, a, static_cast<uint32_t>(gpt), static_cast<uint64_t>(items + 6.0 * std::sqrt(items)) + 128);
-  } else if (mean <= 2048) {
+  } else if (mean <= 512 || (mean <= 2048 && a.ngbx > kSplitGbx)) {
     launch_coll_team<256>(c, a, 1u, 2 * mean);
   } else {
-    launch_coll_team<1024>(c, a, 1u, 2 * mean);
+    // Large gridboxes: as many lanes as the chip has room for, and one more workgroup per 1024 drops
+    // of a gridbox while 128 of them stay free of each other (us by team / 512 lanes / 1024 lanes /
+    // 1024 lanes in shares; 1 gridbox of 1000 drops 16.1 / 13.6 / 13.8 / 14.8, of 2000 26.9 / 19.7 /
+    // 16.6 / 18.2, of 8192 39.7 / 45.1 / 31.9 / 20.7, of 14000 62.8 / 71.4 / 48.6 / 23.2; 64 of 5000
+    // 29.3 / 37.0 / 25.9 / 25.7; 512 of 1500 27.3 / 22.6 / 30.4; 400 of 3000 38.9 / 32.3 / 37.4).
+    if (a.ngbx <= 256 && mean > 1024)
+      launch_coll_split<1024>(c, a, static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(mean / 1024, 128 / a.ngbx))), 2 * mean);
+    else
+      launch_coll_split<512>(c, a, 1u, 2 * mean);
   }
 }
 StatSlots stat_slots(cleo_ctx* c) { return StatSlots{c->sp}; }
@@ -1895,13 +2087,13 @@ void neighbour_sort_to(cleo_ctx* c, const SoA& src, const SoA& dst, int commit_d
 }
 
 void resort_nulls(cleo_ctx* c, uint32_t events) {
-  const uint32_t ngbx = c->grid.ngbx;
-  const SoA &s = c->buf[c->cur], &t = c->buf[1 - c->cur];
-  hipLaunchKernelGGL(k_resort_plan, dim3(1), dim3(1024), 0, c->stream, c->ctl, c->off, c->nact, ngbx, c->off_alt, events);
-  hipLaunchKernelGGL(k_resort_gather, dim3(sparse_blocks(64ull * ngbx)), dim3(256), 0, c->stream, c->ctl, s, t, c->off,
-                     c->nact, c->off_alt, ngbx, c->order);
-  hipLaunchKernelGGL(k_resort_back, dim3(sparse_blocks(std::max<uint64_t>(c->ntot, ngbx + 1ull))), dim3(256), 0, c->stream,
-                     c->ctl, t, s, c->off, c->nact, c->off_alt, ngbx, c->order);
+  const Resort r{c->ctl, c->buf[c->cur], c->buf[1 - c->cur], c->off, c->nact, c->off_alt, c->order, c->grid.ngbx};
+  if (c->ntot <= kResortOneDrops && r.ngbx <= kResortOneDrops) {
+    hipLaunchKernelGGL(k_resort_one, dim3(1), dim3(1024), 0, c->stream, r, events);
+    return;
+  }
+  hipLaunchKernelGGL(k_resort_gather, dim3(std::min<uint32_t>(r.ngbx, 256u)), dim3(1024), 0, c->stream, r, events);
+  hipLaunchKernelGGL(k_resort_back, dim3(sparse_blocks(std::max<uint64_t>(c->ntot, r.ngbx + 1ull))), dim3(256), 0, c->stream, r);
 }
 
 // A pending collision order applied: the domain's drops are gathered into the other buffer in

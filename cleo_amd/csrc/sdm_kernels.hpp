@@ -9,6 +9,8 @@ namespace cleo {
 constexpr uint32_t kTileMaxN = 255;
 constexpr uint32_t kTilePermBytes = 8192;
 constexpr uint32_t kTileMinGbx = 75000;  // gridboxes from which the tiles are the faster variant
+constexpr uint64_t kResortOneDrops = 16384;  // drops up to which one workgroup re-sorts the nulls
+constexpr uint32_t kSplitGbx = 512;  // most gridboxes of 512 to 2048 drops with a larger workgroup each
 constexpr uint32_t kCollTileLdsBytes = kTilePermBytes + 4u * (65u + 4u * 64u);
 constexpr uint32_t kBigGbx = 0xFFFFFFFFu;  // tile LDS marker of a gridbox the whole wave shuffles
 // condensation task ring: prepared drops per wave, and waves per CU of the default grid
@@ -42,7 +44,7 @@ struct CollArgs {
   // in: a pending order of an earlier event (position of the drop at each slot), composed with
   // this event's shuffle; null when the store is in its logical order
   const uint32_t* order_in;
-  const uint32_t* off;
+  uint32_t* off;
   uint32_t* nact;
   const double* vol;
   Solute sol;
@@ -58,6 +60,12 @@ struct CollArgs {
   const uint32_t* inj_op;
   uint32_t* big;   // scratch, two words per drop
   uint32_t* big2;  // the same again
+  // of a single gridbox: non-zero when this is the last event of its microphysics pass, whose `close`
+  // events are then counted and whose nulls re-sorted by the same kernel, with alt and off_new as scratch
+  uint32_t close;
+  SoA alt;
+  uint32_t* off_new;
+  uint32_t* share;  // two words per gridbox, zero between launches
   StatSlots stat;   // ST_COLL_PAIRS .. ST_NULLS
 };
 
