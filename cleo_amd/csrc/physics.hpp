@@ -118,12 +118,16 @@ __device__ __forceinline__ double quotient(double n, double d) {
 // e = 1 - x y^2: at most 0.63 ulp from 1/sqrt(x) over 1M values of 1e-140..1e140, as two
 // Newton-Raphson steps gave, in five instructions instead of eight; for positive finite x; 0 and +inf
 // give the estimate's own inf and 0, negative or NaN x gives NaN, as 1.0 / sqrt(x) does.
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  const double y0 = __builtin_amdgcn_rsq(x);
+__device__ __forceinline__ double rsqrt_step(double x, double y0) {
   const double e = fma(-(x * y0), y0, 1.0);
-  const double y = fma(y0 * e, fma(e, 0.375, 0.5), y0);
+  return fma(y0 * e, fma(e, 0.375, 0.5), y0);
+}
+__device__ __forceinline__ double rsqrt_nr(double x) {
+  const double y0 = __builtin_amdgcn_rsq(x), y = rsqrt_step(x, y0);
   return (x > 0.0 && x < __builtin_huge_val()) ? y : y0;
 }
+// of x known to be positive, normal and finite, or NaN
+__device__ __forceinline__ double rsqrt_normal(double x) { return rsqrt_step(x, __builtin_amdgcn_rsq(x)); }
 // x^p for several exponents p of one positive finite x.  With log2 x = e + lg, |lg| <= 1/2, the integer
 // part of p log2 x is taken out of p e by an FMA, so what is left is rounded at the size of 1 and not
 // of p log2 x: at most 2.7e-16 relative from the power for p = 1.963 and 0.702 over 1e-9..1e-2 (6e-17
@@ -356,22 +360,36 @@ struct NewtonCfg {
 // reference's quotients akoh/r, bkoh/r^3, subdelt/(z ffactor) and rprev/r are products with one
 // reciprocal square root of z (and 1/ffactor per drop): no FP64 division or square root per
 // evaluation instead of six divisions and a root, each term within a few ulp of the reference's.
-__device__ __forceinline__ void ode_g_dg(const ODEConsts& c, double subdelt, double rprev, double rsqrd,
-                                         double& g, double& dg) {
-  // products feeding a sum may fuse into FMAs here (one rounding fewer each)
-#pragma clang fp contract(fast)
-  const double inv_r = rsqrt_nr(rsqrd);
-  const double inv_r2 = inv_r * inv_r;
-  const double a_r = c.akoh * inv_r;
-  const double b_r3 = c.bkoh * (inv_r2 * inv_r);
-  const double alpha = c.s_ratio - 1 - a_r + b_r3;
-  const double beta_d = subdelt * (inv_r2 * c.inv_ffv);
-  const double beta = 2.0 * beta_d;
-  const double q = rprev * inv_r;
-  const double gamma = q * q;
-  g = 1 - gamma - alpha * beta;
-  const double alpha_d = a_r - 3.0 * b_r3;
-  dg = 1 - alpha_d * beta_d;
+// The solves are bound by the issue of these instructions: 13 and the root's 6 per evaluation.  Where
+// a small drop is at equilibrium, alpha's rounding times beta decides the convergence test, so the
+// products and FMAs are written out and every kernel rounds alike (other products of the constants
+// save three instructions and move such drops by 1e-8, the tolerance of the test).
+struct OdeRun {
+  double s1, akoh, bkoh, half_akoh;  // s_ratio - 1, Koehler factors
+  double inv_ffv, subdelt2, rprev;   // ventilation factor / ffactor, 2 subdelt
+};
+__device__ __forceinline__ OdeRun ode_run(const ODEConsts& c, double subdelt, double rprev) {
+  return OdeRun{c.s_ratio - 1, c.akoh, c.bkoh, 0.5 * c.akoh, c.inv_ffv, 2.0 * subdelt, rprev};
+}
+// kStart: rsqrd is any start value, else one of newton_next
+template <bool kStart>
+__device__ __forceinline__ void ode_g_dg(const OdeRun& c, double rsqrd, double& g, double& dg) {
+  const double inv_r = kStart ? rsqrt_nr(rsqrd) : rsqrt_normal(rsqrd);
+  const double inv_r2 = inv_r * inv_r, inv_r3 = inv_r2 * inv_r;
+  const double alpha = fma(c.bkoh, inv_r3, fma(-c.akoh, inv_r, c.s1));
+  const double beta = c.subdelt2 * (inv_r2 * c.inv_ffv);
+  const double q = c.rprev * inv_r;
+  g = fma(-alpha, beta, fma(-q, q, 1.0));
+  const double half_alpha_d = fma(-1.5, c.bkoh * inv_r3, c.half_akoh * inv_r);
+  dg = fma(-half_alpha_d, beta, 1.0);
+}
+// the next z of a Newton iteration (impliciteuler.cpp:240-255), between the reference's lower bound
+// and a value whose reciprocal square root needs no guard
+__device__ __forceinline__ double newton_next(double z, double g, double dg) {
+  return fmin(fmax(z * (1 - quotient(g, dg)), 1e-8), 1e300);
+}
+__device__ __forceinline__ bool newton_converged(const NewtonCfg& cfg, double g1, double g0) {
+  return fabs(g1 - g0) < fma(cfg.rtol, fabs(g1), cfg.atol);
 }
 // Newton state: z with g(z) and g'(z) already evaluated
 struct NewtonState {
@@ -380,15 +398,12 @@ struct NewtonState {
 // one Newton update + convergence test (impliciteuler.cpp:240-255, impliciteuler.hpp:214-219).
 // The reference evaluates g at the new z for the test and again as the next update's numerator;
 // both are the same expression of the same operands, so the value is carried over.
-__device__ __forceinline__ bool newton_iterate(const NewtonCfg& cfg, const ODEConsts& c, double subdelt,
-                                               double rprev, NewtonState& s, uint32_t& iters) {
+__device__ __forceinline__ bool newton_iterate(const NewtonCfg& cfg, const OdeRun& c, NewtonState& s, uint32_t& iters) {
   ++iters;
-  double z = s.z * (1 - quotient(s.g, s.dg));
-  z = fmax(z, 1e-8);
+  const double z = newton_next(s.z, s.g, s.dg);
   double g1, dg1;
-  ode_g_dg(c, subdelt, rprev, z, g1, dg1);
-  const double converged = cfg.rtol * fabs(g1) + cfg.atol;
-  const bool conv = fabs(g1 - s.g) < converged;
+  ode_g_dg<false>(c, z, g1, dg1);
+  const bool conv = newton_converged(cfg, g1, s.g);
   s = NewtonState{z, g1, dg1};
   return conv;
 }
@@ -396,31 +411,39 @@ __device__ __forceinline__ bool newton_iterate(const NewtonCfg& cfg, const ODECo
 // (cfg.budget reached; the drop is then solved again from the start, without a budget).  Returned
 // by value, not through flags passed by reference, which the compiler kept in scratch memory.
 enum : int { kNewtonDeferred = -1, kNewtonLimit = 0, kNewtonConverged = 1 };
-// newtonraphson_untilconverged (impliciteuler.cpp:207-227)
-__device__ __forceinline__ int newton_until(const NewtonCfg& cfg, const ODEConsts& c, uint32_t limit, double subdelt,
-                                            double rprev, NewtonState& s, uint32_t& iters) {
-  for (uint32_t niter = 1;; ++niter) {
+// newtonraphson_untilconverged (impliciteuler.cpp:207-227) from its iteration `niter` on
+__device__ __forceinline__ int newton_until(const NewtonCfg& cfg, const OdeRun& c, uint32_t niter, uint32_t limit,
+                                            NewtonState& s, uint32_t& iters) {
+  for (;; ++niter) {
     if (niter > limit) return kNewtonLimit;
     if (cfg.budget && iters >= cfg.budget) return kNewtonDeferred;
-    if (newton_iterate(cfg, c, subdelt, rprev, s, iters)) return kNewtonConverged;
+    if (newton_iterate(cfg, c, s, iters)) return kNewtonConverged;
   }
 }
 // integrate_condensation_ode (impliciteuler.cpp:128-141): 2 iterations, then restart from the guess
-// (only the second iteration's test decides); the new z and the outcome
+// (only the second iteration's test decides); the new z and the outcome.  The restart's first two
+// iterations are those just made, so their states and tests stand and it goes on from the third: a
+// drop of five counted iterations takes three (64^3 gridboxes of 122 drops 0.72 -> 0.65 ms).
 struct NewtonRun {
   double z;
   int status;
 };
-__device__ __forceinline__ NewtonRun newton_integrate(const NewtonCfg& cfg, const ODEConsts& c, double subdelt,
-                                                      double rprev, double zguess, uint32_t& iters) {
-  NewtonState s0;
-  s0.z = zguess;
-  ode_g_dg(c, subdelt, rprev, zguess, s0.g, s0.dg);
-  NewtonState s = s0;
-  (void)newton_iterate(cfg, c, subdelt, rprev, s, iters);
-  if (newton_iterate(cfg, c, subdelt, rprev, s, iters)) return NewtonRun{s.z, kNewtonConverged};
-  s = s0;
-  const int st = newton_until(cfg, c, cfg.maxniters, subdelt, rprev, s, iters);
+__device__ __forceinline__ NewtonRun newton_integrate(const NewtonCfg& cfg, const OdeRun& c, double zguess, uint32_t& iters) {
+  NewtonState s;
+  s.z = zguess;
+  ode_g_dg<true>(c, zguess, s.g, s.dg);
+  const bool conv1 = newton_iterate(cfg, c, s, iters);
+  const double z1 = s.z;
+  if (newton_iterate(cfg, c, s, iters)) return NewtonRun{s.z, kNewtonConverged};
+  const uint32_t limit = cfg.maxniters;
+  if (limit < 1) return NewtonRun{zguess, kNewtonLimit};
+  if (cfg.budget && iters >= cfg.budget) return NewtonRun{zguess, kNewtonDeferred};
+  ++iters;
+  if (conv1) return NewtonRun{z1, kNewtonConverged};
+  if (limit < 2) return NewtonRun{z1, kNewtonLimit};
+  if (cfg.budget && iters >= cfg.budget) return NewtonRun{z1, kNewtonDeferred};
+  ++iters;
+  const int st = newton_until(cfg, c, 3u, limit, s, iters);
   return NewtonRun{s.z, st};
 }
 __device__ __forceinline__ double initialguess(const ODEConsts& c, double rprev) {
@@ -517,17 +540,18 @@ __device__ __forceinline__ double solve_condensation(const NewtonCfg& cfg, doubl
   double rsqrd;
   NewtonRun run{0.0, kNewtonConverged};
   if (ucrit) {
+    const OdeRun run_c = ode_run(c, cfg.delt, rprev);
     bool plain = true;
     if (warm == warm) {
       // the start: the plain guess where it is already the root to the tolerance, else the learned
       NewtonState s;
       s.z = ziter;
-      ode_g_dg(c, cfg.delt, rprev, ziter, s.g, s.dg);
+      ode_g_dg<true>(run_c, ziter, s.g, s.dg);
       if (!(fabs(s.g) < cfg.atol)) {
         s.z = warm;
-        ode_g_dg(c, cfg.delt, rprev, warm, s.g, s.dg);
+        ode_g_dg<true>(run_c, warm, s.g, s.dg);
       }
-      const int st = newton_until(cfg, c, warm_limit, cfg.delt, rprev, s, o.iters);
+      const int st = newton_until(cfg, run_c, 1u, warm_limit, s, o.iters);
       if (st == kNewtonDeferred) {
         o.deferred = true;
         return 0.0;
@@ -537,7 +561,7 @@ __device__ __forceinline__ double solve_condensation(const NewtonCfg& cfg, doubl
       run.z = s.z;
     }
     if (plain) {
-      run = newton_integrate(cfg, c, cfg.delt, rprev, ziter, o.iters);
+      run = newton_integrate(cfg, run_c, ziter, o.iters);
       if (run.status == kNewtonDeferred) {
         o.deferred = true;
         return 0.0;
@@ -554,7 +578,7 @@ __device__ __forceinline__ double solve_condensation(const NewtonCfg& cfg, doubl
     bool maxed = false;
     while (remdelt > 0.0) {
       const double subdelt = fmin(mindelt, remdelt);
-      run = newton_integrate(cfg, c, subdelt, rp, ziter, o.iters);
+      run = newton_integrate(cfg, ode_run(c, subdelt, rp), ziter, o.iters);
       if (run.status == kNewtonDeferred) {
         o.deferred = true;
         return 0.0;

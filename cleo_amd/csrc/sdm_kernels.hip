@@ -2396,9 +2396,29 @@ __device__ __forceinline__ void finish_deferred(const CondFlatArgs& a, const uin
   }
 }
 
+// The kernel's arguments where the launch put them: Args has the kernel's parameters as its members, all
+// of 8-byte alignment.  After reread_args the compiler reads them again (scalar loads): arguments used
+// throughout a long loop body otherwise move out of the loop, into more scalar registers than there
+// are, and come back one v_readlane at a time, 75 to 100 per 64 drops of the gather with the solves
+// (2.1M drops: 99 -> 94 us; 33M coupled 178 -> 172 ms in 60 steps).
+template <class Args>
+__device__ __forceinline__ const Args* kernel_args() {
+  return reinterpret_cast<const Args*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
+}
+template <class Args>
+__device__ __forceinline__ void reread_args(const Args*& args) {
+  const __attribute__((address_space(4))) Args* p = (const __attribute__((address_space(4))) Args*)args;
+  asm volatile("" : "+s"(p));
+  args = (const Args*)p;
+}
 // per active drop, one thread each
 template <bool kTail>
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(5) k_cond_drops(CondFlatArgs a) {
+__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(5) k_cond_drops(CondFlatArgs) {
+  struct Args {
+    CondFlatArgs a;
+  };
+  auto args = kernel_args<Args>();
+  const CondFlatArgs& a = args->a;
   __shared__ uint32_t ndef;
   if (threadIdx.x == 0) ndef = 0u;
   __syncthreads();
@@ -2406,6 +2426,8 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(5) k_cond_drops(CondFlatAr
   uint64_t k_lo, k_hi;
   block_range(a.off[a.ngbx], k_lo, k_hi);
   for (uint64_t k0 = k_lo; k0 < k_hi; k0 += blockDim.x) {
+    reread_args(args);
+    const CondFlatArgs& a = args->a;
     const uint64_t k = k0 + threadIdx.x;
     bool active = false;
     uint32_t g = 0;
@@ -2461,7 +2483,17 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(5) k_cond_deferred(CondFla
 // the gridbox it reaches, so motion writes nothing of its own.  kLds: the coordinate bounds are read
 // from an LDS copy (dynamic shared memory of nz + nx + ny + 3 doubles).
 template <bool kMove, bool kLds, bool kTail>
-__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gather_cond(NsortArgs n, CondFlatArgs a, MotionArgs m) {
+__global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gather_cond(NsortArgs, CondFlatArgs, MotionArgs) {
+  struct Args {
+    NsortArgs n;
+    CondFlatArgs a;
+    MotionArgs m;
+  };
+  static_assert(sizeof(Args) == sizeof(NsortArgs) + sizeof(CondFlatArgs) + sizeof(MotionArgs) && alignof(Args) == 8, "layout");
+  auto args = kernel_args<Args>();
+  const NsortArgs& n = args->n;
+  const CondFlatArgs& a = args->a;
+  const MotionArgs& m = args->m;
   extern __shared__ double bounds_lds[];
   MotionArgs b = m;
   if constexpr (kMove && kLds) {
@@ -2488,6 +2520,9 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(kMove ? 4 : 5) k_sort_gath
   uint64_t q_lo, q_hi;
   block_range(nsrc, q_lo, q_hi);
   for (uint64_t q0 = q_lo; q0 < q_hi; q0 += blockDim.x) {
+    if constexpr (!kMove) reread_args(args);
+    const NsortArgs& n = args->n;
+    const CondFlatArgs& a = args->a;
     const uint64_t q = q0 + threadIdx.x;
     const bool inq = q < q_hi;
     const uint32_t p = inq ? n.perm[q] : 0u;
@@ -2610,7 +2645,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_cond_queue(CondFlatAr
         double zw = a.warm ? a.warm[kk] : __longlong_as_double(0x7FF8000000000000ll);
         if (uniq && zw == zw) {  // the learned path starts from the plain guess where that is the root
           double gp, dg;       // to the tolerance (solve_condensation)
-          ode_g_dg(cc, cfg.delt, r, zg, gp, dg);
+          ode_g_dg<true>(ode_run(cc, cfg.delt, r), zg, gp, dg);
           if (fabs(gp) < cfg.atol) zw = zg;
         }
         R.zwarm[slot] = zw;
@@ -2678,9 +2713,9 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_cond_queue(CondFlatAr
       // one evaluation of g: the initial state of a segment, or a Newton iteration
       // (newton_iterate, impliciteuler.cpp:240-255)
       double zn = z;
-      if (phase != PH_EVAL) zn = fmax(z * (1 - quotient(gz, dgz)), 1e-8);  // as newton_iterate
+      if (phase != PH_EVAL) zn = newton_next(z, gz, dgz);
       double g1, dg1;
-      ode_g_dg(c, subdelt, rprev, zn, g1, dg1);
+      ode_g_dg<true>(ode_run(c, subdelt, rprev), zn, g1, dg1);
       bool segok = false, segfail = false;
       if (phase == PH_EVAL) {
         z0 = z = zn;
@@ -2695,7 +2730,7 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_cond_queue(CondFlatAr
         }
       } else {
         ++iters;
-        const bool conv = fabs(g1 - gz) < cfg.rtol * fabs(g1) + cfg.atol;
+        const bool conv = newton_converged(cfg, g1, gz);
         z = zn;
         gz = g1;
         dgz = dg1;
@@ -3148,6 +3183,11 @@ static unsigned solve_blocks(const cleo_ctx* c, uint32_t grid_waves) {
   return static_cast<unsigned>(grid_waves ? std::min<uint64_t>(nb, std::max<uint32_t>(1u, grid_waves / 4)) : nb);
 }
 
+// The deferral budget in counted iterations: the two that a restart repeats count for the drop but are
+// not made again (8 that are made: 33M drops coupled 2.43 -> 2.39 ms a step against 8 counted; 6 to 16
+// counted: 2.63, 2.43, 2.39, 2.39, 2.40 ms for 6, 8, 10, 12, 16).
+static uint32_t counted_budget(uint32_t budget) { return budget ? std::min(budget, 0xfffffffdu) + 2u : 0u; }
+
 void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
   if (args.ngbx == 0) return;
   CondFlatArgs a = args;
@@ -3157,7 +3197,7 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
   const uint32_t gw = c->tiles.cond_grid_waves;
   a.gpt = sum_gpt(c);
   const uint32_t budget = c->cond_variant() == 2 ? 0u : c->defer_budget();
-  a.cfg.budget = budget;
+  a.cfg.budget = counted_budget(budget);
   a.dlist = c->dlist;
   a.dcount = c->dcount;
   hipLaunchKernelGGL(k_cond_prep, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
@@ -3223,7 +3263,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   const uint32_t gw = c->tiles.cond_grid_waves;
   a.gpt = sum_gpt(c);
   const uint32_t budget = c->defer_budget();
-  a.cfg.budget = budget;
+  a.cfg.budget = counted_budget(budget);
   a.dlist = c->dlist;
   a.dcount = c->dcount;
   if (a.mlp_inline) {  // learned guesses of the drops where motion left them

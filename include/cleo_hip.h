@@ -411,7 +411,7 @@ typedef struct {
   uint32_t motion_grid_waves;
   uint32_t coll_flat;              /* 0 or 1: collisions by tiles of 64 gridboxes per wave where those
                                       fill the chip, else by a wave or a workgroup per gridbox or few */
-  uint32_t cond_defer;             /* cond_flat 1: Newton iterations after which a drop is set
+  uint32_t cond_defer;             /* cond_flat 1: Newton iterations made after which a drop is set
                                       aside and solved later, packed with others (0: never) */
 } cleo_tiles;
 int cleo_set_tiles(cleo_ctx* ctx, const cleo_tiles* tiles);
