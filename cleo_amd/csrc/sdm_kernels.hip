@@ -1138,11 +1138,21 @@ __device__ __forceinline__ void gbx_thermo(const GState& st, uint32_t g, double*
 // The arrivals and the drops that leave the domain are scanned here within the block of gridboxes, into
 // the new refs and the out-of-domain prefix; k_nsort_apply adds what the blocks before have.  (Separate launches for the fill of the counts, two three-level scans, the refs, the active
 // counts and the condensation inputs, with the same for the re-sort after collisions, made 34 launches
-// of a coupled step, 11 now: 409 -> 349 us on 32^3 gridboxes of 64 drops.)  kThermo: the gridbox's condensation inputs too, for a
-// condensation in the sort's gather (the State is that of before the sort).
+// of a coupled step, 11 now: 409 -> 349 us on 32^3 gridboxes of 64 drops.)  kThermo: the gridboxes' condensation inputs too, for a
+// condensation in the sort's gather (the State is that of before the sort), by workgroups of their own
+// from number nblk on: both are serial chains of a few us (one after the other in each thread: 10.3 us
+// on 3750 gridboxes, 7.4 on 20; now 7.8 and 5.0).
 template <bool kThermo>
 __global__ void __launch_bounds__(kTabBlock) k_nsort_tot(NsortArgs a, GState st, double* gs) {
   __shared__ uint32_t ws[kTabBlock / kWave];
+  if (kThermo && blockIdx.x >= a.nblk) {
+    const uint32_t g = (blockIdx.x - a.nblk) * kTabBlock + threadIdx.x;
+    if (g < a.grid.ngbx) {
+      if (st.temp[g] <= 0) set_error(a.ctl, CLEO_ERR_TEMP_NONPOSITIVE, g, a.off[g]);
+      gbx_thermo(st, g, gs);
+    }
+    return;
+  }
   const uint32_t d = blockIdx.x * kTabBlock + threadIdx.x;
   uint32_t t = 0, gone = 0;
   if (d < a.grid.ngbx) {
@@ -1201,10 +1211,6 @@ __global__ void __launch_bounds__(kTabBlock) k_nsort_tot(NsortArgs a, GState st,
       }
     }
     a.nact[d] = t;
-    if constexpr (kThermo) {
-      if (st.temp[d] <= 0) set_error(a.ctl, CLEO_ERR_TEMP_NONPOSITIVE, d, a.off[d]);
-      gbx_thermo(st, d, gs);
-    }
   }
   uint32_t tsum, gsum;
   const uint32_t tpre = block_excl_scan(t, ws, tsum), gpre = block_excl_scan(gone, ws, gsum);
@@ -1215,7 +1221,7 @@ __global__ void __launch_bounds__(kTabBlock) k_nsort_tot(NsortArgs a, GState st,
   if (threadIdx.x == 0) {
     a.part[2u * blockIdx.x] = tsum;
     a.part[2u * blockIdx.x + 1u] = gsum;
-    if (gridDim.x == 1) a.off_new[a.grid.ngbx] = tsum;  // no k_nsort_apply follows
+    if (a.nblk == 1) a.off_new[a.grid.ngbx] = tsum;  // no k_nsort_apply follows
     if (blockIdx.x == 0) a.ctl->stats[ST_SORTS] += 1;
   }
 }
@@ -2059,7 +2065,7 @@ static NsortArgs nsort_args(cleo_ctx* c, const SoA& src, const SoA& dst) {
 // inputs of every gridbox too
 static void nsort_tables(cleo_ctx* c, const NsortArgs& a, double* gs = nullptr) {
   if (gs)
-    hipLaunchKernelGGL(k_nsort_tot<true>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a, c->st, gs);
+    hipLaunchKernelGGL(k_nsort_tot<true>, dim3(2 * a.nblk), dim3(kTabBlock), 0, c->stream, a, c->st, gs);
   else
     hipLaunchKernelGGL(k_nsort_tot<false>, dim3(a.nblk), dim3(kTabBlock), 0, c->stream, a, GState{}, gs);
   if (a.nblk > kApplyBlocks) {
