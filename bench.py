@@ -37,10 +37,12 @@ BYTES = {
     # read sdgbxindex, r, msol, xi; write r, dm | saturation ratio and diffusion factor, temp, refs
     "k_cond_drops": (44, 2 * 8 + 8 + 8),
     "k_cond_queue": (44, 2 * 8 + 8 + 8),
-    # read xi, r, msol of every paired drop; write its slot of the shuffled order (the drops stay
-    # in place; enacted pairs, a few per cent, also write their attributes) | refs, nact, volume
-    "k_coll_team": (28, 8 + 4 + 8),
-    "k_coll_tiles": (28, 8 + 4 + 8),
+    # read xi and r of every paired drop (msol of the enacted ones, a few in 1e5); write its slot of the
+    # shuffled order (the drops stay in place; enacted pairs also write their attributes) | refs, nact,
+    # volume
+    "k_coll_team": (20, 8 + 4 + 8),
+    "k_coll_split": (20, 8 + 4 + 8),
+    "k_coll_tiles": (20, 8 + 4 + 8),
     # read coords, radius, sdgbxindex; write coords, sdgbxindex | bounds, winds, counts
     "k_motion_flat": (64, 6 * 8 + 6 * 8 + 28 * 4),
     # fused motion + sort, moving pass: read coords, radius, xi, msol, id; write the 60-byte record

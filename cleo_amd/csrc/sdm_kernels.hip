@@ -184,14 +184,14 @@ __device__ __forceinline__ PairOut coll_pair_eval(const CollArgs& a, uint32_t g,
   const uint32_t npairs = n / 2;
   const double scale_p = n * (n - 1.0) / (2.0 * npairs);
   const double VOLUME = a.vol[g] * dimless::VOL0;
-  PairOut o;
-  const DropAttrs A{a.s.xi[ka], a.s.r[ka], a.s.msol[ka]};
-  const DropAttrs B{a.s.xi[kb], a.s.r[kb], a.s.msol[kb]};
-  const bool a_first = !(A.xi < B.xi);  // assign_drops (collisions.hpp:94-101)
+  PairOut o{};
+  const uint64_t xiA = a.s.xi[ka], xiB = a.s.xi[kb];
+  const double rA = a.s.r[ka], rB = a.s.r[kb];
+  const bool a_first = !(xiA < xiB);  // assign_drops (collisions.hpp:94-101)
   // d1 is the drop with the larger multiplicity; selected field by field (a reference picked by a
   // lane-varying flag would put both drops in scratch memory)
-  DropAttrs d1{a_first ? A.xi : B.xi, a_first ? A.r : B.r, a_first ? A.msol : B.msol};
-  DropAttrs d2{a_first ? B.xi : A.xi, a_first ? B.r : A.r, a_first ? B.msol : A.msol};
+  DropAttrs d1{a_first ? xiA : xiB, a_first ? rA : rB, 0.0};
+  DropAttrs d2{a_first ? xiB : xiA, a_first ? rB : rA, 0.0};
   const double prob_jk = pair_probability<Kinetic>(a.k, d1.r, d2.r, VOLUME);
   const double prob = scale_p * static_cast<double>(d1.xi) * prob_jk;
   double phi_coll, phi_out;
@@ -205,7 +205,13 @@ __device__ __forceinline__ PairOut coll_pair_eval(const CollArgs& a, uint32_t g,
     phi_coll = u53(r4[0], r4[1]);
     phi_out = u53(r4[2], r4[3]);
   }
-  o.err = 0;
+  // nothing happens to most pairs (fewer than 1e-4 of the coupled populations' are enacted, 3e-3 of the
+  // Golovin box's): no conversions, no 64-bit division, and the solute masses are not read (k_coll_tiles on
+  // 33.5M drops 299 -> 252 us, k_coll_team on 24679 gridboxes of 300 135 -> 125)
+  if (prob >= 0.0 && prob < 1.0 && !(phi_coll < prob)) return o;
+  const double mA = a.s.msol[ka], mB = a.s.msol[kb];
+  d1.msol = a_first ? mA : mB;
+  d2.msol = a_first ? mB : mA;
   const uint32_t res = enact_pair<Kinetic>(a.k, d1, d2, prob, phi_coll, phi_out, a.sol, o.err);
   o.enacted = (res >> 1) & 1u;
   o.nullA = (res & 1u) && a_first;
