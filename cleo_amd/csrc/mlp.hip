@@ -256,23 +256,31 @@ __global__ void __launch_bounds__(128) k_mlp_grad(TrainArgs a) {
   }
 }
 
-// rows w0 .. w1 - 1 of column p, added in order; the loads of a full chunk are all in flight at once
+// rows w0 .. w1 - 1 of column p, added in order, one running sum; the loads of 32 rows are in flight at
+// once, and with more rows those of the next 32 while these are added
 constexpr uint32_t kReduceChunk = 32;
 __device__ __forceinline__ float sum_rows(const float* rows, uint32_t w0, uint32_t w1, int p) {
   const float* r = rows + static_cast<uint64_t>(w0) * (NPARAM + 1) + p;
+  const uint32_t n = w1 - w0, full = n / kReduceChunk;
   float s = 0.0f;
-  if (w1 - w0 == kReduceChunk) {
-    float v[kReduceChunk];
+  float v[kReduceChunk], next[kReduceChunk];
+  auto load = [&](uint32_t c, float* to) {
+    const float* rc = r + static_cast<uint64_t>(c) * kReduceChunk * (NPARAM + 1);
 #pragma unroll
-    for (uint32_t i = 0; i < kReduceChunk; ++i) v[i] = r[i * (NPARAM + 1)];
+    for (uint32_t i = 0; i < kReduceChunk; ++i) to[i] = rc[i * (NPARAM + 1)];
+  };
+  if (full) load(0u, v);
+  for (uint32_t c = 0; c < full; ++c) {
+    if (c + 1 < full) load(c + 1, next);
 #pragma unroll
     for (uint32_t i = 0; i < kReduceChunk; ++i) s += v[i];
-    return s;
+#pragma unroll
+    for (uint32_t i = 0; i < kReduceChunk; ++i) v[i] = next[i];
   }
-  for (uint32_t i = 0; i < w1 - w0; ++i) s += r[static_cast<uint64_t>(i) * (NPARAM + 1)];
+  for (uint32_t i = full * kReduceChunk; i < n; ++i) s += r[static_cast<uint64_t>(i) * (NPARAM + 1)];
   return s;
 }
-// a level of the gradient sum: chunk c of kReduceChunk rows, summed in row order, for every
+// first level of the gradient sum: chunk c of kReduceChunk rows, summed in row order, for every
 // parameter (and the loss, entry NPARAM); one thread per (parameter, chunk)
 __global__ void k_mlp_reduce_chunks(const float* partial, uint32_t nwaves, float* chunks) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -493,37 +501,30 @@ struct MLPDev {
   MLPWeights weights() const { return MLPWeights{w1p, w2, w2t, master}; }
 };
 
-// the partial gradients of each workgroup, followed by the chunk sums of every level
+// the partial gradients of each workgroup, followed by their chunk sums
 static uint32_t reduce_nchunks(uint32_t waves) { return (waves + kReduceChunk - 1) / kReduceChunk; }
-static uint64_t reduce_rows(uint32_t waves) {
-  uint64_t rows = waves;
-  for (uint32_t n = waves; n > 1; rows += n) n = reduce_nchunks(n);
-  return rows + 1;
-}
 static hipError_t ensure_partial(MLPDev* m, uint32_t waves) {
   if (m->partial_waves >= waves) return hipSuccess;
   hipFree(m->partial);
   m->partial = nullptr;
   m->partial_waves = 0;
-  hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->partial), reduce_rows(waves) * (NPARAM + 1) * 4);
+  hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->partial),
+                           (static_cast<uint64_t>(waves) + reduce_nchunks(waves)) * (NPARAM + 1) * 4);
   if (e == hipSuccess) m->partial_waves = waves;
   return e;
 }
-// The sum of `waves` partials, in levels of chunks of 32 rows until one chunk is left, which the last
-// launch adds (batches up to 65536 samples: one level before it); then Adam when `apply`.
+// The sum of `waves` partials: chunks of 32 rows, then the chunks one after the other (of 2M samples
+// 1024; a further level of chunks would be 17 us faster there, but in another order, that is rounded otherwise); then Adam
+// when `apply`.
 static void launch_reduce_adam(hipStream_t s, MLPDev* m, uint32_t waves, int32_t apply, float lr, float b1, float b2,
                                float eps, float bc1, float bc2) {
-  const float* rows = m->partial;
-  uint32_t n = waves;
-  do {
-    float* next = const_cast<float*>(rows) + static_cast<uint64_t>(n) * (NPARAM + 1);
-    const uint32_t nch = reduce_nchunks(n);
-    hipLaunchKernelGGL(k_mlp_reduce_chunks, dim3((NPARAM + 256) / 256, nch), dim3(256), 0, s, rows, n, next);
-    rows = next;
-    n = nch;
-  } while (n > kReduceChunk);
-  hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 64) / 64), dim3(64), 0, s, rows, n, m->grad, m->loss, m->master,
-                     m->adam_m, m->adam_v, apply, lr, b1, b2, eps, bc1, bc2, m->w1p, m->w2, m->w2t);
+  const uint32_t nch = reduce_nchunks(waves);
+  float* ch = m->partial + static_cast<uint64_t>(m->partial_waves) * (NPARAM + 1);
+  hipLaunchKernelGGL(k_mlp_reduce_chunks, dim3((NPARAM + 256) / 256, nch), dim3(256), 0, s,
+                     static_cast<const float*>(m->partial), waves, ch);
+  hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + 64) / 64), dim3(64), 0, s, static_cast<const float*>(ch), nch,
+                     m->grad, m->loss, m->master, m->adam_m, m->adam_v, apply, lr, b1, b2, eps, bc1, bc2, m->w1p, m->w2,
+                     m->w2t);
 }
 
 hipError_t mlp_create(cleo_ctx* c) {
