@@ -1144,7 +1144,7 @@ __device__ __forceinline__ void gbx_thermo(const GState& st, uint32_t g, double*
 // The arrivals and the drops that leave the domain are scanned here within the block of gridboxes, into
 // the new refs and the out-of-domain prefix; k_nsort_apply adds what the blocks before have.  (Separate launches for the fill of the counts, two three-level scans, the refs, the active
 // counts and the condensation inputs, with the same for the re-sort after collisions, made 34 launches
-// of a coupled step, 11 now: 409 -> 349 us on 32^3 gridboxes of 64 drops.)  kThermo: the gridboxes' condensation inputs too, for a
+// of a coupled step, nine now: 409 -> 349 us on 32^3 gridboxes of 64 drops with eleven of them.)  kThermo: the gridboxes' condensation inputs too, for a
 // condensation in the sort's gather (the State is that of before the sort), by workgroups of their own
 // from number nblk on: both are serial chains of a few us (one after the other in each thread: 10.3 us
 // on 3750 gridboxes, 7.4 on 20; now 7.8 and 5.0).
@@ -1951,7 +1951,8 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   if (args.ngbx == 0) return;
   CollArgs a = args;
   const uint64_t mean = std::max<uint64_t>(1, c->ntot / a.ngbx);
-  // Tiles give the least work per drop (33.5M drops: 0.29 ms against 0.56 ms for the teams), but a
+  // Tiles give the least work per drop (33.5M drops: 0.30 ms against 0.56 ms for the teams, 0.25 ms with
+  // pairs leaving early), but a
   // wave walks through its 64 gridboxes' swaps and pairs in about 1.2 us per drop of the mean, so
   // they need enough gridboxes to fill the chip (32^3 gridboxes of 64: 81 us against 45 us; the
   // lines cross near 75,000 gridboxes at any mean) whose drops fit a tile's 8 KB of permutations.
@@ -2365,10 +2366,10 @@ __global__ void __launch_bounds__(256) k_cond_guess(CondFlatArgs a) {
 // 591 us on 8.4M, and 18 and 31 us more for a launch that solved the list; same-address atomics take
 // about 5 ns each.)  Who solves them:
 // - kTail: the workgroup itself at the end of its range, about 60 drops of 2048, while others fill the
-//   CU: no further launch (2.1M drops: 104 us against 110).
+//   CU: no further launch (2.1M drops: 104 us against 110; 91 with the solves as they are now).
 // - else k_cond_deferred, which packs the lists of several workgroups and keeps the second copy of
 //   the solve, with its registers, out of the main loop (33.5M drops: 1155 us against 1209, 134M:
-//   4.44 ms against 4.64; equal at 8.4M).
+//   4.44 ms against 4.64; equal at 8.4M; 1053 us and 4.0 ms with the solves as they are now).
 __device__ __forceinline__ void defer_drop(uint32_t* ndef, uint32_t* list, bool deferred, uint32_t q) {
   const uint64_t m = ballot(deferred);
   if (!m) return;
