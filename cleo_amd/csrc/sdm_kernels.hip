@@ -18,20 +18,42 @@ namespace cleo {
 // gridboxes' values one after the other, so a tile takes the time of its drops' loads plus its longest
 // sum; tiles of 64 gridboxes leave most of the chip idle below half a million gridboxes (sum_gpt).
 __host__ __device__ __forceinline__ uint32_t sum_tiles(uint32_t ngbx, uint32_t gpt) { return (ngbx + gpt - 1) / gpt; }
-// acc + v[i0] + v[i0+1] + ... + v[i1-1], left to right, eight LDS reads in flight at a time (a read per
-// add waits about 100 cycles for each value)
-template <class T>
-__device__ __forceinline__ T add_in_order(T acc, const T* v, uint32_t i0, uint32_t i1) {
+// acc[c] + v[c][i0] + v[c][i0+1] + ... + v[c][i1-1] for N value sequences, each left to right.  Eight
+// LDS reads of each are in flight while the eight before are added, and the sequences' adds alternate, so
+// neither a read's 100 cycles nor an add's latency is waited for (one sequence after the other, with each
+// eight reads waited for: k_cond_state 11.5 -> 10.5 us on 3750 gridboxes of 128 drops).
+template <int N, class T>
+__device__ __forceinline__ void add_in_order(T* acc, const T* const* v, uint32_t i0, uint32_t i1) {
+  constexpr uint32_t kAhead = 8;
+  const uint32_t full = (i1 - i0) / kAhead;
+  T r[N][kAhead], next[N][kAhead];
+  auto load = [&](uint32_t i, T(&to)[N][kAhead]) {
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j)
+#pragma unroll
+      for (int c = 0; c < N; ++c) to[c][j] = v[c][i + j];
+  };
+  auto add = [&](T(&from)[N][kAhead]) {
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j)
+#pragma unroll
+      for (int c = 0; c < N; ++c) acc[c] += from[c][j];
+  };
   uint32_t i = i0;
-  for (; i + 8 <= i1; i += 8) {
-    T r[8];
-#pragma unroll
-    for (uint32_t j = 0; j < 8; ++j) r[j] = v[i + j];
-#pragma unroll
-    for (uint32_t j = 0; j < 8; ++j) acc += r[j];
+  if (full) load(i, r);
+  for (uint32_t k = 0; k < full; k += 2) {  // two eights per turn: no register moves
+    if (k + 1 < full) load(i + kAhead, next);
+    add(r);
+    i += kAhead;
+    if (k + 1 < full) {
+      if (k + 2 < full) load(i + kAhead, r);
+      add(next);
+      i += kAhead;
+    }
   }
-  for (; i < i1; ++i) acc += v[i];
-  return acc;
+  for (; i < i1; ++i)
+#pragma unroll
+    for (int c = 0; c < N; ++c) acc[c] += v[c][i];
 }
 // Drop-order sums of v(k) over [lo, lo + len) for the gridboxes of a tile (lane i passes its
 // own gridbox's range and gets its sum).  The tile's drops [t_lo, t_hi) are staged through an LDS
@@ -57,7 +79,8 @@ __device__ __forceinline__ double tile_sum(double* win, uint32_t t_lo, uint32_t 
     wave_sync();
     if (we < t_hi) load(we);
     const uint32_t a0 = max(lo, w), a1 = min(lo + len, we);
-    if (a0 < a1) acc = add_in_order(acc, win, a0 - w, a1 - w);
+    const double* const v1[1] = {win};
+    if (a0 < a1) add_in_order<1>(&acc, v1, a0 - w, a1 - w);
     wave_sync();
   }
   return acc;
@@ -68,11 +91,9 @@ template <class V1, class V2>
 __device__ __forceinline__ void tile_sum2(double* win, uint32_t t_lo, uint32_t t_hi, uint32_t lo, uint32_t len, V1 v1,
                                           V2 v2, int lane, double& s1, double& s2) {
   constexpr uint32_t kHalf = kSumWin / 2, kPer = kHalf / kWave;
-  double a1 = 0.0, a2 = 0.0;
-  if (t_lo >= t_hi) {
-    s1 = s2 = 0.0;
-    return;
-  }
+  double acc[2] = {0.0, 0.0};
+  s1 = s2 = 0.0;
+  if (t_lo >= t_hi) return;
   // the next window's values are loaded into registers while the lanes add the current one's
   // (every lane loads, with indices clamped into the tile, so the loads stay in flight)
   double r1[kPer], r2[kPer];
@@ -94,14 +115,60 @@ __device__ __forceinline__ void tile_sum2(double* win, uint32_t t_lo, uint32_t t
     wave_sync();
     if (we < t_hi) load(we);
     const uint32_t b0 = max(lo, w), b1 = min(lo + len, we);
-    if (b0 < b1) {
-      a1 = add_in_order(a1, win, b0 - w, b1 - w);
-      a2 = add_in_order(a2, win + kHalf, b0 - w, b1 - w);
+    const double* const v[2] = {win, win + kHalf};
+    if (b0 < b1) add_in_order<2>(acc, v, b0 - w, b1 - w);
+    wave_sync();
+  }
+  s1 = acc[0];
+  s2 = acc[1];
+}
+// The same for N (one or two) value sequences and tiles of kRows gridboxes, with the next kRowLen values of every
+// gridbox in the window at a time, so that all of the tile's lanes add.  A contiguous window holds the
+// values of a gridbox or two once they have hundreds of drops, and LDS reads, which take the same time
+// for two lanes as for 64, then bound the sums.  Rows of odd length keep the lanes' reads in different banks.
+constexpr uint32_t kRows = 16;
+template <int N, class V>
+__device__ __forceinline__ void tile_rows_sum(double* win, uint32_t t_lo, uint32_t lo, uint32_t len, V v, int lane,
+                                              double* acc) {
+  constexpr uint32_t kHalf = kSumWin / 2, kRowLen = kHalf / kRows - 1, kPer = kHalf / kWave;
+  static_assert(N <= 2 && kRowLen % 2 == 1 && kRows * kRowLen <= kHalf, "rows of the window");
+  uint32_t most = len;
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), o)));
+  if (most == 0) return;
+  uint32_t first[kPer], left[kPer];  // this lane's items: the drop of the first window, the values from it on
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; ++i) {
+    const uint32_t j = static_cast<uint32_t>(lane) + i * kWave, row = min(j / kRowLen, kRows - 1u), at = j - row * kRowLen;
+    const uint32_t n = static_cast<uint32_t>(__shfl(static_cast<int>(len), static_cast<int>(row)));
+    first[i] = static_cast<uint32_t>(__shfl(static_cast<int>(lo), static_cast<int>(row))) + at;
+    left[i] = at < kRowLen && at < n ? n - at : 0u;
+  }
+  double r[N][kPer];
+  auto load = [&](uint32_t w) {  // every lane loads, from the tile's first drop where there is no value
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+      const uint32_t k = w < left[i] ? first[i] + w : t_lo;
+#pragma unroll
+      for (int c = 0; c < N; ++c) r[c][i] = v(c, k);
+    }
+  };
+  load(0u);
+  for (uint32_t w = 0; w < most; w += kRowLen) {
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i)
+#pragma unroll
+      for (int c = 0; c < N; ++c) win[c * kHalf + static_cast<uint32_t>(lane) + i * kWave] = r[c][i];
+    wave_sync();
+    if (w + kRowLen < most) load(w + kRowLen);
+    if (w < len) {
+      const double* rows[N];
+#pragma unroll
+      for (int c = 0; c < N; ++c) rows[c] = win + c * kHalf + static_cast<uint32_t>(lane) * kRowLen;
+      add_in_order<N>(acc, rows, 0u, min(kRowLen, len - w));
     }
     wave_sync();
   }
-  s1 = a1;
-  s2 = a2;
 }
 // condensed water of drop k (condensate_mass * xi, superdrop_attrs.hpp:207-216)
 __device__ __forceinline__ double qcond_term(const SoA& s, const Solute& sol, DevCtl* ctl, uint32_t k) {
@@ -2826,9 +2893,11 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(3) k_cond_queue(CondFlatAr
   }
 }
 
-// per gridbox: Σ dm in drop order and the thermodynamic feedback (condensation.cpp:126-137).
+// per gridbox: Σ dm in drop order and the thermodynamic feedback (condensation.cpp:126-137); kByRows:
+// the sums by tile_rows_sum, tiles of kRows gridboxes.
 // With a.qm, first the qcond recompute after motion from the drops' terms before the solve (the
 // same ordered sum and formula as k_cond_prep's; State is unchanged until here).
+template <bool kByRows>
 __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_state(CondFlatArgs a) {
   __shared__ double win_all[4][kSumWin];
   double* win = win_all[threadIdx.x >> 6];
@@ -2842,15 +2911,25 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(4) k_cond_state(CondFlatAr
     double qc_new = 0.0, tot = 0.0;
     if (a.qm) {
       double totq = 0.0;
-      tile_sum2(win, t_lo, t_hi, lo, n, [&](uint32_t k) { return a.qm[k]; }, [&](uint32_t k) { return a.dm[k]; },
-                lane, totq, tot);
+      if constexpr (kByRows) {
+        double both[2] = {0.0, 0.0};
+        tile_rows_sum<2>(win, t_lo, lo, n, [&](int c, uint32_t k) { return c == 0 ? a.qm[k] : a.dm[k]; }, lane, both);
+        totq = both[0];
+        tot = both[1];
+      } else {
+        tile_sum2(win, t_lo, t_hi, lo, n, [&](uint32_t k) { return a.qm[k]; }, [&](uint32_t k) { return a.dm[k]; },
+                  lane, totq, tot);
+      }
       if (valid) {
         const double rho_cond = totq / a.st.vol[g] * dimless::R0cubed_VOL0;
         qc_new = rho_cond / dry_air_density(a.st.press[g], a.st.temp[g], a.st.qv[g]);
         if (!a.alter) a.st.qc[g] = qc_new;
       }
     } else {
-      tot = tile_sum(win, t_lo, t_hi, lo, n, [&](uint32_t k) { return a.dm[k]; }, lane);
+      if constexpr (kByRows)
+        tile_rows_sum<1>(win, t_lo, lo, n, [&](int, uint32_t k) { return a.dm[k]; }, lane, &tot);
+      else
+        tot = tile_sum(win, t_lo, t_hi, lo, n, [&](uint32_t k) { return a.dm[k]; }, lane);
     }
     if (valid && a.alter) {
       const double temp = a.st.temp[g], press = a.st.press[g];
@@ -2932,7 +3011,7 @@ __global__ void __launch_bounds__(256) k_mass_moments(SoA s, const uint32_t* off
     const uint32_t t_lo = off[g0], t_hi = off[min(g0 + gpt, ngbx)];
     const uint32_t lo = valid ? off[g] : t_hi, hi = valid ? off[g + 1] : t_hi;
     uint64_t m0 = 0;
-    float m1 = 0.f, m2 = 0.f;
+    float m12[2] = {0.f, 0.f};
     if (t_lo >= t_hi) {
       if (valid) {
         mom0[g] = 0;
@@ -2973,16 +3052,17 @@ __global__ void __launch_bounds__(256) k_mass_moments(SoA s, const uint32_t* off
       if (we < t_hi) load(we);
       const uint32_t b0 = max(lo, w), b1 = min(hi, we);
       if (b0 < b1) {
-        m0 = add_in_order(m0, w0, b0 - w, b1 - w);
-        m1 = add_in_order(m1, w1, b0 - w, b1 - w);
-        m2 = add_in_order(m2, w2, b0 - w, b1 - w);
+        const uint64_t* const v0[1] = {w0};
+        const float* const v12[2] = {w1, w2};
+        add_in_order<1>(&m0, v0, b0 - w, b1 - w);
+        add_in_order<2>(m12, v12, b0 - w, b1 - w);
       }
       wave_sync();
     }
     if (valid) {
       mom0[g] = m0;
-      mom1[g] = m1;
-      mom2[g] = m2;
+      mom1[g] = m12[0];
+      mom2[g] = m12[1];
     }
   }
 }
@@ -3196,6 +3276,19 @@ static unsigned solve_blocks(const cleo_ctx* c, uint32_t grid_waves) {
   return static_cast<unsigned>(grid_waves ? std::min<uint64_t>(nb, std::max<uint32_t>(1u, grid_waves / 4)) : nb);
 }
 
+// The sums by rows from 128 drops per gridbox on, where there are 256 tiles of 16 gridboxes to fill the
+// chip (two sums / one sum, contiguous windows against rows, us: 24679 gridboxes of 300 drops 97 / 33
+// against 41 / 21, 8000 of 400 55 / 31 against 24 / 17, 64000 of 128 58 / 24 against 44 / 24, 2000 of 1000
+// 44 / 27 against 48 / 33, 64^3 of 122 181 / 64 against 145 / 76).
+static void launch_cond_state(cleo_ctx* c, CondFlatArgs a, uint32_t gw) {
+  if (a.ngbx >= 256 * kRows && c->ntot / a.ngbx >= 128) {
+    a.gpt = kRows;
+    hipLaunchKernelGGL(k_cond_state<true>, dim3(gbx_blocks(sum_tiles(a.ngbx, kRows), 4, gw)), dim3(256), 0, c->stream, a);
+  } else {
+    hipLaunchKernelGGL(k_cond_state<false>, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
+  }
+}
+
 // The deferral budget in counted iterations: the two that a restart repeats count for the drop but are
 // not made again (8 that are made: 33M drops coupled 2.43 -> 2.39 ms a step against 8 counted; 6 to 16
 // counted: 2.63, 2.43, 2.39, 2.39, 2.40 ms for 6, 8, 10, 12, 16).
@@ -3238,7 +3331,7 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
     if (!tail) launch_deferred(c, a, nb);
     kev_mark(c, 1);
   }
-  hipLaunchKernelGGL(k_cond_state, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
+  launch_cond_state(c, a, gw);
 }
 
 // Motion, the neighbour sort and a condensation that follows at once, with the condensation solve
@@ -3302,7 +3395,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
     nsort_commit(c, commit_dst);
     a.off = c->off;  // the sorted store's refs
   }
-  hipLaunchKernelGGL(k_cond_state, dim3(sum_blocks(c, gw)), dim3(256), 0, c->stream, a);
+  launch_cond_state(c, a, gw);
 }
 
 void launch_motion_flat(cleo_ctx* c, const MotionArgs& args) {
