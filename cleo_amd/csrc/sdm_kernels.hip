@@ -396,7 +396,8 @@ __device__ __forceinline__ void copy_drop(const SoA& src, const SoA& dst, uint64
 struct Resort {
   DevCtl* ctl;
   SoA src, dst;
-  uint32_t *off, *nact, *off_new, *order;
+  uint32_t *off, *nact, *off_new;
+  uint32_t* order;  // the pending order, or null: the store is in its logical order (a condensation applied it)
   uint32_t ngbx;
 };
 __device__ __forceinline__ void resort_begin(const Resort& r, uint32_t events, uint32_t flag) {
@@ -435,7 +436,7 @@ __device__ __forceinline__ void resort_gather(const Resort& r, uint32_t lo, uint
   for (uint32_t g = wide ? lo : lo + tid / kWave; g < hi; g += wide ? 1u : B / kWave) {
     const uint32_t o = r.off[g], n = r.nact[g], nfull = r.off[g + 1] - o, to = r.off_new[g];
     for (uint32_t k = lane; k < nfull; k += lanes) {
-      const uint32_t p = r.order[o + k];
+      const uint32_t p = r.order ? r.order[o + k] : o + k;
       const uint32_t q = k < n ? to + k : active + (o - to) + (k - n);
       if (p < nsrc && q < nsrc) copy_drop(r.src, r.dst, p, q);
     }
@@ -444,7 +445,7 @@ __device__ __forceinline__ void resort_gather(const Resort& r, uint32_t lo, uint
 __device__ __forceinline__ void resort_back(const Resort& r, uint32_t nsrc, uint64_t first, uint64_t stride) {
   for (uint64_t q = first; q < nsrc; q += stride) {
     copy_drop(r.dst, r.src, q, q);
-    r.order[q] = static_cast<uint32_t>(q);
+    if (r.order) r.order[q] = static_cast<uint32_t>(q);
   }
   for (uint64_t g = first; g <= r.ngbx; g += stride) {
     r.off[g] = r.off_new[g];
@@ -2167,7 +2168,8 @@ void neighbour_sort_to(cleo_ctx* c, const SoA& src, const SoA& dst, int commit_d
 }
 
 void resort_nulls(cleo_ctx* c, uint32_t events) {
-  const Resort r{c->ctl, c->buf[c->cur], c->buf[1 - c->cur], c->off, c->nact, c->off_alt, c->order, c->grid.ngbx};
+  const Resort r{c->ctl, c->buf[c->cur], c->buf[1 - c->cur], c->off, c->nact, c->off_alt,
+                 c->order_live ? c->order : nullptr, c->grid.ngbx};
   if (c->ntot <= kResortOneDrops && r.ngbx <= kResortOneDrops) {
     hipLaunchKernelGGL(k_resort_one, dim3(1), dim3(1024), 0, c->stream, r, events);
     return;
