@@ -3341,7 +3341,7 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& args) {
 // the saturation ratios (State only), the gather with the solves, the commit of the sorted store,
 // the deferred drops, then the ordered sums and the State update (with the qcond recompute).
 // margs.s is the store motion reads, `dst` the sorted store; commit_dst >= 0: that buffer becomes
-// current (else, for timing, the refs stay those of the unsorted store).
+// current (else, for timing, the context's refs stay those of the unsorted store).
 void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatArgs& cond, const SoA& dst,
                           int commit_dst) {
   const uint32_t ngbx = c->grid.ngbx;
@@ -3393,10 +3393,8 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
     launch_gather_cond<false>(c, n, a, move_in_gather ? &m : nullptr, nb);
   kev_mark(c, 1);
   if (!tail) launch_deferred(c, a, nb);
-  if (commit_dst >= 0) {
-    nsort_commit(c, commit_dst);
-    a.off = c->off;  // the sorted store's refs
-  }
+  if (commit_dst >= 0) nsort_commit(c, commit_dst);
+  a.off = n.off_new;  // the sorted store's refs, of the same sort as its active counts
   launch_cond_state(c, a, gw);
 }
 
