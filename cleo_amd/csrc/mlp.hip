@@ -479,6 +479,13 @@ __global__ void __launch_bounds__(256) k_order_chase(OrderArgs a) {
     a.perm[i] = x;
   }
 }
+// The order where the state is 0 (the seed equals the constant it is combined with): every draw is then 0,
+// and n-1 swaps with place 0 turn the samples round by one.  One list would hold all of them, which takes
+// n^2 steps to walk.
+__global__ void __launch_bounds__(256) k_order_zero(OrderArgs a) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x)
+    a.perm[i] = i + 1u < a.n ? i + 1u : 0u;
+}
 
 // ------------------------------------------------------------------------------------------------
 struct MLPDev {
@@ -627,12 +634,16 @@ static int sample_order(cleo_ctx* c, uint64_t n, uint64_t state, const uint32_t*
   const OrderArgs a{static_cast<uint32_t>(n), state, m->jump, w, w + n, w + 2 * n, w + 3 * n, w + 4 * n};
   const unsigned nb = static_cast<unsigned>(std::min<uint64_t>((n + 255) / 256, 16384));
   const uint64_t threads = (n + kDrawsPerThread - 1) / kDrawsPerThread;
+  *perm = a.perm;
+  *state_after = xorshift64_after(state, n - 1);
+  if (state == 0) {
+    hipLaunchKernelGGL(k_order_zero, dim3(nb), dim3(256), 0, c->stream, a);
+    return CLEO_OK;
+  }
   hipLaunchKernelGGL(k_order_clear, dim3(nb), dim3(256), 0, c->stream, a);
   hipLaunchKernelGGL(k_order_draw, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, c->stream, a);
   hipLaunchKernelGGL(k_order_link, dim3(nb), dim3(256), 0, c->stream, a);
   hipLaunchKernelGGL(k_order_chase, dim3(nb), dim3(256), 0, c->stream, a);
-  *perm = a.perm;
-  *state_after = xorshift64_after(state, n - 1);
   return CLEO_OK;
 }
 
