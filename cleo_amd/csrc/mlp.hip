@@ -434,8 +434,11 @@ struct OrderArgs {
   uint32_t *head, *nxt, *src, *hop;
   uint32_t* perm;
 };
+// a sample per thread and round; 64-bit, as n may lie less than a stride below 2^32
+__device__ __forceinline__ uint64_t order_first() { return blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; }
+__device__ __forceinline__ uint64_t order_stride() { return static_cast<uint64_t>(gridDim.x) * blockDim.x; }
 __global__ void __launch_bounds__(256) k_order_clear(OrderArgs a) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) a.head[i] = kNoEntry;
+  for (uint64_t i = order_first(); i < a.n; i += order_stride()) a.head[i] = kNoEntry;
 }
 __global__ void __launch_bounds__(256) k_order_draw(OrderArgs a) {
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -453,12 +456,12 @@ __global__ void __launch_bounds__(256) k_order_draw(OrderArgs a) {
   }
 }
 __global__ void __launch_bounds__(256) k_order_link(OrderArgs a) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
+  for (uint64_t i = order_first(); i < a.n; i += order_stride()) {
     uint32_t hop = kNoEntry;
     for (uint32_t e = a.head[i]; e != kNoEntry; e = a.nxt[e])
       if (e != i && e < hop) hop = e;
     a.hop[i] = hop;
-    uint32_t from = i;
+    uint32_t from = static_cast<uint32_t>(i);
     if (i > 0) {
       const uint32_t j = a.src[i];
       if (j != i) {
@@ -472,7 +475,7 @@ __global__ void __launch_bounds__(256) k_order_link(OrderArgs a) {
   }
 }
 __global__ void __launch_bounds__(256) k_order_chase(OrderArgs a) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
+  for (uint64_t i = order_first(); i < a.n; i += order_stride()) {
     uint32_t x = a.src[i];
     if (x == kNoEntry) continue;
     for (uint32_t h = a.hop[x]; h != kNoEntry; h = a.hop[x]) x = h;
@@ -483,8 +486,8 @@ __global__ void __launch_bounds__(256) k_order_chase(OrderArgs a) {
 // and n-1 swaps with place 0 turn the samples round by one.  One list would hold all of them, which takes
 // n^2 steps to walk.
 __global__ void __launch_bounds__(256) k_order_zero(OrderArgs a) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x)
-    a.perm[i] = i + 1u < a.n ? i + 1u : 0u;
+  for (uint64_t i = order_first(); i < a.n; i += order_stride())
+    a.perm[i] = i + 1 < a.n ? static_cast<uint32_t>(i + 1) : 0u;
 }
 
 // ------------------------------------------------------------------------------------------------
