@@ -506,7 +506,7 @@ struct MLPDev {
   uint32_t partial_waves = 0;
   double* moments = nullptr;      // per-block sums of k_mlp_moments
   uint64_t* jump = nullptr;       // the sample order's jump matrices
-  uint32_t* order = nullptr;      // the sample order and its scratch: five words per sample
+  uint32_t* order = nullptr;      // the sample order and its scratch: five words per sample, kept up to kKeepOrder
   uint64_t order_n = 0;
   MLPWeights weights() const { return MLPWeights{w1p, w2, w2t, master}; }
 };
@@ -618,6 +618,8 @@ using namespace cleo;
   } while (0)
 
 constexpr unsigned kMomentBlocks = 256;
+// samples up to which the order's buffer (20 bytes each) stays for the next training
+constexpr uint64_t kKeepOrder = 1u << 22;
 
 // the shuffled order of n samples on the device (see k_order_draw) and the stream's state behind it
 static int sample_order(cleo_ctx* c, uint64_t n, uint64_t state, const uint32_t** perm, uint64_t* state_after) {
@@ -848,6 +850,11 @@ int cleo_mlp_train(cleo_ctx* c, const float* x, const float* y, uint64_t n, cons
   }
   MLP_TRY(c, hipGetLastError());
   MLP_TRY(c, hipStreamSynchronize(c->stream));
+  if (m->order_n > kKeepOrder) {
+    hipFree(m->order);
+    m->order = nullptr;
+    m->order_n = 0;
+  }
   const int rc = mlp_check_ready(c);
   if (rc != CLEO_OK) return rc;
   if (final_loss) {
