@@ -199,6 +199,7 @@ int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p, bool last) {
   if (inj) {
     const int rc = prepare_injected(c);
     if (rc != CLEO_OK) return rc;
+    if (c->ntot > kFyBudget && !c->order_live) pending_identity_order(c);  // for launch_inj_long
   }
   // a pending order of an earlier event is composed with this one's shuffle: the drops stay where
   // they are, and the new order goes to the other order buffer
@@ -229,6 +230,7 @@ int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p, bool last) {
     a.off_new = c->off_alt;
     c->events_pending = 0;
   }
+  if (inj && c->ntot > kFyBudget) launch_inj_long(c, a);
   launch_collisions(c, a);
   if (compose) std::swap(c->order, c->order_alt);
   c->order_live = true;

@@ -1001,6 +1001,64 @@ __global__ void k_inj_sizes(const uint32_t* nact, uint32_t ngbx, uint32_t* nj, u
   np[g] = 2 * (n / 2);
 }
 
+// Injected indices may put any number of swaps on one list (all indices equal) or make a chain of any
+// length (every index one below its swap's place), and the shuffle's passes would take n^2 steps: 1e12 in
+// a gridbox of a million drops.  So before an injected event the lists of every gridbox of more than
+// kFyBudget drops are looked over, and where a place's element is more than kFyBudget list entries away
+// (drawn indices: 4 on average, at most 60 to 120 in 8192 to 200000 drops) one lane makes the swaps on the
+// pending order itself and leaves indices that move nothing.
+template <class Mem>
+__device__ __forceinline__ bool fy_within_budget(const Mem& M, uint32_t k) {
+  using Idx = typename Mem::Idx;
+  constexpr uint32_t kNone = static_cast<uint32_t>(static_cast<Idx>(~Idx(0)));
+  uint32_t x = k, steps = 0;
+  if (k > 0 && M.jst[k] != k) {
+    x = kNone;  // min{ e in L(j) : e > k }
+    for (uint32_t e = M.first(M.jst[k]); e != kNone; e = M.nxt[e]) {
+      if (++steps > kFyBudget) return false;
+      if (e > k && e < x) x = e;
+    }
+  }
+  while (x != kNone) {
+    const uint32_t at = x;
+    x = kNone;  // min(L(at) \ {at})
+    for (uint32_t e = M.first(at); e != kNone; e = M.nxt[e]) {
+      if (++steps > kFyBudget) return false;
+      if (e != at && e < x) x = e;
+    }
+  }
+  return true;
+}
+__global__ void __launch_bounds__(256) k_inj_long(CollArgs a, uint32_t* order, uint32_t* inj_j) {
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t g = blockIdx.x; g < a.ngbx; g += gridDim.x) {
+    const uint32_t base = a.off[g], n = a.nact[g], oj = a.inj_oj[g];
+    if (n <= kFyBudget) continue;
+    const uint64_t b2 = 2ull * base;
+    const FyHbm M{a.big2 + b2, a.big + b2, a.big + b2 + n, nullptr};
+    for (uint32_t k = tid; k < n; k += 256u) M.head[k] = ~0u;
+    __syncthreads();
+    for (uint32_t t = tid; t + 1 < n; t += 256u) {
+      const uint32_t iter = n - 1 - t, j = min(inj_j[oj + t], iter);
+      M.jst[iter] = j;
+      M.nxt[iter] = M.exch(j, iter);
+    }
+    __syncthreads();
+    bool within = true;
+    for (uint32_t k = tid; k < n && within; k += 256u) within = fy_within_budget(M, k);
+    if (__syncthreads_or(!within) && tid == 0) {
+      for (uint32_t t = 0; t + 1 < n; ++t) {
+        const uint32_t iter = n - 1 - t, j = inj_index(a, g, base, n, t);
+        const uint32_t x = order[base + iter];
+        order[base + iter] = order[base + j];
+        order[base + j] = x;
+        inj_j[oj + t] = iter;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // ============================ motion ==========================================================
 // Source gridbox that reaches `d` by the neighbour step `s` (s = (dz+1) + 3(dx+1) + 9(dy+1)),
 // or kOOB when the step would come from outside a finite axis.
@@ -2066,6 +2124,10 @@ void launch_set_event(cleo_ctx* c, uint64_t event) {
 }
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np) {
   hipLaunchKernelGGL(k_inj_sizes, dim3(nblocks(c->grid.ngbx, 256)), dim3(256), 0, c->stream, c->nact, c->grid.ngbx, nj, np);
+}
+
+void launch_inj_long(cleo_ctx* c, const CollArgs& a) {
+  hipLaunchKernelGGL(k_inj_long, dim3(std::min<uint32_t>(a.ngbx, 4096u)), dim3(256), 0, c->stream, a, c->order, c->inj_j);
 }
 
 static size_t scan_words_rec(uint64_t len) {

@@ -10,6 +10,7 @@ constexpr uint32_t kTileMaxN = 255;
 constexpr uint32_t kTilePermBytes = 8192;
 constexpr uint32_t kTileMinGbx = 75000;  // gridboxes from which the tiles are the faster variant
 constexpr uint64_t kResortOneDrops = 16384;  // drops up to which one workgroup re-sorts the nulls
+constexpr uint32_t kFyBudget = 512;  // list entries to a place's element above which injected swaps are made serially
 constexpr uint32_t kSplitGbx = 512;  // most gridboxes of 512 to 2048 drops with a larger workgroup each
 constexpr uint32_t kCollTileLdsBytes = kTilePermBytes + 4u * (65u + 4u * 64u);
 constexpr uint32_t kBigGbx = 0xFFFFFFFFu;  // tile LDS marker of a gridbox the whole wave shuffles
@@ -149,6 +150,8 @@ void launch_collisions(cleo_ctx* c, const CollArgs& a);
 // the statistics rows of the context
 StatSlots stat_slots(cleo_ctx* c);
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np);
+// swaps of an injected event that the parallel shuffle would take too long over, on the pending order
+void launch_inj_long(cleo_ctx* c, const CollArgs& a);
 // exclusive scan of in[i*stride+offset], i < len, into out[0..len] (out[len] = total)
 void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset, uint32_t* out);
 size_t scan_tmp_words(uint64_t len);
