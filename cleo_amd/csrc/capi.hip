@@ -552,10 +552,38 @@ int cleo_upload_supers(cleo_ctx* c, const cleo_supers_soa* h, uint64_t ntot) {
   return sort_upload(c, d, ntot);
 }
 
+// whether the kernels may read `bytes` at p: memory of the current device, within its allocation.  Arrays of
+// which that is not known (pinned host memory, another device's, a null pointer) are left to the runtime's
+// copies, which take what they can reach and report the rest.
+static bool device_readable(const void* p, size_t bytes) {
+  int dev = -1;
+  hipPointerAttribute_t attr{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  const bool known = p && hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&attr, p) == hipSuccess &&
+                     attr.type == hipMemoryTypeDevice && attr.device == dev &&
+                     hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) == hipSuccess;
+  if (!known) {
+    (void)hipGetLastError();  // a query that found nothing is no error
+    return false;
+  }
+  const size_t at = static_cast<size_t>(static_cast<const char*>(p) - static_cast<const char*>(base));
+  return at <= size && bytes <= size - at;
+}
 int cleo_upload_supers_device(cleo_ctx* c, const cleo_supers_soa* h, uint64_t ntot) {
   if (!c || !h) return CLEO_E_ARG;
   if (ntot > c->maxn) return fail(c, CLEO_E_ARG, "ntot exceeds the context capacity");
-  return sort_upload(c, as_soa(*h), ntot);  // sorted from the caller's arrays straight into the store
+  const SoA src = as_soa(*h);
+  bool direct = device_readable(src.gbx, ntot * 4);
+  for (const void* f : {static_cast<const void*>(src.c3), static_cast<const void*>(src.c1), static_cast<const void*>(src.c2),
+                        static_cast<const void*>(src.xi), static_cast<const void*>(src.r), static_cast<const void*>(src.msol),
+                        static_cast<const void*>(src.id)})
+    direct = direct && device_readable(f, ntot * 8);
+  if (direct) return sort_upload(c, src, ntot);  // sorted from the caller's arrays straight into the store
+  c->order_live = false;  // whatever comes of the copies
+  const SoA& d = c->buf[c->cur];
+  HIP_TRY(c, copy_soa(c, d, src, ntot, hipMemcpyDeviceToDevice));
+  return sort_upload(c, d, ntot);
 }
 
 // reference Superdrop layout (superdrop.hpp:36-60): u32 gbx @0, f64 coord3 @8, coord1 @16,
