@@ -62,8 +62,7 @@ void free_soa(SoA& s) {
 
 // the work enqueued so far is done and h_ctl holds the control block as it left it
 hipError_t fetch_ctl(cleo_ctx* c) {
-  launch_publish_ctl(c);
-  const hipError_t e = hipGetLastError();
+  const hipError_t e = launch_publish_ctl(c);
   return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
 }
 // synchronise, then report a recorded device error
@@ -744,8 +743,8 @@ int cleo_set_rng_counter(cleo_ctx* c, uint64_t seed, uint64_t first_event) {
   c->rng_mode = 1;
   c->seed = seed;
   c->events_pending = 0;
-  launch_set_event(c, first_event);
-  return launch_check(c);
+  HIP_TRY(c, launch_set_event(c, first_event));
+  return CLEO_OK;
 }
 
 int cleo_set_rng_injected(cleo_ctx* c, const uint32_t* j, uint64_t nj, const double* phi, uint64_t nphi) {

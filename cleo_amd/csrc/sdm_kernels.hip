@@ -2116,11 +2116,18 @@ void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   }
 }
 StatSlots stat_slots(cleo_ctx* c) { return StatSlots{c->sp}; }
-void launch_publish_ctl(cleo_ctx* c) {
-  hipLaunchKernelGGL(k_publish_ctl, dim3(1), dim3(64), 0, c->stream, c->ctl, c->off, c->grid.ngbx, c->h_ctl);
+// (their own status, as hipGetLastError may hold an error that another call of the thread left)
+hipError_t launch_publish_ctl(cleo_ctx* c) {
+  const DevCtl* ctl = c->ctl;
+  const uint32_t* off = c->off;
+  uint32_t ngbx = c->grid.ngbx;
+  HostCtl* out = c->h_ctl;
+  void* args[] = {&ctl, &off, &ngbx, &out};
+  return hipLaunchKernel(reinterpret_cast<const void*>(k_publish_ctl), dim3(1), dim3(64), args, 0, c->stream);
 }
-void launch_set_event(cleo_ctx* c, uint64_t event) {
-  hipLaunchKernelGGL(k_set_event, dim3(1), dim3(1), 0, c->stream, c->ctl, event);
+hipError_t launch_set_event(cleo_ctx* c, uint64_t event) {
+  void* args[] = {&c->ctl, &event};
+  return hipLaunchKernel(reinterpret_cast<const void*>(k_set_event), dim3(1), dim3(1), args, 0, c->stream);
 }
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np) {
   hipLaunchKernelGGL(k_inj_sizes, dim3(nblocks(c->grid.ngbx, 256)), dim3(256), 0, c->stream, c->nact, c->grid.ngbx, nj, np);

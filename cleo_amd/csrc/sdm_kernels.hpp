@@ -191,9 +191,9 @@ void radix_sort_soa(hipStream_t stream, const SoA& src, const SoA& dst, uint64_t
 // applies a pending collision order to the store (buf[cur] then holds the drops in order)
 void materialize_order(cleo_ctx* c);
 // the control block and the domain's number of drops into the pinned mirror h_ctl, in stream order
-void launch_publish_ctl(cleo_ctx* c);
+hipError_t launch_publish_ctl(cleo_ctx* c);
 // the collision event counter, in stream order
-void launch_set_event(cleo_ctx* c, uint64_t event);
+hipError_t launch_set_event(cleo_ctx* c, uint64_t event);
 // 0th, 1st and 2nd mass moments of every gridbox into device arrays of ngbx entries (raindrops
 // only when rain)
 void launch_mass_moments(cleo_ctx* c, bool rain, uint64_t* mom0, float* mom1, float* mom2);
