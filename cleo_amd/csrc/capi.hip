@@ -62,8 +62,14 @@ void free_soa(SoA& s) {
 
 // the work enqueued so far is done and h_ctl holds the control block as it left it
 hipError_t fetch_ctl(cleo_ctx* c) {
-  const hipError_t e = launch_publish_ctl(c);
-  return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
+  const hipError_t e = launch_publish_ctl(c), w = hipStreamSynchronize(c->stream);
+  return e != hipSuccess ? e : w;
+}
+// e, with what was enqueued before a failure done: copies that read or write the caller's memory end with
+// the call
+hipError_t settled(cleo_ctx* c, hipError_t e) {
+  if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);
+  return e;
 }
 // synchronise, then report a recorded device error
 int sync_check(cleo_ctx* c) {
@@ -529,16 +535,19 @@ static hipError_t copy_soa(cleo_ctx* c, const SoA& d, const SoA& s, uint64_t n, 
   void* dst[7] = {d.c3, d.c1, d.c2, d.xi, d.r, d.msol, d.id};
   const void* src[7] = {s.c3, s.c1, s.c2, s.xi, s.r, s.msol, s.id};
   for (int i = 0; i < 7 && e == hipSuccess; ++i) e = hipMemcpyAsync(dst[i], src[i], n * 8, kind, c->stream);
-  return e;
+  return settled(c, e);
 }
 // the uploaded drops `src` (device memory) replace the store and its pending order, sorted
 static int sort_upload(cleo_ctx* c, const SoA& src, uint64_t ntot) {
   c->order_live = false;
   c->ntot = ntot;
   const int rc = ensure_radix(c, ntot);
-  if (rc != CLEO_OK) return rc;
+  if (rc != CLEO_OK) {
+    (void)hipStreamSynchronize(c->stream);  // the copies of an upload
+    return rc;
+  }
   generic_sort(c, src, true);
-  HIP_TRY(c, hipGetLastError());
+  HIP_TRY(c, settled(c, hipGetLastError()));
   return sync_check(c);
 }
 
@@ -679,9 +688,9 @@ int cleo_mass_moments(cleo_ctx* c, int32_t rain, uint64_t* mom0, float* mom1, fl
     std::memcpy(mom2, d2, ngbx * 4);
     return rc;
   }
-  HIP_TRY(c, hipMemcpyAsync(mom0, d0, ngbx * 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipMemcpyAsync(mom1, d1, ngbx * 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipMemcpyAsync(mom2, d2, ngbx * 4, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, settled(c, hipMemcpyAsync(mom0, d0, ngbx * 8, hipMemcpyDeviceToHost, c->stream)));
+  HIP_TRY(c, settled(c, hipMemcpyAsync(mom1, d1, ngbx * 4, hipMemcpyDeviceToHost, c->stream)));
+  HIP_TRY(c, settled(c, hipMemcpyAsync(mom2, d2, ngbx * 4, hipMemcpyDeviceToHost, c->stream)));
   return sync_check(c);
 }
 
@@ -706,7 +715,7 @@ int cleo_upload_gbx_state(cleo_ctx* c, const cleo_gbx_state* h) {
     HIP_TRY(c, ctx_copy(c, c->d_state, c->stage, 11 * bytes, hipMemcpyHostToDevice));
     return CLEO_OK;
   }
-  for (int i = 0; i < 11; ++i) HIP_TRY(c, hipMemcpyAsync(f[i], src[i], bytes, hipMemcpyHostToDevice, c->stream));
+  for (int i = 0; i < 11; ++i) HIP_TRY(c, settled(c, hipMemcpyAsync(f[i], src[i], bytes, hipMemcpyHostToDevice, c->stream)));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   return CLEO_OK;
 }
@@ -723,7 +732,7 @@ int cleo_download_gbx_state(cleo_ctx* c, cleo_gbx_state* h) {
     HIP_TRY(c, hipMemcpyAsync(c->stage, c->d_state, 11 * bytes, hipMemcpyDeviceToHost, c->stream));
   } else {
     for (int i = 0; i < 11; ++i)
-      if (dst[i]) HIP_TRY(c, hipMemcpyAsync(dst[i], f[i], bytes, hipMemcpyDeviceToHost, c->stream));
+      if (dst[i]) HIP_TRY(c, settled(c, hipMemcpyAsync(dst[i], f[i], bytes, hipMemcpyDeviceToHost, c->stream)));
   }
   const int rc = sync_check(c);
   if (small && (rc == CLEO_OK || rc == CLEO_E_DEVICE))
