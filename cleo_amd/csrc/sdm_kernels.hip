@@ -3347,12 +3347,21 @@ static unsigned solve_blocks(const cleo_ctx* c, uint32_t grid_waves) {
   return static_cast<unsigned>(grid_waves ? std::min<uint64_t>(nb, std::max<uint32_t>(1u, grid_waves / 4)) : nb);
 }
 
-// The sums by rows from 128 drops per gridbox on, where there are 256 tiles of 16 gridboxes to fill the
-// chip (two sums / one sum, contiguous windows against rows, us: 24679 gridboxes of 300 drops 97 / 33
-// against 41 / 21, 8000 of 400 55 / 31 against 24 / 17, 64000 of 128 58 / 24 against 44 / 24, 2000 of 1000
-// 44 / 27 against 48 / 33, 64^3 of 122 181 / 64 against 145 / 76).
+// Whether the State pass sums by rows: from as many drops per gridbox on as make the windows' reads for a
+// lane or two dearer than the rows' extra work, and from 256 tiles of 16 gridboxes that fill the chip.
+// Two sums (after motion) gain from 128 drops on, few gridboxes from 160 (us, windows / rows: 4096 of 128
+// drops 11.1 / 13.5, of 170 14.8 / 14.0; 8192 of 128 13.2 / 13.2; 24679 of 300 93 / 41; 64^3 of 128
+// 169 / 152, of 250 503 / 280).  One sum loses on few gridboxes, and on many, where the windows are near
+// the bandwidth (64^3 of 128 65 / 77, of 150 79 / 86, of 190 105 / 105, of 230 140 / 125; 1M of 130
+// 240 / 292; 8192 of 128 7.1 / 8.3, of 190 11.1 / 10.2; 4096 of 230 9.5 / 11.0; between them 32768 of 128
+// 15.9 / 13.2, 65536 of 128 21.8 / 22.2, of 150 30 / 24, 8000 of 400 30 / 16).
+static bool sums_by_rows(uint64_t ngbx, uint64_t mean, bool two) {
+  if (ngbx < 256 * kRows) return false;
+  if (two) return mean >= (ngbx < 8192 ? 160u : 128u);
+  return mean >= (ngbx < 8192 ? 256u : ngbx < 16384 || ngbx > 65536 ? 192u : 128u);
+}
 static void launch_cond_state(cleo_ctx* c, CondFlatArgs a, uint32_t gw) {
-  if (a.ngbx >= 256 * kRows && c->ntot / a.ngbx >= 128) {
+  if (sums_by_rows(a.ngbx, c->ntot / a.ngbx, a.qm != nullptr)) {
     a.gpt = kRows;
     hipLaunchKernelGGL(k_cond_state<true>, dim3(gbx_blocks(sum_tiles(a.ngbx, kRows), 4, gw)), dim3(256), 0, c->stream, a);
   } else {
