@@ -10,6 +10,7 @@ constexpr uint32_t kTileMaxN = 255;
 constexpr uint32_t kTilePermBytes = 8192;
 constexpr uint32_t kTileMinGbx = 75000;  // gridboxes from which the tiles are the faster variant
 constexpr uint64_t kResortOneDrops = 16384;  // drops up to which one workgroup re-sorts the nulls
+constexpr uint32_t kResortBlocks = 256, kResortSegs = 256;  // workgroups of the re-sort on larger stores, segments of gridboxes
 constexpr uint32_t kFyBudget = 512;  // list entries to a place's element above which injected swaps are made serially
 constexpr uint32_t kSplitGbx = 512;  // most gridboxes of 512 to 2048 drops with a larger workgroup each
 constexpr uint32_t kCollTileLdsBytes = kTilePermBytes + 4u * (65u + 4u * 64u);
