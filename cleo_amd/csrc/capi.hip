@@ -367,7 +367,10 @@ int enqueue_run_step(cleo_ctx* c, uint32_t t_mdl, uint32_t t_mdl_next) {
           rc = enqueue_collision_event(c, q.coll, last);
           any_coll = true;
         }
-        if (rc != CLEO_OK) return rc;
+        if (rc != CLEO_OK) {
+          end_collisions(c);  // the events made so far: no null stays among the domain's drops
+          return rc;
+        }
         pending_qcond = false;
       }
       if (pending_qcond) {
@@ -751,7 +754,6 @@ int cleo_set_rng_counter(cleo_ctx* c, uint64_t seed, uint64_t first_event) {
   if (!c) return CLEO_E_ARG;
   c->rng_mode = 1;
   c->seed = seed;
-  c->events_pending = 0;
   HIP_TRY(c, launch_set_event(c, first_event));
   return CLEO_OK;
 }
@@ -853,9 +855,8 @@ int cleo_condensation(cleo_ctx* c, const cleo_cond_params* p) {
 int cleo_collisions(cleo_ctx* c, const cleo_coll_params* p) {
   if (!c || !p) return CLEO_E_ARG;
   const int rc = enqueue_collision_event(c, *p, true);
-  if (rc != CLEO_OK) return rc;
   end_collisions(c);
-  return launch_check(c);
+  return rc != CLEO_OK ? rc : launch_check(c);
 }
 
 int cleo_run_step(cleo_ctx* c, uint32_t t_mdl, uint32_t t_mdl_next) {
@@ -886,13 +887,6 @@ int cleo_run_steps_graph(cleo_ctx* c, uint32_t t_mdl, uint32_t span, uint32_t ns
     }
   }
   HIP_TRY(c, hipStreamSynchronize(c->stream));
-  if (c->events_pending) {  // events of a call that failed before its end: count them now
-    uint64_t ev = 0;
-    HIP_TRY(c, ctx_copy(c, &ev, &c->ctl->event, 8, hipMemcpyDeviceToHost));
-    ev += c->events_pending;
-    HIP_TRY(c, ctx_copy(c, &c->ctl->event, &ev, 8, hipMemcpyHostToDevice));
-    c->events_pending = 0;
-  }
   // The launches a step enqueues depend on the store's state when it starts (which buffer is
   // current, whether a collision order is pending), so every replay must start in the state the
   // previous one ended in.  One step is captured, or two when one step changes the state; if two
@@ -925,7 +919,6 @@ int cleo_run_steps_graph(cleo_ctx* c, uint32_t t_mdl, uint32_t span, uint32_t ns
     const bool live1 = c->order_live;
     uint32_t* const ord1 = c->order;
     uint32_t* const off1 = c->off;
-    c->events_pending = 0;
     c->cur = cur0;
     c->order_live = live0;
     set_buffers(ord0, off0);

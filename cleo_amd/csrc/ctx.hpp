@@ -155,7 +155,7 @@ struct cleo_ctx {
   uint32_t* order_alt = nullptr;  // the other buffer: a collision event composes order into it
   bool order_live = false;
   uint32_t* coll_share = nullptr;  // k_coll_split: nulls and finished shares of each gridbox, zero between launches
-  uint32_t events_pending = 0;  // collision events since the device's event counter last moved on
+  uint32_t events_pending = 0;  // collision events of the pass under way
   // per drop: condensed mass * xi before a condensation solve (the qcond recompute after motion)
   double* qm = nullptr;
   // mass-moment observer results (ngbx uint64 + 2 * ngbx float, allocated at first use)
