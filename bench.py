@@ -72,12 +72,16 @@ def measured_traffic(kernel, ndims):
     return 1024.0 * (k["fetch_kib"] * t["fetch_scale"] + k["write_kib"] * t["write_scale"])
 
 
-def stage_kernel(stage, tiles):
-    """Name of the main kernel of a stage (0 condensation, 1 collisions, 2 motion) under a tiling."""
+def stage_kernel(stage, tiles, ngbx, ntot):
+    """Name of the main kernel of a stage (0 condensation, 1 collisions, 2 motion) under a tiling.
+    Collisions: by the library's rule on the number of gridboxes and their mean of drops."""
     if stage == 0:
         return {0: "k_cond_drops", 1: "k_cond_drops", 2: "k_cond_queue"}[tiles.cond_flat]
     if stage == 1:
-        return "k_coll_tiles" if tiles.coll_flat else "k_coll_team"
+        mean = max(1, ntot // ngbx)
+        if ngbx >= 75000 and mean <= 132:
+            return "k_coll_tiles"
+        return "k_coll_team" if mean <= 512 or (mean <= 2048 and ngbx > 512) else "k_coll_split"
     return {0: "k_motion_flat", 1: "k_motion_flat", 2: "k_motion_scatter", 3: "k_motion_keys"}[tiles.motion_flat]
 
 
@@ -245,18 +249,18 @@ def run_gpu(args):
                     collisions=elapsed(d, 4, 5))
     # main kernel of each stage alone: HIP events around its launches on the library's stream
     kernel_ms = {}
+    ngbx = int(np.prod(ndims))
     for stage in range(3):
         ms = C.c_float()
         d.check(L.cleo_time_kernel(d.h, stage, 3, C.byref(ms)), "time_kernel")
-        kernel_ms[stage_kernel(stage, tiles)] = float(ms.value)
+        kernel_ms[stage_kernel(stage, tiles, ngbx, d.ntot)] = float(ms.value)
     if tiles.cond_flat == 1 and tiles.motion_flat in (1, 3):
         # the step solves condensation inside the sort's gather (k_sort_gather_cond; with motion
         # variant 3 the drops also move in it) instead of in the separate per-drop kernel
-        del kernel_ms[stage_kernel(0, tiles)]
+        del kernel_ms[stage_kernel(0, tiles, ngbx, d.ntot)]
         ms = C.c_float()
         d.check(L.cleo_time_kernel(d.h, 3, 3, C.byref(ms)), "time_kernel fused")
         kernel_ms["k_sort_gather_cond"] = float(ms.value)
-    ngbx = int(np.prod(ndims))
     nd = ndomain(d)
     # the mass-moment observer's reduction on the state the steps left (not part of the step)
     ms = C.c_float()

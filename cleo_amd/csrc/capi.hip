@@ -260,7 +260,6 @@ int enqueue_motion(cleo_ctx* c, const cleo_motion_params& p, bool qcond) {
   a.st = c->st;
   a.delt = step2dimlesstime(p.interval);
   a.tv = p.terminalv;
-  a.wpb = wpb_or1(c->tiles.motion_waves_per_block);
   a.cnt = c->cnt;
   a.ctl = c->ctl;
   if (c->motion_variant() == 2) {
@@ -275,7 +274,7 @@ int enqueue_motion(cleo_ctx* c, const cleo_motion_params& p, bool qcond) {
     neighbour_sort_to(c, c->buf[c->cur], c->buf[1 - c->cur], 1 - c->cur, a.step);
   }
   if (qcond) {
-    QcondArgs q{c->buf[c->cur], c->off, c->st, c->solute, c->grid.ngbx, wpb_or1(c->tiles.cond_waves_per_block), c->ctl};
+    QcondArgs q{c->buf[c->cur], c->off, c->st, c->solute, c->grid.ngbx, c->ctl};
     launch_qcond(c, q);
   }
   return launch_check(c);
@@ -294,7 +293,6 @@ int enqueue_motion_condensation(cleo_ctx* c, const cleo_motion_params& mp, const
   a.st = c->st;
   a.delt = step2dimlesstime(mp.interval);
   a.tv = mp.terminalv;
-  a.wpb = wpb_or1(c->tiles.motion_waves_per_block);
   a.cnt = c->cnt;
   a.ctl = c->ctl;
   CondFlatArgs f = cond_args(c, cp, true);
@@ -326,7 +324,7 @@ int enqueue_run_step(cleo_ctx* c, uint32_t t_mdl, uint32_t t_mdl_next) {
     return t % iv == 0 && iv != UMAX;
   };
   auto qcond_now = [&]() {
-    QcondArgs q{c->buf[c->cur], c->off, c->st, c->solute, c->grid.ngbx, wpb_or1(c->tiles.cond_waves_per_block), c->ctl};
+    QcondArgs q{c->buf[c->cur], c->off, c->st, c->solute, c->grid.ngbx, c->ctl};
     launch_qcond(c, q);
   };
   uint32_t t_sdm = t_mdl;
@@ -1174,7 +1172,7 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
       a.sol = c->solute;
       a.k = make_collcfg(kp);
       a.ngbx = ngbx;
-      a.wpb = t.coll_waves_per_block ? t.coll_waves_per_block : 1;
+      a.wpb = wpb_or1(t.coll_waves_per_block);
       a.ctl = c->ctl;
       a.seed = c->seed;
       a.inj_oj = c->inj_oj;
@@ -1190,7 +1188,6 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
       a.st = c->st;
       a.delt = step2dimlesstime(mp.interval);
       a.tv = mp.terminalv;
-      a.wpb = t.motion_waves_per_block ? t.motion_waves_per_block : 1;
       a.cnt = c->cnt;
       a.ctl = c->ctl;
       CondFlatArgs f = cond_args(c, cp, true);
@@ -1204,7 +1201,6 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
       a.st = c->st;
       a.delt = step2dimlesstime(mp.interval);
       a.tv = mp.terminalv;
-      a.wpb = t.motion_waves_per_block ? t.motion_waves_per_block : 1;
       a.cnt = c->cnt;
       a.ctl = c->ctl;
       if (c->motion_variant() == 2) {
@@ -1248,7 +1244,7 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
 }
 
 // Times each stage's variants (thread per drop and task ring; motion also fused with the sort and in
-// its gather; collisions with 1 or 4 tiles per workgroup), and grids of one wave per gridbox or of
+// its gather; collisions, where they run by tiles, with 1 or 4 of them per workgroup), and grids of one wave per gridbox or of
 // 8192 / 32768 looping waves, on the resident population, and keeps the fastest.  Drops and State are
 // left unchanged.
 int cleo_autotune(cleo_ctx* c, cleo_tiles* chosen) {
@@ -1257,7 +1253,9 @@ int cleo_autotune(cleo_ctx* c, cleo_tiles* chosen) {
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   const uint32_t grid_waves[3] = {0, 8192, 32768};
   cleo_tiles best_t = c->tiles;
+  best_t.coll_flat = 1;
   for (int kern = 0; kern < 3; ++kern) {
+    if (kern == 1 && !coll_takes_tiles(c)) continue;  // teams and shares have nothing to choose
     float best = 1e30f;
     const uint32_t nvar = kern == 2 ? 3u : 2u;
     for (uint32_t i = 0; i < 3 * nvar; ++i) {
@@ -1267,7 +1265,6 @@ int cleo_autotune(cleo_ctx* c, cleo_tiles* chosen) {
         t.cond_flat = var;
         t.cond_grid_waves = gw;
       } else if (kern == 1) {
-        t.coll_flat = 1;
         t.coll_waves_per_block = var == 1 ? 1 : 4;
         t.coll_grid_waves = gw;
       } else {

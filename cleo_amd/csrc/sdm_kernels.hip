@@ -2098,16 +2098,19 @@ static void launch_coll_split(cleo_ctx* c, const CollArgs& args, uint32_t split,
     hipLaunchKernelGGL((k_coll_split<B, false>), dim3(a.ngbx * split), dim3(B), cap * kSplitItemBytes, c->stream, a, split, cap);
   kev_mark(c, 1);
 }
+// Tiles give the least work per drop (33.5M drops: 0.25 ms, teams 0.56), but a wave walks through its 64
+// gridboxes' swaps and pairs in about 1.2 us per drop of the mean, so they need enough gridboxes to fill
+// the chip (32^3 gridboxes of 64: 81 us against 45 us; the lines cross near 75,000 gridboxes at any mean)
+// whose drops fit a tile's 8 KB of permutations.
+bool coll_takes_tiles(const cleo_ctx* c) {
+  const uint64_t ngbx = c->grid.ngbx;
+  return ngbx >= kTileMinGbx && c->ntot / ngbx <= kTilePermBytes / kWave + 4;
+}
 void launch_collisions(cleo_ctx* c, const CollArgs& args) {
   if (args.ngbx == 0) return;
   CollArgs a = args;
   const uint64_t mean = std::max<uint64_t>(1, c->ntot / a.ngbx);
-  // Tiles give the least work per drop (33.5M drops: 0.30 ms against 0.56 ms for the teams, 0.25 ms with
-  // pairs leaving early), but a
-  // wave walks through its 64 gridboxes' swaps and pairs in about 1.2 us per drop of the mean, so
-  // they need enough gridboxes to fill the chip (32^3 gridboxes of 64: 81 us against 45 us; the
-  // lines cross near 75,000 gridboxes at any mean) whose drops fit a tile's 8 KB of permutations.
-  if (a.ngbx >= kTileMinGbx && mean <= kTilePermBytes / kWave + 4) {
+  if (coll_takes_tiles(c)) {
     const unsigned nb = gbx_blocks((a.ngbx + kWave - 1) / kWave, a.wpb, c->tiles.coll_grid_waves);
     a.stat = stat_slots(c);
     kev_mark(c, 0);

@@ -35,7 +35,6 @@ struct QcondArgs {
   GState st;
   Solute sol;
   uint32_t ngbx;
-  uint32_t wpb;
   DevCtl* ctl;
   uint32_t gpt;  // gridboxes per tile of the sums
 };
@@ -78,7 +77,6 @@ struct MotionArgs {
   GState st;
   double delt;
   int32_t tv;
-  uint32_t wpb;
   uint32_t* cnt;
   DevCtl* ctl;
   StatSlots stat;  // ST_MOTION_DROPS
@@ -148,6 +146,8 @@ void launch_condensation_flat(cleo_ctx* c, const CondFlatArgs& a);
 void launch_motion_flat(cleo_ctx* c, const MotionArgs& a);
 void launch_qcond(cleo_ctx* c, const QcondArgs& a);
 void launch_collisions(cleo_ctx* c, const CollArgs& a);
+// whether launch_collisions runs tiles on the resident drops
+bool coll_takes_tiles(const cleo_ctx* c);
 // the statistics rows of the context
 StatSlots stat_slots(cleo_ctx* c);
 void launch_inj_sizes(cleo_ctx* c, uint32_t* nj, uint32_t* np);

@@ -392,9 +392,9 @@ int cleo_mass_moments(cleo_ctx* ctx, int32_t rain, uint64_t* mom0, float* mom1, 
 
 /* Launch tiling, chosen by the autotuner; values 0 = default. */
 typedef struct {
-  uint32_t cond_waves_per_block;   /* gridboxes (waves) per workgroup, 1..4 */
-  uint32_t coll_waves_per_block;
-  uint32_t motion_waves_per_block;
+  uint32_t cond_waves_per_block;   /* not used; the values 0..4 are accepted */
+  uint32_t coll_waves_per_block;   /* tiles of 64 gridboxes (waves) per workgroup, 1..4 */
+  uint32_t motion_waves_per_block; /* gridboxes (waves) per workgroup of the sort's rank pass, 1..4 */
   uint32_t cond_flat;              /* 0, 1: one thread per drop + per-gridbox prep/sum kernels (0:
                                       with drops set aside after 8 iterations, whatever cond_defer);
                                       2: the same with each wave's drops fed to its lanes from a
@@ -407,10 +407,12 @@ typedef struct {
                                          cond_flat 0 or 1 and a condensation due, the sort's gather
                                          also solves it */
   uint32_t cond_grid_waves;        /* waves per launch; each loops over gridboxes (or drops) */
-  uint32_t coll_grid_waves;        /*   0: one wave per gridbox (one thread per drop) */
+  uint32_t coll_grid_waves;        /*   0: one wave per gridbox (one thread per drop);
+                                      collisions: of tiles only */
   uint32_t motion_grid_waves;
-  uint32_t coll_flat;              /* 0 or 1: collisions by tiles of 64 gridboxes per wave where those
-                                      fill the chip, else by a wave or a workgroup per gridbox or few */
+  uint32_t coll_flat;              /* not used, 0 or 1: collisions run by tiles of 64 gridboxes per wave
+                                      where those fill the chip (75000 gridboxes and more, of at most
+                                      132 drops), else by a wave or a workgroup per gridbox or few */
   uint32_t cond_defer;             /* cond_flat 1: Newton iterations made after which a drop is set
                                       aside and solved later, packed with others (0: never) */
 } cleo_tiles;
