@@ -166,8 +166,6 @@ int prepare_injected(cleo_ctx* c) {
   return CLEO_OK;
 }
 
-// one collision event over every gridbox: the drops stay in buf[cur], their shuffled order goes to
-// c->order (composed with a pending order of an earlier event)
 // the kinds a cleo_coll_params names must be ones the kernels know; the Low-List probabilities
 // and the kinetic-energy NFrags / flags read a terminal velocity formula
 bool tv_known(int32_t tv) { return tv == CLEO_TV_NULL || tv == CLEO_TV_SIMMEL || tv == CLEO_TV_ROGERS_YAU || tv == CLEO_TV_ROGERS_GK; }
@@ -196,7 +194,9 @@ CollCfg make_collcfg(const cleo_coll_params& p) {
   return k;
 }
 
-// one collision event; last: nothing else follows in its microphysics pass
+// one collision event over every gridbox: the drops stay in buf[cur], their shuffled order goes to
+// c->order (composed with a pending order of an earlier event); last: nothing else follows in its
+// microphysics pass
 int enqueue_collision_event(cleo_ctx* c, const cleo_coll_params& p, bool last) {
   if (const char* m = coll_params_error(p)) return fail(c, CLEO_E_ARG, m);
   if (c->rng_mode == 0) return fail(c, CLEO_E_STATE, "no random-number stream set");
@@ -1244,9 +1244,9 @@ static int time_stage(cleo_ctx* c, int kern, const cleo_tiles& t, int reps, bool
 }
 
 // Times each stage's variants (thread per drop and task ring; motion also fused with the sort and in
-// its gather; collisions, where they run by tiles, with 1 or 4 of them per workgroup), and grids of one wave per gridbox or of
-// 8192 / 32768 looping waves, on the resident population, and keeps the fastest.  Drops and State are
-// left unchanged.
+// its gather; collisions, where they run by tiles, with 1 or 4 of them per workgroup), and grids of one
+// wave per gridbox or of 8192 / 32768 looping waves, on the resident population, and keeps the fastest.
+// Drops and State are left unchanged.
 int cleo_autotune(cleo_ctx* c, cleo_tiles* chosen) {
   if (!c) return CLEO_E_ARG;
   if (c->ntot == 0) return fail(c, CLEO_E_STATE, "no superdroplets resident");

@@ -44,18 +44,9 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 // occupancy floor of a kernel: at least W waves per SIMD, so at most 512/W VGPRs per lane
 #define CLEO_OCCUPANCY(W) __attribute__((amdgpu_waves_per_eu(W)))
 
-// v with lane l replaced by the wave-uniform value x
-__device__ __forceinline__ uint32_t writelane_u32(uint32_t v, uint32_t x, uint32_t l) {
-  return static_cast<uint32_t>(lane_id()) == l ? x : v;
-}
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-__device__ __forceinline__ uint32_t wave_or_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o);
   return v;
 }
 

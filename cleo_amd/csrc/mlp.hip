@@ -5,12 +5,13 @@
 // normalised by a (mean, std) pair; output: log(r_new / r), normalised likewise.  The guess
 // handed to Newton is z = r^2 exp(2 y).
 //
-// One wave (64 lanes) owns 64 samples, the M dimension of every MFMA tile.  MFMA lane layout
-// (32x32x8, bf16 operands): A[i][k] from lane (i + 32*(k/4)) element k%4; B[k][j] from lane
-// (j + 32*(k/4)) element k%4; D[i][j] in lane (j + 32*((i/4)%2)) accumulator 4*(i/8) + i%4.
+// 64 samples are the M dimension of every MFMA tile: of one wave in inference, of a workgroup of two
+// waves, with half of the hidden units each, in training.  MFMA lane layout (32x32x8, bf16 operands):
+// A[i][k] from lane (i + 32*(k/4)) element k%4; B[k][j] from lane (j + 32*(k/4)) element k%4; D[i][j] in
+// lane (j + 32*((i/4)%2)) accumulator 4*(i/8) + i%4.
 //
-// Training: each wave computes the loss gradient of its 64 samples; the per-wave partial gradients
-// are summed in a fixed order, in chunks of 32 waves and then the chunk sums in chunk order (the
+// Training: each workgroup computes the loss gradient of its 64 samples; the partial gradients are
+// summed in a fixed order, in chunks of 32 workgroups and then the chunk sums in chunk order (the
 // second kernel also applies Adam), so a run is deterministic.
 #include <hip/hip_runtime.h>
 
@@ -524,8 +525,8 @@ static hipError_t ensure_partial(MLPDev* m, uint32_t waves) {
   return e;
 }
 // The sum of `waves` partials: chunks of 32 rows, then the chunks one after the other (of 2M samples
-// 1024; a further level of chunks would be 17 us faster there, but in another order, that is rounded otherwise); then Adam
-// when `apply`.
+// 1024; a further level of chunks would be 17 us faster there, but in another order, that is rounded
+// otherwise); then Adam when `apply`.
 static void launch_reduce_adam(hipStream_t s, MLPDev* m, uint32_t waves, int32_t apply, float lr, float b1, float b2,
                                float eps, float bc1, float bc2) {
   const uint32_t nch = reduce_nchunks(waves);

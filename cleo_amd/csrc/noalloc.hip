@@ -1,7 +1,8 @@
 // noalloc.hip -- the entry point of libcleo_hip.so that allocates no device memory:
 // cleo_sort_supers_noalloc, the generic superdroplet sort of cleo_upload_supers_device on
-// caller-owned device arrays.  Its scratch (a row per drop, radix keys, indices and digit counts) lives in `scratch`, a fixed device array of this file; every GPU the library runs on
-// holds one copy until the process ends.  Calls that overlap on one GPU share that copy and race.
+// caller-owned device arrays.  Its scratch (a row per drop, radix keys, indices and digit counts) lives
+// in `scratch`, a fixed device array of this file; every GPU the library runs on holds one copy until the
+// process ends.  Calls that overlap on one GPU share that copy and race.
 #include <hip/hip_runtime.h>
 
 #include <mutex>

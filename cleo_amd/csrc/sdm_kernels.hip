@@ -122,10 +122,11 @@ __device__ __forceinline__ void tile_sum2(double* win, uint32_t t_lo, uint32_t t
   s1 = acc[0];
   s2 = acc[1];
 }
-// The same for N (one or two) value sequences and tiles of kRows gridboxes, with the next kRowLen values of every
-// gridbox in the window at a time, so that all of the tile's lanes add.  A contiguous window holds the
-// values of a gridbox or two once they have hundreds of drops, and LDS reads, which take the same time
-// for two lanes as for 64, then bound the sums.  Rows of odd length keep the lanes' reads in different banks.
+// The same for N (one or two) value sequences and tiles of kRows gridboxes, with the next kRowLen values of
+// every gridbox in the window at a time, so that all of the tile's lanes add.  A contiguous window holds
+// the values of a gridbox or two once they have hundreds of drops, and LDS reads, which take the same time
+// for two lanes as for 64, then bound the sums.  Rows of odd length keep the lanes' reads in different
+// banks.
 constexpr uint32_t kRows = 16;
 template <int N, class V>
 __device__ __forceinline__ void tile_rows_sum(double* win, uint32_t t_lo, uint32_t lo, uint32_t len, V v, int lane,
@@ -348,6 +349,7 @@ __device__ __forceinline__ void coll_order_nulls(const CollArgs& a, uint32_t g, 
   }
 }
 
+// exclusive prefix of v over the wave's lanes, and its total
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_t& total) {
   uint32_t x = v;
 #pragma unroll
@@ -358,6 +360,7 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_
   total = readlane_u32(x, kWave - 1);
   return x - v;
 }
+// exclusive prefix of v over the workgroup's threads, and its total (ws: a word per wave)
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* ws, uint32_t& total) {
   uint32_t wt;
   const uint32_t x = wave_excl_scan(v, lane_id(), wt);
@@ -373,6 +376,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* ws, ui
   }
   return pre + x;
 }
+// record p of src to position q of dst
 __device__ __forceinline__ void copy_drop(const SoA& src, const SoA& dst, uint64_t p, uint64_t q) {
   dst.gbx[q] = src.gbx[p];
   dst.c3[q] = src.c3[p];
@@ -537,8 +541,9 @@ __device__ __forceinline__ Resort coll_resort(const CollArgs& a) {
 // entries long on average) only take minima, so the result does not depend on the order of the
 // entries.  The chains of U are one hop long on average (11 at most in 8192 drops).  Serial swaps take
 // one dependent memory round trip each: a gridbox of 8192 drops 1.68 ms for its collisions against
-// 34 us here and 19 us in shares (below), 24679 gridboxes of 300 drops 4.9 ms against 0.13 ms.  What bounds it: LDS (about 30
-// accesses per 64 drops, with bank conflicts) and the latency of its four passes.
+// 34 us here and 19 us in shares (below), 24679 gridboxes of 300 drops 4.9 ms against 0.13 ms.  What
+// bounds it: LDS (about 30 accesses per 64 drops, with bank conflicts) and the latency of its four passes.
+// (Injected indices may make lists and chains of any length: k_inj_long.)
 //
 // A team of B lanes (a wave, or a whole workgroup) shuffles the drops of one or more gridboxes, its
 // items flattened over the lanes.  The lists of a team live in LDS as 16-bit places (kLdsIdx), or,
@@ -878,11 +883,11 @@ __global__ void __launch_bounds__(B) CLEO_OCCUPANCY(Kinetic && B <= 512 ? 3 : 4)
 // Lane i shuffles gridbox 64*tile + i: its permutation (one byte per drop) lives in the wave's LDS
 // tile and the serial swaps of all 64 gridboxes run side by side.  The tile's pairs are then
 // flattened over the lanes (a lane finds its gridbox by binary search over the prefix of per-gridbox
-// pair counts), so every lane evaluates a pair whatever the gridbox sizes.  Gridboxes above kTileMaxN drops, or beyond the tile's LDS, follow one
-// after the other with the whole wave as their team (64^3 gridboxes of 128 drops, where a few of each
-// tile overflow: 433 -> 316 us against their serial swaps in HBM scratch).  The constant-kinetics
-// instantiation runs at four waves per SIMD (1.18 -> 1.07 ms on 134M drops against three), the
-// kinetic-energy one at three.
+// pair counts), so every lane evaluates a pair whatever the gridbox sizes.  Gridboxes above kTileMaxN
+// drops, or beyond the tile's LDS, follow one after the other with the whole wave as their team (64^3
+// gridboxes of 128 drops, where a few of each tile overflow: 433 -> 316 us against their serial swaps in
+// HBM scratch).  The constant-kinetics instantiation runs at four waves per SIMD (1.18 -> 1.07 ms on 134M
+// drops against three), the kinetic-energy one at three.
 struct CollTileLds {
   uint32_t perm32[kTilePermBytes / 4];  // byte permutations, gridbox i from byte loff[i]
   uint32_t ppre[kWave + 1];             // first pair of gridbox i among the tile's pairs
@@ -1272,7 +1277,6 @@ __device__ __forceinline__ Moved move_drop(const MotionArgs& a, uint32_t g, cons
 
 // ============================ neighbour sort ==================================================
 
-// exclusive prefix of v over the block's kTabBlock threads, and the block's total
 // the condensation inputs of a gridbox (condensation.cpp:44-56)
 __device__ __forceinline__ void gbx_thermo(const GState& st, uint32_t g, double* gs) {
   const double temp = st.temp[g], press = st.press[g];
@@ -1287,18 +1291,19 @@ __device__ __forceinline__ void gbx_thermo(const GState& st, uint32_t g, double*
 // Per destination d (thread per d): the drops arriving in d, and for each step s the drops that
 // reach d from source gridboxes of lower index than the source of s (the stable order puts them
 // first).  The counts are destination-major (row d, column s: arrivals at d by the step s), read as
-// one row and, on small domains, left zero for the next motion (counts_stay_clear).  The run offsets are written source-major into `runs`
-// (row g, column s: the offset of g's drops taking the step s), so the rank pass reads its gridbox's
-// 27 offsets as one contiguous row.  Every entry of `runs` belongs to one destination (g + step s): no
-// two threads write the same entry.  Only the entries of steps that some drop takes are written (a
-// source off a finite axis has none); the others keep older values that no pass reads.
-// The arrivals and the drops that leave the domain are scanned here within the block of gridboxes, into
-// the new refs and the out-of-domain prefix; k_nsort_apply adds what the blocks before have.  (Separate launches for the fill of the counts, two three-level scans, the refs, the active
-// counts and the condensation inputs, with the same for the re-sort after collisions, made 34 launches
-// of a coupled step, nine now: 409 -> 349 us on 32^3 gridboxes of 64 drops with eleven of them.)  kThermo: the gridboxes' condensation inputs too, for a
-// condensation in the sort's gather (the State is that of before the sort), by workgroups of their own
-// from number nblk on: both are serial chains of a few us (one after the other in each thread: 10.3 us
-// on 3750 gridboxes, 7.4 on 20; now 7.8 and 5.0).
+// one row and, on small domains, left zero for the next motion (counts_stay_clear).  The run offsets are
+// written source-major into `runs` (row g, column s: the offset of g's drops taking the step s), so the
+// rank pass reads its gridbox's 27 offsets as one contiguous row.  Every entry of `runs` belongs to one
+// destination (g + step s): no two threads write the same entry.  Only the entries of steps that some drop
+// takes are written (a source off a finite axis has none); the others keep older values that no pass reads.
+// The arrivals and the drops that leave the domain are scanned here within the block of gridboxes, into the
+// new refs and the out-of-domain prefix; k_nsort_apply adds what the blocks before have.  (Separate
+// launches for the fill of the counts, two three-level scans, the refs, the active counts and the
+// condensation inputs, with the same for the re-sort after collisions, made 34 launches of a coupled step,
+// nine now: 409 -> 349 us on 32^3 gridboxes of 64 drops with eleven of them.)  kThermo: the gridboxes'
+// condensation inputs too, for a condensation in the sort's gather (the State is that of before the sort),
+// by workgroups of their own from number nblk on: both are serial chains of a few us (one after the other
+// in each thread: 10.3 us on 3750 gridboxes, 7.4 on 20; now 7.8 and 5.0).
 template <bool kThermo>
 __global__ void __launch_bounds__(kTabBlock) k_nsort_tot(NsortArgs a, GState st, double* gs) {
   __shared__ uint32_t ws[kTabBlock / kWave];
@@ -1630,7 +1635,6 @@ __global__ void __launch_bounds__(256) CLEO_OCCUPANCY(6) k_nsort_perm(NsortArgs 
   }
 }
 
-// record p of src to position q of dst
 // The drops that were out of the domain before (positions nsrc on) follow the newly out-of-domain
 // ones; the domain's drops fill the first nsrc positions of the sorted store either way, so they keep
 // their positions.
@@ -1910,8 +1914,9 @@ __global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* key, const u
 }
 
 // The sorted drops to dst, from the store, or from their rows (each drop then touches one line instead
-// of eight: 143 -> 32 us on 1M drops in random order, for 23 us more in the first count), and off[b] = first position with key >= b,
-// b = 0..ngbx (find_refs / find_domainrefs, findrefs.hpp), by bisection of the sorted keys.
+// of eight: 143 -> 32 us on 1M drops in random order, for 23 us more in the first count), and off[b] =
+// first position with key >= b, b = 0..ngbx (find_refs / find_domainrefs, findrefs.hpp), by bisection of
+// the sorted keys.
 __global__ void __launch_bounds__(256) k_rs_gather(SoA src, const DropRow* rows, SoA dst, const uint32_t* key,
                                                    const uint32_t* idx, uint64_t n, uint32_t ngbx, uint32_t* off) {
   const uint64_t first = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x,
@@ -2280,14 +2285,14 @@ void resort_nulls(cleo_ctx* c, uint32_t events) {
   hipLaunchKernelGGL(k_resort_back, dim3(kResortBlocks), dim3(kResortLanes), 0, c->stream, r);
 }
 
-// A pending collision order applied: the domain's drops are gathered into the other buffer in
-// their logical order (the out-of-domain drops are copied as they are) and that buffer becomes
-// current.  Nothing happens when the store is already in order.
 // the store as it is, with the identity as its pending order
 void pending_identity_order(cleo_ctx* c) {
   hipLaunchKernelGGL(k_iota_u32, dim3(stride_blocks(c->ntot)), dim3(256), 0, c->stream, c->order, c->ntot);
   c->order_live = true;
 }
+// A pending collision order applied: the domain's drops are gathered into the other buffer in
+// their logical order (the out-of-domain drops are copied as they are) and that buffer becomes
+// current.  Nothing happens when the store is already in order.
 void materialize_order(cleo_ctx* c) {
   if (!c->order_live) return;
   const int src = c->cur, dst = 1 - c->cur;
@@ -3184,7 +3189,7 @@ void launch_mass_moments(cleo_ctx* c, bool rain, uint64_t* mom0, float* mom1, fl
                        c->solute, c->ctl, mom0, mom1, mom2);
 }
 
-// the thermodynamic functions of k_cond_prep and k_condensation at n states, thread per state
+// the thermodynamic functions of the condensation (gbx_thermo) at n states, thread per state
 __global__ void k_thermo_eval(uint64_t n, const double* temp, const double* press, const double* qvap,
                               double* psat, double* s_ratio, double* ffactor) {
   for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n;
@@ -3465,7 +3470,7 @@ void motion_sort_condense(cleo_ctx* c, const MotionArgs& margs, const CondFlatAr
   const bool on = c->kev_on;
   c->kev_on = false;  // the main kernel of this sequence is the gather with the solves
   if (move_in_gather) {
-      const unsigned mb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
+    const unsigned mb = motion_blocks(c->ntot, c->tiles.motion_grid_waves);
     m.stat = stat_slots(c);
     launch_motion_drops<false>(c, m, mb);
   } else {

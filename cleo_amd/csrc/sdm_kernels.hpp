@@ -157,7 +157,8 @@ void launch_inj_long(cleo_ctx* c, const CollArgs& a);
 void scan_u32(cleo_ctx* c, const uint32_t* in, uint64_t len, uint32_t stride, uint32_t offset, uint32_t* out);
 size_t scan_tmp_words(uint64_t len);
 // after the collision events of a microphysics pass (which leave a pending order, unless a condensation
-// after them has applied it): the event counter moves on by `events`, and if nulls appeared the store is sorted again (SDMMethods, sdmmethods.hpp:213-230)
+// after them has applied it): the event counter moves on by `events`, and if nulls appeared the store is
+// sorted again (SDMMethods, sdmmethods.hpp:213-230)
 void resort_nulls(cleo_ctx* c, uint32_t events);
 // the neighbour sort of `src` (after motion) into `dst`; commit_dst >= 0: that buffer becomes current
 void neighbour_sort_to(cleo_ctx* c, const SoA& src, const SoA& dst, int commit_dst, const uint8_t* step = nullptr);
